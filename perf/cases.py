@@ -2,7 +2,8 @@
 
 A case is a dict of plain values.  `listed()` gives a fixed set over the whole range, `draw(rng)` one more case of the same ranges,
 `prepare(case, seed)` what a program holds before the call (tensors on the device, operators, packed weights, workspace), `run(state)` one
-pass, `work(case)` the bytes and operations a pass cannot do without, `tolerance(case)` how far a correct result may be off.
+pass, `work(case)` the bytes and operations a pass cannot do without, `tolerance(case)` how far a correct result may be off, `exact(case, seed)`
+the same results in 64 bits.
 
 Kinds of case:
   network     a ResNet forward pass: graphs.GraphRunner on one batch of images (image sizes and batches as they are served: one image where
@@ -364,3 +365,106 @@ def tolerance(case):
     if case.get("dtype") == "bfloat16":
         return {"rel": 1.2e-2, "max": 5e-2} if case["kind"] == "network" else {"rel": 1.5e-2, "max": 6e-2}
     return {"rel": 4e-6, "max": 4e-5}
+
+
+# ---- the same results in 64 bits, from torch alone ----
+def _conv64(x, w, s=1, p=0, d=1, g=1):
+    """convolution as one product of matrices per filter tap and group"""
+    b, c, h, wd = x.shape
+    cout, cin_g, k, _ = w.shape
+    oh, ow = _out(h, k, s, p, d), _out(wd, k, s, p, d)
+    x = torch.nn.functional.pad(x, (p, p, p, p))
+    if cin_g == 1 and cout == g:
+        y = torch.zeros((b, cout, oh, ow), dtype=x.dtype, device=x.device)
+        for i in range(k):
+            for j in range(k):
+                y += w[:, 0, i, j].view(1, -1, 1, 1) * x[:, :, i * d:i * d + (oh - 1) * s + 1:s, j * d:j * d + (ow - 1) * s + 1:s]
+        return y
+    y = torch.zeros((b, g, cout // g, oh * ow), dtype=x.dtype, device=x.device)
+    for i in range(k):
+        for j in range(k):
+            taps = x[:, :, i * d:i * d + (oh - 1) * s + 1:s, j * d:j * d + (ow - 1) * s + 1:s].reshape(b, g, cin_g, oh * ow)
+            y += torch.matmul(w[:, :, i, j].reshape(1, g, cout // g, cin_g), taps)
+    return y.view(b, cout, oh, ow)
+
+
+def _conv64_gradients(x, w, dy, s, p, d=1, g=1):
+    b, c, h, wd = x.shape
+    cout, cin_g, k, _ = w.shape
+    oh, ow = dy.shape[2:]
+    x = torch.nn.functional.pad(x, (p, p, p, p))
+    dx, dw = torch.zeros_like(x), torch.zeros_like(w)
+    dyg = dy.reshape(b, g, cout // g, oh * ow)
+    for i in range(k):
+        for j in range(k):
+            rows, cols = slice(i * d, i * d + (oh - 1) * s + 1, s), slice(j * d, j * d + (ow - 1) * s + 1, s)
+            if cin_g == 1 and cout == g:
+                dw[:, 0, i, j] = (x[:, :, rows, cols] * dy).sum((0, 2, 3))
+                dx[:, :, rows, cols] += w[:, 0, i, j].view(1, -1, 1, 1) * dy
+                continue
+            taps = x[:, :, rows, cols].reshape(b, g, cin_g, oh * ow)
+            dw[:, :, i, j] = torch.matmul(dyg, taps.transpose(2, 3).contiguous()).sum(0).reshape(cout, cin_g)
+            wt = w[:, :, i, j].reshape(1, g, cout // g, cin_g).transpose(2, 3).contiguous()
+            dx[:, :, rows, cols] += torch.matmul(wt, dyg).reshape(b, c, oh, ow)
+    return dx[:, :, p:p + h, p:p + wd].contiguous(), dw
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    st = prepare(case, seed)
+    f64 = lambda n: st[n].double()
+    chan = lambda t: t.double().view(1, -1, 1, 1)
+    if kind == "network":
+        runner = st["runner"]
+        ops = getattr(graphs, case["net"])()
+        parts = []
+        for x in st["x"].split(8):
+            t = {"data": x.double()}
+            for o in ops:
+                if o["op"] == "conv":
+                    w, bias = runner.p[o["dst"]]
+                    v = _conv64(t[o["src"]], w.double(), o["s"], o["p"]) + chan(bias)
+                    t[o["dst"]] = v.relu() if o["act"] == "relu" else v
+                elif o["op"] == "maxpool":
+                    t[o["dst"]] = torch.nn.functional.max_pool2d(t[o["src"]], o["k"], o["s"], o["p"])
+                elif o["op"] == "add":
+                    t[o["dst"]] = (t[o["src"][0]] + t[o["src"][1]]).relu()
+                elif o["op"] == "gap":
+                    t[o["dst"]] = t[o["src"]].mean((2, 3))
+                else:
+                    w, bias = runner.p[o["dst"]]
+                    t[o["dst"]] = t[o["src"]] @ w.double().t().contiguous() + bias.double()
+            parts.append(t["logits"])
+        return torch.cat(parts)
+    if kind == "train":
+        s, p, d, g = (case[n] for n in ("s", "p", "d", "g"))
+        dx, dw = _conv64_gradients(f64("x"), f64("w"), f64("dy"), s, p, d, g)
+        return {"y": _conv64(f64("x"), f64("w"), s, p, d, g) + chan(st["b"]), "dx": dx, "dw": dw, "db": f64("dy").sum((0, 2, 3))}
+    if kind == "block":
+        t = (_conv64(f64("x"), f64("w1")) + chan(st["b1"])).clamp(0, 6)
+        t = (_conv64(t, f64("wd"), case["s"], 1, 1, case["hidden"]) + chan(st["bd"])).clamp(0, 6)
+        y = _conv64(t, f64("w2")) + chan(st["b2"])
+        return y + f64("x") if st["skip"] else y
+    if kind == "train_block":
+        c, s = case["c"], case["s"]
+        t = _conv64(f64("x"), f64("wd"), s, 1, 1, c) + chan(st["bd"])
+        dt, dwp = _conv64_gradients(t, f64("wp"), f64("dy"), 1, 0)
+        dx, dwd = _conv64_gradients(f64("x"), f64("wd"), dt, s, 1, 1, c)
+        return {"y": _conv64(t, f64("wp")) + chan(st["bp"]), "dx": dx, "dwd": dwd, "dbd": dt.sum((0, 2, 3)), "dwp": dwp, "dbp": f64("dy").sum((0, 2, 3))}
+    if kind == "head":
+        t = f64("x")
+        for i, (_, w, bias, _) in enumerate(st["layers"]):
+            t = t @ w.double().t().contiguous() + bias.double()
+            t = t.relu() if i < 2 else t
+        return t, torch.softmax(t, 1), torch.nn.functional.cross_entropy(t, st["labels"].long()).reshape(1)
+    k, s, p = case["k"], case["s"], case["p"]
+    x, w = f64("x"), f64("w")
+    b, _, h, wd = x.shape
+    oh, ow = _tconv_out(h, case), _tconv_out(wd, case)
+    full = torch.zeros((b, case["cout"], max((h - 1) * s + k, oh + p), max((wd - 1) * s + k, ow + p)), dtype=x.dtype, device=x.device)
+    for i in range(k):
+        for j in range(k):
+            tap = torch.matmul(w[:, :, i, j].t().contiguous().unsqueeze(0), x.reshape(b, -1, h * wd)).view(b, -1, h, wd)
+            full[:, :, i:i + (h - 1) * s + 1:s, j:j + (wd - 1) * s + 1:s] += tap
+    t = (full[:, :, p:p + oh, p:p + ow] + chan(st["b"])).relu()
+    return t, torch.nn.functional.interpolate(t, scale_factor=2, mode="bilinear", align_corners=False)
