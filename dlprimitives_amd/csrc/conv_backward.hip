@@ -404,25 +404,59 @@ __global__ __launch_bounds__(256) void phase_interleave_kernel(float *__restrict
     }
 }
 
-// db[f] = beta * db[f] + sum over batch and plane of dy[b][f][:]; one workgroup per feature
-__global__ __launch_bounds__(256) void bias_backward_kernel(const float *__restrict__ dy, float *__restrict__ db, int batch, int features, int plane, float beta)
+// db[f] = beta * db[f] + sum over batch and plane of dy[b][f][:]; one workgroup per feature.
+// Bound by how much of dy one compute unit can have on its way: a feature's pixels of all images are walked as one run of V
+// elements per thread (16 bytes where planes and pointer allow it), four of them requested before the first is added, by 1024
+// threads.  A loop over images of 256 threads with one 4-byte load each took, on MI355X, 68.8 us for 64 x 128 x 28 x 28 and
+// 34.7 + 29.2 us for 32 x 32 and 32 x 192 x 28 x 28; with this one the training passes these belong to went from 425 to 363 us and
+// from 140 to 89 us, i.e. to about 6 us per call.
+// seg: images per run, so that a run has fewer than 2^31 elements.
+template <int V>
+__global__ __launch_bounds__(1024) void bias_backward_kernel(const float *__restrict__ dy, float *__restrict__ db, int batch, int features, int plane_v,
+                                                             int seg, uint32_t magic, uint32_t shift, float beta)
 {
-    __shared__ float partial[4];
+    typedef float vec __attribute__((ext_vector_type(V)));
+    __shared__ float partial[16];
     const int f = blockIdx.x;
-    float s = 0.0f;
-    for (int b = 0; b < batch; b++) {
-        const float *p = dy + ((size_t)b * features + f) * plane;
-        for (int i = threadIdx.x; i < plane; i += 256)
-            s += p[i];
+    const uint32_t T = blockDim.x;
+    const size_t skip = (size_t)(features - 1) * plane_v; // from the end of a feature's plane to its plane in the next image
+    vec s[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        s[q] = (vec)0.0f;
+    for (int b0 = 0; b0 < batch; b0 += seg) {
+        const vec *p = reinterpret_cast<const vec *>(dy) + ((size_t)b0 * features + f) * plane_v;
+        const uint32_t n = (uint32_t)min(seg, batch - b0) * (uint32_t)plane_v;
+        uint32_t i = threadIdx.x;
+        for (; i + 3 * T < n; i += 4 * T) {
+            vec v[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                v[q] = p[i + q * T + fast_div(i + q * T, magic, shift) * skip];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                s[q] += v[q];
+        }
+        for (; i < n; i += T)
+            s[0] += p[i + fast_div(i, magic, shift) * skip];
+        if (seg >= batch - b0) // b0 + seg may pass the largest int
+            break;
     }
+    const vec t = (s[0] + s[1]) + (s[2] + s[3]);
+    float sum = t[0];
+#pragma unroll
+    for (int e = 1; e < V; e++)
+        sum += t[e];
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1)
-        s += __shfl_down(s, off);
+        sum += __shfl_down(sum, off);
     if ((threadIdx.x & 63) == 0)
-        partial[threadIdx.x >> 6] = s;
+        partial[threadIdx.x >> 6] = sum;
     __syncthreads();
     if (threadIdx.x == 0) {
-        const float v = (partial[0] + partial[1]) + (partial[2] + partial[3]);
+        float v = partial[0];
+        for (uint32_t w = 1; w < T / 64; w++)
+            v += partial[w];
         db[f] = beta != 0.0f ? fmaf(db[f], beta, v) : v;
     }
 }
@@ -1025,7 +1059,18 @@ int dlp_bias_bwd_enqueue(int dtype, int batch, int features, int plane, const vo
     DLP_REQUIRE(batch >= 0 && features > 0 && plane > 0, "shape");
     DLP_REQUIRE(db != nullptr && (batch == 0 || dy != nullptr), "null tensor pointer");
     TimingScope ts("bias_backward", (hipStream_t)stream);
-    hipLaunchKernelGGL(bias_backward_kernel, dim3((unsigned)features), dim3(256), 0, (hipStream_t)stream, (const float *)dy, db, batch, features, plane, beta);
+    const int v = plane % 4 == 0 && ((uintptr_t)dy & 15) == 0 ? 4 : 1, plane_v = plane / v;
+    const int seg = std::max(1, 0x7FFFFFFF / plane_v);
+    uint32_t magic, shift;
+    make_magic((uint32_t)plane_v, magic, shift);
+    // one wavefront per four loads of a thread, from 4 wavefronts (512 features of 32 x 7 x 7: the launch is its own overhead) to 16
+    const unsigned threads = (long long)batch * plane_v <= 4096 ? 256 : 1024;
+    if (v == 4)
+        hipLaunchKernelGGL(bias_backward_kernel<4>, dim3((unsigned)features), dim3(threads), 0, (hipStream_t)stream, (const float *)dy, db, batch, features,
+                           plane_v, seg, magic, shift, beta);
+    else
+        hipLaunchKernelGGL(bias_backward_kernel<1>, dim3((unsigned)features), dim3(threads), 0, (hipStream_t)stream, (const float *)dy, db, batch, features,
+                           plane_v, seg, magic, shift, beta);
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
 }

@@ -242,3 +242,22 @@ def test_gpu_bias_backward(oracle_mod):
         db = _dev(old)
         dlp.bias_backward(_dev(dy), db, 2.0)
         np.testing.assert_allclose(db.cpu().numpy(), want + 2 * old, rtol=1e-4, atol=1e-4 * np.abs(want).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,features,h,w", [(1, 1, 1, 1), (0, 3, 4, 4), (3, 5, 1, 1), (7, 3, 7, 7), (4, 2, 64, 64), (5, 2, 64, 64), (17, 3, 31, 33), (9, 2, 113, 51)])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_gpu_bias_backward_walk(batch, features, h, w, shifted):
+    """planes of whole 16-byte pieces and others, 4096 elements per feature (the last with 256 threads) and above, an unaligned dy"""
+    import torch
+
+    import dlprimitives_amd as dlp
+
+    gen = torch.Generator().manual_seed(batch * 131 + h)
+    n = batch * features * h * w
+    flat = torch.randint(-8, 9, (n + 1,), generator=gen).float().cuda()  # sums of small whole numbers are exact in any order
+    dy = flat[1:] if shifted else flat[:n]
+    dy = dy.view(batch, features, h, w)
+    db = torch.full((features,), 3.0, device="cuda:0")
+    dlp.bias_backward(dy, db, 2.0)
+    assert torch.equal(db, dy.sum((0, 2, 3)) + 6.0)
