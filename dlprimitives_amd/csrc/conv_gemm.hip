@@ -481,18 +481,19 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
     // ([r][thread], write-through); the workgroup that arrives last at the tile's counter adds up all
     // slices in slice order (deterministic), whoever it is, and goes on to the epilogue.  Nobody waits. ----
     if (splitk > 1 && a.sk_cnt != nullptr) {
-        static_assert(TM == 1 && TN == 1, "one MFMA block per wavefront");
         constexpr int kThrough = 17; // sc0 | sc1: past the caches in both directions
         constexpr uint32_t image_bytes = BM * BN * 4;
         const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(a.sk_part, 0, a.sk_part_bytes, 0x00020000);
         const int tile = (g * a.ntiles + n0 / BN) * a.mtiles + m0 / BM;
         const uint32_t base = image0 * image_bytes;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const float v = acc[0][0][r];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), pr, (uint32_t)tid * 4u,
-                                                  base + (uint32_t)slice * image_bytes + (uint32_t)(r * kThreads * 4), kThrough);
-        }
+        for (int q = 0; q < TM * TN; q++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float v = acc[q / TN][q % TN][r];
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), pr, (uint32_t)tid * 4u,
+                                                      base + (uint32_t)slice * image_bytes + (uint32_t)((q * 16 + r) * kThreads * 4), kThrough);
+            }
         __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this thread's part has been written through
         __syncthreads();
         int *arrived_s = reinterpret_cast<int *>(lds);
@@ -506,23 +507,28 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
         if (tid == 0)
             a.sk_cnt[tile] = 0; // left at zero for the next launch (counters that the operator owns are cleared only once)
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-            acc[0][0][r] = 0.0f;
-        for (int s0 = 0; s0 < splitk; s0 += 4) { // four slices (64 loads) in flight at a time
-            float p[4][16];
+        for (int q = 0; q < TM * TN; q++) {
+            f32x16 sum;
 #pragma unroll
-            for (int ds = 0; ds < 4; ds++)
+            for (int r = 0; r < 16; r++)
+                sum[r] = 0.0f;
+            for (int s0 = 0; s0 < splitk; s0 += 4) { // four slices (64 loads) in flight at a time
+                float p[4][16];
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    p[ds][r] = (s0 + ds < splitk) ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                          pr, (uint32_t)tid * 4u,
-                                                          base + (uint32_t)(s0 + ds) * image_bytes + (uint32_t)(r * kThreads * 4), kThrough))
-                                                    : 0.0f;
+                for (int ds = 0; ds < 4; ds++)
 #pragma unroll
-            for (int ds = 0; ds < 4; ds++)
+                    for (int r = 0; r < 16; r++)
+                        p[ds][r] = (s0 + ds < splitk) ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                              pr, (uint32_t)tid * 4u,
+                                                              base + (uint32_t)(s0 + ds) * image_bytes + (uint32_t)((q * 16 + r) * kThreads * 4), kThrough))
+                                                        : 0.0f;
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    acc[0][0][r] += p[ds][r];
+                for (int ds = 0; ds < 4; ds++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        sum[r] += p[ds][r];
+            }
+            acc[q / TN][q % TN] = sum;
         }
     } else if (splitk > 1) { // raw partial sums in output order, reduced by splitk_reduce_kernel
         if ((a.M & 7) == 0 && a.part_bytes != 0) { // buffer stores with scalar row offsets
@@ -571,40 +577,59 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
     if ((a.factor == 0.0f || (pre && sizeof(T) == 4)) && (a.M & 7) == 0 && a.y_bytes != 0) {
         const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, a.y_bytes, 0x00020000);
         const bool clamp = a.act != DLP_ACT_IDENTITY;
+        auto store_all = [&](auto pre_c) {
+            constexpr bool PRE = decltype(pre_c)::value;
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn * WTN + j * 32 + l32;
-            const int b = (int)fast_div((uint32_t)n, a.ohw_magic, a.ohw_shift);
-            const int pix = n - b * a.OHW;
-            const uint32_t voff =
-                n < a.N ? (uint32_t)(((b * a.Cout + g * a.M + m0 + wm * WTM + 4 * h) * a.OHW + pix) * (int)sizeof(T)) : kOutOfRange;
+            for (int j = 0; j < TN; j++) {
+                const int n = n0 + wn * WTN + j * 32 + l32;
+                const int b = (int)fast_div((uint32_t)n, a.ohw_magic, a.ohw_shift);
+                const int pix = n - b * a.OHW;
+                const uint32_t voff =
+                    n < a.N ? (uint32_t)(((b * a.Cout + g * a.M + m0 + wm * WTM + 4 * h) * a.OHW + pix) * (int)sizeof(T)) : kOutOfRange;
+                // the old values of all the column's rows are requested before the first is used: one by one, each waited for its own trip
+                // to memory (64->256 1x1 at 56x56 with its residual sum, batch 16, in tiles of 128x128: 56 -> 33 us)
+                float old[TM][16];
+                if (PRE) {
 #pragma unroll
-            for (int i = 0; i < TM; i++) {
+                    for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    const int mrow = wm * WTM + i * 32 + 8 * rq; // + 4*h + (r & 3); this part is uniform
-                    if (m0 + mrow >= a.M)
-                        continue;
-                    const f32x4 bv = *(const f32x4 *)&bias_s[mrow + 4 * h];
+                        for (int r = 0; r < 16; r++)
+                            if (m0 + wm * WTM + i * 32 + 8 * (r >> 2) < a.M)
+                                old[i][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                                          yr, voff, (uint32_t)((i * 32 + 8 * (r >> 2) + (r & 3)) * a.OHW * (int)sizeof(T)), 0));
+                }
 #pragma unroll
-                    for (int rr = 0; rr < 4; rr++) {
-                        float v = acc[i][j][4 * rq + rr] + bv[rr];
-                        const uint32_t soff = (uint32_t)((i * 32 + 8 * rq + rr) * a.OHW * (int)sizeof(T));
-                        if (pre)
-                            v = fmaf(__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(yr, voff, soff, 0)), a.factor, v);
-                        if (ACT == ACT_CLAMP) {
-                            if (clamp) // identity must keep NaNs: no min/max
-                                v = clamp_med3(v, a.clamp_lo, a.clamp_hi);
-                        } else
-                            v = apply_act(v, a.act);
-                        if (sizeof(T) == 4)
-                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr, voff, soff, 0);
-                        else
-                            __builtin_amdgcn_raw_buffer_store_b16((short)to_bf16(v).bits, yr, voff, soff, 0);
+                for (int i = 0; i < TM; i++) {
+#pragma unroll
+                    for (int rq = 0; rq < 4; rq++) {
+                        const int mrow = wm * WTM + i * 32 + 8 * rq; // + 4*h + (r & 3); this part is uniform
+                        if (m0 + mrow >= a.M)
+                            continue;
+                        const f32x4 bv = *(const f32x4 *)&bias_s[mrow + 4 * h];
+#pragma unroll
+                        for (int rr = 0; rr < 4; rr++) {
+                            float v = acc[i][j][4 * rq + rr] + bv[rr];
+                            const uint32_t soff = (uint32_t)((i * 32 + 8 * rq + rr) * a.OHW * (int)sizeof(T));
+                            if (PRE)
+                                v = fmaf(old[i][4 * rq + rr], a.factor, v);
+                            if (ACT == ACT_CLAMP) {
+                                if (clamp) // identity must keep NaNs: no min/max
+                                    v = clamp_med3(v, a.clamp_lo, a.clamp_hi);
+                            } else
+                                v = apply_act(v, a.act);
+                            if (sizeof(T) == 4)
+                                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr, voff, soff, 0);
+                            else
+                                __builtin_amdgcn_raw_buffer_store_b16((short)to_bf16(v).bits, yr, voff, soff, 0);
+                        }
                     }
                 }
             }
-        }
+        };
+        if (pre) // (two copies: the test alone, inside the loops, cost launches without a sum 1.5 %)
+            store_all(std::true_type{});
+        else
+            store_all(std::false_type{});
         return;
     }
     // accumulator register r of a 32x32 block holds row 8*(r/4) + 4*h + r%4, column l32
@@ -999,6 +1024,8 @@ __global__ __launch_bounds__(kThreads) void conv_patch_f32_kernel(GemmArgs a)
 // The sum over k is accumulated in fp32 exactly as in the fp32 kernel (products of bf16 values
 // are exact in fp32), only in a different order.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+#include "conv_gemm_split.hpp"
+
 // Register sets of tiles in flight (2 or 4).  Measured: 4 sets (two more K steps of load latency
 // hidden, 148 instead of 102 VGPRs) are not faster -- the kernel is bound by the vector-memory
 // access rate, not by latency -- so 2 sets and three workgroups per CU it is.
@@ -2409,11 +2436,64 @@ void set_tile_magics(GemmArgs &a, int groups)
     make_magic((uint32_t)std::max(a.tail_tiles, 1), a.tt_magic, a.tt_shift);
 }
 
+// How a launch of conv_split_f32_kernel is cut: `tiles` tiles of nkt K tiles in s slices each, but the tiles that would make up the last,
+// partial round of workgroups (one per CU and round: the workgroups of a CU share its matrix units) in s2 finer ones.  `cost`: K tiles the
+// busiest CU works through, and what the partial sums cost -- about a twentieth of a K tile per piece for its trip through
+// the workspace, and once the time the last piece to arrive takes to add the others up.
+struct SplitCut {
+    int s, tail, s2;
+    double cost;
+};
+SplitCut split_cut(long long tiles, int nkt, int cus)
+{
+    SplitCut best = {1, 0, 1, 0.0};
+    if (tiles > 64ll * cus)
+        return best;
+    // a CU with one workgroup works at little over half its rate, with two at nine tenths
+    auto rate = [&](long long wgs) { return wgs <= cus ? 0.6 : wgs <= 2ll * cus ? 0.9 : 1.0; };
+    best.cost = (double)((tiles + cus - 1) / cus) * nkt / rate(tiles);
+    for (int s = 1; s <= 16 && nkt / s >= 8; s++) {
+        const long long wgs = tiles * s, rounds = wgs / cus;
+        const int kt = (nkt + s - 1) / s;
+        const double piece = 0.05;
+        const double whole = (double)((wgs + cus - 1) / cus) * kt / rate(wgs) + 6.0 + piece * wgs;
+        if (s > 1 && whole < best.cost)
+            best = {s, 0, 1, whole};
+        const long long tail = tiles - rounds * cus / s;
+        if (rounds == 0 || tail == 0)
+            continue;
+        for (int s2 = s + 1; s2 <= 16 && nkt / s2 >= 4; s2++) {
+            const long long pieces = tail * s2;
+            const double cost = ((double)rounds * kt + (double)((pieces + cus - 1) / cus) * ((nkt + s2 - 1) / s2)) / rate(rounds * cus + pieces) + 6.0 +
+                                piece * (pieces + (s > 1 ? rounds * cus : 0));
+            if (cost < best.cost)
+                best = {s, (int)tail, s2, cost};
+        }
+    }
+    return best;
+}
+
 void plan_split(const GemmPlan &p, GemmArgs &a, int groups, bool have_ws, size_t ws_bytes)
 {
     a.mtiles = p.mtiles;
     a.ntiles = (a.N + p.BN - 1) / p.BN;
     const long long tiles = (long long)a.mtiles * a.ntiles * groups;
+    if (p.split) {
+        const SplitCut c = have_ws ? split_cut(tiles, a.nkt, device_cu_count()) : SplitCut{1, 0, 1, 0.0};
+        auto cut = [&](int s, int tail, int s2) { // every slice starts inside the K range
+            a.kt_per_slice = (a.nkt + s - 1) / s;
+            a.splitk = (a.nkt + a.kt_per_slice - 1) / a.kt_per_slice;
+            a.tail_tiles = tail;
+            a.tail_kt = tail ? (a.nkt + s2 - 1) / s2 : a.kt_per_slice;
+            a.tail_splitk = tail ? (a.nkt + a.tail_kt - 1) / a.tail_kt : 1;
+        };
+        cut(c.s, c.tail, c.s2);
+        if (split_total_bytes(p, a, groups) > ws_bytes || split_total_bytes(p, a, groups) >= kOutOfRange)
+            cut(1, 0, 1); // no (or too small a) workspace: run unsplit
+        a.main_wgs = (int)((tiles - a.tail_tiles) * a.splitk);
+        set_tile_magics(a, groups);
+        return;
+    }
     int s = choose_splitk(tiles, a.nkt, p.order);
     if (s > 1 && (!have_ws || ws_bytes < split_workspace_bytes(p, a, groups, s)))
         s = 1; // no (or too small a) workspace: run unsplit
@@ -2762,6 +2842,31 @@ int launch_patch(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t 
     return DLP_OK;
 }
 
+template <int BM, int BN, int WM, int WN>
+void launch_split_inst(TimingScope &ts, const GemmArgs &a, unsigned blocks, hipStream_t stream)
+{
+    if (a.wdirect)
+        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, true>), dim3(blocks), dim3(kThreads), 0, stream, a);
+    else
+        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, false>), dim3(blocks), dim3(kThreads), 0, stream, a);
+}
+
+int launch_split(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t stream)
+{
+    const long long blocks = (long long)a.main_wgs + (long long)a.tail_tiles * a.tail_splitk;
+    if ((long long)a.mtiles * a.ntiles * g.groups * a.splitk > 0x7fffffffLL)
+        return fail(DLP_ERR_NOT_IMPLEMENTED, "convolution too large for a single launch");
+    {
+        TimingScope ts("conv_gemm", stream);
+        if (p.tile == 4)
+            launch_split_inst<128, 128, 2, 2>(ts, a, (unsigned)blocks, stream);
+        else
+            launch_split_inst<64, 128, 1, 4>(ts, a, (unsigned)blocks, stream);
+    }
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
+}
+
 template <class T, int BM, int BN, int WM, int WN>
 int launch_tile(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, int act, hipStream_t stream)
 {
@@ -2786,7 +2891,8 @@ int launch_tile(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, int act, hipS
 struct TileShape {
     int id, BM, BN;
 };
-constexpr TileShape kTiles[] = {{0, 64, 64}, {1, 32, 128}, {2, 128, 128}, {3, 64, 256}}; // 2, 3: bf16 matrix-instruction path
+constexpr TileShape kTiles[] = {{0, 64, 64}, {1, 32, 128}, {2, 128, 128}, {3, 64, 256}, // 2, 3: bf16 matrix-instruction path
+                                {4, 128, 128}, {5, 64, 128}}; // conv_split_f32_kernel
 
 int tile_choice(int M) { return M > 32 ? 0 : 1; }
 
@@ -2805,6 +2911,8 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
 {
     GemmPlan p;
     p.wdirect = 0;
+    p.split = 0;
+    p.patch_layer = 0;
     p.stem = conv_stem_supported(g) ? 1 : 0;
     p.dense_pxl = 0;
     p.dense_sx = 1;
@@ -2882,6 +2990,27 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
         p.xt = tap_major && p.dense_pxl == 0 && p.patch_bf16 == 0 && g.Cin <= 65535 * 64 &&
                (size_t)g.H * g.W * g.Cin * sizeof(bf16_t) < kOutOfRange / 2;
     }
+    p.patch_layer = p.patch;
+    // fp32 as three bf16 parts (conv_split_f32_kernel), from the size on at which its larger tiles fill the chip.  Counted in tiles of
+    // 64 filters x 128 pixels at the batch of the settings (packed weights stay valid at every other one).  Measured, batch 64 unless
+    // said, filters packed, patch or gathering kernel / 64x128 / 128x128 tiles: 3x3 64->64 at 56x56 120 / 91 / - us, 128->128 at 28x28
+    // 114 / 93 / 85, 256->256 at 14x14 111 / 101 / 99, 512->512 at 7x7 112 / 95 / 92, stride 2 64->128 at 56x56 67 / 61 / 51, 1x1
+    // 256->64 at 56x56 62 / 55 / -, 64->256 at batch 128 201 / 186 / 166.  Below 350 tiles a launch needs K slices, which only long
+    // reductions pay for: 1x1 512->2048 at 7x7, batch 16 (224 tiles x 32 K tiles) 22 / 26 / 28, 5x5 32->64 at 28x28, batch 32
+    // (196 x 50) 31 / 34 / -, but 5x5 48->80 at 35x35, batch 9 (174 x 75) 40 / 32 / - and 3x3 256->256 at 14x14, batch 16 (100 x 144)
+    // 39 / 39 / 45.  128x128 tiles want twice as much work: 3x3 128->128 at batch 32 (392 x 72) 63 / 53 / 57, 256->256 at 14x14,
+    // batch 40 (248 x 144) 81 / 99 / 69.
+    if (g.dtype == DLP_FLOAT && p.order == GEMM_ORDER_TAP && !p.stem && !p.pointwise && p.M > 32) {
+        const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)g.B_hint * g.OH * g.OW + 127) / 128), work = tiles * p.nkt;
+        const int rest = p.M % 128;
+        const int tile = (rest == 0 || rest > 64) && (tiles >= 700 || work >= 30000) ? 4 : 5;
+        const int bm = tile == 4 ? 128 : 64;
+        if ((tiles >= 350 || work >= (p.patch ? 20000 : 12000)) && (size_t)g.groups * ((p.M + bm - 1) / bm) * p.nkt * bm * 96 < kOutOfRange) {
+            p.split = 1;
+            p.patch = 0;
+            p.tile = tile;
+        }
+    }
     p.BM = 64;
     p.BN = 64;
     for (const TileShape &ts : kTiles)
@@ -2893,6 +3022,8 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
     p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * BK * p.BM * sizeof(float);
     if (bf16_mfma_order(p.order))
         p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * BK2 * p.BM * sizeof(bf16_t);
+    if (p.split)
+        p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * p.BM * 96;
     p.wpack_bytes = (p.wpack_bytes + 255) / 256 * 256;
     return p;
 }
@@ -3028,7 +3159,13 @@ int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, 
         return fail(DLP_ERR_NOT_IMPLEMENTED, "weight tensor too large");
     TimingScope ts("pack_weights", stream);
     const int khw = g.KH * g.KW;
-    if ((p.order == GEMM_ORDER_TAP || p.order == GEMM_ORDER_TAP_BF16) && ((uintptr_t)w & 15) == 0) {
+    if (p.split) {
+        const int ncb = p.nkt / khw;
+        hipLaunchKernelGGL(pack_weights_split_kernel, dim3((unsigned)((long long)g.groups * p.mtiles * ncb * (p.BM / 16))), dim3(256),
+                           16 * (BK * khw + 1) * sizeof(float), stream, p, ncb, khw, ((uintptr_t)w & 15) == 0 ? 1 : 0, (const float *)w, (u32x4 *)wpacked);
+        if (zero != nullptr)
+            hipLaunchKernelGGL(clear_counters_kernel, dim3((unsigned)((nzero + 255) / 256)), dim3(256), 0, stream, zero, nzero);
+    } else if ((p.order == GEMM_ORDER_TAP || p.order == GEMM_ORDER_TAP_BF16) && ((uintptr_t)w & 15) == 0) {
         const int ncb = p.nkt / khw;
         const dim3 grid((unsigned)((long long)g.groups * p.mtiles * ncb * (p.BM / 16)));
         if (p.order == GEMM_ORDER_TAP_BF16)
@@ -3211,6 +3348,8 @@ int conv_gemm_launch(const ConvGeom &g, const GemmPlan &p, const KTabEntry *dev_
         const int pxl = ((uintptr_t)x & 3) == 0 ? p.dense_pxl : 0;
         return launch_bf16_mfma(g, p, pxl, a, stream, xt);
     }
+    if (p.split)
+        return launch_split(g, p, a, stream);
     return with_tile(p.tile, [&](auto bm, auto bn, auto wm, auto wn) {
         if (g.dtype == DLP_BFLOAT16)
             return launch_tile<bf16_t, decltype(bm)::value, decltype(bn)::value, decltype(wm)::value, decltype(wn)::value>(g, p, a, act, stream);

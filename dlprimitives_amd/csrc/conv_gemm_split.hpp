@@ -1,0 +1,401 @@
+// fp32 convolutions on the bf16 matrix instruction, without loss of precision.  Included by conv_gemm.hip.
+//
+// A float is the exact sum of three bf16 numbers (3 x 8 significant bits, each piece rounded to nearest, so that the next one takes what
+// is left over): a = a0 + a1 + a2 with |a1| <= 2^-8 |a0| and |a2| <= 2^-16 |a0|.  A product a * b is then the sum of nine products of
+// bf16 numbers, each exact in fp32; the three smallest (a1 b2, a2 b1, a2 b2: at most 2^-23 of a * b together, without bias, 2^-25 in the
+// root mean square) are left out, six remain.  v_mfma_f32_32x32x16_bf16 is sixteen times as fast per product as the fp32 instruction,
+// so six of them leave it 2.7 times ahead -- and it adds several k of a product to the accumulator at once, where the fp32 instruction
+// rounds after every k; with the five small products in an accumulator of their own the error against 64 bits is smaller than the fp32
+// instruction's (2-norm, K = 64 / 576 / 1152: 4.8e-8 / 1.1e-7 / 1.6e-7 against 1.0e-7 / 3.1e-7 / 4.0e-7).
+//
+// What does not split is computed on the fp32 instruction: an operand that is infinite, not a number, or so close to the largest float
+// that its first piece rounds to infinity leaves an infinity or a NaN in the sums, and a tile whose sums are not all finite is
+// computed again, whole, from the same operands as they were (the three pieces of a packed weight add up to it).  Pieces below the
+// smallest normal number may be lost: operands below 2^-100 carry fewer than 24 bits.
+//
+//  * K tile = one filter tap x 16 channels = one matrix step; the input is gathered as in conv_gemm_f32_kernel (one masked pixel per
+//    lane, a channel per load), split in registers by the thread that loaded it, and stored as three 16-byte pieces of eight channels;
+//    the weights are split once, by the packing kernel, into the image of the LDS tile ([piece][half of the channels][row][8]);
+//    1x1 convolutions whose weights are not packed ahead read and split the weight tensor in place.
+//  * LDS holds [piece][half][row][8 k]: an operand is one 16-byte read per lane, 32 lanes read 512 consecutive bytes.
+//  * A wavefront owns 64x64 of the output (64x32 with tiles of 64x128): at six matrix instructions per operand pair of 32x32x16 (192
+//    clocks) a 32x32 tile would want 128 bytes per clock and CU from LDS, all there is; 64x64 wants half of that.
+//
+// Reaches 200 TFLOP/s of products on long launches (1x1 1024->1024 at 28x28, batch 128: 1673 -> 1056 us; 3x3 256->256 at 14x14, batch 512:
+// 858 -> 591 us): 1.2e15 bf16 operations a second on operands of random bits, what the library's bf16 product reaches on the same card.
+// Loads two K tiles further ahead, or a second set of registers for them, made no difference.
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t round_pair(float lo, float hi)
+{
+    bf16x2 v; // one v_cvt_pk_bf16_f32
+    v[0] = (__bf16)lo;
+    v[1] = (__bf16)hi;
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// eight consecutive k of a row -> the 16-byte pieces of its three parts
+__device__ __forceinline__ void split8(const float *v, u32x4 (&o)[3])
+{
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        float lo = v[2 * q], hi = v[2 * q + 1];
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++) {
+            const uint32_t r = opaque(round_pair(lo, hi)); // (else the compiler rounds the lower element a second time to shift it)
+            o[pl][q] = r;
+            lo -= __builtin_bit_cast(float, r << 16);
+            hi -= __builtin_bit_cast(float, r & 0xFFFF0000u);
+        }
+    }
+}
+
+template <int BM, int BN, int WM, int WN, bool ADIR>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_split_f32_kernel(GemmArgs a)
+{
+    static_assert(WM * WN == 4 && BN == 128 && (BM == 64 || BM == 128), "tile shape");
+    constexpr int WTM = BM / WM, WTN = BN / WN;
+    constexpr int TM = WTM / 32, TN = WTN / 32;
+    constexpr int A_BYTES = BM * 96, B_BYTES = BN * 96, BUF = A_BYTES + B_BYTES;
+    constexpr int A_PIECES = BM * 6;
+    constexpr int A_LD = ADIR ? 2 : (A_PIECES + kThreads - 1) / kThreads;
+
+    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * BUF];
+    __shared__ float bias_early[BM];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31;
+    const int h = lane >> 5;
+    const int wm = wave / WN, wn = wave % WN;
+
+    // tile and K slice of this workgroup: as in conv_gemm_f32_kernel
+    int t, slice, splitk = a.splitk, kt_per_slice = a.kt_per_slice;
+    uint32_t image0;
+    {
+        const int tiles = a.mtiles * a.ntiles * a.groups, tiles_main = tiles - a.tail_tiles;
+        const int bid = blockIdx.x;
+        if (bid < a.main_wgs) {
+            const int nb = a.main_wgs;
+            const int q = nb >> 3, r = nb & 7;
+            const int xcd = bid & 7, slot = bid >> 3;
+            t = (xcd < r) ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
+            slice = (int)fast_div((uint32_t)t, a.tm_magic, a.tm_shift);
+            t -= slice * tiles_main;
+            image0 = (uint32_t)(t * splitk);
+        } else {
+            t = bid - a.main_wgs;
+            slice = (int)fast_div((uint32_t)t, a.tt_magic, a.tt_shift);
+            t -= slice * a.tail_tiles;
+            image0 = (uint32_t)((splitk > 1 ? tiles_main * splitk : 0) + t * a.tail_splitk);
+            t += tiles_main;
+            splitk = a.tail_splitk;
+            kt_per_slice = a.tail_kt;
+        }
+    }
+    const int tm = (int)fast_div((uint32_t)t, a.mt_magic, a.mt_shift);
+    const int mt = t - tm * a.mtiles;
+    const int g = (int)fast_div((uint32_t)tm, a.ntl_magic, a.ntl_shift);
+    const int nt = tm - g * a.ntiles;
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int kt_begin = slice * kt_per_slice;
+    const int kt_end = min(kt_begin + kt_per_slice, a.nkt);
+    if (tid < BM)
+        bias_early[tid] = (a.bias && m0 + tid < a.M) ? a.bias[g * a.M + m0 + tid] : 0.0f;
+
+    const __amdgpu_buffer_rsrc_t xr =
+        __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)a.x - a.x_shift), 0, a.x_bytes + a.x_shift, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)a.wp, 0, a.wp_bytes, 0x00020000);
+    ConstInt *ktab = (ConstInt *)a.ktab;
+
+    // ---- the input: one output pixel per thread, its window origin and the mask of its taps inside the image ----
+    const int p = tid % BN;
+    const int half = __builtin_amdgcn_readfirstlane(tid / BN); // of a K tile's channels
+    uint32_t vbase, my = 0;
+    {
+        const int n = n0 + p;
+        const int b = (int)fast_div((uint32_t)n, a.ohw_magic, a.ohw_shift);
+        const int pix = n - b * a.OHW;
+        const int oy = (int)fast_div((uint32_t)pix, a.ow_magic, a.ow_shift);
+        const int ox = pix - oy * a.OW;
+        vbase = (uint32_t)((((b * a.Cin + g * a.Cin_g) * a.H + oy * a.sh) * a.W + ox * a.sw) * 4);
+        if (n < a.N) {
+            uint32_t rx = 0;
+            for (int kx = 0; kx < a.KW; kx++) {
+                const int xx = ox * a.sw - a.pw + kx * a.dw;
+                rx |= (xx >= 0 && xx < a.W ? 1u : 0u) << kx;
+            }
+            for (int ky = 0; ky < a.KH; ky++) {
+                const int yy = oy * a.sh - a.ph + ky * a.dh;
+                if (yy >= 0 && yy < a.H)
+                    my |= rx << (ky * a.KW);
+            }
+        }
+    }
+    // ---- the weights: 16-byte pieces of the packed tile in order, or (ADIR) eight channels of a row of the weight tensor ----
+    const uint32_t a_tile_bytes = ADIR ? (uint32_t)(BK * 4) : (uint32_t)A_BYTES;
+    const uint32_t a_row_base = ADIR ? 0u : (uint32_t)((g * a.mtiles + mt) * a.nkt) * a_tile_bytes;
+    const int arow = tid % BM, ahalf = tid / BM;
+    uint32_t a_voff[A_LD];
+#pragma unroll
+    for (int j = 0; j < A_LD; j++) {
+        if (ADIR)
+            a_voff[j] = (ahalf < 2 && m0 + arow < a.M) ? (uint32_t)(((g * a.M + m0 + arow) * a.K + 8 * ahalf + 4 * j) * 4) : kOutOfRange;
+        else
+            a_voff[j] = tid + j * kThreads < A_PIECES ? (uint32_t)((tid + j * kThreads) * 16) : kOutOfRange;
+    }
+
+    float rb[8];
+    u32x4 ra[A_LD];
+    auto load_b = [&](int kt) {
+        ConstInt *e = ktab + min(kt, a.nkt + 1) * 4; // (tiles past the end of K are never multiplied)
+        const uint32_t xoff = (uint32_t)e[0], tap = (uint32_t)e[1];
+        const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)my, tap, 1u);
+        const uint32_t v = opaque((vbase & m) | (kOutOfRange & ~m));
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            rb[i] = buf_load<float>(xr, v, xoff + (uint32_t)(half * 8 + i) * a.hw4);
+    };
+    auto load_a = [&](int kt) {
+        const uint32_t soff = a_row_base + (uint32_t)min(kt, a.nkt - 1) * a_tile_bytes;
+#pragma unroll
+        for (int j = 0; j < A_LD; j++)
+            ra[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, a_voff[j], soff, 0);
+    };
+    auto store_tile = [&](auto buf_c) {
+        unsigned char *const buf = smem + decltype(buf_c)::value * BUF;
+        u32x4 o[3];
+        if (ADIR) {
+            const f32x4 lo = __builtin_bit_cast(f32x4, ra[0]), hi = __builtin_bit_cast(f32x4, ra[1]);
+            const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            if (BM == 128 || tid < 2 * BM) {
+                split8(v, o);
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++)
+                    *(u32x4 *)(buf + ((pl * 2 + ahalf) * BM + arow) * 16) = o[pl];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < A_LD; j++)
+                if (A_PIECES % kThreads == 0 || tid + j * kThreads < A_PIECES)
+                    *(u32x4 *)(buf + (tid + j * kThreads) * 16) = ra[j];
+        }
+        split8(rb, o);
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++)
+            *(u32x4 *)(buf + A_BYTES + ((pl * 2 + half) * BN + p) * 16) = o[pl];
+    };
+
+    // the five small products are summed on their own: in one accumulator with the large one, every step would round the sum six
+    // times as often, at its full size
+    f32x16 acc[TM][TN], small[TM][TN];
+    auto clear = [&](f32x16 (&v)[TM][TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    v[i][j][r] = 0.0f;
+    };
+    clear(acc);
+    clear(small);
+
+    bf16x8 fa[3][TM], fb[3][TN]; // operands of the K tile at hand, by piece
+    auto read_piece = [&](auto buf_c, int pl) {
+        const unsigned char *const buf = smem + decltype(buf_c)::value * BUF;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+            fa[pl][i] = *(const bf16x8 *)(buf + ((pl * 2 + h) * BM + wm * WTM + i * 32 + l32) * 16);
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            fb[pl][j] = *(const bf16x8 *)(buf + A_BYTES + ((pl * 2 + h) * BN + wn * WTN + j * 32 + l32) * 16);
+    };
+    auto multiply = [&](f32x16 (&c)[TM][TN], int pa, int pb) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa][i], fb[pb][j], c[i][j], 0, 0, 0);
+    };
+    // One K tile, its operands in registers.  One barrier, in the middle: before it the next tile is split and goes from its registers to
+    // LDS[P ^ 1] (and the one after is requested); behind it the next tile's operands replace this one's, piece by piece, as soon as the
+    // last product that wants a piece has been issued, so that a wavefront alone on its SIMD does not wait for LDS either.
+    auto k_step = [&](auto par, int kt) {
+        using Other = std::integral_constant<int, decltype(par)::value ^ 1>;
+        multiply(small, 1, 1);
+        multiply(small, 1, 0);
+        store_tile(Other{});
+        load_b(kt + 2);
+        load_a(kt + 2);
+        __syncthreads();
+        multiply(small, 0, 1);
+        __builtin_amdgcn_sched_barrier(0); // keep this order: the scheduler would sink the operand reads to their uses
+        read_piece(Other{}, 1);
+        multiply(small, 2, 0);
+        multiply(small, 0, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        read_piece(Other{}, 2);
+        multiply(acc, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        read_piece(Other{}, 0);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    load_b(kt_begin);
+    load_a(kt_begin);
+    store_tile(I0{});
+    load_b(kt_begin + 1);
+    load_a(kt_begin + 1);
+    __syncthreads();
+    read_piece(I0{}, 1);
+    read_piece(I0{}, 2);
+    read_piece(I0{}, 0);
+    int kt = kt_begin;
+    for (; kt + 1 < kt_end; kt += 2) {
+        k_step(I0{}, kt);
+        k_step(I1{}, kt + 1);
+    }
+    if (kt < kt_end)
+        k_step(I0{}, kt);
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            acc[i][j] += small[i][j];
+
+    // sums that are not finite: the tile again on the fp32 instruction
+    float finite = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                finite = fmaf(acc[i][j][r], 0.0f, finite);
+    if (__syncthreads_or(finite != 0.0f)) { // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+        clear(acc);
+        float *const Af = reinterpret_cast<float *>(smem), *const Bf = Af + BK * BM; // [k][row], [k][pixel]
+        for (kt = kt_begin; kt < kt_end; kt++) {
+            load_b(kt);
+            if (tid < 2 * BM) {
+                const uint32_t soff = a_row_base + (uint32_t)kt * a_tile_bytes;
+                float v[8];
+                if (ADIR) {
+                    load_a(kt);
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        v[e] = __builtin_bit_cast(f32x4, ra[e / 4])[e % 4];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        v[e] = 0.0f;
+#pragma unroll
+                    for (int pl = 0; pl < 3; pl++) {
+                        const u32x4 o = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)(((pl * 2 + ahalf) * BM + arow) * 16), soff, 0);
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            v[e] += __builtin_bit_cast(float, (e & 1) ? o[e / 2] & 0xFFFF0000u : o[e / 2] << 16);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    Af[(ahalf * 8 + e) * BM + arow] = v[e];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                Bf[(half * 8 + i) * BN + p] = rb[i];
+            __syncthreads();
+#pragma unroll
+            for (int kk = 0; kk < BK / 2; kk++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(Af[(2 * kk + h) * BM + wm * WTM + i * 32 + l32],
+                                                                         Bf[(2 * kk + h) * BN + wn * WTN + j * 32 + l32], acc[i][j], 0, 0, 0);
+            __syncthreads();
+        }
+    }
+    gemm_tile_output<float, BM, BN, WM, WN, ACT_CLAMP>(a, acc, reinterpret_cast<float *>(smem), m0, n0, g, slice, splitk, image0, wm, wn, h, l32, tid,
+                                                       bias_early);
+}
+
+// Weights -> [group][m tile][K tile][piece][half][row][8 channels of one tap], zero padded.  One workgroup moves 16 filters x 16 channels
+// through LDS (read in runs of whole filter rows, 16 bytes per lane where the tensor is aligned); a thread then splits eight channels
+// of a filter at a time.  A weight whose first piece would round to infinity is cut instead, so that the pieces always add up to it.
+__global__ __launch_bounds__(256) void pack_weights_split_kernel(GemmPlan p, int ncb, int khw, int aligned, const float *__restrict__ w,
+                                                                 u32x4 *__restrict__ out)
+{
+    extern __shared__ __align__(16) unsigned char split_smem[];
+    float *lds = reinterpret_cast<float *>(split_smem);
+    const int run = BK * khw, ld = run + 1;
+    const int mchunks = p.BM / 16;
+    int bid = (int)blockIdx.x;
+    const int mc = bid % mchunks;
+    bid /= mchunks;
+    const int cb = bid % ncb;
+    bid /= ncb;
+    const int mt = bid % p.mtiles;
+    const int g = bid / p.mtiles;
+    const int m_base = mt * p.BM + mc * 16;
+    const float *src = w + (size_t)g * p.M * p.K + (size_t)cb * run;
+    const int wv = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    if (aligned) {
+        for (int j = lane * 4; j < run; j += 256) {
+            f32x4 v[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int m = m_base + wv + 4 * q;
+                v[q] = (f32x4)0.0f;
+                if (m < p.M)
+                    v[q] = *reinterpret_cast<const f32x4 *>(src + (size_t)m * p.K + j);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    lds[(wv + 4 * q) * ld + j + e] = v[q][e];
+        }
+    } else {
+        for (int j = lane; j < run; j += 64)
+            for (int q = 0; q < 4; q++) {
+                const int m = m_base + wv + 4 * q;
+                lds[(wv + 4 * q) * ld + j] = m < p.M ? src[(size_t)m * p.K + j] : 0.0f;
+            }
+    }
+    __syncthreads();
+    u32x4 *const tile0 = out + ((size_t)(g * p.mtiles + mt) * p.nkt + (size_t)cb * khw) * (6 * p.BM) + mc * 16;
+    for (int idx = (int)threadIdx.x; idx < 32 * khw; idx += 256) {
+        const int r = idx % 16, half = (idx / 16) % 2, tap = idx / 32;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            v[e] = lds[r * ld + (half * 8 + e) * khw + tap];
+        u32x4 o[3];
+        split8(v, o);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int sh = (e & 1) * 16;
+            if (((o[0][e / 2] >> sh) & 0x7F80u) != 0x7F80u)
+                continue;
+            // infinite, not a number, or rounded to infinity
+            const uint32_t bits = __builtin_bit_cast(uint32_t, v[e]);
+            float part[3] = {v[e], 0.0f, 0.0f};
+            if ((bits & 0x7F800000u) != 0x7F800000u) {
+                part[0] = __builtin_bit_cast(float, bits & 0xFFFF0000u);
+                part[1] = to_float(to_bf16(v[e] - part[0]));
+                part[2] = v[e] - part[0] - part[1];
+            }
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++)
+                o[pl][e / 2] = (o[pl][e / 2] & ~(0xFFFFu << sh)) | ((uint32_t)to_bf16(part[pl]).bits << sh);
+        }
+        u32x4 *const dst = tile0 + (size_t)tap * (6 * p.BM) + half * p.BM + r;
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++)
+            dst[(size_t)pl * 2 * p.BM] = o[pl];
+    }
+}

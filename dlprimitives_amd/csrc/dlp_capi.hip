@@ -206,6 +206,7 @@ static int make_geom(const dlp_conv2d_settings &c, const int x_shape[4], ConvGeo
     if (rc != DLP_OK)
         return rc;
     g.B = x_shape[0];
+    g.B_hint = c.shape[0];
     g.Cin = c.channels_in;
     g.H = x_shape[2];
     g.W = x_shape[3];
@@ -534,7 +535,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     // 256->256 at 14x14 123 / 97, 512->512 at 7x7 124 / 105; at batch 16: 49 / 40, 45 / 39, 47 / 46 (200 workgroups), 48 / 77 (128).
     const int cin_g = cfg->channels_in / cfg->groups;
     bool gemm_faster = false;
-    if (gplan.patch && win) {
+    if (gplan.patch_layer && win) {
         const WinoPlan wp = winograd_plan(g);
         const long long wgs = winograd_workgroups(g, wp, winograd_blocks_per_workgroup(g, wp));
         gemm_faster = cin_g < 64 || (cin_g < 128 && cfg->channels_out % 64 != 0) || wgs * 2 < 3ll * dlp_cu_count();
@@ -651,7 +652,7 @@ static void layout_of(const GemmPlan &p, int (&sig)[6])
     sig[1] = p.BM;
     sig[2] = p.nkt;
     sig[3] = p.mtiles;
-    sig[4] = p.patch;
+    sig[4] = p.patch + 2 * p.split;
     sig[5] = p.wdirect;
 }
 

@@ -51,6 +51,7 @@ int dlp_cu_count();
 // Geometry of one forward convolution call (whole tensor, all groups).
 struct ConvGeom {
     int B, Cin, H, W;
+    int B_hint = 0; // batch of the shape an operator was created with: chooses between kernels whose packed weights differ (B may change from call to call)
     int Cout, OH, OW;
     int KH, KW;
     int sh, sw, ph, pw, dh, dw;
@@ -177,6 +178,8 @@ struct GemmPlan {
     int M, K, nkt;      // per group: rows, reduction length, K tiles of 16
     int mtiles;         // ceil(M / BM)
     int patch;          // 1: stride-1 "same" convolution run by the LDS-patch kernel (tap-major packed weights)
+    int patch_layer;    // 1: the shape is one that the LDS-patch kernel serves, whichever kernel runs it
+    int split;          // 1: conv_split_f32_kernel (fp32 as three bf16 parts; tap-major packed weights of its own)
     int stem;           // 1: 3-channel 7x7 stride-2 convolution run by conv_stem_f32_kernel (reads the weight tensor in place, nothing is packed)
     int wdirect;        // bf16 matrix-instruction path, 1x1: the kernel reads the weight tensor in place, nothing is packed
     int dense_pxl;      // bf16 matrix-instruction path, 1x1 stride 1 pad 0: input pixels per load of the dense loader (8, 4; 0 = gather)

@@ -1,0 +1,117 @@
+"""fp32 convolutions on the bf16 matrix instruction (conv_split_f32_kernel: three bf16 parts per operand) at the sizes where its tiles,
+K slices and masks can go wrong, against torch in 64 bits."""
+import pytest
+import torch
+
+import dlprimitives_amd as dlp
+
+
+def _geometry(c):
+    cin, cout, k, s, p, d, g, b, h, w = c
+    oh, ow = ((n + 2 * p - d * (k - 1) - 1) // s + 1 for n in (h, w))
+    return (b, cin, h, w), (cout, cin // g, k, k), (b, cout, oh, ow)
+
+
+def _run(c, x, w, bias, packed, act="identity", factor=0.0, y0=None, shift=0, hint=None):
+    cin, cout, k, s, p, d, g, b, h, wd = c
+    xs, ws_, ys = _geometry(c)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, ((hint or b),) + xs[1:]), bias is not None, act, "gemm")
+    wbuf = torch.empty(w.numel() + shift, device="cuda:0")  # shift: a weight tensor off its 16-byte boundary
+    wbuf[shift:].copy_(w.reshape(-1))
+    wdev = wbuf[shift:].view(ws_)
+    y = torch.full(ys, float("nan"), device="cuda:0") if y0 is None else y0.float().cuda()
+    ws = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    bd = None if bias is None else bias.float().cuda()
+    if packed:
+        buf = torch.empty(max(op.packed_size(), 1), dtype=torch.uint8, device="cuda:0")
+        op.pack(wdev, buf)
+        op.enqueue_packed(x.float().cuda(), wdev, buf, bd, y, ws, factor)
+    else:
+        op.enqueue(x.float().cuda(), wdev, bd, y, ws, factor)
+    torch.cuda.synchronize()
+    return y.cpu().double()
+
+
+def _conv64(c, x, w, bias):
+    cin, cout, k, s, p, d, g, b, h, wd = c
+    return torch.nn.functional.conv2d(x.double(), w.double(), None if bias is None else bias.double(), s, p, d, g)
+
+
+# every one large enough for these kernels: 350 tiles of 64 filters x 128 pixels, or 20000 K tiles in all
+# (cin, cout, k, stride, pad, dilate, groups, batch, h, w)
+CASES = [
+    (16, 64, 1, 1, 0, 1, 1, 32, 38, 38),     # one K tile, 64x128 tiles
+    (16, 33, 1, 1, 0, 1, 1, 47, 31, 33),     # rows and pixels off the tile
+    (32, 80, 1, 2, 0, 1, 1, 90, 31, 33),     # two tiles of 64 rows, the second mostly empty; strided
+    (48, 128, 1, 1, 0, 1, 1, 32, 38, 38),    # 128x128 tiles, three K tiles
+    (16, 200, 3, 1, 1, 1, 1, 20, 31, 30),    # rows off 128, taps outside the image
+    (16, 97, 3, 2, 1, 1, 1, 64, 39, 41),
+    (64, 64, 3, 1, 1, 1, 1, 16, 53, 53),     # a last round of few tiles, cut into K slices
+    (192, 96, 3, 1, 1, 1, 1, 5, 61, 43),     # K slices throughout
+    (640, 128, 3, 1, 1, 1, 1, 5, 27, 27),
+    (32, 48, 5, 1, 4, 2, 1, 40, 31, 33),     # dilation
+    (64, 320, 3, 1, 1, 1, 4, 9, 33, 31),     # groups
+    (16, 40, 5, 3, 0, 1, 1, 81, 75, 75),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", CASES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("packed", [False, True])
+def test_gpu_split_parity(c, packed):
+    gen = torch.Generator().manual_seed(sum(c))
+    xs, ws, ys = _geometry(c)
+    x, w, bias = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen), torch.randn(c[1], generator=gen)
+    want = _conv64(c, x, w, bias)
+    got = _run(c, x, w, bias, packed, shift=0 if packed else 1)
+    # a product is off by 2^-23 at most; the sums, none above sum |x||w|, round by 2^-24 of themselves once per four k and a few times behind
+    scale = _conv64(c, x.abs(), w.abs(), bias.abs())
+    bound = (w[0].numel() / 4 + 8) * 2.0 ** -24
+    assert ((got - want).abs() <= scale * bound).all()
+    # roundings of either sign add up as their squares: sqrt(K / 4) of them, each a third of 2^-24 or so of a sum that has grown to sqrt(K)
+    # products, stay below 2^-22 of the result up to K = 6000; a piece too few would show as 2^-17, a lost small product as 2^-17 to 2^-9
+    assert (got - want).norm() <= want.norm() * 2.0 ** -22
+    old = torch.randn(ys, generator=gen)
+    got = _run(c, x, w, None, packed, "relu", 0.5, old)
+    want = _conv64(c, x, w, None).relu() + 0.5 * old.double()
+    assert ((got - want).abs() <= (scale + old.abs()) * bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("c", [(32, 64, 1, 1, 0, 1, 1, 32, 38, 38), (48, 128, 1, 1, 0, 1, 1, 32, 38, 38), (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)],
+                         ids=["64x128", "128x128", "slices"])
+def test_gpu_split_not_finite(c, packed):
+    """infinities, NaN and values next to the largest float come out as the definition has them"""
+    gen = torch.Generator().manual_seed(5)
+    xs, ws, ys = _geometry(c)
+    x, w = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+    x[0, 3, 4, 5], x[0, 7, 20, 9], x[1, 1, 30, 30], x[2, 2, 11, 3] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w[:, 2] *= 1e-3  # the products with 3.4e38 stay finite
+    want = _conv64(c, x, w, None)
+    got = _run(c, x, w, None, packed)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(want))
+    scale = _conv64(c, torch.nan_to_num(x, 0.0, 0.0, 0.0).abs(), w.abs(), None)
+    ok = torch.isfinite(want)
+    assert ((got - want).abs()[ok] <= scale[ok] * 2.0 ** -18).all()  # an fp32 sum of K terms where the tile is computed again
+    w[3, 1], w[5, 2], w[9, 0] = float("inf"), float("nan"), 3.4e38
+    x = torch.rand(xs, generator=gen) * 1e-3 + 1e-3
+    want = _conv64(c, x, w, None)
+    got = _run(c, x, w, None, packed)
+    inside = (slice(None), slice(None), slice(1, -1), slice(1, -1))  # (infinity times the padding's zeros is left to either)
+    for f in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(f(got[inside]), f(want[inside]))
+
+
+@pytest.mark.gpu
+def test_gpu_split_other_batches():
+    """weights packed at the batch of the settings stay valid at others; a workspace of a smaller batch runs unsplit"""
+    c = (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)
+    gen = torch.Generator().manual_seed(6)
+    for batch in (1, 4, 9):
+        cb = c[:7] + (batch,) + c[8:]
+        xs, ws, _ = _geometry(cb)
+        x, w = torch.randint(-4, 5, xs, generator=gen).float(), torch.randint(-4, 5, ws, generator=gen).float()
+        for packed in (False, True):
+            assert torch.equal(_run(cb, x, w, None, packed, hint=5), _conv64(cb, x, w, None))  # whole numbers are exact
