@@ -3190,6 +3190,32 @@ int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, 
     return DLP_OK;
 }
 
+int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream)
+{
+    PhasePackArgs a;
+    a.n = n;
+    a.cout_g = cout_g;
+    a.cin_g = cin_g;
+    a.KH = KH;
+    a.KW = KW;
+    unsigned long long blocks = 0;
+    for (int i = 0; i < n; i++) {
+        const GemmPlan &p = ph[i].plan;
+        const unsigned long long units = (unsigned long long)groups * p.mtiles * p.nkt * (p.split ? 2 : BK) * p.BM;
+        if (units >= kOutOfRange)
+            return fail(DLP_ERR_NOT_IMPLEMENTED, "weight tensor too large");
+        a.ph[i] = {ph[i].packed, ph[i].nh, ph[i].nw, ph[i].rh0, ph[i].rhstep, ph[i].rw0, ph[i].rwstep, p.BM, p.nkt, p.mtiles, p.split, (uint32_t)units,
+                   (uint32_t)blocks};
+        blocks += (units + 255) / 256;
+    }
+    if (n == 0)
+        return DLP_OK;
+    TimingScope ts("pack_weights", stream);
+    hipLaunchKernelGGL(phase_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, w, a);
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
+}
+
 // Channels-last x and / or y: served by the bf16 matrix-instruction kernels only (x: the channels-last loader, i.e. input
 // channels per group in multiples of 32 and a kernel extent the tap masks hold; y: output channels per group in eights).
 static bool layouts_supported(const ConvGeom &g, const GemmPlan &p);

@@ -25,29 +25,39 @@
 // 858 -> 591 us): 1.2e15 bf16 operations a second on operands of random bits, what the library's bf16 product reaches on the same card.
 // Loads two K tiles further ahead, or a second set of registers for them, made no difference.
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t round_pair(float lo, float hi)
-{
-    bf16x2 v; // one v_cvt_pk_bf16_f32
-    v[0] = (__bf16)lo;
-    v[1] = (__bf16)hi;
-    return __builtin_bit_cast(uint32_t, v);
-}
-
 // eight consecutive k of a row -> the 16-byte pieces of its three parts
 __device__ __forceinline__ void split8(const float *v, u32x4 (&o)[3])
 {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        float lo = v[2 * q], hi = v[2 * q + 1];
+        uint32_t r[3];
+        split_pair(v[2 * q], v[2 * q + 1], r);
 #pragma unroll
-        for (int pl = 0; pl < 3; pl++) {
-            const uint32_t r = opaque(round_pair(lo, hi)); // (else the compiler rounds the lower element a second time to shift it)
-            o[pl][q] = r;
-            lo -= __builtin_bit_cast(float, r << 16);
-            hi -= __builtin_bit_cast(float, r & 0xFFFF0000u);
+        for (int pl = 0; pl < 3; pl++)
+            o[pl][q] = r[pl];
+    }
+}
+
+// ... for weights: one whose first piece would round to infinity is cut instead, so that the pieces always add up to it
+__device__ __forceinline__ void split8_weights(const float *v, u32x4 (&o)[3])
+{
+    split8(v, o);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int sh = (e & 1) * 16;
+        if (((o[0][e / 2] >> sh) & 0x7F80u) != 0x7F80u)
+            continue;
+        // infinite, not a number, or rounded to infinity
+        const uint32_t bits = __builtin_bit_cast(uint32_t, v[e]);
+        float part[3] = {v[e], 0.0f, 0.0f};
+        if ((bits & 0x7F800000u) != 0x7F800000u) {
+            part[0] = __builtin_bit_cast(float, bits & 0xFFFF0000u);
+            part[1] = to_float(to_bf16(v[e] - part[0]));
+            part[2] = v[e] - part[0] - part[1];
         }
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++)
+            o[pl][e / 2] = (o[pl][e / 2] & ~(0xFFFFu << sh)) | ((uint32_t)to_bf16(part[pl]).bits << sh);
     }
 }
 
@@ -325,7 +335,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
 // Weights -> [group][m tile][K tile][piece][half][row][8 channels of one tap], zero padded.  One workgroup moves 16 filters x 16 channels
 // through LDS (read in runs of whole filter rows, 16 bytes per lane where the tensor is aligned); a thread then splits eight channels
-// of a filter at a time.  A weight whose first piece would round to infinity is cut instead, so that the pieces always add up to it.
+// of a filter at a time.
 __global__ __launch_bounds__(256) void pack_weights_split_kernel(GemmPlan p, int ncb, int khw, int aligned, const float *__restrict__ w,
                                                                  u32x4 *__restrict__ out)
 {
@@ -375,27 +385,65 @@ __global__ __launch_bounds__(256) void pack_weights_split_kernel(GemmPlan p, int
         for (int e = 0; e < 8; e++)
             v[e] = lds[r * ld + (half * 8 + e) * khw + tap];
         u32x4 o[3];
-        split8(v, o);
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int sh = (e & 1) * 16;
-            if (((o[0][e / 2] >> sh) & 0x7F80u) != 0x7F80u)
-                continue;
-            // infinite, not a number, or rounded to infinity
-            const uint32_t bits = __builtin_bit_cast(uint32_t, v[e]);
-            float part[3] = {v[e], 0.0f, 0.0f};
-            if ((bits & 0x7F800000u) != 0x7F800000u) {
-                part[0] = __builtin_bit_cast(float, bits & 0xFFFF0000u);
-                part[1] = to_float(to_bf16(v[e] - part[0]));
-                part[2] = v[e] - part[0] - part[1];
-            }
-#pragma unroll
-            for (int pl = 0; pl < 3; pl++)
-                o[pl][e / 2] = (o[pl][e / 2] & ~(0xFFFFu << sh)) | ((uint32_t)to_bf16(part[pl]).bits << sh);
-        }
+        split8_weights(v, o);
         u32x4 *const dst = tile0 + (size_t)tap * (6 * p.BM) + half * p.BM + r;
 #pragma unroll
         for (int pl = 0; pl < 3; pl++)
             dst[(size_t)pl * 2 * p.BM] = o[pl];
     }
+}
+
+// Filters of a backward-data pass, packed straight from w[group][k][c][KH][KW]: a phase's convolution maps dy (channels k) to dx (rows c)
+// with the taps (rh0 + (nh - 1 - jh) * rhstep, rw0 + (nw - 1 - jw) * rwstep).  One launch for all phases, about 5 us, in the place of one
+// transposing and one packing launch per phase at 4 to 5 us each whatever their size.  A thread has one k (float tiles) or eight
+// consecutive k (split tiles) of one row; rows are contiguous in the packed tile, so the stores coalesce and the caches serve the loads.
+struct PhasePack {
+    void *out;
+    int nh, nw, rh0, rhstep, rw0, rwstep;
+    int BM, nkt, mtiles, split;
+    uint32_t units, block0; // threads with something to do, first workgroup
+};
+struct PhasePackArgs {
+    int n, cout_g, cin_g, KH, KW;
+    PhasePack ph[kMaxPhases];
+};
+__global__ __launch_bounds__(256) void phase_pack_kernel(const float *__restrict__ w, PhasePackArgs a)
+{
+    int i = 0;
+    while (i + 1 < a.n && blockIdx.x >= a.ph[i + 1].block0)
+        i++;
+    const PhasePack &p = a.ph[i];
+    const uint32_t unit = (blockIdx.x - p.block0) * 256u + threadIdx.x;
+    if (unit >= p.units)
+        return;
+    const uint32_t per_row = p.split ? 2 : BK;
+    uint32_t q = unit / (uint32_t)p.BM;
+    const int row = (int)(unit - q * (uint32_t)p.BM);
+    const int k = (int)(q % per_row);
+    q /= per_row;
+    const uint32_t tile = q; // (group, m tile, K tile)
+    const int kt = (int)(q % (uint32_t)p.nkt);
+    q /= (uint32_t)p.nkt;
+    const int mt = (int)(q % (uint32_t)p.mtiles), g = (int)(q / (uint32_t)p.mtiles);
+    const int taps = p.nh * p.nw, cb = kt / taps, tap = kt - cb * taps;
+    const int jh = tap / p.nw, jw = tap - jh * p.nw;
+    const int rh = p.rh0 + (p.nh - 1 - jh) * p.rhstep, rw = p.rw0 + (p.nw - 1 - jw) * p.rwstep;
+    const int c = mt * p.BM + row;
+    const bool ok = c < a.cin_g;
+    const size_t step = (size_t)a.cin_g * a.KH * a.KW; // from one k to the next
+    const float *src = w + (size_t)(g * a.cout_g + cb * BK) * step + ((size_t)c * a.KH + rh) * a.KW + rw;
+    if (!p.split) {
+        ((float *)p.out)[unit] = ok ? src[k * step] : 0.0f;
+        return;
+    }
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        v[e] = ok ? src[(k * 8 + e) * step] : 0.0f;
+    u32x4 o[3];
+    split8_weights(v, o);
+    u32x4 *const dst = (u32x4 *)p.out + (size_t)tile * (6 * p.BM) + k * p.BM + row;
+#pragma unroll
+    for (int pl = 0; pl < 3; pl++)
+        dst[(size_t)pl * 2 * p.BM] = o[pl];
 }

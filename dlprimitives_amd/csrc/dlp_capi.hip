@@ -266,6 +266,31 @@ __global__ void clear_ints_kernel(int *p, int n)
 }
 } // namespace
 
+// what a packed buffer's layout depends on
+static void layout_of(const GemmPlan &p, int (&sig)[6])
+{
+    sig[0] = p.order;
+    sig[1] = p.BM;
+    sig[2] = p.nkt;
+    sig[3] = p.mtiles;
+    sig[4] = p.patch + 2 * p.split;
+    sig[5] = p.wdirect;
+}
+
+namespace dlp {
+bool conv_fwd_packable(dlp_conv2d_fwd *op, GemmPlan *plan)
+{
+    ConvGeom g;
+    if (op == nullptr || op->algo != ALGO_GEMM || op_geom(op, op->cfg.shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
+        return false;
+    *plan = conv_gemm_plan(g, op->activation);
+    if (plan->order != GEMM_ORDER_TAP || plan->stem || plan->pointwise)
+        return false;
+    layout_of(*plan, op->packed_layout);
+    return true;
+}
+} // namespace dlp
+
 extern "C" {
 
 const char *dlp_last_error(void) { return g_last_error.c_str(); }
@@ -646,16 +671,6 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
 }
 
 // ---- weights that stay constant between calls: transformed once into a buffer of the caller ----
-static void layout_of(const GemmPlan &p, int (&sig)[6])
-{
-    sig[0] = p.order;
-    sig[1] = p.BM;
-    sig[2] = p.nkt;
-    sig[3] = p.mtiles;
-    sig[4] = p.patch + 2 * p.split;
-    sig[5] = p.wdirect;
-}
-
 int dlp_conv2d_fwd_set_accumulate_first(dlp_conv2d_fwd *op, int on)
 {
     DLP_REQUIRE(op != nullptr, "null argument");

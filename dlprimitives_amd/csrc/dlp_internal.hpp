@@ -119,6 +119,24 @@ __device__ __forceinline__ bf16_t to_bf16(float f)
     return r;
 }
 
+// A float as the exact sum of three bf16 numbers (8 significant bits each, rounded to nearest, the next taking what is left over): the
+// parts of lo in the lower, those of hi in the upper halves of o[0..2].
+__device__ __forceinline__ void split_pair(float lo, float hi, uint32_t (&o)[3])
+{
+    typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int pl = 0; pl < 3; pl++) {
+        pair_t v; // one v_cvt_pk_bf16_f32
+        v[0] = (__bf16)lo;
+        v[1] = (__bf16)hi;
+        uint32_t r = __builtin_bit_cast(uint32_t, v);
+        asm("" : "+v"(r)); // (else the compiler rounds the lower element a second time to shift it)
+        o[pl] = r;
+        lo -= __builtin_bit_cast(float, r << 16);
+        hi -= __builtin_bit_cast(float, r & 0xFFFF0000u);
+    }
+}
+
 __device__ __forceinline__ void store_out(bf16_t *p, float v, float factor)
 {
     if (factor != 0.0f)
@@ -207,6 +225,19 @@ enum { GEMM_PACK_AND_CLEAR = 0, GEMM_PACK_ONLY = 1, GEMM_CLEAR_ONLY = 2 };
 // counters_owned: conv_gemm_launch will be given counters of the operator's own (see there): none are cleared here.
 int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, void *wpacked, hipStream_t stream,
                            void *part_ws = nullptr, size_t part_bytes = 0, int mode = GEMM_PACK_AND_CLEAR, bool counters_owned = false);
+// One phase of a backward-data pass (a stride-1 pass is one phase): the plan of its convolution dy -> dx, where its packed filter goes, and
+// which filter rows and columns it takes: r0 + j * step, in reverse order.
+constexpr int kMaxPhases = 16;
+struct PhaseFilter {
+    GemmPlan plan;
+    void *packed;
+    int nh, nw, rh0, rhstep, rw0, rwstep;
+};
+// packs the filters of n phases from w[groups * cout_g][cin_g][KH][KW] in one launch; plans as conv_fwd_packable gives them
+int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream);
+// Whether conv_gemm_pack_phases can fill the buffer that dlp_conv2d_fwd_enqueue_packed takes for this operator (float, algorithm gemm, K
+// tiles of one tap x 16 channels, packed tiles the only form of the weights it reads); if so the operator expects that layout from now on.
+bool conv_fwd_packable(dlp_conv2d_fwd *op, GemmPlan *plan);
 // Tile counters a launch at this batch may use (0: none).  A caller that keeps that many zeroed ints per operator and
 // hands them to conv_gemm_launch as own_counters saves the clearing before every launch: the kernels leave them at zero.
 // Such an operator must not run on two streams at once.

@@ -115,3 +115,29 @@ def test_gpu_split_other_batches():
         x, w = torch.randint(-4, 5, xs, generator=gen).float(), torch.randint(-4, 5, ws, generator=gen).float()
         for packed in (False, True):
             assert torch.equal(_run(cb, x, w, None, packed, hint=5), _conv64(cb, x, w, None))  # whole numbers are exact
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(48, 64, 3, 2, 1, 1, 1, 24, 79, 81), (40, 32, 4, 2, 1, 1, 1, 3, 18, 22), (64, 48, 3, 1, 1, 1, 2, 33, 40, 40), (20, 16, 5, 3, 2, 1, 1, 2, 17, 19)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_gpu_backward_data_phase_packing(c):
+    """filters of all stride phases packed by one launch, in float and in split tiles; bias and activation behind the interleaving"""
+    cin, cout, k, s, p, d, g, b, h, wd = c
+    gen = torch.Generator().manual_seed(sum(c))
+    xs, ws, ys = _geometry(c)
+    w, dy, bias = torch.randn(ws, generator=gen), torch.randn(ys, generator=gen), torch.randn(cin, generator=gen)
+    extra = tuple(n - ((o - 1) * s - 2 * p + d * (k - 1) + 1) for n, o in zip(xs[2:], ys[2:]))
+    want = torch.nn.functional.conv_transpose2d(dy.double(), w.double(), None, s, p, extra, g, d)
+    scale = torch.nn.functional.conv_transpose2d(dy.double().abs(), w.double().abs(), None, s, p, extra, g, d) + bias.double().abs().view(1, -1, 1, 1)
+    bound = (cout // g * k * k + 8) * 2.0 ** -24  # one rounding per product and a few behind
+    op = dlp.Conv2DBackwardData.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs), "gemm")
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    dx = torch.full(xs, float("nan"), device="cuda:0")
+    op.enqueue(dx, w.cuda(), dy.cuda(), work)
+    assert ((dx.cpu().double() - want).abs() <= scale * bound).all()
+    tr = dlp.TransposedConv2DForward.create(dlp.Conv2DSettings(cout, cin, k, s, d, p, g, ys), extra, True, "relu", "gemm")
+    work = torch.empty(max(tr.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    y = torch.full(xs, float("nan"), device="cuda:0")
+    tr.enqueue(dy.cuda(), w.cuda(), bias.cuda(), y, work)
+    assert ((y.cpu().double() - (want + bias.double().view(1, -1, 1, 1)).relu()).abs() <= scale * bound).all()
+
