@@ -32,6 +32,7 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int KC = 32;        // reduction indices (pixels of the batch, image after image) per staged chunk
 constexpr int PITCH = KC + 4; // LDS row pitch in floats: 16-byte reads of 8 consecutive lanes cover all banks
@@ -53,14 +54,22 @@ struct WgradArgs {
 // AVEC: OH * OW is a multiple of 4, dy rows are read 16 bytes per lane.
 // MASKED: the padding test of a gathered element is one bit of a per-lane tap mask: 1 = KH * KW <= 31 (one word),
 // 2 = KH * KW <= 63 (two words); 0 = row and column comparisons per element.
-template <int BM, int BN, bool AVEC, int MASKED>
-__global__ __launch_bounds__(256) void conv_wgrad_f32_kernel(WgradArgs a)
+// SPLIT: the operands as three bf16 parts on the bf16 matrix instruction, six products per k, the five small ones in an accumulator of
+// their own, and a tile whose sums are not all finite again on the fp32 instruction -- as conv_gemm_split.hpp explains for the forward
+// pass.  A chunk's 32 k of a row then lie in LDS as 64 bytes per part (rows of 80: 16-byte reads of 8 consecutive lanes cover all banks).
+// x arrives one pixel per lane: neighbouring lanes trade elements of two rows, so that each has two consecutive k of one row to split and
+// store as a word.  Tiles of 128x128 only: smaller ones leave a wavefront 32x32 of the output, which LDS cannot feed at that rate.
+// 3x3 128->128 at 28x28, batch 64: 152 -> 101 us; stride 2 128->256, batch 32: 52 -> 28 us; 5x5 48->80 at 35x27, batch 9: 43 -> 34 us.
+template <int BM, int BN, bool AVEC, int MASKED, bool SPLIT = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : 1))) void conv_wgrad_f32_kernel(WgradArgs a)
 {
     constexpr int TM = BM / 64, TN = BN / 64; // 32x32 MFMA blocks per wavefront (wavefronts 2 x 2)
     constexpr int RB = BN / 8;                // gathered rows per thread: two rows per wavefront load
     constexpr int RA = AVEC ? BM / 32 : BM / 8;
-    __shared__ __attribute__((aligned(16))) float As[BM * PITCH];
-    __shared__ __attribute__((aligned(16))) float Bs[BN * PITCH];
+    constexpr int SROW = 80; // bytes of a row of one part (SPLIT)
+    __shared__ __attribute__((aligned(16))) unsigned char smem[SPLIT ? 3 * (BM + BN) * SROW : (BM + BN) * PITCH * 4];
+    float *const As = reinterpret_cast<float *>(smem), *const Bs = As + BM * PITCH;
+    unsigned char *const At = smem, *const Bt = smem + 3 * BM * SROW; // SPLIT: [part][row][k]
     __shared__ __attribute__((aligned(16))) int rowtab[BN * 4]; // per column: x offset of the tap, tap bit (or 31), row and column shift
 
     const int tid = threadIdx.x;
@@ -189,43 +198,134 @@ __global__ __launch_bounds__(256) void conv_wgrad_f32_kernel(WgradArgs a)
             for (int r = 0; r < 16; r++)
                 acc[i][j][r] = 0.0f;
 
-    if (ck_begin < ck_end)
-        fetch(ck_begin);
-    for (int ck = ck_begin; ck < ck_end; ck++) {
-        __syncthreads(); // the previous chunk has been read
-        if (AVEC) {
+    bool in_floats = !SPLIT;
+    if constexpr (SPLIT) {
+        f32x16 small[TM][TN];
 #pragma unroll
-            for (int i = 0; i < RA; i++)
-                *reinterpret_cast<f32x4 *>(&As[(arow + 32 * i) * PITCH + 4 * (lane & 7)]) = ra4[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < RA; i++)
-                As[(arow + 8 * i) * PITCH + l32] = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < RB; i++)
-            Bs[(brow + 8 * i) * PITCH + l32] = rb[i];
-        __syncthreads();
-        if (ck + 1 < ck_end)
-            fetch(ck + 1); // lands while this chunk is multiplied
-        // k order inside a chunk: MFMA step 4*kq + e takes index 8*kq + e from the lower half-wave and
-        // 8*kq + 4 + e from the upper one, for both operands alike
-#pragma unroll
-        for (int kq = 0; kq < KC / 8; kq++) {
-            f32x4 av[TM], bv[TN];
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-                av[i] = *reinterpret_cast<const f32x4 *>(&As[(wm * (BM / 2) + i * 32 + l32) * PITCH + kq * 8 + h * 4]);
+        for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++)
-                bv[j] = *reinterpret_cast<const f32x4 *>(&Bs[(wn * (BN / 2) + j * 32 + l32) * PITCH + kq * 8 + h * 4]);
+                small[i][j] = acc[i][j];
+        // rows r0 and r1 of one k per lane -> the lane's row of the two, two consecutive k: split and stored
+        auto store_pair = [&](unsigned char *t, int rows, float v0, float v1, int r0, int r1) {
+            const bool odd = lane & 1;
+            const float got = __shfl_xor(odd ? v0 : v1, 1);
+            uint32_t o[3];
+            split_pair(odd ? got : v0, odd ? v1 : got, o);
+            unsigned char *const dst = t + (odd ? r1 : r0) * SROW + (l32 & ~1) * 2;
 #pragma unroll
-            for (int e = 0; e < 4; e++)
+            for (int pl = 0; pl < 3; pl++)
+                *reinterpret_cast<uint32_t *>(dst + pl * rows * SROW) = o[pl];
+        };
+        if (ck_begin < ck_end)
+            fetch(ck_begin);
+        for (int ck = ck_begin; ck < ck_end; ck++) {
+            __syncthreads(); // the previous chunk has been read
+            if (AVEC) {
 #pragma unroll
-                for (int i = 0; i < TM; i++)
+                for (int i = 0; i < RA; i++) {
+                    uint32_t lo[3], hi[3];
+                    split_pair(ra4[i][0], ra4[i][1], lo);
+                    split_pair(ra4[i][2], ra4[i][3], hi);
+#pragma unroll
+                    for (int pl = 0; pl < 3; pl++)
+                        *reinterpret_cast<uint2 *>(At + (pl * BM + arow + 32 * i) * SROW + (lane & 7) * 8) = make_uint2(lo[pl], hi[pl]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < RA; i += 2)
+                    store_pair(At, BM, ra[AVEC ? 0 : i], ra[AVEC ? 0 : i + 1], arow + 8 * i, arow + 8 * (i + 1));
+            }
+#pragma unroll
+            for (int i = 0; i < RB; i += 2)
+                store_pair(Bt, BN, rb[i], rb[i + 1], brow + 8 * i, brow + 8 * (i + 1));
+            __syncthreads();
+            if (ck + 1 < ck_end)
+                fetch(ck + 1); // lands while this chunk is multiplied
+#pragma unroll
+            for (int ks = 0; ks < KC / 16; ks++) {
+                bf16x8 fa[3][TM], fb[3][TN];
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++) {
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+                        fa[pl][i] = *reinterpret_cast<const bf16x8 *>(At + (pl * BM + wm * (BM / 2) + i * 32 + l32) * SROW + ks * 32 + h * 16);
 #pragma unroll
                     for (int j = 0; j < TN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
+                        fb[pl][j] = *reinterpret_cast<const bf16x8 *>(Bt + (pl * BN + wn * (BN / 2) + j * 32 + l32) * SROW + ks * 32 + h * 16);
+                }
+                constexpr int PA[6] = {0, 1, 0, 1, 2, 0}, PB[6] = {0, 0, 1, 1, 0, 2};
+#pragma unroll
+                for (int q = 0; q < 6; q++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++) {
+                            f32x16 &c = q == 0 ? acc[i][j] : small[i][j];
+                            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[PA[q]][i], fb[PB[q]][j], c, 0, 0, 0);
+                        }
+            }
+        }
+        float finite = 0.0f; // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                acc[i][j] += small[i][j];
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    finite = fmaf(acc[i][j][r], 0.0f, finite);
+            }
+        in_floats = __syncthreads_or(finite != 0.0f);
+        if (in_floats) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        acc[i][j][r] = 0.0f;
+        }
+    }
+    if (in_floats) {
+        if (ck_begin < ck_end)
+            fetch(ck_begin);
+        for (int ck = ck_begin; ck < ck_end; ck++) {
+            __syncthreads(); // the previous chunk has been read
+            if (AVEC) {
+#pragma unroll
+                for (int i = 0; i < RA; i++)
+                    *reinterpret_cast<f32x4 *>(&As[(arow + 32 * i) * PITCH + 4 * (lane & 7)]) = ra4[i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < RA; i++)
+                    As[(arow + 8 * i) * PITCH + l32] = ra[i];
+            }
+#pragma unroll
+            for (int i = 0; i < RB; i++)
+                Bs[(brow + 8 * i) * PITCH + l32] = rb[i];
+            __syncthreads();
+            if (ck + 1 < ck_end)
+                fetch(ck + 1); // lands while this chunk is multiplied
+            // k order inside a chunk: MFMA step 4*kq + e takes index 8*kq + e from the lower half-wave and
+            // 8*kq + 4 + e from the upper one, for both operands alike
+#pragma unroll
+            for (int kq = 0; kq < KC / 8; kq++) {
+                f32x4 av[TM], bv[TN];
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+                    av[i] = *reinterpret_cast<const f32x4 *>(&As[(wm * (BM / 2) + i * 32 + l32) * PITCH + kq * 8 + h * 4]);
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    bv[j] = *reinterpret_cast<const f32x4 *>(&Bs[(wn * (BN / 2) + j * 32 + l32) * PITCH + kq * 8 + h * 4]);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
+            }
         }
     }
 
@@ -487,7 +587,8 @@ struct WgradPlan {
     size_t part_bytes;
 };
 
-constexpr int kWgradSlots = 256 * 3; // workgroups resident at once: three per compute unit
+constexpr int kWgradSlots = 256 * 3;      // workgroups resident at once: three per compute unit
+constexpr int kWgradSlotsSplit = 256 * 2; // ... two of the 128x128 tiles in bf16 parts
 
 // Slices: one full round of resident workgroups where the tiles allow it, at least two chunks each.
 WgradPlan wgrad_plan(const dlp_conv2d_settings &c, int batch, int OH, int OW)
@@ -509,7 +610,7 @@ WgradPlan wgrad_plan(const dlp_conv2d_settings &c, int batch, int OH, int OW)
     p.ntiles = (ncol + p.BN - 1) / p.BN;
     p.chunks = (int)(((long long)batch * OH * OW + KC - 1) / KC);
     const long long tiles = (long long)p.mtiles * p.ntiles * c.groups;
-    long long want = std::max<long long>(1, kWgradSlots / tiles);
+    long long want = std::max<long long>(1, (p.BM == 128 && p.BN == 128 ? kWgradSlotsSplit : kWgradSlots) / tiles);
     want = std::min<long long>(want, std::max(1, p.chunks / 2));
     p.cps = (int)((p.chunks + want - 1) / want);
     p.slices = (p.chunks + p.cps - 1) / p.cps;
@@ -966,30 +1067,30 @@ int dlp_conv2d_bwd_filter_enqueue(dlp_conv2d_bwd_filter *op, const int x_shape[4
         const bool avec = a.OHW % 4 == 0 && ((uintptr_t)dy & 15) == 0;
         const int taps = a.KH * a.KW;
         const int masked = taps <= 31 ? 1 : taps <= 63 ? 2 : 0;
-#define DLP_WGRAD_LAUNCH_M(BM_, BN_, AV_)                                                                      \
+#define DLP_WGRAD_LAUNCH_M(BM_, BN_, AV_, SP_)                                                                    \
     do {                                                                                                       \
         if (masked == 1)                                                                                       \
-            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 1>), grid, block, 0, st, a);              \
+            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 1, SP_>), grid, block, 0, st, a);         \
         else if (masked == 2)                                                                                  \
-            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 2>), grid, block, 0, st, a);              \
+            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 2, SP_>), grid, block, 0, st, a);         \
         else                                                                                                   \
-            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 0>), grid, block, 0, st, a);              \
+            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 0, SP_>), grid, block, 0, st, a);         \
     } while (0)
-#define DLP_WGRAD_LAUNCH(BM_, BN_)                                                                             \
+#define DLP_WGRAD_LAUNCH(BM_, BN_, SP_)                                                                           \
     do {                                                                                                       \
         if (avec)                                                                                              \
-            DLP_WGRAD_LAUNCH_M(BM_, BN_, true);                                                                \
+            DLP_WGRAD_LAUNCH_M(BM_, BN_, true, SP_);                                                           \
         else                                                                                                   \
-            DLP_WGRAD_LAUNCH_M(BM_, BN_, false);                                                               \
+            DLP_WGRAD_LAUNCH_M(BM_, BN_, false, SP_);                                                          \
     } while (0)
         if (p.BM == 128 && p.BN == 128)
-            DLP_WGRAD_LAUNCH(128, 128);
+            DLP_WGRAD_LAUNCH(128, 128, true);
         else if (p.BM == 128)
-            DLP_WGRAD_LAUNCH(128, 64);
+            DLP_WGRAD_LAUNCH(128, 64, false);
         else if (p.BN == 128)
-            DLP_WGRAD_LAUNCH(64, 128);
+            DLP_WGRAD_LAUNCH(64, 128, false);
         else
-            DLP_WGRAD_LAUNCH(64, 64);
+            DLP_WGRAD_LAUNCH(64, 64, false);
 #undef DLP_WGRAD_LAUNCH
 #undef DLP_WGRAD_LAUNCH_M
     }

@@ -141,3 +141,35 @@ def test_gpu_backward_data_phase_packing(c):
     tr.enqueue(dy.cuda(), w.cuda(), bias.cuda(), y, work)
     assert ((y.cpu().double() - (want + bias.double().view(1, -1, 1, 1)).relu()).abs() <= scale * bound).all()
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(32, 80, 3, 1, 1, 1, 1, 3, 12, 12), (33, 130, 3, 2, 1, 1, 1, 2, 15, 13), (48, 70, 5, 1, 2, 1, 1, 1, 9, 7), (16, 65, 7, 1, 3, 1, 1, 2, 10, 8),
+                               (256, 72, 1, 1, 0, 1, 2, 5, 8, 8), (128, 128, 1, 1, 0, 1, 1, 1, 1, 1), (20, 200, 8, 1, 4, 1, 1, 2, 9, 9)], ids=lambda c: "x".join(map(str, c)))
+def test_gpu_split_filter_gradient(c):
+    """filter gradients in tiles of 128x128 (more than 64 filters and 64 columns): remainders in rows, columns and pixels, planes of whole
+    16-byte pieces and others, one and two words of tap mask and none; then infinities and NaN"""
+    cin, cout, k, s, p, d, g, b, h, wd = c
+    gen = torch.Generator().manual_seed(sum(c))
+    xs, ws, ys = _geometry(c)
+    x, dy = torch.randn(xs, generator=gen), torch.randn(ys, generator=gen)
+    op = dlp.Conv2DBackwardFilter.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs))
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+
+    def got(x):
+        dw = torch.full(ws, float("nan"), device="cuda:0")
+        op.enqueue(x.cuda(), dw, dy.cuda(), work)
+        return dw.cpu().double()
+
+    grad = lambda x, dy: torch.nn.grad.conv2d_weight(x.double(), ws, dy.double(), s, p, d, g)
+    want, scale = grad(x, dy), grad(x.abs(), dy.abs())
+    n = ys[0] * ys[2] * ys[3]
+    err = (got(x) - want).abs()
+    assert (err <= scale * (n / 4 + 8) * 2.0 ** -24).all()  # as for the forward pass
+    x[0, 1, 0, 0], x[0, 3, xs[2] // 2, xs[3] // 2] = float("inf"), float("nan")
+    dy = dy.abs() + 0.5  # no product of infinity and zero inside the image
+    mine, want = got(x), grad(torch.nan_to_num(x, nan=0.0, posinf=0.0), dy)
+    clean = [i for i in range(cin // g) if not (i == 1 or i == 3)]
+    assert torch.isfinite(mine[:, clean][cout // g:] if g > 1 else mine[:, clean]).all()
+    first = mine[: cout // g]
+    assert (torch.isposinf(first[:, 1]) | torch.isfinite(first[:, 1])).all() and torch.isposinf(first[:, 1]).any()
+    assert torch.isnan(first[:, 3]).any() and (torch.isnan(first[:, 3]) | torch.isfinite(first[:, 3])).all()
