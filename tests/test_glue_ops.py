@@ -404,3 +404,21 @@ def test_gpu_eltwise_broadcast(dtype):
     with pytest.raises(dlp.NotImplementedErrorDlprim):  # five runs of dimensions that alternate between the operands
         dlp.eltwise_forward(torch.zeros((2, 1, 2, 1, 2), device="cuda:0"), torch.zeros((1, 2, 1, 2, 1), device="cuda:0"), torch.zeros((2, 2, 2, 2, 2), device="cuda:0"))
 
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(5, 1000), (3, 1024), (3, 1025), (2, 64), (2, 65), (1, 1), (3, 130, 7)], ids=str)
+@pytest.mark.parametrize("log", [False, True])
+def test_gpu_softmax_in_registers(shape, log):
+    """class counts around a wavefront's multiples and around the 1024 that are held in registers, planes of one pixel and more"""
+    import torch
+
+    import dlprimitives_amd as dlp
+
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(sum(shape))) * 4
+    x.view(-1)[0] = 80.0
+    y = torch.full(shape, float("nan"), device="cuda:0")
+    dlp.softmax_forward(x.cuda(), y, log)
+    want = torch.log_softmax(x.double(), 1) if log else torch.softmax(x.double(), 1)
+    # the exponent is off by half a unit of its largest difference (2^7 * 2^-24), the sum by a rounding per step of 16 + 6
+    np.testing.assert_allclose(y.cpu().double().numpy(), want.numpy(), rtol=2.0 ** -16, atol=2.0 ** -120)
