@@ -633,9 +633,7 @@ struct PhaseAxis {
 struct BwdPhase {
     PhaseAxis h, w;
     dlp_conv2d_fwd *fwd;
-    size_t wt_bytes, fwd_ws;
-    bool packable; // conv_gemm_pack_phases fills the filter region
-    GemmPlan plan; // ... by this plan
+    size_t wt_bytes, fwd_ws; // filter region: packed tiles or, in calls whose kernel reads a filter, the phase's filter
 };
 
 struct dlp_conv2d_bwd_data {
@@ -644,8 +642,6 @@ struct dlp_conv2d_bwd_data {
     bool strided;            // one stride-1 convolution per phase, then interleaved into dx
     dlp_conv2d_fwd *fwd;     // stride 1: the convolution dy -> dx on the transposed, flipped filter
     size_t wt_bytes, fwd_ws; // stride 1
-    bool packable;           // ... as in BwdPhase
-    GemmPlan plan;
     BwdPhase phase[kMaxPhases];
     int nphases;
 };
@@ -745,9 +741,8 @@ int dlp_conv2d_bwd_data_create(const dlp_conv2d_settings *cfg, const char *algo,
             delete op;
             return rc;
         }
-        op->packable = conv_fwd_packable(op->fwd, &op->plan);
-        op->wt_bytes = op->packable ? dlp_conv2d_fwd_packed_bytes(op->fwd)
-                                    : round256((size_t)cfg->channels_out * cin_g * cfg->kernel[0] * cfg->kernel[1] * sizeof(float));
+        op->wt_bytes = std::max(conv_fwd_tiles_bytes(op->fwd),
+                                round256((size_t)cfg->channels_out * cin_g * cfg->kernel[0] * cfg->kernel[1] * sizeof(float)));
         op->fwd_ws = round256(dlp_conv2d_fwd_workspace(op->fwd));
         *out = op;
         return DLP_OK;
@@ -779,8 +774,7 @@ int dlp_conv2d_bwd_data_create(const dlp_conv2d_settings *cfg, const char *algo,
                 bwd_data_free(op);
                 return rc;
             }
-            ph.packable = conv_fwd_packable(ph.fwd, &ph.plan);
-            ph.wt_bytes = ph.packable ? dlp_conv2d_fwd_packed_bytes(ph.fwd) : round256((size_t)cfg->channels_out * cin_g * ph.h.n * ph.w.n * sizeof(float));
+            ph.wt_bytes = std::max(conv_fwd_tiles_bytes(ph.fwd), round256((size_t)cfg->channels_out * cin_g * ph.h.n * ph.w.n * sizeof(float)));
             ph.fwd_ws = round256(dlp_conv2d_fwd_workspace(ph.fwd));
         }
     *out = op;
@@ -844,12 +838,12 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
     if (!op->strided) {
         float *wt = (float *)ws;
         void *fws = (char *)ws + op->wt_bytes;
-        if (op->packable) {
-            const PhaseFilter pf = {op->plan, wt, c.kernel[0], c.kernel[1], 0, 1, 0, 1};
+        PhaseFilter pf = {{}, wt, c.kernel[0], c.kernel[1], 0, 1, 0, 1};
+        if (conv_fwd_tiles_plan(op->fwd, batch, &pf.plan)) {
             const int rc = conv_gemm_pack_phases((const float *)w, c.groups, cout_g, cin_g, c.kernel[0], c.kernel[1], &pf, 1, st);
             if (rc != DLP_OK)
                 return rc;
-            return dlp_conv2d_fwd_enqueue_packed(op->fwd, in_shape, dy, wt, wt, nullptr, dx, op->fwd_ws ? fws : nullptr, op->fwd_ws, factor, stream);
+            return conv_fwd_enqueue_tiles(op->fwd, batch, pf.plan, dy, wt, dx, fws, op->fwd_ws, factor, st);
         }
         {
             TimingScope ts("bwd_data_filter_transpose", st);
@@ -885,7 +879,7 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
     }
     float *wt[kMaxPhases], *outp[kMaxPhases];
     PhaseFilter pf[kMaxPhases];
-    int npf = 0;
+    int npf = 0, packed_as[kMaxPhases]; // place in pf, -1: a phase whose kernel reads a filter
     for (int i = 0; i < op->nphases; i++) {
         const BwdPhase &ph = op->phase[i];
         if (!ph.fwd)
@@ -894,8 +888,12 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
         cursor += ph.wt_bytes;
         outp[i] = (float *)cursor;
         cursor += round256(planes * ph.h.out * ph.w.out * sizeof(float));
-        if (ph.packable)
-            pf[npf++] = {ph.plan, wt[i], ph.h.n, ph.w.n, ph.h.r0, ph.h.rstep, ph.w.r0, ph.w.rstep};
+        GemmPlan plan;
+        packed_as[i] = -1;
+        if (conv_fwd_tiles_plan(ph.fwd, batch, &plan)) {
+            packed_as[i] = npf;
+            pf[npf++] = {plan, wt[i], ph.h.n, ph.w.n, ph.h.r0, ph.h.rstep, ph.w.r0, ph.w.rstep};
+        }
     }
     int rc = conv_gemm_pack_phases((const float *)w, c.groups, cout_g, cin_g, c.kernel[0], c.kernel[1], pf, npf, st);
     if (rc != DLP_OK)
@@ -904,8 +902,8 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
         const BwdPhase &ph = op->phase[i];
         if (!ph.fwd)
             continue;
-        if (ph.packable)
-            rc = dlp_conv2d_fwd_enqueue_packed(ph.fwd, in_shape, dy, wt[i], wt[i], nullptr, outp[i], ph.fwd_ws ? fws : nullptr, ph.fwd_ws, 0.0f, stream);
+        if (packed_as[i] >= 0)
+            rc = conv_fwd_enqueue_tiles(ph.fwd, batch, pf[packed_as[i]].plan, dy, wt[i], outp[i], fws, ph.fwd_ws, 0.0f, st);
         else {
             PhaseFilterArgs fa = {c.groups, cout_g, cin_g, c.kernel[0], c.kernel[1], ph.h.n, ph.w.n, ph.h.r0, ph.h.rstep, ph.w.r0, ph.w.rstep};
             {

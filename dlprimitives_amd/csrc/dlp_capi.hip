@@ -278,16 +278,43 @@ static void layout_of(const GemmPlan &p, int (&sig)[6])
 }
 
 namespace dlp {
-bool conv_fwd_packable(dlp_conv2d_fwd *op, GemmPlan *plan)
+bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan)
 {
     ConvGeom g;
-    if (op == nullptr || op->algo != ALGO_GEMM || op_geom(op, op->cfg.shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
+    const int x_shape[4] = {batch, op->cfg.channels_in, op->cfg.shape[2], op->cfg.shape[3]};
+    if (op->algo != ALGO_GEMM || op_geom(op, x_shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
         return false;
     *plan = conv_gemm_plan(g, op->activation);
-    if (plan->order != GEMM_ORDER_TAP || plan->stem || plan->pointwise)
-        return false;
-    layout_of(*plan, op->packed_layout);
-    return true;
+    return plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise;
+}
+
+size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op)
+{
+    ConvGeom g;
+    if (op->algo != ALGO_GEMM || op_geom(op, op->cfg.shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
+        return 0;
+    return round256(conv_gemm_plan(g, op->activation).wpack_bytes);
+}
+
+int conv_fwd_enqueue_tiles(dlp_conv2d_fwd *op, int batch, const GemmPlan &plan, const void *x, const void *tiles, void *y, void *ws, size_t ws_bytes,
+                           float factor, hipStream_t stream)
+{
+    ConvGeom g;
+    const int x_shape[4] = {batch, op->cfg.channels_in, op->cfg.shape[2], op->cfg.shape[3]};
+    int rc = op_geom(op, x_shape, g);
+    if (rc != DLP_OK)
+        return rc;
+    Epilogue ep;
+    ep.bias = nullptr;
+    ep.factor = factor;
+    ep.activation = op->activation;
+    ep.accumulate_first = op->accumulate_first;
+    int *counters = nullptr;
+    rc = own_counters(op, g, plan, &counters);
+    if (rc != DLP_OK)
+        return rc;
+    // no filter tensor: there are only the tiles
+    return conv_gemm_launch(g, plan, op->ktab, x, tiles, y, ep, stream, -1, ws_bytes > 0 ? ws : nullptr, ws_bytes, nullptr, counters);
 }
 } // namespace dlp
 

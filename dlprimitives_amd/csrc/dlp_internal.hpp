@@ -225,7 +225,7 @@ enum { GEMM_PACK_AND_CLEAR = 0, GEMM_PACK_ONLY = 1, GEMM_CLEAR_ONLY = 2 };
 // counters_owned: conv_gemm_launch will be given counters of the operator's own (see there): none are cleared here.
 int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, void *wpacked, hipStream_t stream,
                            void *part_ws = nullptr, size_t part_bytes = 0, int mode = GEMM_PACK_AND_CLEAR, bool counters_owned = false);
-// One phase of a backward-data pass (a stride-1 pass is one phase): the plan of its convolution dy -> dx, where its packed filter goes, and
+// One phase of a backward-data pass (a stride-1 pass is one phase): the plan of its convolution dy -> dx in this call, where its packed filter goes, and
 // which filter rows and columns it takes: r0 + j * step, in reverse order.
 constexpr int kMaxPhases = 16;
 struct PhaseFilter {
@@ -233,11 +233,16 @@ struct PhaseFilter {
     void *packed;
     int nh, nw, rh0, rhstep, rw0, rwstep;
 };
-// packs the filters of n phases from w[groups * cout_g][cin_g][KH][KW] in one launch; plans as conv_fwd_packable gives them
+// packs the filters of n phases from w[groups * cout_g][cin_g][KH][KW] in one launch; plans as conv_fwd_tiles_plan gives them
 int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream);
-// Whether conv_gemm_pack_phases can fill the buffer that dlp_conv2d_fwd_enqueue_packed takes for this operator (float, algorithm gemm, K
-// tiles of one tap x 16 channels, packed tiles the only form of the weights it reads); if so the operator expects that layout from now on.
-bool conv_fwd_packable(dlp_conv2d_fwd *op, GemmPlan *plan);
+// Whether a call at this batch can run on tiles that conv_gemm_pack_phases writes, and by which plan (float, algorithm gemm, K tiles of one
+// tap x 16 channels; not where the kernel of the call reads the filter as it is, which depends on the batch too).
+bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan);
+// ... the bytes of the tiles, enough for every batch (0: no call of this operator runs on them)
+size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op);
+// ... and the call (an operator without bias)
+int conv_fwd_enqueue_tiles(dlp_conv2d_fwd *op, int batch, const GemmPlan &plan, const void *x, const void *tiles, void *y, void *ws, size_t ws_bytes,
+                           float factor, hipStream_t stream);
 // Tile counters a launch at this batch may use (0: none).  A caller that keeps that many zeroed ints per operator and
 // hands them to conv_gemm_launch as own_counters saves the clearing before every launch: the kernels leave them at zero.
 // Such an operator must not run on two streams at once.

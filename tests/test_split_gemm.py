@@ -173,3 +173,32 @@ def test_gpu_split_filter_gradient(c):
     first = mine[: cout // g]
     assert (torch.isposinf(first[:, 1]) | torch.isfinite(first[:, 1])).all() and torch.isposinf(first[:, 1]).any()
     assert torch.isnan(first[:, 3]).any() and (torch.isnan(first[:, 3]) | torch.isfinite(first[:, 3])).all()
+
+
+# (cin, cout, k, stride, pad, create batch, call batch, h, w): gradients and transposed convolutions whose kernel reads the filter as it is
+# from 131072 pixels and at most 32 rows on, and packed tiles below
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(32, 16, 1, 1, 0, 2, 42, 56, 56), (24, 32, 1, 1, 0, 1, 140, 32, 32), (32, 16, 2, 2, 0, 2, 170, 56, 56), (16, 48, 3, 2, 1, 1, 44, 111, 111)],
+                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("grow", [False, True])
+def test_gpu_backward_data_batch_other_than_created(c, grow):
+    """created at a small batch and called at a large one, and the other way round"""
+    cin, cout, k, s, p, small, large, h, w = c
+    create, batch = (small, large) if grow else (large, small)
+    gen = torch.Generator().manual_seed(sum(c))
+    f = torch.randint(-4, 5, (cout, cin, k, k), generator=gen).float()
+    oh, ow = ((n + 2 * p - k) // s + 1 for n in (h, w))
+    dy = torch.randint(-4, 5, (batch, cout, oh, ow), generator=gen).float()
+    extra = tuple(n - ((o - 1) * s - 2 * p + k) for n, o in zip((h, w), (oh, ow)))
+    want = torch.nn.functional.conv_transpose2d(dy, f, None, s, p, extra)  # whole numbers: exact in any order
+    op = dlp.Conv2DBackwardData.create(dlp.Conv2DSettings(cin, cout, k, s, 1, p, 1, (create, cin, h, w)), "gemm")
+    # the part for phase outputs grows with the batch
+    work = torch.empty(max(op.workspace(), 1) * max(1, -(-batch // create)), dtype=torch.uint8, device="cuda:0")
+    dx = torch.full((batch, cin, h, w), float("nan"), device="cuda:0")
+    op.enqueue(dx, f.cuda(), dy.cuda(), work)
+    assert torch.equal(dx.cpu(), want)
+    tr = dlp.TransposedConv2DForward.create(dlp.Conv2DSettings(cout, cin, k, s, 1, p, 1, (create, cout, oh, ow)), extra, False, "identity", "gemm")
+    work = torch.empty(max(tr.workspace(), 1) * max(1, -(-batch // create)), dtype=torch.uint8, device="cuda:0")
+    y = torch.full((batch, cin, h, w), float("nan"), device="cuda:0")
+    tr.enqueue(dy.cuda(), f.cuda(), None, y, work)
+    assert torch.equal(y.cpu(), want)
