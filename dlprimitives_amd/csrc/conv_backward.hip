@@ -55,8 +55,9 @@ struct WgradArgs {
 // MASKED: the padding test of a gathered element is one bit of a per-lane tap mask: 1 = KH * KW <= 31 (one word),
 // 2 = KH * KW <= 63 (two words); 0 = row and column comparisons per element.
 // SPLIT: the operands as three bf16 parts on the bf16 matrix instruction, six products per k, the five small ones in an accumulator of
-// their own, and a tile whose sums are not all finite again on the fp32 instruction -- as conv_gemm_split.hpp explains for the forward
-// pass.  A chunk's 32 k of a row then lie in LDS as 64 bytes per part (rows of 80: 16-byte reads of 8 consecutive lanes cover all banks).
+// their own, and a tile whose sums are not finite or too small for the bits that small operands lose, or which has operands above 2^16, again
+// on the fp32 instruction -- as conv_gemm_split.hpp explains for the forward pass.  A chunk's 32 k of a row then lie in LDS as 64 bytes
+// per part (rows of 80: 16-byte reads of 8 consecutive lanes cover all banks).
 // x arrives one pixel per lane: neighbouring lanes trade elements of two rows, so that each has two consecutive k of one row to split and
 // store as a word.  Tiles of 128x128 only: smaller ones leave a wavefront 32x32 of the output, which LDS cannot feed at that rate.
 // 3x3 128->128 at 28x28, batch 64: 152 -> 101 us; stride 2 128->256, batch 32: 52 -> 28 us; 5x5 48->80 at 35x27, batch 9: 43 -> 34 us.
@@ -206,9 +207,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
 #pragma unroll
             for (int j = 0; j < TN; j++)
                 small[i][j] = acc[i][j];
+        float largest = 0.0f; // of this thread's operands
         // rows r0 and r1 of one k per lane -> the lane's row of the two, two consecutive k: split and stored
         auto store_pair = [&](unsigned char *t, int rows, float v0, float v1, int r0, int r1) {
             const bool odd = lane & 1;
+            largest = split_largest(largest, v0, v1);
             const float got = __shfl_xor(odd ? v0 : v1, 1);
             uint32_t o[3];
             split_pair(odd ? got : v0, odd ? v1 : got, o);
@@ -224,6 +227,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
             if (AVEC) {
 #pragma unroll
                 for (int i = 0; i < RA; i++) {
+                    largest = split_largest(split_largest(largest, ra4[i][0], ra4[i][1]), ra4[i][2], ra4[i][3]);
                     uint32_t lo[3], hi[3];
                     split_pair(ra4[i][0], ra4[i][1], lo);
                     split_pair(ra4[i][2], ra4[i][3], hi);
@@ -266,6 +270,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
                         }
             }
         }
+        uint32_t smallest = kSplitNoSum;
         float finite = 0.0f; // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -273,10 +278,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
             for (int j = 0; j < TN; j++) {
                 acc[i][j] += small[i][j];
 #pragma unroll
-                for (int r = 0; r < 16; r++)
+                for (int r = 0; r < 16; r++) {
                     finite = fmaf(acc[i][j][r], 0.0f, finite);
+                    smallest = split_smallest(smallest, acc[i][j][r]);
+                }
             }
-        in_floats = __syncthreads_or(finite != 0.0f);
+        in_floats = __syncthreads_or(finite != 0.0f || smallest < kSplitSmallSum || largest > kSplitLarge);
         if (in_floats) {
 #pragma unroll
             for (int i = 0; i < TM; i++)

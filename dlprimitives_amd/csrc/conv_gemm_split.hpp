@@ -10,8 +10,9 @@
 //
 // What does not split is computed on the fp32 instruction: an operand that is infinite, not a number, or so close to the largest float
 // that its first piece rounds to infinity leaves an infinity or a NaN in the sums, and a tile whose sums are not all finite is
-// computed again, whole, from the same operands as they were (the three pieces of a packed weight add up to it).  Pieces below the
-// smallest normal number may be lost: operands below 2^-100 carry fewer than 24 bits.
+// computed again, whole, from the same operands as they were (the three pieces of a packed weight add up to it).  So is a tile whose sums
+// are so small that bits lost from operands below 2^-110 could count (dlp_internal.hpp), and one with a weight below 2^-110 or above
+// 2^16: the packing kernel writes such a weight as a NaN and its 32 bits; weights read in place are looked at as they pass, and so is the input then.
 //
 //  * K tile = one filter tap x 16 channels = one matrix step; the input is gathered as in conv_gemm_f32_kernel (one masked pixel per
 //    lane, a channel per load), split in registers by the thread that loaded it, and stored as three 16-byte pieces of eight channels;
@@ -38,26 +39,30 @@ __device__ __forceinline__ void split8(const float *v, u32x4 (&o)[3])
     }
 }
 
-// ... for weights: one whose first piece would round to infinity is cut instead, so that the pieces always add up to it
+// ... for weights: one that is too small to be split, or too large, is left as kWholeWeight (a NaN, which no other weight becomes) and its
+// upper and lower 16 bits
+constexpr uint32_t kWholeWeight = 0x7FFFu;
 __device__ __forceinline__ void split8_weights(const float *v, u32x4 (&o)[3])
 {
     split8(v, o);
+    uint32_t smallest = kSplitNoSum, largest = 0;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        smallest = split_smallest(smallest, v[e]);
+        largest = max(largest, __builtin_bit_cast(uint32_t, v[e]) & 0x7FFFFFFFu);
+    }
+    if (smallest >= kSplitSmall && largest <= __builtin_bit_cast(uint32_t, kSplitLarge))
+        return;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
         const int sh = (e & 1) * 16;
-        if (((o[0][e / 2] >> sh) & 0x7F80u) != 0x7F80u)
-            continue;
-        // infinite, not a number, or rounded to infinity
         const uint32_t bits = __builtin_bit_cast(uint32_t, v[e]);
-        float part[3] = {v[e], 0.0f, 0.0f};
-        if ((bits & 0x7F800000u) != 0x7F800000u) {
-            part[0] = __builtin_bit_cast(float, bits & 0xFFFF0000u);
-            part[1] = to_float(to_bf16(v[e] - part[0]));
-            part[2] = v[e] - part[0] - part[1];
-        }
+        if (split_smallest(kSplitNoSum, v[e]) >= kSplitSmall && (bits & 0x7FFFFFFFu) <= __builtin_bit_cast(uint32_t, kSplitLarge))
+            continue;
+        const uint32_t piece[3] = {kWholeWeight, bits >> 16, bits & 0xFFFFu};
 #pragma unroll
         for (int pl = 0; pl < 3; pl++)
-            o[pl][e / 2] = (o[pl][e / 2] & ~(0xFFFFu << sh)) | ((uint32_t)to_bf16(part[pl]).bits << sh);
+            o[pl][e / 2] = (o[pl][e / 2] & ~(0xFFFFu << sh)) | (piece[pl] << sh);
     }
 }
 
@@ -159,6 +164,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
     float rb[8];
     u32x4 ra[A_LD];
+    float largest = 0.0f; // ADIR: of this thread's operands
     auto load_b = [&](int kt) {
         ConstInt *e = ktab + min(kt, a.nkt + 1) * 4; // (tiles past the end of K are never multiplied)
         const uint32_t xoff = (uint32_t)e[0], tap = (uint32_t)e[1];
@@ -181,6 +187,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             const f32x4 lo = __builtin_bit_cast(f32x4, ra[0]), hi = __builtin_bit_cast(f32x4, ra[1]);
             const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             if (BM == 128 || tid < 2 * BM) {
+#pragma unroll
+                for (int e = 0; e < 8; e += 2)
+                    largest = split_largest(largest, v[e], v[e + 1]);
                 split8(v, o);
 #pragma unroll
                 for (int pl = 0; pl < 3; pl++)
@@ -192,12 +201,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                 if (A_PIECES % kThreads == 0 || tid + j * kThreads < A_PIECES)
                     *(u32x4 *)(buf + (tid + j * kThreads) * 16) = ra[j];
         }
+        if (ADIR)
+#pragma unroll
+            for (int i = 0; i < 8; i += 2)
+                largest = split_largest(largest, rb[i], rb[i + 1]);
         split8(rb, o);
 #pragma unroll
         for (int pl = 0; pl < 3; pl++)
             *(u32x4 *)(buf + A_BYTES + ((pl * 2 + half) * BN + p) * 16) = o[pl];
     };
-
     // the five small products are summed on their own: in one accumulator with the large one, every step would round the sum six
     // times as often, at its full size
     f32x16 acc[TM][TN], small[TM][TN];
@@ -276,16 +288,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int j = 0; j < TN; j++)
             acc[i][j] += small[i][j];
 
-    // sums that are not finite: the tile again on the fp32 instruction
+    // sums that are not finite or too small, operands too large: the tile again on the fp32 instruction
     float finite = 0.0f;
+    uint32_t smallest = kSplitNoSum;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++)
+            for (int r = 0; r < 16; r++) {
                 finite = fmaf(acc[i][j][r], 0.0f, finite);
-    if (__syncthreads_or(finite != 0.0f)) { // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+                smallest = split_smallest(smallest, acc[i][j][r]);
+            }
+    if (__syncthreads_or(finite != 0.0f || smallest < kSplitSmallSum || largest > kSplitLarge)) { // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
         clear(acc);
         float *const Af = reinterpret_cast<float *>(smem), *const Bf = Af + BK * BM; // [k][row], [k][pixel]
         for (kt = kt_begin; kt < kt_end; kt++) {
@@ -299,15 +314,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                     for (int e = 0; e < 8; e++)
                         v[e] = __builtin_bit_cast(f32x4, ra[e / 4])[e % 4];
                 } else {
+                    u32x4 o[3];
 #pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        v[e] = 0.0f;
+                    for (int pl = 0; pl < 3; pl++)
+                        o[pl] = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)(((pl * 2 + ahalf) * BM + arow) * 16), soff, 0);
 #pragma unroll
-                    for (int pl = 0; pl < 3; pl++) {
-                        const u32x4 o = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)(((pl * 2 + ahalf) * BM + arow) * 16), soff, 0);
+                    for (int e = 0; e < 8; e++) {
+                        uint32_t piece[3]; // in the upper half
 #pragma unroll
-                        for (int e = 0; e < 8; e++)
-                            v[e] += __builtin_bit_cast(float, (e & 1) ? o[e / 2] & 0xFFFF0000u : o[e / 2] << 16);
+                        for (int pl = 0; pl < 3; pl++)
+                            piece[pl] = (e & 1) ? o[pl][e / 2] & 0xFFFF0000u : o[pl][e / 2] << 16;
+                        v[e] = __builtin_bit_cast(float, piece[0]) + __builtin_bit_cast(float, piece[1]) + __builtin_bit_cast(float, piece[2]);
+                        if (piece[0] == kWholeWeight << 16)
+                            v[e] = __builtin_bit_cast(float, piece[1] | (piece[2] >> 16));
                     }
                 }
 #pragma unroll

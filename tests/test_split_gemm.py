@@ -105,6 +105,40 @@ def test_gpu_split_not_finite(c, packed):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["packed", "raw", "in_place"])
+@pytest.mark.parametrize("c", [(32, 64, 1, 1, 0, 1, 1, 32, 38, 38), (48, 128, 1, 1, 0, 1, 1, 32, 38, 38), (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)],
+                         ids=["64x128", "128x128", "slices"])
+def test_gpu_split_small_operands(c, mode):
+    """operands too small for three bf16 parts (a float below 2^-110 is no multiple of the smallest bf16 number, 2^-133) lose nothing"""
+    gen = torch.Generator().manual_seed(11)
+    xs, ws, ys = _geometry(c)
+    x0, w0 = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+    k = w0[0].numel()
+
+    def check(x, w):
+        got, want = _run(c, x, w, None, mode == "packed", shift=int(mode == "raw")), _conv64(c, x, w, None)
+        scale = _conv64(c, x.abs(), w.abs(), None)
+        # the fp32 instruction rounds once per product; the last bits of 2^-120 lost would show as 2^-15
+        assert ((got - want).abs() <= scale * ((k + 8) * 2.0 ** -24)).all()
+        assert (got - want).norm() <= want.norm() * 2.0 ** -19
+
+    check(x0 * 2.0 ** -120, w0 * 2.0 ** 60)
+    check(x0 * 2.0 ** 60, w0 * 2.0 ** -120)
+    x, w = x0.clone(), w0.clone()
+    x[:, 3] *= 2.0 ** -120  # one channel of the input, as large in the sums as the others
+    w[:, 3] *= 2.0 ** 120
+    check(x, w)
+    x, w = x0.clone(), w0.clone()
+    x[:, 5] *= 2.0 ** 120
+    w[:, 5] *= 2.0 ** -120
+    w[7] *= 2.0 ** -115  # and a filter that is small throughout
+    check(x, w)
+    x = x0.clone()
+    x[1, 2, 3, 4] = 2.0 ** -149  # one operand of one tile: the tile is computed again, its neighbours are not
+    check(x, w0)
+
+
+@pytest.mark.gpu
 def test_gpu_split_other_batches():
     """weights packed at the batch of the settings stay valid at others; a workspace of a smaller batch runs unsplit"""
     c = (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)
@@ -173,6 +207,28 @@ def test_gpu_split_filter_gradient(c):
     first = mine[: cout // g]
     assert (torch.isposinf(first[:, 1]) | torch.isfinite(first[:, 1])).all() and torch.isposinf(first[:, 1]).any()
     assert torch.isnan(first[:, 3]).any() and (torch.isnan(first[:, 3]) | torch.isfinite(first[:, 3])).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(32, 80, 3, 1, 1, 1, 1, 3, 12, 12), (33, 130, 3, 2, 1, 1, 1, 2, 15, 13), (256, 144, 1, 1, 0, 1, 2, 5, 8, 8)], ids=lambda c: "x".join(map(str, c)))
+def test_gpu_split_filter_gradient_small_operands(c):
+    cin, cout, k, s, p, d, g, b, h, wd = c
+    gen = torch.Generator().manual_seed(sum(c))
+    xs, ws, ys = _geometry(c)
+    x0, dy0 = torch.randn(xs, generator=gen), torch.randn(ys, generator=gen)
+    op = dlp.Conv2DBackwardFilter.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs))
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    one_x, one_dy = x0.clone(), dy0.clone()
+    one_x[:, :, h // 2] *= 2.0 ** -120  # one row of the image
+    one_dy[:, 3] *= 2.0 ** -120
+    for x, dy in [(x0 * 2.0 ** -120, dy0 * 2.0 ** 60), (x0 * 2.0 ** 60, dy0 * 2.0 ** -120), (one_x, dy0), (x0, one_dy)]:
+        dw = torch.full(ws, float("nan"), device="cuda:0")
+        op.enqueue(x.cuda(), dw, dy.cuda(), work)
+        grad = lambda x, dy: torch.nn.grad.conv2d_weight(x.double(), ws, dy.double(), s, p, d, g)
+        want, scale = grad(x, dy), grad(x.abs(), dy.abs())
+        err = (dw.cpu().double() - want).abs()
+        assert (err <= scale * ((ys[0] * ys[2] * ys[3] + 8) * 2.0 ** -24)).all()
+        assert (err.norm() <= want.norm() * 2.0 ** -20) and (err[3].norm() <= want[3].norm() * 2.0 ** -20)
 
 
 # (cin, cout, k, stride, pad, create batch, call batch, h, w): gradients and transposed convolutions whose kernel reads the filter as it is
