@@ -231,6 +231,21 @@ def test_gpu_split_filter_gradient_small_operands(c):
         assert (err.norm() <= want.norm() * 2.0 ** -20) and (err[3].norm() <= want[3].norm() * 2.0 ** -20)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 2])
+def test_gpu_filter_gradient_of_single_products(batch):
+    """one product is rounded once, two at most three times, as on the fp32 instruction"""
+    gen = torch.Generator().manual_seed(batch)
+    x, dy = torch.randn((batch, 160, 1, 1), generator=gen), torch.randn((batch, 144, 1, 1), generator=gen)
+    x = torch.cat([x] * 2, 1)[:, :256]
+    op = dlp.Conv2DBackwardFilter.create(dlp.Conv2DSettings(256, 144, 1, 1, 1, 0, 1, tuple(x.shape)))
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    dw = torch.full((144, 256, 1, 1), float("nan"), device="cuda:0")
+    op.enqueue(x.cuda(), dw, dy.cuda(), work)
+    got, terms = dw.cpu().double()[:, :, 0, 0], dy.double()[:, :, 0, 0].unsqueeze(2) * x.double()[:, :, 0, 0].unsqueeze(1)
+    assert ((got - terms.sum(0)).abs() <= terms.abs().sum(0) * (2 * batch - 1) * 2.0 ** -24).all()
+
+
 # (cin, cout, k, stride, pad, create batch, call batch, h, w): gradients and transposed convolutions whose kernel reads the filter as it is
 # from 131072 pixels and at most 32 rows on, and packed tiles below
 @pytest.mark.gpu
