@@ -84,6 +84,7 @@ struct GemmArgs {
     int pxv;                  // bf16 matrix-instruction kernels: pixels per output store (0 = one element per store)
     int pp_nbr;               // conv_patch_bf16_kernel: blocks of PXP rows in the largest patch of the launch
     int wdirect;              // conv_gemm_bf16_kernel: wp is the weight tensor itself (1x1 convolution), not packed tiles
+    int pack_bm, pack_mtiles; // conv_split_f32_kernel: rows and number (per group) of the packed tiles
     int y_cl;                 // bf16 matrix-instruction kernels: y is [image][pixel][channel]
     int Cin, Cin_g, H, W, Cout, OW, OHW, groups;
     int sh, sw, ph, pw, dh, dw, KH, KW;
@@ -2992,8 +2993,9 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
     }
     p.patch_layer = p.patch;
     // fp32 as three bf16 parts (conv_split_f32_kernel), from the size on at which its larger tiles fill the chip.  Counted in tiles of
-    // 64 filters x 128 pixels at the batch of the settings (packed weights stay valid at every other one).  Measured, batch 64 unless
-    // said, filters packed, patch or gathering kernel / 64x128 / 128x128 tiles: 3x3 64->64 at 56x56 120 / 91 / - us, 128->128 at 28x28
+    // 64 filters x 128 pixels at the batch of the call, at most that of the settings (for which workspace and packed weights are laid out):
+    // an operator created at batch 64 and run on one image took 50 us instead of 18 on these kernels (3x3 512->512 at 7x7), 34 instead of
+    // 15 (128->128 at 28x28), 18 instead of 9 (1x1 256->1024 at 14x14).  Measured, batch 64 unless said, filters packed, patch or gathering kernel / 64x128 / 128x128 tiles: 3x3 64->64 at 56x56 120 / 91 / - us, 128->128 at 28x28
     // 114 / 93 / 85, 256->256 at 14x14 111 / 101 / 99, 512->512 at 7x7 112 / 95 / 92, stride 2 64->128 at 56x56 67 / 61 / 51, 1x1
     // 256->64 at 56x56 62 / 55 / -, 64->256 at batch 128 201 / 186 / 166.  Below 350 tiles a launch needs K slices, which only long
     // reductions pay for: 1x1 512->2048 at 7x7, batch 16 (224 tiles x 32 K tiles) 22 / 26 / 28, 5x5 32->64 at 28x28, batch 32
@@ -3001,7 +3003,7 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
     // 39 / 39 / 45.  128x128 tiles want twice as much work: 3x3 128->128 at batch 32 (392 x 72) 63 / 53 / 57, 256->256 at 14x14,
     // batch 40 (248 x 144) 81 / 99 / 69.
     if (g.dtype == DLP_FLOAT && p.order == GEMM_ORDER_TAP && !p.stem && !p.pointwise && p.M > 32) {
-        const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)g.B_hint * g.OH * g.OW + 127) / 128), work = tiles * p.nkt;
+        const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 127) / 128), work = tiles * p.nkt;
         const int rest = p.M % 128;
         const int tile = (rest == 0 || rest > 64) && (tiles >= 700 || work >= 30000) ? 4 : 5;
         const int bm = tile == 4 ? 128 : 64;
@@ -3019,12 +3021,46 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
             p.BN = ts.BN;
         }
     p.mtiles = (p.M + p.BM - 1) / p.BM;
+    p.pack_bm = p.BM;
     p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * BK * p.BM * sizeof(float);
     if (bf16_mfma_order(p.order))
         p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * BK2 * p.BM * sizeof(bf16_t);
     if (p.split)
         p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * p.BM * 96;
     p.wpack_bytes = (p.wpack_bytes + 255) / 256 * 256;
+    return p;
+}
+
+// the plan on the fp32 instruction
+static GemmPlan float_plan(ConvGeom g, int activation)
+{
+    g.B_hint = 0;
+    return conv_gemm_plan(g, activation);
+}
+
+GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation)
+{
+    GemmPackPlan pp;
+    ConvGeom at_hint = g;
+    at_hint.B = g.B_hint;
+    pp.p = conv_gemm_plan(at_hint, activation);
+    pp.bytes = pp.p.wpack_bytes;
+    if (pp.p.split) {
+        pp.floats = float_plan(g, activation);
+        pp.bytes += pp.floats.wpack_bytes;
+    }
+    return pp;
+}
+
+GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPackPlan &pp, size_t &offset)
+{
+    GemmPlan p = conv_gemm_plan(g, activation);
+    offset = 0;
+    if (pp.p.split && p.split) { // (tiles of no more rows than packed ones: the batch is no larger)
+        p.pack_bm = pp.p.BM;
+        p.wpack_bytes = pp.p.wpack_bytes;
+    } else if (pp.p.split)
+        offset = pp.p.wpack_bytes;
     return p;
 }
 
@@ -3109,7 +3145,7 @@ __global__ __launch_bounds__(256) void clear_counters_kernel(int *p, int n)
 } // namespace
 
 int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, void *wpacked, hipStream_t stream, void *part_ws,
-                           size_t part_bytes, int mode, bool counters_owned)
+                           size_t part_bytes, int mode, bool counters_owned, const GemmPlan *floats)
 {
     if (p.wdirect && ((uintptr_t)w & 15) == 0) { // conv_gemm_launch reads w in place: only the counters are left to do
         // (a buffer packed ahead of time is filled all the same: a later call may come with a weight pointer that cannot be read in place)
@@ -3162,7 +3198,8 @@ int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, 
     if (p.split) {
         const int ncb = p.nkt / khw;
         hipLaunchKernelGGL(pack_weights_split_kernel, dim3((unsigned)((long long)g.groups * p.mtiles * ncb * (p.BM / 16))), dim3(256),
-                           16 * (BK * khw + 1) * sizeof(float), stream, p, ncb, khw, ((uintptr_t)w & 15) == 0 ? 1 : 0, (const float *)w, (u32x4 *)wpacked);
+                           16 * (BK * khw + 1) * sizeof(float), stream, p, ncb, khw, ((uintptr_t)w & 15) == 0 ? 1 : 0, (const float *)w, (u32x4 *)wpacked,
+                           floats ? (float *)((char *)wpacked + p.wpack_bytes) : nullptr, floats ? floats->BM : 64, floats ? floats->mtiles : 0);
         if (zero != nullptr)
             hipLaunchKernelGGL(clear_counters_kernel, dim3((unsigned)((nzero + 255) / 256)), dim3(256), 0, stream, zero, nzero);
     } else if ((p.order == GEMM_ORDER_TAP || p.order == GEMM_ORDER_TAP_BF16) && ((uintptr_t)w & 15) == 0) {
@@ -3304,6 +3341,8 @@ int conv_gemm_launch(const ConvGeom &g, const GemmPlan &p, const KTabEntry *dev_
     a.x_bytes = (uint32_t)(x_elems * esize);
     a.wp_bytes = (uint32_t)p.wpack_bytes;
     a.wdirect = 0;
+    a.pack_bm = p.pack_bm;
+    a.pack_mtiles = (p.M + p.pack_bm - 1) / p.pack_bm;
     if (p.wdirect && w != nullptr && ((uintptr_t)w & 15) == 0) { // same test as in conv_gemm_pack_weights
         a.wdirect = 1;
         a.wp = (const float *)w;

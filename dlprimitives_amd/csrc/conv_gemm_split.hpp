@@ -150,16 +150,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         }
     }
     // ---- the weights: 16-byte pieces of the packed tile in order, or (ADIR) eight channels of a row of the weight tensor ----
-    const uint32_t a_tile_bytes = ADIR ? (uint32_t)(BK * 4) : (uint32_t)A_BYTES;
-    const uint32_t a_row_base = ADIR ? 0u : (uint32_t)((g * a.mtiles + mt) * a.nkt) * a_tile_bytes;
+    const uint32_t a_tile_bytes = ADIR ? (uint32_t)(BK * 4) : (uint32_t)(a.pack_bm * 96);
+    const uint32_t a_row_base = ADIR ? 0u : (uint32_t)((g * a.pack_mtiles + m0 / a.pack_bm) * a.nkt) * a_tile_bytes;
     const int arow = tid % BM, ahalf = tid / BM;
+    const int pack_row = m0 % a.pack_bm; // of the packed tile, first row of this one
     uint32_t a_voff[A_LD];
 #pragma unroll
     for (int j = 0; j < A_LD; j++) {
         if (ADIR)
             a_voff[j] = (ahalf < 2 && m0 + arow < a.M) ? (uint32_t)(((g * a.M + m0 + arow) * a.K + 8 * ahalf + 4 * j) * 4) : kOutOfRange;
         else
-            a_voff[j] = tid + j * kThreads < A_PIECES ? (uint32_t)((tid + j * kThreads) * 16) : kOutOfRange;
+            a_voff[j] = tid + j * kThreads < A_PIECES
+                            ? (uint32_t)(((tid + j * kThreads) / BM * a.pack_bm + pack_row + (tid + j * kThreads) % BM) * 16)
+                            : kOutOfRange;
     }
 
     float rb[8];
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                     u32x4 o[3];
 #pragma unroll
                     for (int pl = 0; pl < 3; pl++)
-                        o[pl] = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)(((pl * 2 + ahalf) * BM + arow) * 16), soff, 0);
+                        o[pl] = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)(((pl * 2 + ahalf) * a.pack_bm + pack_row + arow) * 16), soff, 0);
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
                         uint32_t piece[3]; // in the upper half
@@ -354,9 +357,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
 // Weights -> [group][m tile][K tile][piece][half][row][8 channels of one tap], zero padded.  One workgroup moves 16 filters x 16 channels
 // through LDS (read in runs of whole filter rows, 16 bytes per lane where the tensor is aligned); a thread then splits eight channels
-// of a filter at a time.
+// of a filter at a time.  floats: the same weights once more, as tiles of f_bm rows for the kernels on the fp32 instruction.
 __global__ __launch_bounds__(256) void pack_weights_split_kernel(GemmPlan p, int ncb, int khw, int aligned, const float *__restrict__ w,
-                                                                 u32x4 *__restrict__ out)
+                                                                 u32x4 *__restrict__ out, float *__restrict__ floats, int f_bm, int f_mtiles)
 {
     extern __shared__ __align__(16) unsigned char split_smem[];
     float *lds = reinterpret_cast<float *>(split_smem);
@@ -409,6 +412,13 @@ __global__ __launch_bounds__(256) void pack_weights_split_kernel(GemmPlan p, int
 #pragma unroll
         for (int pl = 0; pl < 3; pl++)
             dst[(size_t)pl * 2 * p.BM] = o[pl];
+    }
+    if (floats != nullptr && m_base / f_bm < f_mtiles) { // rows 16 at a time: f_bm is a multiple
+        float *const ftile0 = floats + ((size_t)(g * f_mtiles + m_base / f_bm) * p.nkt + (size_t)cb * khw) * (BK * f_bm) + m_base % f_bm;
+        for (int idx = (int)threadIdx.x; idx < 16 * BK * khw; idx += 256) {
+            const int r = idx % 16, k = (idx / 16) % BK, tap = idx / (16 * BK);
+            ftile0[(size_t)tap * (BK * f_bm) + k * f_bm + r] = lds[r * ld + k * khw + tap];
+        }
     }
 }
 

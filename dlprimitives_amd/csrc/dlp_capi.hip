@@ -266,7 +266,7 @@ __global__ void clear_ints_kernel(int *p, int n)
 }
 } // namespace
 
-// what a packed buffer's layout depends on
+// what a packed buffer's layout depends on (plan of the settings' batch)
 static void layout_of(const GemmPlan &p, int (&sig)[6])
 {
     sig[0] = p.order;
@@ -293,7 +293,9 @@ size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op)
     ConvGeom g;
     if (op->algo != ALGO_GEMM || op_geom(op, op->cfg.shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
         return 0;
-    return round256(conv_gemm_plan(g, op->activation).wpack_bytes);
+    // (either form; a smaller batch needs no more than the settings' one)
+    const GemmPackPlan pp = conv_gemm_pack_plan(g, op->activation);
+    return round256(pp.p.split ? std::max(pp.p.wpack_bytes, pp.floats.wpack_bytes) : pp.p.wpack_bytes);
 }
 
 int conv_fwd_enqueue_tiles(dlp_conv2d_fwd *op, int batch, const GemmPlan &plan, const void *x, const void *tiles, void *y, void *ws, size_t ws_bytes,
@@ -621,7 +623,9 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
         rc = upload_ktab(g, activation, &op->ktab);
         int *unused = nullptr;
         if (rc == DLP_OK) // counters for the batch of the hint, so that a first call inside a stream capture allocates nothing
-            rc = own_counters(op, g, conv_gemm_plan(g, activation), &unused);
+            rc = own_counters(op, g, gplan, &unused);
+        if (rc == DLP_OK && gplan.split) // ... and for the smaller tiles of smaller batches
+            rc = own_counters(op, g, conv_gemm_pack_plan(g, activation).floats, &unused);
     } else if (chosen == ALGO_WINOGRAD) {
         op->wino = winograd_plan(g);
         op->workspace = op->wino.ws_bytes;
@@ -769,7 +773,7 @@ size_t dlp_conv2d_fwd_packed_bytes(const dlp_conv2d_fwd *op)
     ConvGeom g;
     if (op_geom(op, op->cfg.shape, g) != DLP_OK)
         return 0;
-    return round256(conv_gemm_plan(g, op->activation).wpack_bytes);
+    return round256(conv_gemm_pack_plan(g, op->activation).bytes);
 }
 
 int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *stream)
@@ -786,9 +790,9 @@ int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *s
         Epilogue ep = {nullptr, 0.0f, op->activation};
         return winograd_launch(g, op->wino, nullptr, w, nullptr, packed, op->wino.ws_bytes, ep, (hipStream_t)stream, WINO_FILTER_ONLY);
     }
-    const GemmPlan plan = conv_gemm_plan(g, op->activation);
-    layout_of(plan, op->packed_layout);
-    return conv_gemm_pack_weights(g, plan, w, packed, (hipStream_t)stream, nullptr, 0, GEMM_PACK_ONLY);
+    const GemmPackPlan pp = conv_gemm_pack_plan(g, op->activation);
+    layout_of(pp.p, op->packed_layout);
+    return conv_gemm_pack_weights(g, pp.p, w, packed, (hipStream_t)stream, nullptr, 0, GEMM_PACK_ONLY, false, pp.p.split ? &pp.floats : nullptr);
 }
 
 int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], const void *x, const void *w, const void *packed, const void *bias,
@@ -819,9 +823,11 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
     case ALGO_DEPTHWISE:
         return depthwise_launch(g, x, w, y, ep, s);
     default: {
-        const GemmPlan plan = conv_gemm_plan(g, op->activation);
+        const GemmPackPlan pp = conv_gemm_pack_plan(g, op->activation);
+        size_t offset;
+        const GemmPlan plan = conv_gemm_plan_on_packed(g, op->activation, pp, offset);
         int sig[6];
-        layout_of(plan, sig);
+        layout_of(pp.p, sig);
         for (int i = 0; i < 6; i++)
             DLP_REQUIRE(sig[i] == op->packed_layout[i], "the weights were packed for another tile plan (pack again for this batch)");
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
@@ -832,7 +838,7 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
             return rc;
         // fp32 1x1 convolutions could read w in place, but the packed tiles are there and load faster: no w, no in-place reading
         const void *w_arg = (plan.wdirect && plan.order < GEMM_ORDER_TAP_BF16 && !plan.pointwise) ? nullptr : w;
-        return conv_gemm_launch(g, plan, op->ktab, x, packed, y, ep, s, -1, part, ws_bytes, w_arg, counters);
+        return conv_gemm_launch(g, plan, op->ktab, x, (const char *)packed + offset, y, ep, s, -1, part, ws_bytes, w_arg, counters);
     }
     }
 }

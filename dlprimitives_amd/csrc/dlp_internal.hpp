@@ -51,7 +51,7 @@ int dlp_cu_count();
 // Geometry of one forward convolution call (whole tensor, all groups).
 struct ConvGeom {
     int B, Cin, H, W;
-    int B_hint = 0; // batch of the shape an operator was created with: chooses between kernels whose packed weights differ (B may change from call to call)
+    int B_hint = 0; // batch of the shape an operator was created with (B may change from call to call)
     int Cout, OH, OW;
     int KH, KW;
     int sh, sw, ph, pw, dh, dw;
@@ -217,6 +217,7 @@ struct GemmPlan {
     int patch;          // 1: stride-1 "same" convolution run by the LDS-patch kernel (tap-major packed weights)
     int patch_layer;    // 1: the shape is one that the LDS-patch kernel serves, whichever kernel runs it
     int split;          // 1: conv_split_f32_kernel (fp32 as three bf16 parts; tap-major packed weights of its own)
+    int pack_bm;        // ... rows of a packed tile: BM, or 128 where a launch of 64-row tiles runs on weights packed for 128-row ones
     int stem;           // 1: 3-channel 7x7 stride-2 convolution run by conv_stem_f32_kernel (reads the weight tensor in place, nothing is packed)
     int wdirect;        // bf16 matrix-instruction path, 1x1: the kernel reads the weight tensor in place, nothing is packed
     int dense_pxl;      // bf16 matrix-instruction path, 1x1 stride 1 pad 0: input pixels per load of the dense loader (8, 4; 0 = gather)
@@ -230,6 +231,16 @@ struct GemmPlan {
     size_t wpack_bytes; // packed weights [group][m tile][K tile][16][BM] floats, 256-byte rounded
 };
 GemmPlan conv_gemm_plan(const ConvGeom &g, int activation);
+// Weights that are packed once serve every batch: how they are packed, and which part of them a call runs on.  Tiles for
+// conv_split_f32_kernel are followed by tiles for the batches that the fp32 instruction serves.
+struct GemmPackPlan {
+    GemmPlan p;      // of the settings' batch
+    GemmPlan floats; // p.split: of the tiles that follow
+    size_t bytes;
+};
+GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation);
+// plan of a call on weights packed that way, with its tiles `offset` bytes into them
+GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPackPlan &pp, size_t &offset);
 size_t conv_gemm_ktab_entries(const ConvGeom &g);
 // The table layout depends on the geometry AND on the activation the op was created with.
 void conv_gemm_fill_ktab(const ConvGeom &g, int activation, KTabEntry *host_tab);
@@ -242,8 +253,10 @@ size_t conv_gemm_workspace_bytes(const ConvGeom &g, int activation);
 // mode: both steps, the packing alone (weights that stay constant are packed once), or the counters alone.
 enum { GEMM_PACK_AND_CLEAR = 0, GEMM_PACK_ONLY = 1, GEMM_CLEAR_ONLY = 2 };
 // counters_owned: conv_gemm_launch will be given counters of the operator's own (see there): none are cleared here.
+// floats: also write the tiles of this plan behind those of p (GemmPackPlan)
 int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, void *wpacked, hipStream_t stream,
-                           void *part_ws = nullptr, size_t part_bytes = 0, int mode = GEMM_PACK_AND_CLEAR, bool counters_owned = false);
+                           void *part_ws = nullptr, size_t part_bytes = 0, int mode = GEMM_PACK_AND_CLEAR, bool counters_owned = false,
+                           const GemmPlan *floats = nullptr);
 // One phase of a backward-data pass (a stride-1 pass is one phase): the plan of its convolution dy -> dx in this call, where its packed filter goes, and
 // which filter rows and columns it takes: r0 + j * step, in reverse order.
 constexpr int kMaxPhases = 16;

@@ -151,6 +151,44 @@ def test_gpu_split_other_batches():
             assert torch.equal(_run(cb, x, w, None, packed, hint=5), _conv64(cb, x, w, None))  # whole numbers are exact
 
 
+def _kernels(f):
+    """names of the kernels that f launches, without packing"""
+    dlp.timing_enable(True)
+    dlp.timing_reset()
+    try:
+        f()
+        return [k for section, _, k in dlp.timing_records(kernels=True) if section == "conv_gemm"]
+    finally:
+        dlp.timing_enable(False)
+        dlp.timing_reset()
+
+
+# (cin, cout, k, stride, pad, h, batch of the settings, batch of the call): on either side of the lines between the kernels at the
+# call's batch, weights packed for 128 rows run in tiles of 64 and in fp32 tiles (of 64 and of 32 rows, stream and slices)
+OTHER = [(128, 128, 3, 1, 1, 28, 64, 64), (128, 128, 3, 1, 1, 28, 64, 20), (128, 128, 3, 1, 1, 28, 64, 5), (512, 512, 3, 1, 1, 7, 64, 33),
+         (128, 200, 3, 2, 1, 28, 64, 40), (128, 200, 3, 2, 1, 28, 64, 3), (64, 256, 1, 1, 0, 56, 32, 8), (64, 256, 1, 1, 0, 56, 32, 1),
+         (256, 96, 1, 1, 0, 28, 64, 60), (256, 96, 1, 1, 0, 28, 64, 2), (48, 80, 5, 1, 2, 35, 9, 9), (48, 80, 5, 1, 2, 35, 9, 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", OTHER, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("packed", [False, True])
+def test_gpu_kernel_of_the_call_s_batch(c, packed):
+    """an operator runs the kernel at any batch that one created for that batch runs, on weights packed once"""
+    cin, cout, k, s, p, h, hint, batch = c
+    cb = (cin, cout, k, s, p, 1, 1, batch, h, h)
+    gen = torch.Generator().manual_seed(sum(c))
+    xs, ws, _ = _geometry(cb)
+    x, w, bias = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen), torch.randn(cout, generator=gen)
+    out = {}
+    names = {n: _kernels(lambda: out.update({n: _run(cb, x, w, bias, packed, shift=1, hint=n)})) for n in (hint, batch)}
+    assert names[hint] == names[batch] and len(names[hint]) == 1
+    want, scale = _conv64(cb, x, w, bias), _conv64(cb, x.abs(), w.abs(), bias.abs())
+    for n in (hint, batch):
+        # fp32 sums of K products, one rounding each
+        assert ((out[n] - want).abs() <= scale * ((w[0].numel() + 8) * 2.0 ** -24)).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("c", [(48, 64, 3, 2, 1, 1, 1, 24, 79, 81), (40, 32, 4, 2, 1, 1, 1, 3, 18, 22), (64, 48, 3, 1, 1, 1, 2, 33, 40, 40), (20, 16, 5, 3, 2, 1, 1, 2, 17, 19)],
                          ids=lambda c: "x".join(map(str, c)))
