@@ -685,7 +685,9 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
         return depthwise_launch(g, x, w, y, ep, s);
     default: {
         // workspace = packed weights | split-K partial sums
-        const GemmPlan plan = conv_gemm_plan(g, op->activation);
+        GemmPlan plan = conv_gemm_plan(g, op->activation);
+        if (plan.split && ws_bytes < plan.wpack_bytes) // the smaller tiles may still fit
+            plan = conv_gemm_pack_plan(g, op->activation).floats;
         DLP_REQUIRE(ws != nullptr && ws_bytes >= plan.wpack_bytes, "workspace smaller than workspace()");
         const size_t used = round256(plan.wpack_bytes);
         void *part = ws_bytes > used ? (char *)ws + used : nullptr;

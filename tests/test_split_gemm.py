@@ -140,7 +140,7 @@ def test_gpu_split_small_operands(c, mode):
 
 @pytest.mark.gpu
 def test_gpu_split_other_batches():
-    """weights packed at the batch of the settings stay valid at others; a workspace of a smaller batch runs unsplit"""
+    """weights packed at the batch of the settings stay valid at others"""
     c = (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)
     gen = torch.Generator().manual_seed(6)
     for batch in (1, 4, 9):
@@ -187,6 +187,40 @@ def test_gpu_kernel_of_the_call_s_batch(c, packed):
     for n in (hint, batch):
         # fp32 sums of K products, one rounding each
         assert ((out[n] - want).abs() <= scale * ((w[0].numel() + 8) * 2.0 ** -24)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("c", [(512, 512, 3, 1, 1, 7, 64), (128, 128, 3, 1, 1, 28, 64), (64, 128, 3, 2, 1, 56, 64), (256, 512, 3, 2, 1, 14, 64), (1024, 256, 1, 1, 0, 14, 64),
+                               (48, 80, 5, 1, 2, 21, 33)], ids=lambda c: "x".join(map(str, c)))
+def test_gpu_slices_of_the_call_s_batch(c, packed):
+    """a workspace sized for the batch of the settings has room for the K slices of every smaller one: the same bits as from an operator
+    created for that batch (another cut adds up in another order)"""
+    cin, cout, k, s, p, h, hint = c
+    gen = torch.Generator().manual_seed(sum(c))
+    for batch in sorted({1, 2, 3, 5, 8, 12, 16, 21, hint // 2, hint - 9, hint - 1}):
+        cb = (cin, cout, k, s, p, 1, 1, batch, h, h)
+        xs, ws, _ = _geometry(cb)
+        x, w = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+        assert torch.equal(_run(cb, x, w, None, packed, hint=hint), _run(cb, x, w, None, packed)), batch
+
+
+@pytest.mark.gpu
+def test_gpu_split_small_workspaces():
+    """as many K slices as there is room for, fp32 tiles where the split ones find none, an error below that"""
+    c = (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)
+    gen = torch.Generator().manual_seed(3)
+    xs, ws, ys = _geometry(c)
+    x, w = torch.randint(-4, 5, xs, generator=gen).float(), torch.randint(-4, 5, ws, generator=gen).float()
+    want = _conv64(c, x, w, None)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(192, 96, 3, 1, 1, 1, 1, xs), False, "identity", "gemm")
+    floats, split = 2 * 108 * 16 * 64 * 4, 2 * 108 * 64 * 96  # two row tiles of 108 K tiles
+    for size in (op.workspace(), op.workspace() - 256, split + (op.workspace() - split) // 2, split + 200000, split, split - 256, floats):
+        y = torch.full(ys, float("nan"), device="cuda:0")
+        op.enqueue(x.cuda(), w.cuda(), None, y, torch.empty(size, dtype=torch.uint8, device="cuda:0"))
+        assert torch.equal(y.cpu().double(), want), size  # whole numbers are exact
+    with pytest.raises(dlp.DlprimError):
+        op.enqueue(x.cuda(), w.cuda(), None, y, torch.empty(floats - 256, dtype=torch.uint8, device="cuda:0"))
 
 
 @pytest.mark.gpu
