@@ -270,20 +270,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
                         }
             }
         }
-        uint32_t smallest = kSplitNoSum;
         float finite = 0.0f; // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+        bool small_sum = false;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 acc[i][j] += small[i][j];
+                float v[16];
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    finite = fmaf(acc[i][j][r], 0.0f, finite);
-                    smallest = split_smallest(smallest, acc[i][j][r]);
+                    v[r] = acc[i][j][r];
+                    finite = fmaf(v[r], 0.0f, finite);
                 }
+                small_sum |= split_small_sum(v);
             }
-        in_floats = __syncthreads_or(finite != 0.0f || smallest < kSplitSmallSum || largest > kSplitLarge);
+        in_floats = __syncthreads_or(finite != 0.0f || small_sum || largest > kSplitLarge);
         if (in_floats) {
 #pragma unroll
             for (int i = 0; i < TM; i++)

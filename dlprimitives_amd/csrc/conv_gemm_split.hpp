@@ -292,18 +292,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             acc[i][j] += small[i][j];
 
     // sums that are not finite or too small, operands too large: the tile again on the fp32 instruction
-    float finite = 0.0f;
-    uint32_t smallest = kSplitNoSum;
+    float finite = 0.0f; // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+    bool small_sum = false;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++) {
+            float v[16];
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                finite = fmaf(acc[i][j][r], 0.0f, finite);
-                smallest = split_smallest(smallest, acc[i][j][r]);
+                v[r] = acc[i][j][r];
+                finite = fmaf(v[r], 0.0f, finite);
             }
-    if (__syncthreads_or(finite != 0.0f || smallest < kSplitSmallSum || largest > kSplitLarge)) { // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+            small_sum |= split_small_sum(v);
+        }
+    if (__syncthreads_or(finite != 0.0f || small_sum || largest > kSplitLarge)) {
         clear(acc);
         float *const Af = reinterpret_cast<float *>(smem), *const Bf = Af + BK * BM; // [k][row], [k][pixel]
         for (kt = kt_begin; kt < kt_end; kt++) {

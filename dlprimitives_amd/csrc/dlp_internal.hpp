@@ -150,6 +150,22 @@ __device__ __forceinline__ uint32_t split_smallest(uint32_t smallest, float v)
 {
     return min(smallest, 2u * __builtin_bit_cast(uint32_t, v) - 1u);
 }
+// whether there is a sum among the N that is not zero and too small.  Half an instruction for each where none is zero.
+template <int N>
+__device__ __forceinline__ bool split_small_sum(const float (&v)[N])
+{
+    float low = 1.0f;
+#pragma unroll
+    for (int e = 0; e < N; e += 2)
+        asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(v[e]), "v"(v[e + 1]));
+    if (low >= 0x1p-72f)
+        return false;
+    uint32_t smallest = kSplitNoSum;
+#pragma unroll
+    for (int e = 0; e < N; e++)
+        smallest = split_smallest(smallest, v[e]);
+    return smallest < kSplitSmallSum;
+}
 __device__ __forceinline__ float split_largest(float largest, float v, float w) // one instruction; fmaxf would quiet each operand first
 {
     asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(v), "v"(w));
