@@ -160,7 +160,7 @@ __device__ __forceinline__ void static_for_all(F &&f)
     f(std::integral_constant<int, 7>{});
 }
 
-template <class T, int BM, int BN, int WM, int WN, int ACT>
+template <class T, int BM, int BN, int WM, int WN, int ACT, bool RAGGED = false>
 __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc)[BM / WM / 32][BN / WN / 32], float *lds, int m0, int n0,
                                                  int g, int slice, int splitk, uint32_t image0, int wm, int wn, int h, int l32, int tid,
                                                  const float *bias_s);
@@ -471,7 +471,8 @@ __global__ __launch_bounds__(kThreads) void conv_gemm_f32_kernel(GemmArgs a)
 // epilogue (bias, activation, factor) and the NCHW store.  `lds` is LDS that is free after the
 // last barrier of the main loop (at least BM floats).  `bias_s`: the bias of the tile's BM rows in LDS (zero past M), staged by the
 // kernel when it starts on the tile: requested here, its trip to memory stood between the last matrix instruction and the first store.
-template <class T, int BM, int BN, int WM, int WN, int ACT>
+// RAGGED: built for M off multiples of 8 too (a kernel of its own: as one more copy of the stores it cost the other launches up to 10 %).
+template <class T, int BM, int BN, int WM, int WN, int ACT, bool RAGGED>
 __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc)[BM / WM / 32][BN / WN / 32], float *lds, int m0, int n0,
                                                  int g, int slice, int splitk, uint32_t image0, int wm, int wn, int h, int l32, int tid,
                                                  const float *bias_s)
@@ -571,15 +572,14 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
     }
 
     // ---- epilogue: bias, activation, factor, NCHW store ----
-    // Fast path (no factor, M a multiple of 8, y below 2 GiB): the bias of the tile's rows goes
-    // through LDS (free after the last barrier) and the stores are buffer stores whose row offset
-    // is scalar, instead of a bias load and 64-bit address arithmetic per value.
+    // Fast path (float, or no factor; M a multiple of 8 or RAGGED; y below 2 GiB): the bias of the tile's rows has gone through LDS and the stores are buffer
+    // stores whose row offset is scalar, instead of a bias load and 64-bit address arithmetic per value.
     const bool pre = a.pre != 0 && a.factor != 0.0f;
-    if ((a.factor == 0.0f || (pre && sizeof(T) == 4)) && (a.M & 7) == 0 && a.y_bytes != 0) {
+    if ((a.factor == 0.0f || sizeof(T) == 4) && (RAGGED || (a.M & 7) == 0) && a.y_bytes != 0) {
         const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, a.y_bytes, 0x00020000);
         const bool clamp = a.act != DLP_ACT_IDENTITY;
-        auto store_all = [&](auto pre_c) {
-            constexpr bool PRE = decltype(pre_c)::value;
+        auto store_all = [&](auto sum_c) {
+            constexpr int SUM = decltype(sum_c)::value; // factor * y: 0 none, 1 added before the activation, 2 behind it
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const int n = n0 + wn * WTN + j * 32 + l32;
@@ -590,7 +590,7 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
                 // the old values of all the column's rows are requested before the first is used: one by one, each waited for its own trip
                 // to memory (64->256 1x1 at 56x56 with its residual sum, batch 16, in tiles of 128x128: 56 -> 33 us)
                 float old[TM][16];
-                if (PRE) {
+                if (SUM) {
 #pragma unroll
                     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -607,30 +607,40 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
                         if (m0 + mrow >= a.M)
                             continue;
                         const f32x4 bv = *(const f32x4 *)&bias_s[mrow + 4 * h];
+                        uint32_t vr[4] = {voff, voff, voff, voff};
+                        if (RAGGED)
+#pragma unroll
+                            for (int rr = 0; rr < 4; rr++)
+                                vr[rr] = m0 + mrow + 4 * h + rr < a.M ? voff : kOutOfRange;
 #pragma unroll
                         for (int rr = 0; rr < 4; rr++) {
                             float v = acc[i][j][4 * rq + rr] + bv[rr];
                             const uint32_t soff = (uint32_t)((i * 32 + 8 * rq + rr) * a.OHW * (int)sizeof(T));
-                            if (PRE)
+                            if (SUM == 1)
                                 v = fmaf(old[i][4 * rq + rr], a.factor, v);
                             if (ACT == ACT_CLAMP) {
                                 if (clamp) // identity must keep NaNs: no min/max
                                     v = clamp_med3(v, a.clamp_lo, a.clamp_hi);
                             } else
                                 v = apply_act(v, a.act);
+                            if (SUM == 2)
+                                v = fmaf(old[i][4 * rq + rr], a.factor, v);
                             if (sizeof(T) == 4)
-                                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr, voff, soff, 0);
+                                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yr, vr[rr], soff, 0);
                             else
-                                __builtin_amdgcn_raw_buffer_store_b16((short)to_bf16(v).bits, yr, voff, soff, 0);
+                                __builtin_amdgcn_raw_buffer_store_b16((short)to_bf16(v).bits, yr, vr[rr], soff, 0);
                         }
                     }
                 }
             }
         };
-        if (pre) // (two copies: the test alone, inside the loops, cost launches without a sum 1.5 %)
-            store_all(std::true_type{});
+        // (copies: the test alone, inside the loops, cost launches without a sum 1.5 %)
+        if (a.factor == 0.0f)
+            store_all(std::integral_constant<int, 0>{});
+        else if (pre)
+            store_all(std::integral_constant<int, 1>{});
         else
-            store_all(std::false_type{});
+            store_all(std::integral_constant<int, 2>{});
         return;
     }
     // accumulator register r of a 32x32 block holds row 8*(r/4) + 4*h + r%4, column l32
@@ -2845,13 +2855,13 @@ int launch_patch(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t 
     return DLP_OK;
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, bool RAGGED>
 void launch_split_inst(TimingScope &ts, const GemmArgs &a, unsigned blocks, hipStream_t stream)
 {
     if (a.wdirect)
-        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, true>), dim3(blocks), dim3(kThreads), 0, stream, a);
+        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, true, RAGGED>), dim3(blocks), dim3(kThreads), 0, stream, a);
     else
-        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, false>), dim3(blocks), dim3(kThreads), 0, stream, a);
+        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, false, RAGGED>), dim3(blocks), dim3(kThreads), 0, stream, a);
 }
 
 int launch_split(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t stream)
@@ -2861,10 +2871,15 @@ int launch_split(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t 
         return fail(DLP_ERR_NOT_IMPLEMENTED, "convolution too large for a single launch");
     {
         TimingScope ts("conv_gemm", stream);
-        if (p.tile == 4)
-            launch_split_inst<128, 128, 2, 2>(ts, a, (unsigned)blocks, stream);
+        const bool ragged = (a.M & 7) != 0;
+        if (p.tile == 4 && ragged)
+            launch_split_inst<128, 128, 2, 2, true>(ts, a, (unsigned)blocks, stream);
+        else if (p.tile == 4)
+            launch_split_inst<128, 128, 2, 2, false>(ts, a, (unsigned)blocks, stream);
+        else if (ragged)
+            launch_split_inst<64, 128, 1, 4, true>(ts, a, (unsigned)blocks, stream);
         else
-            launch_split_inst<64, 128, 1, 4>(ts, a, (unsigned)blocks, stream);
+            launch_split_inst<64, 128, 1, 4, false>(ts, a, (unsigned)blocks, stream);
     }
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;

@@ -66,7 +66,7 @@ __device__ __forceinline__ void split8_weights(const float *v, u32x4 (&o)[3])
     }
 }
 
-template <int BM, int BN, int WM, int WN, bool ADIR>
+template <int BM, int BN, int WM, int WN, bool ADIR, bool RAGGED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_split_f32_kernel(GemmArgs a)
 {
     static_assert(WM * WN == 4 && BN == 128 && (BM == 64 || BM == 128), "tile shape");
@@ -354,8 +354,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             __syncthreads();
         }
     }
-    gemm_tile_output<float, BM, BN, WM, WN, ACT_CLAMP>(a, acc, reinterpret_cast<float *>(smem), m0, n0, g, slice, splitk, image0, wm, wn, h, l32, tid,
-                                                       bias_early);
+    gemm_tile_output<float, BM, BN, WM, WN, ACT_CLAMP, RAGGED>(a, acc, reinterpret_cast<float *>(smem), m0, n0, g, slice, splitk, image0, wm, wn, h,
+                                                               l32, tid, bias_early);
 }
 
 // Weights -> [group][m tile][K tile][piece][half][row][8 channels of one tap], zero padded.  One workgroup moves 16 filters x 16 channels

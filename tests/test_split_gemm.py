@@ -12,10 +12,12 @@ def _geometry(c):
     return (b, cin, h, w), (cout, cin // g, k, k), (b, cout, oh, ow)
 
 
-def _run(c, x, w, bias, packed, act="identity", factor=0.0, y0=None, shift=0, hint=None):
+def _run(c, x, w, bias, packed, act="identity", factor=0.0, y0=None, shift=0, hint=None, first=False):
     cin, cout, k, s, p, d, g, b, h, wd = c
     xs, ws_, ys = _geometry(c)
     op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, ((hint or b),) + xs[1:]), bias is not None, act, "gemm")
+    if first:
+        op.accumulate_before_activation(True)
     wbuf = torch.empty(w.numel() + shift, device="cuda:0")  # shift: a weight tensor off its 16-byte boundary
     wbuf[shift:].copy_(w.reshape(-1))
     wdev = wbuf[shift:].view(ws_)
@@ -75,6 +77,23 @@ def test_gpu_split_parity(c, packed):
     got = _run(c, x, w, None, packed, "relu", 0.5, old)
     want = _conv64(c, x, w, None).relu() + 0.5 * old.double()
     assert ((got - want).abs() <= (scale + old.abs()) * bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["identity", "relu", "relu6"])
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("c", [(16, 64, 1, 1, 0, 1, 1, 32, 38, 38), (48, 248, 1, 1, 0, 1, 1, 32, 38, 38), (16, 33, 1, 1, 0, 1, 1, 47, 31, 33), (64, 500, 1, 1, 0, 1, 2, 33, 38, 38),
+                               (32, 100, 3, 1, 1, 1, 1, 3, 9, 11)], ids=lambda c: "x".join(map(str, c)))
+def test_gpu_residual_sums(c, first, act):
+    """factor * y before and behind the activation: rows in whole eights and not, tiles of 64 and 128 rows, the fp32 instruction (last)"""
+    gen = torch.Generator().manual_seed(sum(c))
+    xs, ws, ys = _geometry(c)
+    x, w, bias = torch.randint(-3, 4, xs, generator=gen).float(), torch.randint(-3, 4, ws, generator=gen).float(), torch.randint(-9, 10, (c[1],), generator=gen).float()
+    old = torch.randint(-9, 10, ys, generator=gen).float()
+    f = {"identity": lambda t: t, "relu": torch.relu, "relu6": lambda t: t.clamp(0, 6)}[act]
+    conv = _conv64(c, x, w, bias)
+    want = f(conv - 2 * old.double()) if first else f(conv) - 2 * old.double()
+    assert torch.equal(_run(c, x, w, bias, True, act, -2.0, old, first=first), want)  # whole numbers are exact
 
 
 @pytest.mark.gpu
