@@ -458,7 +458,11 @@ __global__ __launch_bounds__(256) void channel_affine_kernel(size_t packs, int C
 
 // Softmax over dimension 1 of x[B][C][S] (S = 1 for a matrix): one wavefront per (b, s) column;
 // max, sum of exp(x - max), then exp(x - max) / sum or, for the log variant, x - max - log(sum).
-template <class T>
+// NV: up to NV * 64 classes stay in registers: all of a lane's loads are on their way at once and the exponentials are taken once.  0: loops
+// that wait for memory three times over, element by element (16 x 1000: 11.5 us, nearly all of it that wait; 5.0 us so).  The same
+// operations in the same order, the same bits.  NV no larger than the classes ask for: with 16 for all, 2 classes of 4 x 512 x 512 took
+// 275 us instead of 251 in loops (bf16 291 instead of 256).
+template <class T, int NV>
 __global__ __launch_bounds__(256) void softmax_kernel(int B, int C, int S, int log_softmax, const T *__restrict__ x, T *__restrict__ y)
 {
     const int lane = threadIdx.x & 63;
@@ -469,11 +473,7 @@ __global__ __launch_bounds__(256) void softmax_kernel(int B, int C, int S, int l
     const T *xp = x + ((size_t)b * C) * S + sp;
     T *yp = y + ((size_t)b * C) * S + sp;
     float m = -3.402823466e+38f;
-    // Up to 1024 classes stay in registers: all of a lane's loads are on their way at once and the exponentials are taken once.  The loops
-    // below wait for memory three times over, element by element: 16 x 1000 took 11.5 us, nearly all of it that wait (5.0 us so).  The same
-    // operations in the same order, the same bits.
-    constexpr int NV = 16;
-    if (C <= NV * 64) {
+    if constexpr (NV > 0) {
         float v[NV];
 #pragma unroll
         for (int q = 0; q < NV; q++)
@@ -500,27 +500,27 @@ __global__ __launch_bounds__(256) void softmax_kernel(int B, int C, int S, int l
         for (int q = 0; q < NV; q++)
             if (lane + 64 * q < C)
                 store_plain(yp + (size_t)(lane + 64 * q) * S, log_softmax ? v[q] + shift : v[q] * inv);
-        return;
-    }
-    for (int j = lane; j < C; j += 64)
-        m = fmaxf(m, to_float(xp[(size_t)j * S]));
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-        m = fmaxf(m, __shfl_xor(m, off));
-    float sum = 0.0f;
-    for (int j = lane; j < C; j += 64)
-        sum += expf(to_float(xp[(size_t)j * S]) - m);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-        sum += __shfl_xor(sum, off);
-    if (log_softmax) {
-        const float shift = -m - logf(sum);
-        for (int j = lane; j < C; j += 64)
-            store_plain(yp + (size_t)j * S, to_float(xp[(size_t)j * S]) + shift);
     } else {
-        const float inv = 1.0f / sum;
         for (int j = lane; j < C; j += 64)
-            store_plain(yp + (size_t)j * S, expf(to_float(xp[(size_t)j * S]) - m) * inv);
+            m = fmaxf(m, to_float(xp[(size_t)j * S]));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1)
+            m = fmaxf(m, __shfl_xor(m, off));
+        float sum = 0.0f;
+        for (int j = lane; j < C; j += 64)
+            sum += expf(to_float(xp[(size_t)j * S]) - m);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1)
+            sum += __shfl_xor(sum, off);
+        if (log_softmax) {
+            const float shift = -m - logf(sum);
+            for (int j = lane; j < C; j += 64)
+                store_plain(yp + (size_t)j * S, to_float(xp[(size_t)j * S]) + shift);
+        } else {
+            const float inv = 1.0f / sum;
+            for (int j = lane; j < C; j += 64)
+                store_plain(yp + (size_t)j * S, expf(to_float(xp[(size_t)j * S]) - m) * inv);
+        }
     }
 }
 
@@ -876,12 +876,22 @@ int dlp_softmax_fwd_enqueue(int dtype, int log_softmax, int batch, int classes, 
     DLP_REQUIRE((cols + 3) / 4 < (1ll << 31), "too many columns");
     hipStream_t st = (hipStream_t)stream;
     TimingScope ts("softmax", st);
-    if (dtype == DLP_BFLOAT16)
-        hipLaunchKernelGGL(softmax_kernel<bf16_t>, dim3((unsigned)((cols + 3) / 4)), dim3(256), 0, st, batch, classes, inner, log_softmax,
-                           (const bf16_t *)x, (bf16_t *)y);
+    const dim3 grid((unsigned)((cols + 3) / 4));
+    auto launch = [&](auto nv) {
+        constexpr int NV = decltype(nv)::value;
+        if (dtype == DLP_BFLOAT16)
+            hipLaunchKernelGGL((softmax_kernel<bf16_t, NV>), grid, dim3(256), 0, st, batch, classes, inner, log_softmax, (const bf16_t *)x, (bf16_t *)y);
+        else
+            hipLaunchKernelGGL((softmax_kernel<float, NV>), grid, dim3(256), 0, st, batch, classes, inner, log_softmax, (const float *)x, (float *)y);
+    };
+    if (classes <= 64)
+        launch(std::integral_constant<int, 1>{});
+    else if (classes <= 256)
+        launch(std::integral_constant<int, 4>{});
+    else if (classes <= 1024)
+        launch(std::integral_constant<int, 16>{});
     else
-        hipLaunchKernelGGL(softmax_kernel<float>, dim3((unsigned)((cols + 3) / 4)), dim3(256), 0, st, batch, classes, inner, log_softmax,
-                           (const float *)x, (float *)y);
+        launch(std::integral_constant<int, 0>{});
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
 }

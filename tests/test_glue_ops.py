@@ -422,3 +422,26 @@ def test_gpu_softmax_in_registers(shape, log):
     want = torch.log_softmax(x.double(), 1) if log else torch.softmax(x.double(), 1)
     # the exponent is off by half a unit of its largest difference (2^7 * 2^-24), the sum by a rounding per step of 16 + 6
     np.testing.assert_allclose(y.cpu().double().numpy(), want.numpy(), rtol=2.0 ** -16, atol=2.0 ** -120)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(5, 256), (5, 257), (3, 2, 50), (2, 64, 9), (7, 3)], ids=str)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_gpu_softmax_registers_per_lane(shape, dtype):
+    """class counts around the lines between one, four and sixteen registers a lane, few classes of many pixels"""
+    import torch
+
+    import dlprimitives_amd as dlp
+
+    dt = getattr(torch, dtype)
+    x = (torch.randn(shape, generator=torch.Generator().manual_seed(sum(shape))) * 4).to(dt)
+    y = torch.full(shape, float("nan"), dtype=dt, device="cuda:0")
+    half = 2.0 ** -24 if dtype == "float32" else 2.0 ** -8  # half a unit in the last of 24 or 8 significant bits
+    dlp.softmax_forward(x.cuda(), y, False)
+    want = torch.softmax(x.double(), 1)
+    np.testing.assert_allclose(y.cpu().double().numpy(), want.numpy(), rtol=2.0 ** -16 + half, atol=2.0 ** -120)  # as above, rounded for storage
+    dlp.softmax_forward(x.cuda(), y, True)
+    want = torch.log_softmax(x.double(), 1)
+    # x + (-max - log(sum)): one rounding each of two terms no larger than 2 * max|x| + log(classes), and the logarithm's own
+    largest = 2 * float(x.abs().max()) + 8
+    np.testing.assert_allclose(y.cpu().double().numpy(), want.numpy(), rtol=half, atol=3 * largest * 2.0 ** -24)
