@@ -245,10 +245,10 @@ def test_gpu_bias_backward(oracle_mod):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("batch,features,h,w", [(1, 1, 1, 1), (0, 3, 4, 4), (3, 5, 1, 1), (7, 3, 7, 7), (4, 2, 64, 64), (5, 2, 64, 64), (17, 3, 31, 33), (9, 2, 113, 51)])
+@pytest.mark.parametrize("batch,features,h,w", [(1, 1, 1, 1), (0, 3, 4, 4), (3, 5, 1, 1), (65, 2, 1, 1), (4, 3, 8, 8), (64, 2, 1, 1), (7, 3, 7, 7), (4, 2, 64, 64), (5, 2, 64, 64), (17, 3, 31, 33), (9, 2, 113, 51)])
 @pytest.mark.parametrize("shifted", [False, True])
 def test_gpu_bias_backward_walk(batch, features, h, w, shifted):
-    """planes of whole 16-byte pieces and others, 4096 elements per feature (the last with 256 threads) and above, an unaligned dy"""
+    """planes of whole 16-byte pieces and others, runs of 64 (the last with 64 threads) and 4096 (with 256) and above, an unaligned dy"""
     import torch
 
     import dlprimitives_amd as dlp
