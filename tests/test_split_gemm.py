@@ -12,7 +12,7 @@ def _geometry(c):
     return (b, cin, h, w), (cout, cin // g, k, k), (b, cout, oh, ow)
 
 
-def _run(c, x, w, bias, packed, act="identity", factor=0.0, y0=None, shift=0, hint=None, first=False):
+def _run(c, x, w, bias, packed, act="identity", factor=0.0, y0=None, shift=0, hint=None, first=False, room=None):
     cin, cout, k, s, p, d, g, b, h, wd = c
     xs, ws_, ys = _geometry(c)
     op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, ((hint or b),) + xs[1:]), bias is not None, act, "gemm")
@@ -22,7 +22,7 @@ def _run(c, x, w, bias, packed, act="identity", factor=0.0, y0=None, shift=0, hi
     wbuf[shift:].copy_(w.reshape(-1))
     wdev = wbuf[shift:].view(ws_)
     y = torch.full(ys, float("nan"), device="cuda:0") if y0 is None else y0.float().cuda()
-    ws = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    ws = torch.empty(max(op.workspace(), 1) if room is None else room, dtype=torch.uint8, device="cuda:0")
     bd = None if bias is None else bias.float().cuda()
     if packed:
         buf = torch.empty(max(op.packed_size(), 1), dtype=torch.uint8, device="cuda:0")
@@ -39,6 +39,26 @@ def _conv64(c, x, w, bias):
     return torch.nn.functional.conv2d(x.double(), w.double(), None if bias is None else bias.double(), s, p, d, g)
 
 
+def _kernels(f):
+    """names of the kernels that f launches, without packing"""
+    dlp.timing_enable(True)
+    dlp.timing_reset()
+    try:
+        f()
+        return [k for section, _, k in dlp.timing_records(kernels=True) if section == "conv_gemm"]
+    finally:
+        dlp.timing_enable(False)
+        dlp.timing_reset()
+
+
+def _tile(names):
+    """rows of the tiles of the one launch, which is one of conv_split_f32_kernel<rows, pixels, wavefronts, weights in place, ..>"""
+    (name,) = names
+    assert name.startswith("conv_split_f32_kernel<"), name
+    args = name[name.index("<") + 1:].split(", ")
+    return int(args[0]), args[4] == "true"
+
+
 # every one large enough for these kernels: 350 tiles of 64 filters x 128 pixels, or 20000 K tiles in all
 # (cin, cout, k, stride, pad, dilate, groups, batch, h, w)
 CASES = [
@@ -46,7 +66,7 @@ CASES = [
     (16, 33, 1, 1, 0, 1, 1, 47, 31, 33),     # rows and pixels off the tile
     (32, 80, 1, 2, 0, 1, 1, 90, 31, 33),     # two tiles of 64 rows, the second mostly empty; strided
     (48, 128, 1, 1, 0, 1, 1, 32, 38, 38),    # 128x128 tiles, three K tiles
-    (16, 200, 3, 1, 1, 1, 1, 20, 31, 30),    # rows off 128, taps outside the image
+    (16, 200, 3, 1, 1, 1, 1, 20, 31, 30),    # rows off 64, taps outside the image
     (16, 97, 3, 2, 1, 1, 1, 64, 39, 41),
     (64, 64, 3, 1, 1, 1, 1, 16, 53, 53),     # a last round of few tiles, cut into K slices
     (192, 96, 3, 1, 1, 1, 1, 5, 61, 43),     # K slices throughout
@@ -54,29 +74,93 @@ CASES = [
     (32, 48, 5, 1, 4, 2, 1, 40, 31, 33),     # dilation
     (64, 320, 3, 1, 1, 1, 4, 9, 33, 31),     # groups
     (16, 40, 5, 3, 0, 1, 1, 81, 75, 75),
+    (64, 128, 3, 1, 1, 1, 1, 16, 53, 53),    # 128x128 tiles: filter taps outside the image
+    (32, 200, 3, 1, 1, 1, 1, 25, 31, 30),    # ... rows off 128
+    (256, 96, 3, 1, 1, 1, 1, 10, 37, 37),    # ... K slices, rows off 128
+    (128, 512, 1, 1, 0, 1, 4, 16, 33, 33),   # ... groups
+    (64, 160, 1, 1, 0, 1, 2, 21, 33, 33),    # ... groups whose rows are off 128
 ]
+ROWS = {c: 128 for c in CASES[-5:]}
+ROWS[(48, 128, 1, 1, 0, 1, 1, 32, 38, 38)] = 128
+SLICES = {(64, 64, 3, 1, 1, 1, 1, 16, 53, 53), (64, 128, 3, 1, 1, 1, 1, 16, 53, 53), (32, 48, 5, 1, 4, 2, 1, 40, 31, 33), (192, 96, 3, 1, 1, 1, 1, 5, 61, 43),
+          (640, 128, 3, 1, 1, 1, 1, 5, 27, 27), (256, 96, 3, 1, 1, 1, 1, 10, 37, 37)}
+
+
+def _bounds(want, scale, k):
+    """elementwise and in the 2-norm"""
+    # a product is off by 2^-23 at most; the sums, none above sum |x||w|, round by 2^-24 of themselves once per four k and a few times behind
+    each = scale * ((k / 4 + 8) * 2.0 ** -24)
+    # roundings of either sign add up as their squares: sqrt(K / 4) of them, each a third of 2^-24 or so of a sum that has grown to sqrt(K)
+    # products, stay below 2^-22 of the result up to K = 6000; a piece too few would show as 2^-17, a lost small product as 2^-17 to 2^-9
+    return each, want.norm() * 2.0 ** -22
+
+
+def _parts(t):
+    """a float as three bf16 numbers, as the kernels cut it"""
+    out = []
+    rest = t.float()
+    for _ in range(3):
+        out.append(rest.bfloat16().float())
+        rest = rest - out[-1]
+    assert not rest.any()
+    return [p.double() for p in out]
+
+
+def test_bounds_see_a_lost_product():
+    """the parity bounds hold for the six products of the kernels and for no five of them, nor with two parts exchanged"""
+    gen = torch.Generator().manual_seed(1)
+    kept = [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)]
+    for k in (16, 144, 1728):
+        a, b = torch.randn((96, k), generator=gen), torch.randn((k, 80), generator=gen)
+        pa, pb = _parts(a), _parts(b)
+        want, scale = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+        each, norm = _bounds(want, scale, k)
+        holds = lambda pairs: bool(((sum(pa[i] @ pb[j] for i, j in pairs) - want).abs() <= each).all()) and (sum(pa[i] @ pb[j] for i, j in pairs) - want).norm() <= norm
+        assert holds(kept)
+        for lost in kept:
+            assert not holds([p for p in kept if p != lost])
+        assert not holds([(0, 0), (0, 2), (1, 0), (1, 2), (0, 1), (2, 0)])  # second and third part of b in each other's place
+
+
+def test_parts_of_small_floats():
+    """three bf16 numbers hold a float from 2^-110 on, below it they lose bits"""
+    gen = torch.Generator().manual_seed(2)
+    t = (torch.rand(4096, generator=gen) + 1) * torch.where(torch.rand(4096, generator=gen) < 0.5, -1.0, 1.0)
+    for e in (-110, -100, 0, 126):
+        x = t * 2.0 ** e
+        assert torch.equal(sum(_parts(x)), x.double())
+    lost = 0
+    rest = t * 2.0 ** -111
+    for _ in range(3):
+        rest = rest - rest.bfloat16().float()
+    assert rest.any()
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", CASES, ids=lambda c: "x".join(map(str, c)))
-@pytest.mark.parametrize("packed", [False, True])
-def test_gpu_split_parity(c, packed):
+@pytest.mark.parametrize("mode,c", [(m, c) for m in ("packed", "raw", "in_place") for c in CASES if m != "in_place" or c[2] == 1],  # 1x1: read in place
+                         ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_gpu_split_parity(mode, c):
+    packed, shift = mode == "packed", int(mode == "raw")
     gen = torch.Generator().manual_seed(sum(c))
     xs, ws, ys = _geometry(c)
     x, w, bias = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen), torch.randn(c[1], generator=gen)
     want = _conv64(c, x, w, bias)
-    got = _run(c, x, w, bias, packed, shift=0 if packed else 1)
-    # a product is off by 2^-23 at most; the sums, none above sum |x||w|, round by 2^-24 of themselves once per four k and a few times behind
+    got = []
+    names = _kernels(lambda: got.append(_run(c, x, w, bias, packed, shift=shift)))
+    assert _tile(names) == (ROWS.get(c, 64), mode == "in_place")
+    got = got[0]
     scale = _conv64(c, x.abs(), w.abs(), bias.abs())
-    bound = (w[0].numel() / 4 + 8) * 2.0 ** -24
-    assert ((got - want).abs() <= scale * bound).all()
-    # roundings of either sign add up as their squares: sqrt(K / 4) of them, each a third of 2^-24 or so of a sum that has grown to sqrt(K)
-    # products, stay below 2^-22 of the result up to K = 6000; a piece too few would show as 2^-17, a lost small product as 2^-17 to 2^-9
-    assert (got - want).norm() <= want.norm() * 2.0 ** -22
+    each, norm = _bounds(want, scale, w[0].numel())
+    assert ((got - want).abs() <= each).all()
+    assert (got - want).norm() <= norm
+    if packed:  # without a workspace there is one slice: other bits where there are more
+        assert torch.equal(_run(c, x, w, bias, True, room=0), got) == (c not in SLICES)
     old = torch.randn(ys, generator=gen)
-    got = _run(c, x, w, None, packed, "relu", 0.5, old)
-    want = _conv64(c, x, w, None).relu() + 0.5 * old.double()
-    assert ((got - want).abs() <= (scale + old.abs()) * bound).all()
+    for first in (False, True):
+        got = _run(c, x, w, None, packed, "relu", 0.5, old, shift=shift, first=first)
+        want = _conv64(c, x, w, None)
+        want = (want + 0.5 * old.double()).relu() if first else want.relu() + 0.5 * old.double()
+        assert ((got - want).abs() <= each + old.abs() * 2.0 ** -22).all()
 
 
 @pytest.mark.gpu
@@ -98,8 +182,8 @@ def test_gpu_residual_sums(c, first, act):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("packed", [False, True])
-@pytest.mark.parametrize("c", [(32, 64, 1, 1, 0, 1, 1, 32, 38, 38), (48, 128, 1, 1, 0, 1, 1, 32, 38, 38), (192, 96, 3, 1, 1, 1, 1, 5, 61, 43)],
-                         ids=["64x128", "128x128", "slices"])
+@pytest.mark.parametrize("c", [(32, 64, 1, 1, 0, 1, 1, 32, 38, 38), (48, 128, 1, 1, 0, 1, 1, 32, 38, 38), (192, 96, 3, 1, 1, 1, 1, 5, 61, 43),
+                               (256, 96, 3, 1, 1, 1, 1, 10, 37, 37)], ids=["64x128", "128x128", "slices", "128x128 slices"])
 def test_gpu_split_not_finite(c, packed):
     """infinities, NaN and values next to the largest float come out as the definition has them"""
     gen = torch.Generator().manual_seed(5)
@@ -170,18 +254,6 @@ def test_gpu_split_other_batches():
             assert torch.equal(_run(cb, x, w, None, packed, hint=5), _conv64(cb, x, w, None))  # whole numbers are exact
 
 
-def _kernels(f):
-    """names of the kernels that f launches, without packing"""
-    dlp.timing_enable(True)
-    dlp.timing_reset()
-    try:
-        f()
-        return [k for section, _, k in dlp.timing_records(kernels=True) if section == "conv_gemm"]
-    finally:
-        dlp.timing_enable(False)
-        dlp.timing_reset()
-
-
 # (cin, cout, k, stride, pad, h, batch of the settings, batch of the call): on either side of the lines between the kernels at the
 # call's batch, weights packed for 128 rows run in tiles of 64 and in fp32 tiles (of 64 and of 32 rows, stream and slices)
 OTHER = [(128, 128, 3, 1, 1, 28, 64, 64), (128, 128, 3, 1, 1, 28, 64, 20), (128, 128, 3, 1, 1, 28, 64, 5), (512, 512, 3, 1, 1, 7, 64, 33),
@@ -242,9 +314,17 @@ def test_gpu_split_small_workspaces():
         op.enqueue(x.cuda(), w.cuda(), None, y, torch.empty(floats - 256, dtype=torch.uint8, device="cuda:0"))
 
 
+# the kernels that the phases run on: float tiles, split tiles of 64 and 128 rows
+PHASES = {
+    (48, 64, 3, 2, 1, 1, 1, 24, 79, 81): {0}, (40, 32, 4, 2, 1, 1, 1, 3, 18, 22): {0}, (64, 48, 3, 1, 1, 1, 2, 33, 40, 40): set(),  # (24 channels a group are not packed)
+    (20, 16, 5, 3, 2, 1, 1, 2, 17, 19): {0}, (36, 64, 3, 2, 1, 1, 2, 4, 18, 18): {0},  # groups
+    (128, 48, 4, 2, 1, 1, 1, 32, 56, 56): {64}, (96, 64, 3, 2, 1, 1, 1, 33, 55, 57): {64}, (128, 64, 4, 2, 1, 1, 2, 32, 56, 56): {64},
+    (200, 32, 4, 2, 1, 1, 1, 32, 56, 54): {128}, (160, 64, 2, 2, 0, 1, 2, 64, 56, 56): {128}, (72, 32, 3, 1, 1, 1, 1, 40, 38, 38): {128},
+}
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", [(48, 64, 3, 2, 1, 1, 1, 24, 79, 81), (40, 32, 4, 2, 1, 1, 1, 3, 18, 22), (64, 48, 3, 1, 1, 1, 2, 33, 40, 40), (20, 16, 5, 3, 2, 1, 1, 2, 17, 19)],
-                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("c", PHASES, ids=lambda c: "x".join(map(str, c)))
 def test_gpu_backward_data_phase_packing(c):
     """filters of all stride phases packed by one launch, in float and in split tiles; bias and activation behind the interleaving"""
     cin, cout, k, s, p, d, g, b, h, wd = c
@@ -258,7 +338,11 @@ def test_gpu_backward_data_phase_packing(c):
     op = dlp.Conv2DBackwardData.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs), "gemm")
     work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
     dx = torch.full(xs, float("nan"), device="cuda:0")
-    op.enqueue(dx, w.cuda(), dy.cuda(), work)
+    names = _kernels(lambda: op.enqueue(dx, w.cuda(), dy.cuda(), work))
+    if PHASES[c]:
+        assert {_tile([n])[0] if n.startswith("conv_split") else 0 for n in names} == PHASES[c]
+    if 0 not in PHASES[c]:
+        bound = (cout // g * k * k / 4 + 8) * 2.0 ** -24  # (_bounds)
     assert ((dx.cpu().double() - want).abs() <= scale * bound).all()
     tr = dlp.TransposedConv2DForward.create(dlp.Conv2DSettings(cout, cin, k, s, d, p, g, ys), extra, True, "relu", "gemm")
     work = torch.empty(max(tr.workspace(), 1), dtype=torch.uint8, device="cuda:0")
@@ -290,14 +374,18 @@ def test_gpu_split_filter_gradient(c):
     n = ys[0] * ys[2] * ys[3]
     err = (got(x) - want).abs()
     assert (err <= scale * (n / 4 + 8) * 2.0 ** -24).all()  # as for the forward pass
-    x[0, 1, 0, 0], x[0, 3, xs[2] // 2, xs[3] // 2] = float("inf"), float("nan")
     dy = dy.abs() + 0.5  # no product of infinity and zero inside the image
-    mine, want = got(x), grad(torch.nan_to_num(x, nan=0.0, posinf=0.0), dy)
-    clean = [i for i in range(cin // g) if not (i == 1 or i == 3)]
-    assert torch.isfinite(mine[:, clean][cout // g:] if g > 1 else mine[:, clean]).all()
-    first = mine[: cout // g]
-    assert (torch.isposinf(first[:, 1]) | torch.isfinite(first[:, 1])).all() and torch.isposinf(first[:, 1]).any()
-    assert torch.isnan(first[:, 3]).any() and (torch.isnan(first[:, 3]) | torch.isfinite(first[:, 3])).all()
+    for values in [(float("inf"), float("nan")), (float("-inf"), 3.4e38), (float("nan"), float("inf"))]:
+        # the first pixel that a tap meets, and one in the middle
+        x[0, 1, 0, 0], x[0, 3, xs[2] // 2, xs[3] // 2] = values
+        mine, want = got(x), grad(x, dy)
+        for f in (torch.isnan, torch.isposinf, torch.isneginf):
+            # (a sum that the fp32 instruction rounds to infinity is finite in 64 bits)
+            assert torch.equal(f(mine), f(want.float().double()))
+        ok = torch.isfinite(mine)
+        scale = grad(torch.nan_to_num(x, 0.0, 0.0, 0.0).abs(), dy)
+        # the tile is computed again: one rounding per product
+        assert ((mine - want).abs()[ok] <= scale[ok] * (n + 8) * 2.0 ** -24).all()
 
 
 @pytest.mark.gpu
