@@ -135,7 +135,8 @@ def build_layers(layer_list, batch, seed, bf16=False):
 
 
 def matrix_peak_tflops(kernel_name):
-    if kernel_name.startswith("conv_split_f32_kernel"):  # float products, each as six products of bf16 parts on the bf16 matrix instruction
+    # float products, each as six products of bf16 parts on the bf16 matrix instruction
+    if kernel_name.startswith("conv_split_f32_kernel") or (kernel_name.startswith("conv_wgrad_f32_kernel") and kernel_name.endswith("true>")):
         return round(BF16_MATRIX_PEAK_TFLOPS / 6, 1)
     return BF16_MATRIX_PEAK_TFLOPS if kernel_name.startswith(("conv_gemm_bf16_kernel", "conv_patch_bf16_kernel", "conv_stem_bf16_kernel")) else FP32_MATRIX_PEAK_TFLOPS
 
@@ -281,11 +282,16 @@ def run_backward_workload(args):
     torch.cuda.synchronize()
     dlp.timing_enable(False)
     sections = {}
-    for (section, ms) in dlp.timing_records():
+    wgrad_kernels = []
+    for (section, ms, kname) in dlp.timing_records(kernels=True):
         sections[section] = round(sections.get(section, 0.0) + ms, 4)
+        if section == "wgrad":
+            wgrad_kernels.append(kname)
     dlp.timing_reset()
     flops_f = sum(conv_flops(e["L"], args.batch) for e in layers)
     flops_d = sum(conv_flops(e["L"], args.batch) for e in layers if e["bd"])
+    # the filter gradients' own peak: every launch's flops at the rate of the instruction that it runs on
+    peak = round(flops_f / sum(conv_flops(e["L"], args.batch) / matrix_peak_tflops(k) for e, k in zip(layers, wgrad_kernels)), 1)
     wgrad_ms = sections.get("wgrad", 0.0)
     out = {
         "metric": BASELINE_METRIC, "value": round(args.batch / (ms_per_step * 1e-3), 1), "unit": "images/s", "n_gpus": 1,
@@ -298,8 +304,7 @@ def run_backward_workload(args):
         "frac_of_fp32_matrix_peak": round((flops_f + flops_d) / (ms_per_step * 1e-3) / 1e12 / FP32_MATRIX_PEAK_TFLOPS, 4),
         "kernel_ms_by_section": sections,
         "roofline": {"bound": "mfma", "kernel": "conv_wgrad_f32_kernel (20 launches)", "achieved": round(flops_f / (wgrad_ms * 1e-3) / 1e12, 2) if wgrad_ms else None,
-                     "peak": FP32_MATRIX_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(flops_f / (wgrad_ms * 1e-3) / 1e12 / FP32_MATRIX_PEAK_TFLOPS, 4) if wgrad_ms else None, "traffic": None},
+                     "peak": peak, "unit": "TFLOP/s", "frac": round(flops_f / (wgrad_ms * 1e-3) / 1e12 / peak, 4) if wgrad_ms else None, "traffic": None},
         "cpu_baseline": None,
     }
     print(json.dumps(out))

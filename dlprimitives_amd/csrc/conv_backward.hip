@@ -1077,11 +1077,11 @@ int dlp_conv2d_bwd_filter_enqueue(dlp_conv2d_bwd_filter *op, const int x_shape[4
 #define DLP_WGRAD_LAUNCH_M(BM_, BN_, AV_, SP_)                                                                    \
     do {                                                                                                       \
         if (masked == 1)                                                                                       \
-            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 1, SP_>), grid, block, 0, st, a);         \
+            DLP_LAUNCH_TIMED(ts, (conv_wgrad_f32_kernel<BM_, BN_, AV_, 1, SP_>), grid, block, 0, st, a);       \
         else if (masked == 2)                                                                                  \
-            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 2, SP_>), grid, block, 0, st, a);         \
+            DLP_LAUNCH_TIMED(ts, (conv_wgrad_f32_kernel<BM_, BN_, AV_, 2, SP_>), grid, block, 0, st, a);       \
         else                                                                                                   \
-            hipLaunchKernelGGL((conv_wgrad_f32_kernel<BM_, BN_, AV_, 0, SP_>), grid, block, 0, st, a);         \
+            DLP_LAUNCH_TIMED(ts, (conv_wgrad_f32_kernel<BM_, BN_, AV_, 0, SP_>), grid, block, 0, st, a);       \
     } while (0)
 #define DLP_WGRAD_LAUNCH(BM_, BN_, SP_)                                                                           \
     do {                                                                                                       \

@@ -588,7 +588,7 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
                 const uint32_t voff =
                     n < a.N ? (uint32_t)(((b * a.Cout + g * a.M + m0 + wm * WTM + 4 * h) * a.OHW + pix) * (int)sizeof(T)) : kOutOfRange;
                 // the old values of all the column's rows are requested before the first is used: one by one, each waited for its own trip
-                // to memory (64->256 1x1 at 56x56 with its residual sum, batch 16, in tiles of 128x128: 56 -> 33 us)
+                // to memory (64->256 1x1 at 56x56 in tiles of 128x128, sum behind the activation: 277 -> 99 us at batch 64, 87 -> 32 at 16)
                 float old[TM][16];
                 if (SUM) {
 #pragma unroll
@@ -2449,8 +2449,11 @@ void set_tile_magics(GemmArgs &a, int groups)
 
 // How a launch of conv_split_f32_kernel is cut: `tiles` tiles of nkt K tiles in s slices each, but the tiles that would make up the last,
 // partial round of workgroups (one per CU and round: the workgroups of a CU share its matrix units) in s2 finer ones.  `cost`: K tiles the
-// busiest CU works through, and what the partial sums cost -- about a twentieth of a K tile per piece for its trip through
-// the workspace, and once the time the last piece to arrive takes to add the others up.
+// busiest CU works through, and what the partial sums cost -- a twentieth of a K tile per piece of the launch for its trip through
+// the workspace (which all pieces share), and six K tiles once for the last piece to arrive, which adds the others up.  The constants were set
+// by hand to the layers of ResNet-18 and ResNet-50 and are no more exact than this (filters packed, best cut / none): 3x3 64->64 at
+// 56x56, batch 64, 102 / 106 us, 256->256 at 14x14 105 / 114, 512->512 at 7x7 97 / 219, stride 2 256->512 at 14x14 67 / 100, 1x1
+// 2048->512 at 7x7 52 / 84; batch 32 56 / 64, 57 / 95, 64 / 188; but stride 2 128->256 at 28x28 66 / 60 and 64->128 at 56x56 55 / 53.
 // Only cuts whose partial sums number at most max_images (BM x BN accumulators) are considered.
 struct SplitCut {
     int s, tail, s2;
@@ -3055,12 +3058,17 @@ static GemmPlan float_plan(ConvGeom g, int activation)
     return conv_gemm_plan(g, activation);
 }
 
+GemmPlan conv_gemm_hint_plan(const ConvGeom &g, int activation)
+{
+    ConvGeom at_hint = g;
+    at_hint.B = g.B_hint;
+    return conv_gemm_plan(at_hint, activation);
+}
+
 GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation)
 {
     GemmPackPlan pp;
-    ConvGeom at_hint = g;
-    at_hint.B = g.B_hint;
-    pp.p = conv_gemm_plan(at_hint, activation);
+    pp.p = conv_gemm_hint_plan(g, activation);
     pp.bytes = pp.p.wpack_bytes;
     if (pp.p.split) {
         pp.floats = float_plan(g, activation);
@@ -3069,15 +3077,15 @@ GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation)
     return pp;
 }
 
-GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPackPlan &pp, size_t &offset)
+GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPlan &packed, size_t &offset)
 {
     GemmPlan p = conv_gemm_plan(g, activation);
     offset = 0;
-    if (pp.p.split && p.split) { // (tiles of no more rows than packed ones: the batch is no larger)
-        p.pack_bm = pp.p.BM;
-        p.wpack_bytes = pp.p.wpack_bytes;
-    } else if (pp.p.split)
-        offset = pp.p.wpack_bytes;
+    if (packed.split && p.split) { // (tiles of no more rows than packed ones: the batch is no larger)
+        p.pack_bm = packed.BM;
+        p.wpack_bytes = packed.wpack_bytes;
+    } else if (packed.split)
+        offset = packed.wpack_bytes;
     return p;
 }
 

@@ -22,8 +22,11 @@
 //  * A wavefront owns 64x64 of the output (64x32 with tiles of 64x128): at six matrix instructions per operand pair of 32x32x16 (192
 //    clocks) a 32x32 tile would want 128 bytes per clock and CU from LDS, all there is; 64x64 wants half of that.
 //
-// Reaches 200 TFLOP/s of products on long launches (1x1 1024->1024 at 28x28, batch 128: 1673 -> 1056 us; 3x3 256->256 at 14x14, batch 512:
-// 858 -> 591 us): 1.2e15 bf16 operations a second on operands of random bits, what the library's bf16 product reaches on the same card.
+// Reaches 200 to 215 TFLOP/s of products on long launches (1x1 1024->1024 at 28x28, batch 128: 1662 us on the fp32 instruction, 1038 here; 3x3
+// 256->256 at 14x14, batch 512: 825, 563): 1.2e15 bf16 operations a second on operands of random bits, what the library's bf16 product
+// reaches on the same card.  At batch 64 (128->128 at 28x28: 151 to 168 TFLOP/s) the matrix units are busy 43 % of the time: a
+// launch is little more than one round of workgroups, a SIMD has 1.4 wavefronts on average (2.3 in tiles of 64x128), and a wavefront spends half
+// its life ready but not issued, a fifth at barriers and waits, 7 % of it on LDS (11 % in tiles of 64x128; no bank conflicts).
 // Loads two K tiles further ahead, or a second set of registers for them, made no difference.
 
 // eight consecutive k of a row -> the 16-byte pieces of its three parts

@@ -582,11 +582,12 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     const GemmPlan gplan = conv_gemm_plan(g, activation);
     const bool bf16_mfma = gplan.order >= GEMM_ORDER_TAP_BF16;
     // Where the reference rule would pick Winograd (src/core/conv.cpp:714-718), the automatic choice here keeps "gemm" for layers that
-    // the LDS-patch kernel serves and that (a) have fewer than 64 input channels, or fewer than 128 with a filter count off 64 (the
+    // the LDS-patch kernel can serve and that (a) have fewer than 64 input channels, or fewer than 128 with a filter count off 64 (the
     // Winograd kernel then gives a workgroup 32 output channels: 130 against 126 us on 64->64 at 56x56, batch 64), or (b) leave the
-    // Winograd kernel fewer than one and a half workgroups per compute unit at the batch of the settings.  Whole layers, weights
-    // transformed in the call, cold tensors, gemm / winograd, at batch 64: 64->64 at 56x56 150 / 125 us, 128->128 at 28x28 129 / 108,
-    // 256->256 at 14x14 123 / 97, 512->512 at 7x7 124 / 105; at batch 16: 49 / 40, 45 / 39, 47 / 46 (200 workgroups), 48 / 77 (128).
+    // Winograd kernel fewer than one and a half workgroups per compute unit at the batch of the settings.  These lines were drawn against the
+    // LDS-patch kernel.  From batch 32 to 64 on such layers run on conv_split_f32_kernel, and the choice is then not the faster one
+    // throughout: weights transformed in the call, gemm / winograd, at batch 64 64->64 at 56x56 97 / 111 us, 128->128 at 28x28 91 / 104,
+    // 256->256 at 14x14 107 / 94, 512->512 at 7x7 104 / 106; at batch 16 37 / 37, 42 / 38, 44 / 44 (200 workgroups), 49 / 77 (128).
     const int cin_g = cfg->channels_in / cfg->groups;
     bool gemm_faster = false;
     if (gplan.patch_layer && win) {
@@ -825,11 +826,11 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
     case ALGO_DEPTHWISE:
         return depthwise_launch(g, x, w, y, ep, s);
     default: {
-        const GemmPackPlan pp = conv_gemm_pack_plan(g, op->activation);
+        const GemmPlan hint_plan = conv_gemm_hint_plan(g, op->activation);
         size_t offset;
-        const GemmPlan plan = conv_gemm_plan_on_packed(g, op->activation, pp, offset);
+        const GemmPlan plan = conv_gemm_plan_on_packed(g, op->activation, hint_plan, offset);
         int sig[6];
-        layout_of(pp.p, sig);
+        layout_of(hint_plan, sig);
         for (int i = 0; i < 6; i++)
             DLP_REQUIRE(sig[i] == op->packed_layout[i], "the weights were packed for another tile plan (pack again for this batch)");
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");

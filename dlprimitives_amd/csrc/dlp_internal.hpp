@@ -255,8 +255,9 @@ struct GemmPackPlan {
     size_t bytes;
 };
 GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation);
-// plan of a call on weights packed that way, with its tiles `offset` bytes into them
-GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPackPlan &pp, size_t &offset);
+GemmPlan conv_gemm_hint_plan(const ConvGeom &g, int activation); // its p alone
+// plan of a call on weights packed by `packed`, a hint plan, with its tiles `offset` bytes into them
+GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPlan &packed, size_t &offset);
 size_t conv_gemm_ktab_entries(const ConvGeom &g);
 // The table layout depends on the geometry AND on the activation the op was created with.
 void conv_gemm_fill_ktab(const ConvGeom &g, int activation, KTabEntry *host_tab);

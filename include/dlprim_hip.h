@@ -123,19 +123,23 @@ int dlp_conv2d_output_shape(const dlp_conv2d_settings *cfg, const int in_shape[4
  *      to "gemm" exactly as the reference does (:725-727).  The automatic
  *      choice ("" / "auto") differs from the reference's rule (:714-718) in one
  *      place: a Winograd-compatible fp32 convolution that the LDS-patch GEMM
- *      kernel serves (image at most 62 wide, Cin a multiple of 16, more than 32
- *      filters) stays "gemm" where that is the faster of the two on gfx950:
- *      with fewer than 64 input channels, with fewer than 128 and a filter count
- *      that is no multiple of 64, and when the batch of the settings leaves the
- *      Winograd kernel fewer than one and a half workgroups per compute unit;
- *      algo() reports what was chosen. ------ */
+ *      kernel can serve (image at most 62 wide, Cin a multiple of 16, more than
+ *      32 filters) stays "gemm" with fewer than 64 input channels, with fewer
+ *      than 128 and a filter count that is no multiple of 64, and when the batch
+ *      of the settings leaves the Winograd kernel fewer than one and a half
+ *      workgroups per compute unit; algo() reports what was chosen.  (Large
+ *      launches of "gemm" run on the bf16 matrix instruction, every float as three
+ *      bf16 parts, and are then the faster of the two on some layers that the rule
+ *      gives to Winograd: name the algorithm where that counts.) ------ */
 int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activation,
                           const char *algo, dlp_conv2d_fwd **out);
 
 /* Conv2DBase::algo(), include/dlprim/core/conv.hpp:33 */
 const char *dlp_conv2d_fwd_algo(const dlp_conv2d_fwd *op);
 
-/* Conv2DBase::workspace() in bytes, include/dlprim/core/conv.hpp:34 */
+/* Conv2DBase::workspace() in bytes, include/dlprim/core/conv.hpp:34: enough for every batch
+ * up to that of the shape given at create, and for larger ones.  "gemm" on a smaller one than it
+ * asks for cuts long sums less finely, down to the size of the tile-ordered weights alone. */
 size_t dlp_conv2d_fwd_workspace(const dlp_conv2d_fwd *op);
 
 /* core::Conv2DForward::enqueue, include/dlprim/core/conv.hpp:48.
@@ -158,8 +162,9 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4],
  * (tile-ordered weights of "gemm", the transformed filter of "winograd") and that
  * dlp_conv2d_fwd_enqueue_packed reads instead of transforming `w` again (`w` is still passed: 1x1
  * bf16 convolutions read it in place).  `ws` then only holds the per-call scratch: workspace() bytes
- * are always enough, and convolutions that run one after another on a stream may share it.  Pack
- * again after the weights change. */
+ * are always enough, and convolutions that run one after another on a stream may share it.  The
+ * buffer serves every batch (float "gemm" weights that a large batch wants as three bf16 parts are
+ * held as fp32 tiles too, for small ones).  Pack again after the weights change. */
 size_t dlp_conv2d_fwd_packed_bytes(const dlp_conv2d_fwd *op);
 int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *stream);
 int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], const void *x, const void *w,
@@ -412,7 +417,10 @@ int dlp_softmax_loss_fwd_enqueue(int dtype, int label_dtype, int batch, int clas
 
 /* ===== data types ==================================================================
  * DLP_FLOAT: everything fp32, as in the reference (its conv/GEMM reject other types,
- * src/gemm.cpp:577,593).  DLP_BFLOAT16 (an extension): x, w, y of Conv2DForward and
+ * src/gemm.cpp:577,593).  Large "gemm" convolutions and filter gradients multiply each float
+ * as three bf16 parts (six of the nine products of parts, summed in fp32), with errors below
+ * the fp32 matrix instruction's; infinities, NaN, sums below 2^-72 and operands at the ends of
+ * the range are computed on that instruction.  DLP_BFLOAT16 (an extension): x, w, y of Conv2DForward and
  * IPForward and the tensors of the glue operators are stored as bfloat16; bias stays
  * fp32; products are accumulated in fp32 on the matrix cores and the epilogue runs in
  * fp32 before one round-to-nearest-even conversion of the result.  All three algorithms

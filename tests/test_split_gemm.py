@@ -39,13 +39,13 @@ def _conv64(c, x, w, bias):
     return torch.nn.functional.conv2d(x.double(), w.double(), None if bias is None else bias.double(), s, p, d, g)
 
 
-def _kernels(f):
-    """names of the kernels that f launches, without packing"""
+def _kernels(f, section="conv_gemm"):
+    """names of the kernels that f launches in a section of the timing records"""
     dlp.timing_enable(True)
     dlp.timing_reset()
     try:
         f()
-        return [k for section, _, k in dlp.timing_records(kernels=True) if section == "conv_gemm"]
+        return [k for s, _, k in dlp.timing_records(kernels=True) if s == section]
     finally:
         dlp.timing_enable(False)
         dlp.timing_reset()
@@ -353,7 +353,7 @@ def test_gpu_backward_data_phase_packing(c):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("c", [(32, 80, 3, 1, 1, 1, 1, 3, 12, 12), (33, 130, 3, 2, 1, 1, 1, 2, 15, 13), (48, 70, 5, 1, 2, 1, 1, 1, 9, 7), (16, 65, 7, 1, 3, 1, 1, 2, 10, 8),
-                               (256, 72, 1, 1, 0, 1, 2, 5, 8, 8), (128, 128, 1, 1, 0, 1, 1, 1, 1, 1), (20, 200, 8, 1, 4, 1, 1, 2, 9, 9)], ids=lambda c: "x".join(map(str, c)))
+                               (256, 144, 1, 1, 0, 1, 2, 5, 8, 8), (128, 128, 1, 1, 0, 1, 1, 1, 1, 1), (20, 200, 8, 1, 4, 1, 1, 2, 9, 9)], ids=lambda c: "x".join(map(str, c)))
 def test_gpu_split_filter_gradient(c):
     """filter gradients in tiles of 128x128 (more than 64 filters and 64 columns): remainders in rows, columns and pixels, planes of whole
     16-byte pieces and others, one and two words of tap mask and none; then infinities and NaN"""
@@ -369,6 +369,8 @@ def test_gpu_split_filter_gradient(c):
         op.enqueue(x.cuda(), dw, dy.cuda(), work)
         return dw.cpu().double()
 
+    (name,) = _kernels(lambda: got(x), "wgrad")
+    assert name.startswith("conv_wgrad_f32_kernel<128, 128,") and name.endswith(", true>") == (ys[0] * ys[2] * ys[3] >= 3), name
     grad = lambda x, dy: torch.nn.grad.conv2d_weight(x.double(), ws, dy.double(), s, p, d, g)
     want, scale = grad(x, dy), grad(x.abs(), dy.abs())
     n = ys[0] * ys[2] * ys[3]
@@ -452,3 +454,31 @@ def test_gpu_backward_data_batch_other_than_created(c, grow):
     y = torch.full((batch, cin, h, w), float("nan"), device="cuda:0")
     tr.enqueue(dy.cuda(), f.cuda(), None, y, work)
     assert torch.equal(y.cpu(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+def test_gpu_first_call_of_a_smaller_batch_in_a_capture(packed):
+    """an operator's first call may sit in a capture at any batch up to the settings' one: nothing is allocated, replays repeat"""
+    gen = torch.Generator().manual_seed(4)
+    w = torch.randint(-4, 5, (128, 128, 3, 3), generator=gen).float()
+    for batch in (64, 20, 3):
+        op = dlp.Conv2DForward.create(dlp.Conv2DSettings(128, 128, 3, 1, 1, 1, 1, (64, 128, 14, 14)), False, "identity", "gemm")
+        x, wd = torch.randint(-4, 5, (batch, 128, 14, 14), generator=gen).float().cuda(), w.cuda()
+        y = torch.empty_like(x)
+        ws = torch.empty(op.workspace(), dtype=torch.uint8, device="cuda:0")
+        buf = torch.empty(op.packed_size(), dtype=torch.uint8, device="cuda:0")
+        op.pack(wd, buf)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            if packed:
+                op.enqueue_packed(x, wd, buf, None, y, ws)
+            else:
+                op.enqueue(x, wd, None, y, ws)
+        for _ in range(3):
+            x.copy_(torch.randint(-4, 5, x.shape, generator=gen).float())
+            y.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y.cpu().double(), torch.nn.functional.conv2d(x.cpu().double(), w.double(), None, 1, 1))
