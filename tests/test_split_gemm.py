@@ -482,3 +482,26 @@ def test_gpu_first_call_of_a_smaller_batch_in_a_capture(packed):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y.cpu().double(), torch.nn.functional.conv2d(x.cpu().double(), w.double(), None, 1, 1))
+
+
+@pytest.mark.gpu
+def test_gpu_rows_of_128_in_tiles_of_64_computed_again():
+    """weights packed for 128-row tiles, a call in 64-row ones: infinities, NaN, and weights that are kept whole"""
+    c = (128, 200, 3, 1, 1, 1, 1, 14, 28, 28)
+    gen = torch.Generator().manual_seed(8)
+    xs, ws, _ = _geometry(c)
+    x, w = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+    x[0, 3, 4, 5], x[5, 7, 20, 9] = float("inf"), float("nan")
+    w[70] *= 2.0 ** -118  # second tile of 64, in the first packed one
+    w[150, 5] *= 2.0 ** 40  # first tile of the second
+    w[199, 2] = float("inf")
+    got = []
+    names = _kernels(lambda: got.append(_run(c, x, w, None, True, hint=64)))
+    assert _tile(names) == (64, False)
+    want = _conv64(c, x, w, None)
+    inside = (slice(None), slice(None), slice(1, -1), slice(1, -1))  # (infinity times the padding's zeros is left to either)
+    for f in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(f(got[0][inside]), f(want[inside]))
+    scale = _conv64(c, torch.nan_to_num(x, 0.0, 0.0, 0.0).abs(), torch.nan_to_num(w, 0.0, 0.0, 0.0).abs(), None)
+    ok = torch.isfinite(want)
+    assert ((got[0] - want).abs()[ok] <= scale[ok] * ((128 * 9 + 8) * 2.0 ** -24)).all()  # one rounding per product
