@@ -823,7 +823,49 @@ static size_t bwd_data_need(const dlp_conv2d_bwd_data *op, int batch, size_t *fw
     return total + fws;
 }
 
-size_t dlp_conv2d_bwd_data_workspace(const dlp_conv2d_bwd_data *op) { return op ? bwd_data_need(op, std::max(op->cfg.shape[0], 1), nullptr) : 0; }
+// The phases as one launch, longest first (place[i]: of phase i), where all of them have filter taps and are convolutions on tiles of 16 channels
+// of a tap (conv_gemm_phases_plan).
+static bool merged_phases(const dlp_conv2d_bwd_data *op, int batch, int act, size_t ws_bytes, PhaseConv *ph, int *order, PhasesPlan &plan)
+{
+    if (!op->strided || op->nphases > kMaxPhases)
+        return false;
+    for (int i = 0; i < op->nphases; i++) {
+        if (!op->phase[i].fwd)
+            return false;
+        order[i] = i;
+    }
+    std::stable_sort(order, order + op->nphases, [&](int x, int y) {
+        return op->phase[x].h.n * op->phase[x].w.n > op->phase[y].h.n * op->phase[y].w.n;
+    });
+    const dlp_conv2d_settings &c = op->cfg;
+    for (int j = 0; j < op->nphases; j++) {
+        const BwdPhase &p = op->phase[order[j]];
+        if (!conv_fwd_tap_table(p.fwd, batch, ph[j].g, &ph[j].ktab))
+            return false;
+        ph[j].off_h = p.h.off;
+        ph[j].off_w = p.w.off;
+        ph[j].len_h = p.h.len;
+        ph[j].len_w = p.w.len;
+        ph[j].out_off = order[j] / c.stride[1] * c.shape[3] + order[j] % c.stride[1];
+    }
+    return conv_gemm_phases_plan(ph, op->nphases, act, ws_bytes, plan);
+}
+
+size_t dlp_conv2d_bwd_data_workspace(const dlp_conv2d_bwd_data *op)
+{
+    if (!op)
+        return 0;
+    const int batch = std::max(op->cfg.shape[0], 1);
+    size_t need = bwd_data_need(op, batch, nullptr);
+    // as one launch, with the K slices of this batch and of smaller ones
+    PhaseConv ph[kMaxPhases];
+    int order[kMaxPhases];
+    PhasesPlan plan;
+    for (int b = batch; b >= 1; b /= 2)
+        if (merged_phases(op, b, DLP_ACT_IDENTITY, (size_t)-1, ph, order, plan))
+            need = std::max(need, plan.bytes);
+    return need;
+}
 
 // bias and act: of a transposed convolution, applied by the interleaving kernel (strided passes only)
 static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx, const void *w, const void *dy, void *ws, size_t ws_bytes, float factor,
@@ -864,6 +906,28 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
     }
     const size_t planes = (size_t)batch * c.channels_in;
     DLP_REQUIRE(planes * c.shape[2] * c.shape[3] < (1ull << 31) / 4, "tensor of 2 GiB or more");
+    PhaseConv conv[kMaxPhases];
+    int order[kMaxPhases];
+    PhasesPlan merged;
+    if (((uintptr_t)ws & 15) == 0 && merged_phases(op, batch, act, ws_bytes, conv, order, merged)) {
+        int *const counters = (int *)((char *)ws + merged.packed_bytes);
+        PhaseFilter pf[kMaxPhases];
+        size_t at = 0;
+        for (int j = 0; j < op->nphases; j++) {
+            const BwdPhase &p = op->phase[order[j]];
+            pf[j] = {merged.plan[j], (char *)ws + at, p.h.n, p.w.n, p.h.r0, p.h.rstep, p.w.r0, p.w.rstep};
+            at += merged.plan[j].wpack_bytes;
+        }
+        const int rc = conv_gemm_pack_phases((const float *)w, c.groups, cout_g, cin_g, c.kernel[0], c.kernel[1], pf, op->nphases, st, counters, merged.counters);
+        if (rc != DLP_OK)
+            return rc;
+        Epilogue ep;
+        ep.bias = bias;
+        ep.factor = factor;
+        ep.activation = act;
+        return conv_gemm_phases_launch(conv, op->nphases, merged, dy, ws, counters, (float *)((char *)counters + round256(merged.counters * sizeof(int))), dx,
+                                       c.shape[2], c.shape[3], c.stride[0], c.stride[1], ep, st);
+    }
     InterleaveArgs ia;
     ia.H = c.shape[2];
     ia.W = c.shape[3];

@@ -101,6 +101,9 @@ struct GemmArgs {
     int pre; // the old value of y is added before the activation (Epilogue::accumulate_first)
     int act;
     float clamp_lo, clamp_hi;
+    // conv_phases_f32_kernel: pixel (i, j) of a phase is computed as output (i + off_h, j + off_w) of its convolution and stored as pixel
+    // (i * out_sh, j * out_sw) of y + out_off, whose planes have out_hw pixels in rows of out_w
+    int off_h, off_w, out_hw, out_w, out_sh, out_sw, out_off;
 };
 
 typedef __attribute__((address_space(4))) const int32_t ConstInt;
@@ -160,7 +163,7 @@ __device__ __forceinline__ void static_for_all(F &&f)
     f(std::integral_constant<int, 7>{});
 }
 
-template <class T, int BM, int BN, int WM, int WN, int ACT, bool RAGGED = false>
+template <class T, int BM, int BN, int WM, int WN, int ACT, bool RAGGED = false, bool STRIDED = false>
 __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc)[BM / WM / 32][BN / WN / 32], float *lds, int m0, int n0,
                                                  int g, int slice, int splitk, uint32_t image0, int wm, int wn, int h, int l32, int tid,
                                                  const float *bias_s);
@@ -472,7 +475,8 @@ __global__ __launch_bounds__(kThreads) void conv_gemm_f32_kernel(GemmArgs a)
 // last barrier of the main loop (at least BM floats).  `bias_s`: the bias of the tile's BM rows in LDS (zero past M), staged by the
 // kernel when it starts on the tile: requested here, its trip to memory stood between the last matrix instruction and the first store.
 // RAGGED: built for M off multiples of 8 too (a kernel of its own: as one more copy of the stores it cost the other launches up to 10 %).
-template <class T, int BM, int BN, int WM, int WN, int ACT, bool RAGGED>
+// STRIDED: the pixels of one stride phase, out_sh rows and out_sw columns apart (float, y below 2 GiB).
+template <class T, int BM, int BN, int WM, int WN, int ACT, bool RAGGED, bool STRIDED>
 __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc)[BM / WM / 32][BN / WN / 32], float *lds, int m0, int n0,
                                                  int g, int slice, int splitk, uint32_t image0, int wm, int wn, int h, int l32, int tid,
                                                  const float *bias_s)
@@ -575,7 +579,8 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
     // Fast path (float, or no factor; M a multiple of 8 or RAGGED; y below 2 GiB): the bias of the tile's rows has gone through LDS and the stores are buffer
     // stores whose row offset is scalar, instead of a bias load and 64-bit address arithmetic per value.
     const bool pre = a.pre != 0 && a.factor != 0.0f;
-    if ((a.factor == 0.0f || sizeof(T) == 4) && (RAGGED || (a.M & 7) == 0) && a.y_bytes != 0) {
+    if (STRIDED || ((a.factor == 0.0f || sizeof(T) == 4) && (RAGGED || (a.M & 7) == 0) && a.y_bytes != 0)) {
+        const int plane = STRIDED ? a.out_hw : a.OHW;
         const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, a.y_bytes, 0x00020000);
         const bool clamp = a.act != DLP_ACT_IDENTITY;
         auto store_all = [&](auto sum_c) {
@@ -584,9 +589,13 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
             for (int j = 0; j < TN; j++) {
                 const int n = n0 + wn * WTN + j * 32 + l32;
                 const int b = (int)fast_div((uint32_t)n, a.ohw_magic, a.ohw_shift);
-                const int pix = n - b * a.OHW;
+                int pix = n - b * a.OHW;
+                if (STRIDED) {
+                    const int oy = (int)fast_div((uint32_t)pix, a.ow_magic, a.ow_shift);
+                    pix = oy * a.out_sh * a.out_w + (pix - oy * a.OW) * a.out_sw + a.out_off;
+                }
                 const uint32_t voff =
-                    n < a.N ? (uint32_t)(((b * a.Cout + g * a.M + m0 + wm * WTM + 4 * h) * a.OHW + pix) * (int)sizeof(T)) : kOutOfRange;
+                    n < a.N ? (uint32_t)(((b * a.Cout + g * a.M + m0 + wm * WTM + 4 * h) * plane + pix) * (int)sizeof(T)) : kOutOfRange;
                 // the old values of all the column's rows are requested before the first is used: one by one, each waited for its own trip
                 // to memory (64->256 1x1 at 56x56 in tiles of 128x128, sum behind the activation: 277 -> 99 us at batch 64, 87 -> 32 at 16)
                 float old[TM][16];
@@ -597,7 +606,7 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
                         for (int r = 0; r < 16; r++)
                             if (m0 + wm * WTM + i * 32 + 8 * (r >> 2) < a.M)
                                 old[i][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                                          yr, voff, (uint32_t)((i * 32 + 8 * (r >> 2) + (r & 3)) * a.OHW * (int)sizeof(T)), 0));
+                                                                          yr, voff, (uint32_t)((i * 32 + 8 * (r >> 2) + (r & 3)) * plane * (int)sizeof(T)), 0));
                 }
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
@@ -615,7 +624,7 @@ __device__ __forceinline__ void gemm_tile_output(const GemmArgs &a, f32x16 (&acc
 #pragma unroll
                         for (int rr = 0; rr < 4; rr++) {
                             float v = acc[i][j][4 * rq + rr] + bv[rr];
-                            const uint32_t soff = (uint32_t)((i * 32 + 8 * rq + rr) * a.OHW * (int)sizeof(T));
+                            const uint32_t soff = (uint32_t)((i * 32 + 8 * rq + rr) * plane * (int)sizeof(T));
                             if (SUM == 1)
                                 v = fmaf(old[i][4 * rq + rr], a.factor, v);
                             if (ACT == ACT_CLAMP) {
@@ -2861,10 +2870,10 @@ int launch_patch(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t 
 template <int BM, int BN, int WM, int WN, bool RAGGED>
 void launch_split_inst(TimingScope &ts, const GemmArgs &a, unsigned blocks, hipStream_t stream)
 {
+    void (*kernel)(GemmArgs) = conv_split_f32_kernel<BM, BN, WM, WN, false, RAGGED>;
     if (a.wdirect)
-        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, true, RAGGED>), dim3(blocks), dim3(kThreads), 0, stream, a);
-    else
-        DLP_LAUNCH_TIMED(ts, (conv_split_f32_kernel<BM, BN, WM, WN, false, RAGGED>), dim3(blocks), dim3(kThreads), 0, stream, a);
+        kernel = conv_split_f32_kernel<BM, BN, WM, WN, true, RAGGED>;
+    DLP_LAUNCH_TIMED(ts, kernel, dim3(blocks), dim3(kThreads), 0, stream, a);
 }
 
 int launch_split(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t stream)
@@ -3267,9 +3276,12 @@ int conv_gemm_pack_weights(const ConvGeom &g, const GemmPlan &p, const void *w, 
     return DLP_OK;
 }
 
-int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream)
+int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream, int *zero,
+                          int nzero)
 {
     PhasePackArgs a;
+    a.zero = zero;
+    a.nzero = nzero;
     a.n = n;
     a.cout_g = cout_g;
     a.cin_g = cin_g;
@@ -3289,6 +3301,188 @@ int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int
         return DLP_OK;
     TimingScope ts("pack_weights", stream);
     hipLaunchKernelGGL(phase_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, w, a);
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
+}
+
+// How the phases are cut: every phase in slices of about q K tiles, longest first; the cost is what split_cut counts, here by dealing the
+// workgroups out to the CUs in their order.
+static double phases_cut(const PhaseConv *ph, int n, int q, int cus, PhasesPlan &pl, long long &images)
+{
+    long long at = 0, next = 0, sliced = 0;
+    double busiest = 0.0;
+    images = 0;
+    for (int i = 0; i < n; i++) {
+        const GemmPlan &p = pl.plan[i];
+        int s = std::max(1, std::min(16, (p.nkt + q - 1) / q));
+        pl.kt_per_slice[i] = (p.nkt + s - 1) / s;
+        pl.splitk[i] = s = (p.nkt + pl.kt_per_slice[i] - 1) / pl.kt_per_slice[i];
+        const long long N = (long long)ph[i].g.B * ph[i].len_h * ph[i].len_w, wgs = (long long)ph[i].g.groups * p.mtiles * ((N + p.BN - 1) / p.BN) * s;
+        for (at += wgs; next < at; next += cus)
+            busiest += pl.kt_per_slice[i];
+        if (s > 1) {
+            sliced += wgs;
+            images += wgs;
+        }
+    }
+    const double rate = at <= cus ? 0.6 : at <= 2ll * cus ? 0.9 : 1.0;
+    return busiest / rate + (sliced ? 6.0 : 0.0) + 0.05 * sliced;
+}
+
+bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws_bytes, PhasesPlan &pl)
+{
+    if (n < 2 || n > kMaxMergedPhases || generic_act(activation))
+        return false;
+    const ConvGeom &g0 = ph[0].g;
+    const int M = g0.Cout / g0.groups;
+    int tile = 4; // of the smallest any phase would take by itself (0: the fp32 instruction)
+    for (int i = 0; i < n; i++) {
+        const ConvGeom &g = ph[i].g;
+        if (g.Cin / g.groups % BK != 0 || g.KH * g.KW > 31 || (size_t)g.B * g.Cin * g.H * g.W * 4 + ((size_t)g.ph * g.W + g.pw) * 4 >= kOutOfRange)
+            return false;
+        const GemmPlan p = conv_gemm_plan(g, activation);
+        tile = !p.split ? 0 : tile == 4 ? p.tile : tile;
+    }
+    // Tiles: what the phases would take by themselves, and 64x64 below that, measured against one launch a phase and the interleaving (transposed,
+    // packing included, us; interleaved / 64x64 / 64x128 / 128x128): 256->128 at 14x14, 4x4, batch 1 73 / 22 / 28 / 37, batch 4 77 / 26 / 31 / 40, batch
+    // 16 91 / 45 / 46 / 49; 512->256 at 7x7, 4x4, batch 8 87 / 36 / 42 / 53; 512->16 at 20x20, 3x3, batch 4 72 / 24 / 31 / 41; 128->128 at 28x28,
+    // 4x4, batch 32 175 / 120 / 115 / 108, 128->64 at 56x56 278 / 202 / 195 / 264.  No size was found where one launch a phase is the better one.
+    const int bm = tile == 4 ? 128 : 64, bn = tile == 0 ? 64 : 128;
+    pl.packed_bytes = 0;
+    long long ntiles = 0;
+    for (int i = 0; i < n; i++) {
+        const ConvGeom &g = ph[i].g;
+        GemmPlan &p = pl.plan[i];
+        p = GemmPlan();
+        p.order = GEMM_ORDER_TAP;
+        p.mask = GEMM_MASK_TAPS;
+        p.split = 1;
+        p.tile = tile;
+        p.BM = p.pack_bm = bm;
+        p.BN = bn;
+        p.M = M;
+        p.K = g.Cin / g.groups * g.KH * g.KW;
+        p.nkt = p.K / BK;
+        p.mtiles = (M + bm - 1) / bm;
+        p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * bm * 96;
+        pl.packed_bytes += p.wpack_bytes;
+        ntiles += (long long)g.groups * p.mtiles * (((long long)g.B * ph[i].len_h * ph[i].len_w + p.BN - 1) / p.BN);
+    }
+    pl.packed_bytes = (pl.packed_bytes + 255) / 256 * 256;
+    const size_t fixed = pl.packed_bytes + split_counter_bytes(ntiles);
+    if (pl.packed_bytes >= kOutOfRange || ntiles * 16 > 0x7fffffffLL || fixed > ws_bytes)
+        return false;
+    pl.counters = (int)ntiles;
+    const size_t image = (size_t)bm * bn * sizeof(float);
+    const long long room = (long long)(std::min<size_t>(ws_bytes - fixed, kOutOfRange - 1) / image);
+    int longest = 0, best_q = 0;
+    for (int i = 0; i < n; i++)
+        longest = std::max(longest, pl.plan[i].nkt);
+    double best = 0.0;
+    long long images = 0;
+    for (int s = 1; s <= 16 && (s == 1 || longest / s >= 8); s++) {
+        const int q = (longest + s - 1) / s;
+        const double cost = phases_cut(ph, n, q, device_cu_count(), pl, images);
+        if (images <= room && (best_q == 0 || cost < best)) {
+            best = cost;
+            best_q = q;
+        }
+    }
+    phases_cut(ph, n, best_q, device_cu_count(), pl, images);
+    pl.bytes = fixed + (size_t)images * image;
+    return true;
+}
+
+int conv_gemm_phases_launch(const PhaseConv *ph, int n, const PhasesPlan &pl, const void *dy, const void *packed, int *counters, float *images, void *dx,
+                            int out_h, int out_w, int out_sh, int out_sw, const Epilogue &ep, hipStream_t stream)
+{
+    const ConvGeom &g = ph[0].g;
+    PhasesArgs args;
+    GemmArgs &a = args.a;
+    a = GemmArgs();
+    a.x = dy;
+    a.wp = (const float *)packed;
+    a.bias = ep.bias;
+    a.y = dx;
+    a.M = pl.plan[0].M;
+    a.mtiles = pl.plan[0].mtiles;
+    a.Cout = g.Cout;
+    a.groups = g.groups;
+    a.Cin = g.Cin;
+    a.Cin_g = g.Cin / g.groups;
+    a.H = g.H;
+    a.W = g.W;
+    a.sh = a.sw = 1;
+    a.pack_bm = pl.plan[0].pack_bm;
+    a.pack_mtiles = a.mtiles;
+    a.x_bytes = (uint32_t)((size_t)g.B * g.Cin * g.H * g.W * 4);
+    a.wp_bytes = (uint32_t)pl.packed_bytes;
+    a.y_bytes = (uint32_t)((size_t)g.B * g.Cout * out_h * out_w * 4);
+    a.hw4 = (uint32_t)(g.H * g.W * 4);
+    a.out_hw = out_h * out_w;
+    a.out_w = out_w;
+    a.out_sh = out_sh;
+    a.out_sw = out_sw;
+    a.factor = ep.factor;
+    a.act = ep.activation;
+    a.clamp_lo = -__builtin_huge_valf();
+    a.clamp_hi = __builtin_huge_valf();
+    if (ep.activation == DLP_ACT_RELU || ep.activation == DLP_ACT_RELU6)
+        a.clamp_lo = 0.0f;
+    if (ep.activation == DLP_ACT_RELU6)
+        a.clamp_hi = 6.0f;
+    a.sk_cnt = counters;
+    a.sk_part = images;
+    a.sk_part_bytes = (uint32_t)(pl.bytes - pl.packed_bytes - split_counter_bytes(pl.counters));
+    make_magic((uint32_t)a.mtiles, a.mt_magic, a.mt_shift);
+    args.n = n;
+    long long blocks = 0, image0 = 0;
+    size_t wp = 0;
+    int counter0 = 0;
+    for (int i = 0; i < n; i++) {
+        SplitPhase &p = args.ph[i];
+        const GemmPlan &t = pl.plan[i];
+        p.ktab = (const int32_t *)ph[i].ktab;
+        p.wp_offset = (uint32_t)wp;
+        wp += t.wpack_bytes;
+        p.nkt = t.nkt;
+        p.N = g.B * ph[i].len_h * ph[i].len_w;
+        p.ntiles = (p.N + t.BN - 1) / t.BN;
+        p.KH = ph[i].g.KH; p.KW = ph[i].g.KW; p.ph = ph[i].g.ph; p.pw = ph[i].g.pw; p.dh = ph[i].g.dh; p.dw = ph[i].g.dw;
+        p.off_h = ph[i].off_h; p.off_w = ph[i].off_w; p.OW = ph[i].len_w; p.OHW = ph[i].len_h * ph[i].len_w; p.out_off = ph[i].out_off;
+        p.x_shift = (uint32_t)((p.ph * g.W + p.pw) * 4);
+        const int tiles = t.mtiles * p.ntiles * g.groups;
+        make_magic((uint32_t)p.OHW, p.ohw_magic, p.ohw_shift);
+        make_magic((uint32_t)p.OW, p.ow_magic, p.ow_shift);
+        make_magic((uint32_t)p.ntiles, p.ntl_magic, p.ntl_shift);
+        make_magic((uint32_t)tiles, p.tm_magic, p.tm_shift);
+        p.splitk = pl.splitk[i];
+        p.kt_per_slice = pl.kt_per_slice[i];
+        p.block0 = (int)blocks;
+        p.blocks = tiles * p.splitk;
+        p.counter0 = counter0;
+        p.image0 = (uint32_t)image0;
+        blocks += p.blocks;
+        counter0 += tiles;
+        image0 += p.splitk > 1 ? p.blocks : 0;
+    }
+    TimingScope ts("conv_gemm", stream);
+    const bool ragged = (a.M & 7) != 0;
+    const dim3 grid((unsigned)blocks), block(kThreads);
+    void (*kernel)(PhasesArgs);
+    if (pl.plan[0].tile == 4 && ragged)
+        kernel = conv_split_f32_kernel<128, 128, 2, 2, false, true>;
+    else if (pl.plan[0].tile == 4)
+        kernel = conv_split_f32_kernel<128, 128, 2, 2, false, false>;
+    else if (pl.plan[0].tile == 5 && ragged)
+        kernel = conv_split_f32_kernel<64, 128, 1, 4, false, true>;
+    else if (pl.plan[0].tile == 5)
+        kernel = conv_split_f32_kernel<64, 128, 1, 4, false, false>;
+    else if (ragged)
+        kernel = conv_phases_f32_kernel<64, 64, 2, 2, true>;
+    else
+        kernel = conv_phases_f32_kernel<64, 64, 2, 2, false>;
+    DLP_LAUNCH_TIMED(ts, kernel, grid, block, 0, stream, args);
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
 }

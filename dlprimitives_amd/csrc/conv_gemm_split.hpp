@@ -69,10 +69,13 @@ __device__ __forceinline__ void split8_weights(const float *v, u32x4 (&o)[3])
     }
 }
 
-template <int BM, int BN, int WM, int WN, bool ADIR, bool RAGGED>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_split_f32_kernel(GemmArgs a)
+// PHASED: the workgroups of one of several convolutions of one launch (conv_phases_f32_kernel): `a` is that convolution, its workgroups are
+// numbered from zero, its counters and images begin at a.sk_cnt and image_base.
+template <int BM, int BN, int WM, int WN, bool ADIR, bool RAGGED, bool PHASED>
+__device__ __forceinline__ void conv_split_tile(const GemmArgs &a, const int bid, const uint32_t image_base)
 {
-    static_assert(WM * WN == 4 && BN == 128 && (BM == 64 || BM == 128), "tile shape");
+    static_assert(WM * WN == 4 && (BN == 128 || BN == 64) && (BM == 64 || BM == 128), "tile shape");
+    constexpr int CH = BN / 16; // channels of its pixel that a thread loads
     constexpr int WTM = BM / WM, WTN = BN / WN;
     constexpr int TM = WTM / 32, TN = WTN / 32;
     constexpr int A_BYTES = BM * 96, B_BYTES = BN * 96, BUF = A_BYTES + B_BYTES;
@@ -94,15 +97,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     uint32_t image0;
     {
         const int tiles = a.mtiles * a.ntiles * a.groups, tiles_main = tiles - a.tail_tiles;
-        const int bid = blockIdx.x;
-        if (bid < a.main_wgs) {
+        if (PHASED || bid < a.main_wgs) {
             const int nb = a.main_wgs;
             const int q = nb >> 3, r = nb & 7;
             const int xcd = bid & 7, slot = bid >> 3;
             t = (xcd < r) ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
             slice = (int)fast_div((uint32_t)t, a.tm_magic, a.tm_shift);
             t -= slice * tiles_main;
-            image0 = (uint32_t)(t * splitk);
+            image0 = image_base + (uint32_t)(t * splitk);
         } else {
             t = bid - a.main_wgs;
             slice = (int)fast_div((uint32_t)t, a.tt_magic, a.tt_shift);
@@ -130,7 +132,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
     // ---- the input: one output pixel per thread, its window origin and the mask of its taps inside the image ----
     const int p = tid % BN;
-    const int half = __builtin_amdgcn_readfirstlane(tid / BN); // of a K tile's channels
+    const int part = __builtin_amdgcn_readfirstlane(tid / BN); // of a K tile's channels, CH of them
     uint32_t vbase, my = 0;
     {
         const int n = n0 + p;
@@ -138,15 +140,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const int pix = n - b * a.OHW;
         const int oy = (int)fast_div((uint32_t)pix, a.ow_magic, a.ow_shift);
         const int ox = pix - oy * a.OW;
-        vbase = (uint32_t)((((b * a.Cin + g * a.Cin_g) * a.H + oy * a.sh) * a.W + ox * a.sw) * 4);
+        const int iy = PHASED ? oy + a.off_h : oy * a.sh, ix = PHASED ? ox + a.off_w : ox * a.sw;
+        vbase = (uint32_t)((((b * a.Cin + g * a.Cin_g) * a.H + iy) * a.W + ix) * 4);
         if (n < a.N) {
             uint32_t rx = 0;
             for (int kx = 0; kx < a.KW; kx++) {
-                const int xx = ox * a.sw - a.pw + kx * a.dw;
+                const int xx = ix - a.pw + kx * a.dw;
                 rx |= (xx >= 0 && xx < a.W ? 1u : 0u) << kx;
             }
             for (int ky = 0; ky < a.KH; ky++) {
-                const int yy = oy * a.sh - a.ph + ky * a.dh;
+                const int yy = iy - a.ph + ky * a.dh;
                 if (yy >= 0 && yy < a.H)
                     my |= rx << (ky * a.KW);
             }
@@ -168,7 +171,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                             : kOutOfRange;
     }
 
-    float rb[8];
+    float rb[CH];
     u32x4 ra[A_LD];
     float largest = 0.0f; // ADIR: of this thread's operands
     auto load_b = [&](int kt) {
@@ -177,8 +180,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)my, tap, 1u);
         const uint32_t v = opaque((vbase & m) | (kOutOfRange & ~m));
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            rb[i] = buf_load<float>(xr, v, xoff + (uint32_t)(half * 8 + i) * a.hw4);
+        for (int i = 0; i < CH; i++)
+            rb[i] = buf_load<float>(xr, v, xoff + (uint32_t)(part * CH + i) * a.hw4);
     };
     auto load_a = [&](int kt) {
         const uint32_t soff = a_row_base + (uint32_t)min(kt, a.nkt - 1) * a_tile_bytes;
@@ -209,12 +212,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         }
         if (ADIR)
 #pragma unroll
-            for (int i = 0; i < 8; i += 2)
+            for (int i = 0; i < CH; i += 2)
                 largest = split_largest(largest, rb[i], rb[i + 1]);
-        split8(rb, o);
+        if constexpr (CH == 8) {
+            split8(rb, o);
 #pragma unroll
-        for (int pl = 0; pl < 3; pl++)
-            *(u32x4 *)(buf + A_BYTES + ((pl * 2 + half) * BN + p) * 16) = o[pl];
+            for (int pl = 0; pl < 3; pl++)
+                *(u32x4 *)(buf + A_BYTES + ((pl * 2 + part) * BN + p) * 16) = o[pl];
+        } else {
+            uint32_t lo[3], hi[3];
+            split_pair(rb[0], rb[1], lo);
+            split_pair(rb[2], rb[3], hi);
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++)
+                *(u32x2 *)(buf + A_BYTES + ((pl * 2 + part / 2) * BN + p) * 16 + part % 2 * 8) = (u32x2){lo[pl], hi[pl]};
+        }
     };
     // the five small products are summed on their own: in one accumulator with the large one, every step would round the sum six
     // times as often, at its full size
@@ -343,8 +355,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                     Af[(ahalf * 8 + e) * BM + arow] = v[e];
             }
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-                Bf[(half * 8 + i) * BN + p] = rb[i];
+            for (int i = 0; i < CH; i++)
+                Bf[(part * CH + i) * BN + p] = rb[i];
             __syncthreads();
 #pragma unroll
             for (int kk = 0; kk < BK / 2; kk++)
@@ -357,8 +369,71 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             __syncthreads();
         }
     }
-    gemm_tile_output<float, BM, BN, WM, WN, ACT_CLAMP, RAGGED>(a, acc, reinterpret_cast<float *>(smem), m0, n0, g, slice, splitk, image0, wm, wn, h,
-                                                               l32, tid, bias_early);
+    gemm_tile_output<float, BM, BN, WM, WN, ACT_CLAMP, RAGGED, PHASED>(a, acc, reinterpret_cast<float *>(smem), m0, n0, g, slice, splitk, image0, wm, wn,
+                                                                       h, l32, tid, bias_early);
+}
+
+template <int BM, int BN, int WM, int WN, bool ADIR, bool RAGGED>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_split_f32_kernel(GemmArgs a)
+{
+    conv_split_tile<BM, BN, WM, WN, ADIR, RAGGED, false>(a, blockIdx.x, 0);
+}
+
+// All stride phases of a backward-data pass or transposed convolution in one launch: stride-1 convolutions of one input with filters,
+// extents and paddings of their own, every one storing its share of the pixels of y, with bias, activation and old value.  One launch a phase
+// into planes that another kernel interleaved left the chip half empty four times over (BM x BN tiles of one phase: 100 to 230 workgroups)
+// and took the output through memory twice more.
+struct SplitPhase {
+    const int32_t *ktab;
+    uint32_t wp_offset; // bytes into the packed weights
+    int nkt, N, ntiles, KH, KW, ph, pw, dh, dw, off_h, off_w, OW, OHW, out_off;
+    uint32_t x_shift, ohw_magic, ohw_shift, ow_magic, ow_shift, ntl_magic, ntl_shift, tm_magic, tm_shift;
+    int block0, blocks;    // workgroups
+    int splitk, kt_per_slice, counter0;
+    uint32_t image0;
+};
+constexpr int kMaxMergedPhases = 9;
+struct PhasesArgs {
+    GemmArgs a; // what the phases have in common
+    int n;
+    SplitPhase ph[kMaxMergedPhases];
+};
+template <int BM, int BN, int WM, int WN, bool RAGGED>
+__device__ __forceinline__ void conv_phases_tile(const PhasesArgs &args)
+{
+    int i = 0;
+    while (i + 1 < args.n && (int)blockIdx.x >= args.ph[i + 1].block0)
+        i++;
+    const SplitPhase &p = args.ph[i];
+    GemmArgs a = args.a;
+    a.ktab = p.ktab;
+    a.wp = (const float *)((const char *)a.wp + p.wp_offset);
+    a.wp_bytes -= p.wp_offset;
+    a.nkt = p.nkt;
+    a.N = p.N;
+    a.ntiles = p.ntiles;
+    a.KH = p.KH; a.KW = p.KW; a.ph = p.ph; a.pw = p.pw; a.dh = p.dh; a.dw = p.dw;
+    a.off_h = p.off_h; a.off_w = p.off_w; a.OW = p.OW; a.OHW = p.OHW; a.out_off = p.out_off;
+    a.x_shift = p.x_shift;
+    a.ohw_magic = p.ohw_magic; a.ohw_shift = p.ohw_shift; a.ow_magic = p.ow_magic; a.ow_shift = p.ow_shift;
+    a.ntl_magic = p.ntl_magic; a.ntl_shift = p.ntl_shift; a.tm_magic = p.tm_magic; a.tm_shift = p.tm_shift;
+    a.splitk = p.splitk;
+    a.kt_per_slice = p.kt_per_slice;
+    a.tail_tiles = 0;
+    a.main_wgs = p.blocks;
+    a.sk_cnt = p.splitk > 1 ? a.sk_cnt + p.counter0 : nullptr;
+    conv_split_tile<BM, BN, WM, WN, false, RAGGED, true>(a, (int)blockIdx.x - p.block0, p.image0);
+}
+// tiles as conv_split_f32_kernel has them for one convolution, and smaller ones for launches below its sizes
+template <int BM, int BN, int WM, int WN, bool ADIR, bool RAGGED>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_split_f32_kernel(PhasesArgs args)
+{
+    conv_phases_tile<BM, BN, WM, WN, RAGGED>(args);
+}
+template <int BM, int BN, int WM, int WN, bool RAGGED>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_phases_f32_kernel(PhasesArgs args)
+{
+    conv_phases_tile<BM, BN, WM, WN, RAGGED>(args);
 }
 
 // Weights -> [group][m tile][K tile][piece][half][row][8 channels of one tap], zero padded.  One workgroup moves 16 filters x 16 channels
@@ -440,10 +515,14 @@ struct PhasePack {
 };
 struct PhasePackArgs {
     int n, cout_g, cin_g, KH, KW;
+    int *zero; // tile counters of the launch that follows
+    int nzero;
     PhasePack ph[kMaxPhases];
 };
 __global__ __launch_bounds__(256) void phase_pack_kernel(const float *__restrict__ w, PhasePackArgs a)
 {
+    for (int z = blockIdx.x * 256 + threadIdx.x; z < a.nzero; z += gridDim.x * 256)
+        a.zero[z] = 0;
     int i = 0;
     while (i + 1 < a.n && blockIdx.x >= a.ph[i + 1].block0)
         i++;

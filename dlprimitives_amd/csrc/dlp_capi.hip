@@ -288,6 +288,14 @@ bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan)
     return plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise;
 }
 
+bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab)
+{
+    const int x_shape[4] = {batch, op->cfg.channels_in, op->cfg.shape[2], op->cfg.shape[3]};
+    GemmPlan plan;
+    *ktab = op->ktab;
+    return conv_fwd_tiles_plan(op, batch, &plan) && op_geom(op, x_shape, g) == DLP_OK;
+}
+
 size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op)
 {
     ConvGeom g;

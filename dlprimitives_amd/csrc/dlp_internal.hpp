@@ -283,7 +283,29 @@ struct PhaseFilter {
     int nh, nw, rh0, rhstep, rw0, rwstep;
 };
 // packs the filters of n phases from w[groups * cout_g][cin_g][KH][KW] in one launch; plans as conv_fwd_tiles_plan gives them
-int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream);
+// (zero: nzero ints to clear along the way)
+int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int KH, int KW, const PhaseFilter *ph, int n, hipStream_t stream,
+                          int *zero = nullptr, int nzero = 0);
+// All phases in one launch that stores dx itself (conv_phases_f32_kernel).  A phase: its convolution of dy, of whose outputs those of len_h rows
+// from off_h on and len_w columns from off_w on are pixels (i * out_sh, j * out_sw) of dx + out_off.
+struct PhaseConv {
+    ConvGeom g;
+    const KTabEntry *ktab;
+    int off_h, off_w, len_h, len_w, out_off;
+};
+struct PhasesPlan {
+    GemmPlan plan[kMaxPhases];     // tiles that conv_gemm_pack_phases writes, one phase behind the other
+    int splitk[kMaxPhases], kt_per_slice[kMaxPhases];
+    size_t packed_bytes, bytes;    // of the workspace: packed filters | tile counters | accumulator images
+    int counters;
+};
+// whether the phases run that way, in as many K slices as pay within ws_bytes of workspace
+bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws_bytes, PhasesPlan &plan);
+// dx: planes of out_h x out_w pixels
+int conv_gemm_phases_launch(const PhaseConv *ph, int n, const PhasesPlan &plan, const void *dy, const void *packed, int *counters, float *images, void *dx,
+                            int out_h, int out_w, int out_sh, int out_sw, const Epilogue &ep, hipStream_t stream);
+// the gather table of an operator that conv_fwd_tiles_plan accepts, and the geometry of its convolution at this batch
+bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab);
 // Whether a call at this batch can run on tiles that conv_gemm_pack_phases writes, and by which plan (float, algorithm gemm, K tiles of one
 // tap x 16 channels; not where the kernel of the call reads the filter as it is, which depends on the batch too).
 bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan);
