@@ -1391,6 +1391,8 @@ __device__ __forceinline__ void bf16_tile_output(const GemmArgs &a, f32x16 (&acc
     }
 }
 
+#include "conv_gemm_wave.hpp"
+
 // PXL > 0 selects the dense loader (1x1, stride 1, no padding: a plain GEMM W * X per image):
 // a lane loads PXL consecutive pixels of 8 consecutive channels with 8- or 16-byte loads (the
 // texture path handles four lanes per clock whatever the width of the load, so a 16-bit load per
@@ -2688,7 +2690,57 @@ size_t xt_bytes(const ConvGeom &g, int batch)
     return ((size_t)batch * t.H * t.W * g.Cin * sizeof(bf16_t) + 255) / 256 * 256;
 }
 
-int launch_bf16_mfma(const ConvGeom &g, const GemmPlan &p, int pxl, GemmArgs &a, hipStream_t stream, void *xt)
+template <int TILE, int KW>
+void launch_wave_bf16(TimingScope &ts, const GemmArgs &a, unsigned blocks, hipStream_t stream)
+{
+    if (a.y_cl)
+        DLP_LAUNCH_TIMED(ts, (conv_wave_bf16_kernel<TILE, KW, true>), dim3(blocks), dim3(KW * 64), 0, stream, a);
+    else
+        DLP_LAUNCH_TIMED(ts, (conv_wave_bf16_kernel<TILE, KW, false>), dim3(blocks), dim3(KW * 64), 0, stream, a);
+}
+
+// Whether a channels-last input of N pixels is convolved in 32x32 tiles (conv_wave_bf16_kernel).  The time of such a launch goes with tiles x K
+// tiles, 3 us + 0.35 us per thousand; what the tiles of 128x128 or 64x256 take hardly depends on the batch until they fill the chip.  Layers
+// of ResNet-50, us, those / these: 3x3 512->512 at 7x7 (144 K tiles) batch 1 13.9 / 6.4, batch 16 24.5 / 16.7, batch 32 28.3 / 28.3; 1x1
+// 1024->256 at 14x14 (32) batch 1 10.2 / 3.8, 16 17.6 / 13.5, 32 22.9 / 20.6; 1x1 512->256 at 28x28 (16) batch 8 19.1 / 12.8, 32 15.2 / 35.4.
+// Short reductions end sooner: 1x1 256->64 at 56x56 (8) batch 4 7.4 / 5.6, 8 7.8 / 7.4, 16 8.8 / 13.7; 64->256 (2) batch 1 5.2 / 4.5, 4 5.9 / 8.7.
+bool bf16_wave(const GemmPlan &p, long long N, int groups)
+{
+    const long long tiles = (long long)groups * ((p.M + 31) / 32) * ((N + 31) / 32);
+    return p.nkt >= 16 ? tiles * p.nkt <= 58000 : tiles <= (p.nkt >= 8 ? 1600 : 1000);
+}
+
+int launch_wave_bf16(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t stream)
+{
+    // tiles of 16x16 where those of 32x32 would leave half of the CUs idle through a long reduction: every CU reads at its own rate (3x3 512->512
+    // at 7x7, one image: 32 tiles 9.8 us, 128 of 16x16 6.2; 1x1 512->256 at 28x28, 200 tiles 4.3, 700 of 16x16 4.6)
+    const bool small = (long long)g.groups * ((p.M + 31) / 32) * ((a.N + 31) / 32) <= 128 && p.nkt >= 16;
+    const int tile = small ? 16 : 32;
+    a.mtiles = (p.M + tile - 1) / tile;
+    a.ntiles = (a.N + tile - 1) / tile;
+    set_tile_magics(a, g.groups);
+    make_magic((uint32_t)(a.nkt / (g.KH * g.KW)), a.ncb_magic, a.ncb_shift);
+    const long long tiles = (long long)a.mtiles * a.ntiles * g.groups;
+    if (tiles > 0x7fffffffLL)
+        return fail(DLP_ERR_NOT_IMPLEMENTED, "convolution too large for a single launch");
+    TimingScope ts("conv_gemm", stream);
+    // more wavefronts share a reduction where few workgroups do not fill the CUs with wavefronts (3x3 512->512 at 7x7, batch 8, 208 tiles: 17.2 / 11.9 /
+    // 10.2 us with 2 / 4 / 8; 64->256 at 56x56, one image, 784 tiles of two K tiles: 4.5 / 4.9 / 7.3)
+    if (small && p.nkt < 24)
+        launch_wave_bf16<16, 4>(ts, a, (unsigned)tiles, stream);
+    else if (small)
+        launch_wave_bf16<16, 8>(ts, a, (unsigned)tiles, stream);
+    else if (tiles <= 256 && p.nkt >= 32)
+        launch_wave_bf16<32, 8>(ts, a, (unsigned)tiles, stream);
+    else if (tiles <= 512)
+        launch_wave_bf16<32, 4>(ts, a, (unsigned)tiles, stream);
+    else
+        launch_wave_bf16<32, 2>(ts, a, (unsigned)tiles, stream);
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
+}
+
+int launch_bf16_mfma(const ConvGeom &g, const GemmPlan &p, int pxl, GemmArgs &a, hipStream_t stream, void *xt, bool wave)
 {
     long long blocks = (long long)a.mtiles * a.ntiles * g.groups * a.splitk;
     if (blocks > 0x7fffffffLL)
@@ -2726,6 +2778,8 @@ int launch_bf16_mfma(const ConvGeom &g, const GemmPlan &p, int pxl, GemmArgs &a,
         a.x_shift = (uint32_t)(((size_t)g.ph * t.W + g.pw) * g.Cin * sizeof(bf16_t));
         a.ktab += (p.nkt + 2) * BK2; // the second table of conv_gemm_fill_ktab
     }
+    if (wave)
+        return launch_wave_bf16(g, p, a, stream);
     {
         TimingScope ts("conv_gemm", stream);
         const Bf16Kernel kernel = bf16_kernel(p.tile, p.order, pxl, p.dense_sx, xt != nullptr);
@@ -3612,7 +3666,8 @@ int conv_gemm_launch(const ConvGeom &g, const GemmPlan &p, const KTabEntry *dev_
         part_bytes -= xt_bytes(g, g.B);
         a.part = (float *)part_ws;
     }
-    plan_split(p, a, g.groups, part_ws != nullptr, part_bytes);
+    const bool wave = xt != nullptr && a.y_bytes != 0 && bf16_wave(p, a.N, g.groups);
+    plan_split(p, a, g.groups, part_ws != nullptr && !wave, part_bytes);
     a.sk_cnt = nullptr;
     a.part_bytes = 0;
     if ((a.splitk > 1 || a.tail_tiles > 0) && !bf16_mfma_order(p.order)) {
@@ -3645,7 +3700,7 @@ int conv_gemm_launch(const ConvGeom &g, const GemmPlan &p, const KTabEntry *dev_
         if (p.patch_bf16 && ((uintptr_t)x & 3) == 0)
             return launch_patch_bf16(g, p, a, stream);
         const int pxl = ((uintptr_t)x & 3) == 0 ? p.dense_pxl : 0;
-        return launch_bf16_mfma(g, p, pxl, a, stream, xt);
+        return launch_bf16_mfma(g, p, pxl, a, stream, xt, wave);
     }
     if (p.split)
         return launch_split(g, p, a, stream);
