@@ -103,6 +103,9 @@ def lib():
             getattr(L, pre + "destroy").restype = None
         L.dlp_bias_bwd_enqueue.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float,
                                            ctypes.c_void_p]
+        L.dlp_conv2d_fwd_enqueue_packed.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                                    ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_float,
+                                                    ctypes.c_void_p]
         L.dlp_conv2d_output_shape.argtypes = [ctypes.POINTER(_Settings), ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]
         L.dlp_ip_fwd_create.argtypes = [ctypes.POINTER(_IPSettings), ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_void_p)]
         L.dlp_ip_fwd_enqueue.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
@@ -176,7 +179,8 @@ def _stream(stream):
     if stream is None:
         import torch
 
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        # the handle of torch.cuda.current_stream() without the Stream object around it: 0.4 us instead of 2.8, of the 9 a call takes
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return ctypes.c_void_p(int(stream))
 
 
@@ -273,9 +277,6 @@ class Conv2DForward:
 
     def enqueue_packed(self, x, w, packed, bias, y, ws=None, factor=0.0, stream=None):
         """enqueue() on weights that pack() transformed earlier; ws is per-call scratch only"""
-        lib().dlp_conv2d_fwd_enqueue_packed.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
-                                                        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_float,
-                                                        ctypes.c_void_p]
         xs = self._x_shape(x)
         ws_bytes = ws.numel() * ws.element_size() if ws is not None else 0
         _check(lib().dlp_conv2d_fwd_enqueue_packed(self._h, xs, _ptr(x), _ptr(w), _ptr(packed), _ptr(bias), _ptr(y), _ptr(ws), ws_bytes,

@@ -2817,7 +2817,10 @@ static int strided_patch_rows(const ConvGeom &g)
     if (ohw > (1 << 16))
         return 1 << 30;
     int worst = 0;
-    for (int nt = 0; nt < ohw; nt++) { // n0 = 64 nt takes every residue modulo the plane that a tile start can have
+    int tiles = ohw; // n0 = 64 nt takes every residue modulo the plane that a tile start can have, then repeats
+    for (int two = 0; two < 6 && tiles % 2 == 0; two++)
+        tiles /= 2;
+    for (int nt = 0; nt < tiles; nt++) {
         const long long n0 = 64ll * nt, n_last = n0 + 63;
         const long long b0 = n0 / ohw;
         int total = 0;
@@ -3055,7 +3058,7 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
             }
         }
         // stride-1 3x3 "same" convolutions whose largest patch fits the LDS rows and one block per lane: LDS-patch kernel
-        if (tap_major && g.KH == 3 && g.KW == 3 && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && g.ph == 1 && g.pw == 1 &&
+        if (tap_major && !g.x_channels_last && g.KH == 3 && g.KW == 3 && g.sh == 1 && g.sw == 1 && g.dh == 1 && g.dw == 1 && g.ph == 1 && g.pw == 1 &&
             (g.H * g.W) % 4 == 0 && g.B > 0) {
             const int pxp = (g.H * g.W) % 8 == 0 ? 8 : 4;
             const int BN = p.tile == 2 ? 128 : 256, pitch = p.tile == 2 ? kPatchPitchBf16_128 : kPatchPitchBf16_256;
