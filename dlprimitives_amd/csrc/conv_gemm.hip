@@ -2740,6 +2740,22 @@ int launch_wave_bf16(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStrea
     return DLP_OK;
 }
 
+template <int TILE, int KW>
+int launch_wave_f32(const GemmArgs &a, unsigned blocks, hipStream_t stream)
+{
+    constexpr int KT = TILE == 32 ? 16 : 32;
+    constexpr size_t operands = (size_t)KW * TILE * KT * 4, sums = (size_t)KW * TILE * TILE * 4;
+    const bool point = a.KH * a.KW == 1;
+    const size_t lds = std::max(operands, sums) + (point ? 0 : (size_t)(a.K + KT - 1) / KT * KT * 8);
+    void (*kernel)(GemmArgs) = conv_wave_f32_kernel<TILE, KW, false>;
+    if (point)
+        kernel = conv_wave_f32_kernel<TILE, KW, true>;
+    TimingScope ts("conv_gemm", stream);
+    DLP_LAUNCH_TIMED(ts, kernel, dim3(blocks), dim3(KW * 64), lds, stream, a);
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
+}
+
 int launch_bf16_mfma(const ConvGeom &g, const GemmPlan &p, int pxl, GemmArgs &a, hipStream_t stream, void *xt, bool wave)
 {
     long long blocks = (long long)a.mtiles * a.ntiles * g.groups * a.splitk;
@@ -3542,6 +3558,86 @@ int conv_gemm_phases_launch(const PhaseConv *ph, int n, const PhasesPlan &pl, co
     DLP_LAUNCH_TIMED(ts, kernel, grid, block, 0, stream, args);
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
+}
+
+// Which float convolutions run on conv_wave_f32_kernel: long reductions in few tiles.  Its time goes with U = tiles of 32x32 x K tiles of 16,
+// about 4 us + 0.35 us per thousand; the other kernels take 9 to 30 us however small the layer, and a packing launch where the filter comes
+// raw.  Measured, us, raw filters, others / this one: 3x3 512->512 at 7x7 batch 1 (U 9200) 26 / 21, 256->256 at 14x14 batch 1 20 / 13, batch 4
+// (29000) 22 / 19, 64->64 at 56x56 batch 1 16 / 10, batch 4 (28000) 16 / 19, 160->100 at 17x17 batch 8 (26000) 25 / 21; 1x1 1024->256 at 14x14 batch 1
+// 17 / 6, batch 16 (50000) 26 / 28, 256->64 at 56x56 batch 2 (6300, 16 K tiles) 9.3 / 7.0, 192->32 at 28x28 batch 32 (9400, 12) 8.8 / 10.5, 64->256 at 56x56 (4) 5.3 / 8;
+// channels off multiples of 16, which the others gather k by k: 3x3 52->16 at 107x107 batch 5 (54000) 31 / 26, 215->489 at 7x8 33 / 14.  With filters
+// packed ahead: 3x3 64->64 at 56x56 batch 1 13 / 10, 512->512 at 7x7 (32 tiles) 18 / 21.
+bool conv_wave_f32_serves(const ConvGeom &g, bool packed)
+{
+    const int cin_g = g.Cin / g.groups, M = g.Cout / g.groups, taps = g.KH * g.KW;
+    const long long K = (long long)cin_g * taps;
+    if (g.dtype != DLP_FLOAT || g.B <= 0 || taps > 31 || K > 8192 || conv_stem_supported(g) || (cin_g == 1 && M == 1))
+        return false;
+    const long long N = (long long)g.B * g.OH * g.OW;
+    if (((size_t)g.B * g.Cin * g.H * g.W + (size_t)g.ph * g.W + g.pw) * 4 >= kOutOfRange || (size_t)N * g.Cout * 4 >= kOutOfRange ||
+        (size_t)g.Cout * K * 4 >= kOutOfRange)
+        return false;
+    const long long tiles = (long long)g.groups * ((M + 31) / 32) * ((N + 31) / 32), kt = (K + 15) / 16, u = tiles * kt;
+    if (taps == 1) // (not filters that leave conv_gemm_f32_kernel's last tile of 64 half empty: it has tiles of 32 rows for those)
+        return kt >= 14 && (M <= 32 || M % 64 == 0 || M % 64 > 32) && u <= (kt >= 32 ? 20000 : 8000);
+    if (kt < 9)
+        return false;
+    if (cin_g % BK != 0)
+        return u <= 54000;
+    if (kt < 14 && M <= 32) // 3x3 of 16 channels: 64 filters at 40x40, batch 6, 26 / 10; 16 at 60x60, batch 12, 14 / 16
+        return false;
+    return packed ? u <= 10000 && tiles >= 48 : u <= 24000;
+}
+
+int conv_wave_f32_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream)
+{
+    GemmArgs a = GemmArgs();
+    a.x = x;
+    a.wp = (const float *)w;
+    a.bias = ep.bias;
+    a.y = y;
+    a.M = g.Cout / g.groups;
+    a.K = g.Cin / g.groups * g.KH * g.KW;
+    a.N = g.B * g.OH * g.OW;
+    a.Cout = g.Cout;
+    a.groups = g.groups;
+    a.Cin = g.Cin;
+    a.Cin_g = g.Cin / g.groups;
+    a.H = g.H;
+    a.W = g.W;
+    a.OW = g.OW;
+    a.OHW = g.OH * g.OW;
+    a.sh = g.sh; a.sw = g.sw; a.ph = g.ph; a.pw = g.pw; a.dh = g.dh; a.dw = g.dw;
+    a.KH = g.KH; a.KW = g.KW;
+    a.x_bytes = (uint32_t)((size_t)g.B * g.Cin * g.H * g.W * 4);
+    a.wp_bytes = (uint32_t)((size_t)g.Cout * a.K * 4);
+    a.y_bytes = (uint32_t)((size_t)a.N * g.Cout * 4);
+    a.x_shift = (uint32_t)((g.ph * g.W + g.pw) * 4);
+    a.hw4 = (uint32_t)(g.H * g.W * 4);
+    make_magic((uint32_t)a.OHW, a.ohw_magic, a.ohw_shift);
+    make_magic((uint32_t)a.OW, a.ow_magic, a.ow_shift);
+    make_magic((uint32_t)(g.KH * g.KW), a.ncb_magic, a.ncb_shift);
+    make_magic((uint32_t)g.KW, a.nt_magic, a.nt_shift);
+    a.factor = ep.factor;
+    a.pre = ep.accumulate_first;
+    a.act = ep.activation;
+    a.clamp_lo = -__builtin_huge_valf();
+    a.clamp_hi = __builtin_huge_valf();
+    if (ep.activation == DLP_ACT_RELU || ep.activation == DLP_ACT_RELU6)
+        a.clamp_lo = 0.0f;
+    if (ep.activation == DLP_ACT_RELU6)
+        a.clamp_hi = 6.0f;
+    // tiles of 16x16 where those of 32x32 would leave half of the CUs idle (3x3 256->256 at 14x14, one image, 56 tiles: 18.3 us, in tiles of 16x16 12.7;
+    // 64->64 at 56x56, 196 tiles: 10.1 and 11.8); four wavefronts for short reductions (15 K tiles, 750 tiles: 11.8 us, eight 12.4)
+    const long long tiles32 = (long long)g.groups * ((a.M + 31) / 32) * ((a.N + 31) / 32);
+    const int tile = tiles32 <= 128 ? 16 : 32;
+    a.mtiles = (a.M + tile - 1) / tile;
+    a.ntiles = (a.N + tile - 1) / tile;
+    set_tile_magics(a, g.groups);
+    const unsigned tiles = (unsigned)((long long)a.mtiles * a.ntiles * g.groups); // (conv_wave_f32_serves bounds them)
+    if (tile == 16)
+        return launch_wave_f32<16, 8>(a, tiles, stream);
+    return a.K > 15 * 16 ? launch_wave_f32<32, 8>(a, tiles, stream) : launch_wave_f32<32, 4>(a, tiles, stream);
 }
 
 // Channels-last x and / or y: served by the bf16 matrix-instruction kernels only (x: the channels-last loader, i.e. input

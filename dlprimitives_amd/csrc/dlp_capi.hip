@@ -107,6 +107,7 @@ struct dlp_conv2d_fwd {
     bool bias;
     int activation;
     ConvAlgo algo;
+    bool automatic; // the algorithm was not asked for by name
     int device;
     KTabEntry *ktab; // device gather table of the GEMM stage
     WinoPlan wino;
@@ -285,15 +286,17 @@ bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan)
     if (op->algo != ALGO_GEMM || op_geom(op, x_shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
         return false;
     *plan = conv_gemm_plan(g, op->activation);
-    return plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise;
+    return plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise && !conv_wave_f32_serves(g, false);
 }
 
 bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab)
 {
     const int x_shape[4] = {batch, op->cfg.channels_in, op->cfg.shape[2], op->cfg.shape[3]};
-    GemmPlan plan;
     *ktab = op->ktab;
-    return conv_fwd_tiles_plan(op, batch, &plan) && op_geom(op, x_shape, g) == DLP_OK;
+    if (op->algo != ALGO_GEMM || op_geom(op, x_shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
+        return false;
+    const GemmPlan plan = conv_gemm_plan(g, op->activation);
+    return plan.order == GEMM_ORDER_TAP && !plan.stem && !plan.pointwise;
 }
 
 size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op)
@@ -615,6 +618,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     op->bias = bias != 0;
     op->activation = activation;
     op->algo = chosen;
+    op->automatic = auto_algo;
     op->ktab = nullptr;
     op->workspace = 0;
     for (int i = 0; i < 6; i++)
@@ -689,6 +693,8 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
     hipStream_t s = (hipStream_t)stream;
     switch (op->algo) {
     case ALGO_WINOGRAD:
+        if (op->automatic && ws != nullptr && ws_bytes >= op->wino.ws_bytes && conv_wave_f32_serves(g, false))
+            return conv_wave_f32_launch(g, x, w, y, ep, s); // (direct: no less exact)
         return winograd_launch(g, op->wino, x, w, y, ws, ws_bytes, ep, s);
     case ALGO_DEPTHWISE:
         return depthwise_launch(g, x, w, y, ep, s);
@@ -698,6 +704,8 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
         if (plan.split && ws_bytes < plan.wpack_bytes) // the smaller tiles may still fit
             plan = conv_gemm_pack_plan(g, op->activation).floats;
         DLP_REQUIRE(ws != nullptr && ws_bytes >= plan.wpack_bytes, "workspace smaller than workspace()");
+        if (conv_wave_f32_serves(g, false))
+            return conv_wave_f32_launch(g, x, w, y, ep, s);
         const size_t used = round256(plan.wpack_bytes);
         void *part = ws_bytes > used ? (char *)ws + used : nullptr;
         int *counters = nullptr;
@@ -830,6 +838,8 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
     switch (op->algo) {
     case ALGO_WINOGRAD:
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
+        if (op->automatic && conv_wave_f32_serves(g, true))
+            return conv_wave_f32_launch(g, x, w, y, ep, s);
         return winograd_launch(g, op->wino, x, w, y, const_cast<void *>(packed), op->wino.ws_bytes, ep, s, WINO_RUN_ONLY);
     case ALGO_DEPTHWISE:
         return depthwise_launch(g, x, w, y, ep, s);
@@ -842,6 +852,8 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
         for (int i = 0; i < 6; i++)
             DLP_REQUIRE(sig[i] == op->packed_layout[i], "the weights were packed for another tile plan (pack again for this batch)");
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
+        if (conv_wave_f32_serves(g, true))
+            return conv_wave_f32_launch(g, x, w, y, ep, s);
         void *part = ws_bytes > 0 ? ws : nullptr;
         int *counters = nullptr;
         rc = own_counters(op, g, plan, &counters);

@@ -304,7 +304,11 @@ bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws
 // dx: planes of out_h x out_w pixels
 int conv_gemm_phases_launch(const PhaseConv *ph, int n, const PhasesPlan &plan, const void *dy, const void *packed, int *counters, float *images, void *dx,
                             int out_h, int out_w, int out_sh, int out_sw, const Epilogue &ep, hipStream_t stream);
-// the gather table of an operator that conv_fwd_tiles_plan accepts, and the geometry of its convolution at this batch
+// Small float convolutions, read as they lie (conv_wave_f32_kernel): whether a call is one, given that its filter could be packed ahead or has to be
+// in the call, and the call.
+bool conv_wave_f32_serves(const ConvGeom &g, bool packed);
+int conv_wave_f32_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream);
+// the gather table of a float operator of algorithm gemm in the tap-major order (not where the kernel reads the filter as it is), and the geometry of its convolution at this batch
 bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab);
 // Whether a call at this batch can run on tiles that conv_gemm_pack_phases writes, and by which plan (float, algorithm gemm, K tiles of one
 // tap x 16 channels; not where the kernel of the call reads the filter as it is, which depends on the batch too).
