@@ -2503,6 +2503,27 @@ SplitCut split_cut(long long tiles, int nkt, int cus, long long max_images)
     return best;
 }
 
+// us that a CU takes for a K tile of 64x64 among n workgroups of its own: alone, a workgroup waits for its barrier and LDS most of the time
+double split64_k_tile(long long n) { return n <= 1 ? 0.40 : n == 2 ? 0.26 : n == 3 ? 0.235 : 0.23; }
+// what K slices of 64x64 tiles cost, us: the trip through the workspace of every piece, and of the last one of a tile that adds the others up
+double split64_slices(long long pieces, int s) { return s > 1 ? 3.0 + 0.006 * pieces + 0.35 * s : 0.0; }
+
+// ... in tiles of 64x64, in equal slices.  Measured / by this count, filters packed, us: 5x5 48->80 at 31x31, batch 9 (272 tiles of 75 K tiles), s = 1 36
+// / 39, 2 30 / 33, 3 28 / 32, 4 31 / 33; 3x3 256->256 at 14x14, batch 16 (196 of 144), 1 61 / 58, 3 38 / 41, 5 34 / 37, 6 39 / 40; 512->512 at 7x7, batch 16 (104
+// of 288), 4 41 / 44, 6 40 / 43, 8 42 / 44; 3x3 stride 2 128->256 at 28x28, batch 32 (392 of 72), 1 36 / 37, 2 44 / 42.
+SplitCut split_cut_64(long long tiles, int nkt, int cus, long long max_images)
+{
+    SplitCut best = {1, 0, 1, 0.0};
+    for (int s = 1; s <= 8 && (s == 1 || nkt / s >= 6); s++) {
+        const int kt = (nkt + s - 1) / s;
+        const long long pieces = tiles * ((nkt + kt - 1) / kt), n = (pieces + cus - 1) / cus;
+        const double cost = (double)n * kt * split64_k_tile(n) + split64_slices(pieces, s);
+        if (s == 1 || (cost < best.cost && pieces <= max_images))
+            best = {s, 0, 1, cost};
+    }
+    return best;
+}
+
 void plan_split(const GemmPlan &p, GemmArgs &a, int groups, bool have_ws, size_t ws_bytes)
 {
     a.mtiles = p.mtiles;
@@ -2511,7 +2532,8 @@ void plan_split(const GemmPlan &p, GemmArgs &a, int groups, bool have_ws, size_t
     if (p.split) {
         // the best cut that the workspace (below 2 GiB of it) has room for
         const size_t room = have_ws ? std::min<size_t>(ws_bytes, kOutOfRange - 1) : 0, counters = split_counter_bytes(tiles);
-        const SplitCut c = split_cut(tiles, a.nkt, device_cu_count(), room > counters ? (long long)((room - counters) / ((size_t)p.BM * p.BN * sizeof(float))) : 0);
+        const long long images = room > counters ? (long long)((room - counters) / ((size_t)p.BM * p.BN * sizeof(float))) : 0;
+        const SplitCut c = p.tile == 6 ? split_cut_64(tiles, a.nkt, device_cu_count(), images) : split_cut(tiles, a.nkt, device_cu_count(), images);
         a.kt_per_slice = (a.nkt + c.s - 1) / c.s;
         a.splitk = (a.nkt + a.kt_per_slice - 1) / a.kt_per_slice; // every slice starts inside the K range
         a.tail_tiles = c.tail;
@@ -2961,6 +2983,10 @@ int launch_split(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t 
             launch_split_inst<128, 128, 2, 2, true>(ts, a, (unsigned)blocks, stream);
         else if (p.tile == 4)
             launch_split_inst<128, 128, 2, 2, false>(ts, a, (unsigned)blocks, stream);
+        else if (p.tile == 6 && ragged)
+            launch_split_inst<64, 64, 2, 2, true>(ts, a, (unsigned)blocks, stream);
+        else if (p.tile == 6)
+            launch_split_inst<64, 64, 2, 2, false>(ts, a, (unsigned)blocks, stream);
         else if (ragged)
             launch_split_inst<64, 128, 1, 4, true>(ts, a, (unsigned)blocks, stream);
         else
@@ -2995,7 +3021,7 @@ struct TileShape {
     int id, BM, BN;
 };
 constexpr TileShape kTiles[] = {{0, 64, 64}, {1, 32, 128}, {2, 128, 128}, {3, 64, 256}, // 2, 3: bf16 matrix-instruction path
-                                {4, 128, 128}, {5, 64, 128}}; // conv_split_f32_kernel
+                                {4, 128, 128}, {5, 64, 128}, {6, 64, 64}}; // conv_split_f32_kernel
 
 int tile_choice(int M) { return M > 32 ? 0 : 1; }
 
@@ -3106,6 +3132,7 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
     // batch 40 (248 x 144) 81 / 99 / 69.
     if (g.dtype == DLP_FLOAT && p.order == GEMM_ORDER_TAP && !p.stem && !p.pointwise && p.M > 32) {
         const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 127) / 128), work = tiles * p.nkt;
+        const long long tiles64 = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 63) / 64);
         const int rest = p.M % 128;
         const int tile = (rest == 0 || rest > 64) && (tiles >= 700 || work >= 30000) ? 4 : 5;
         const int bm = tile == 4 ? 128 : 64;
@@ -3113,6 +3140,14 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
             p.split = 1;
             p.patch = 0;
             p.tile = tile;
+        } else if (tiles64 * p.nkt >= 12000 && p.nkt >= 24 && (size_t)g.groups * ((p.M + 63) / 64) * p.nkt * 64 * 96 < kOutOfRange) {
+            // below that, long reductions in tiles of 64x64, from some 50 K tiles a CU on.  Filters packed, fp32 instruction / these: 3x3 256->256 at
+            // 14x14, batch 16 (196 x 144) 42 / 34 us, batch 4 (52 x 144) 17 / 21, 512->512 at 7x7, batch 16 (104 x 288) 42 / 40, 128->128 at 28x28, batch
+            // 16 (392 x 72) 41 / 35, 64->64 at 56x56, batch 4 (196 x 36) 13 / 17, 5x5 48->80 at 31x31, batch 9 (272 x 75) 34 / 28, 1x1 512->128 at 28x28,
+            // batch 16 (392 x 32) 24 / 19, 2048->512 at 7x7 (104 x 128) 28 / 24.  (1x1 filters read in place: 24 / 23, 29 / 32.  Those calls stay.)
+            p.split = 1;
+            p.patch = 0;
+            p.tile = 6;
         }
     }
     p.BM = 64;
@@ -3134,7 +3169,7 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
 }
 
 // the plan on the fp32 instruction
-static GemmPlan float_plan(ConvGeom g, int activation)
+GemmPlan conv_gemm_float_plan(ConvGeom g, int activation)
 {
     g.B_hint = 0;
     return conv_gemm_plan(g, activation);
@@ -3153,7 +3188,7 @@ GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation)
     pp.p = conv_gemm_hint_plan(g, activation);
     pp.bytes = pp.p.wpack_bytes;
     if (pp.p.split) {
-        pp.floats = float_plan(g, activation);
+        pp.floats = conv_gemm_float_plan(g, activation);
         pp.bytes += pp.floats.wpack_bytes;
     }
     return pp;
@@ -3383,6 +3418,7 @@ int conv_gemm_pack_phases(const float *w, int groups, int cout_g, int cin_g, int
 static double phases_cut(const PhaseConv *ph, int n, int q, int cus, PhasesPlan &pl, long long &images)
 {
     long long at = 0, next = 0, sliced = 0;
+    int most = 1;
     double busiest = 0.0;
     images = 0;
     for (int i = 0; i < n; i++) {
@@ -3395,9 +3431,12 @@ static double phases_cut(const PhaseConv *ph, int n, int q, int cus, PhasesPlan 
             busiest += pl.kt_per_slice[i];
         if (s > 1) {
             sliced += wgs;
+            most = std::max(most, s);
             images += wgs;
         }
     }
+    if (pl.plan[0].BN == 64)
+        return busiest * split64_k_tile((at + cus - 1) / cus) + split64_slices(sliced, most);
     const double rate = at <= cus ? 0.6 : at <= 2ll * cus ? 0.9 : 1.0;
     return busiest / rate + (sliced ? 6.0 : 0.0) + 0.05 * sliced;
 }
@@ -3414,7 +3453,7 @@ bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws
         if (g.Cin / g.groups % BK != 0 || g.KH * g.KW > 31 || (size_t)g.B * g.Cin * g.H * g.W * 4 + ((size_t)g.ph * g.W + g.pw) * 4 >= kOutOfRange)
             return false;
         const GemmPlan p = conv_gemm_plan(g, activation);
-        tile = !p.split ? 0 : tile == 4 ? p.tile : tile;
+        tile = !p.split || p.tile == 6 ? 0 : tile == 4 ? p.tile : tile;
     }
     // Tiles: what the phases would take by themselves, and 64x64 below that, measured against one launch a phase and the interleaving (transposed,
     // packing included, us; interleaved / 64x64 / 64x128 / 128x128): 256->128 at 14x14, 4x4, batch 1 73 / 22 / 28 / 37, batch 4 77 / 26 / 31 / 40, batch

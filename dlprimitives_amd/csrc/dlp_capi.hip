@@ -639,6 +639,12 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
             rc = own_counters(op, g, gplan, &unused);
         if (rc == DLP_OK && gplan.split) // ... and for the smaller tiles of smaller batches
             rc = own_counters(op, g, conv_gemm_pack_plan(g, activation).floats, &unused);
+        if (rc == DLP_OK && gplan.split) {
+            GemmPlan small = gplan;
+            small.mtiles = (small.M + 63) / 64;
+            small.BN = 64;
+            rc = own_counters(op, g, small, &unused);
+        }
     } else if (chosen == ALGO_WINOGRAD) {
         op->wino = winograd_plan(g);
         op->workspace = op->wino.ws_bytes;
@@ -701,8 +707,9 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
     default: {
         // workspace = packed weights | split-K partial sums
         GemmPlan plan = conv_gemm_plan(g, op->activation);
-        if (plan.split && ws_bytes < plan.wpack_bytes) // the smaller tiles may still fit
-            plan = conv_gemm_pack_plan(g, op->activation).floats;
+        // the smaller tiles may still fit; and tiles of 64x64 want 1x1 filters split ahead, not by every workgroup that reads them
+        if (plan.split && (ws_bytes < plan.wpack_bytes || (plan.tile == 6 && plan.wdirect && ((uintptr_t)w & 15) == 0)))
+            plan = conv_gemm_float_plan(g, op->activation);
         DLP_REQUIRE(ws != nullptr && ws_bytes >= plan.wpack_bytes, "workspace smaller than workspace()");
         if (conv_wave_f32_serves(g, false))
             return conv_wave_f32_launch(g, x, w, y, ep, s);

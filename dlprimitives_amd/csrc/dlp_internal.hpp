@@ -256,6 +256,7 @@ struct GemmPackPlan {
 };
 GemmPackPlan conv_gemm_pack_plan(const ConvGeom &g, int activation);
 GemmPlan conv_gemm_hint_plan(const ConvGeom &g, int activation); // its p alone
+GemmPlan conv_gemm_float_plan(ConvGeom g, int activation);        // on the fp32 instruction
 // plan of a call on weights packed by `packed`, a hint plan, with its tiles `offset` bytes into them
 GemmPlan conv_gemm_plan_on_packed(const ConvGeom &g, int activation, const GemmPlan &packed, size_t &offset);
 size_t conv_gemm_ktab_entries(const ConvGeom &g);
