@@ -256,14 +256,13 @@ __global__ __launch_bounds__(256) void ip_direct_kernel(IpArgs a)
 // accumulators are added in wavefront order through LDS; wavefront 0 then finishes the slice like the direct kernel does.
 constexpr int kIpRowBytes = 1024;            // bytes of a row per chunk
 constexpr int kIpLdsRow = kIpRowBytes + 16;  // LDS bytes per row
-// LDS of an instance: the tile of w and XR (+ 1 row of zeros when XR < 32) rows of x.  32 rows of x: 65 KB, two workgroups per
-// compute unit; 16 rows (batches of at most 16): 50 KB, three.
-constexpr int ip_stream_lds_bytes(int xr) { return (32 + xr + (xr < 32 ? 1 : 0)) * kIpLdsRow; }
+// LDS: the tiles of w and x, 65 KB, two workgroups per compute unit.
+constexpr int kIpStreamLds = 64 * kIpLdsRow;
 
-template <class T, int XR>
+template <class T>
 __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
 {
-    extern __shared__ __attribute__((aligned(16))) unsigned char ip_lds[]; // ip_stream_lds_bytes(XR), asked for at launch
+    extern __shared__ __attribute__((aligned(16))) unsigned char ip_lds[]; // kIpStreamLds, asked for at launch
     unsigned char *Ws = ip_lds, *Xs = ip_lds + 32 * kIpLdsRow;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -287,25 +286,16 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
         w_off[i] = (uint32_t)min(m0 + r, a.Out - 1) * row_bytes + (uint32_t)lane * 16u;
         x_off[i] = n0 + r < a.B ? (uint32_t)(n0 + r) * row_bytes + (uint32_t)lane * 16u : kIpOutOfRange;
     }
-    constexpr int XP = XR / 4; // pieces of x per thread
-    ip_u32x4 rw[8], rx[XP];
+    ip_u32x4 rw[8], rx[8];
     auto load_chunk = [&](int c) {
         const uint32_t soff = (uint32_t)c * (uint32_t)kIpRowBytes;
         const bool inside = soff + (uint32_t)lane * 16u < row_bytes; // the last chunk of a row may be short: what follows is the next row
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             rw[i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, inside ? w_off[i] : kIpOutOfRange, soff, 0));
-            if (i < XP)
-                rx[i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, inside ? x_off[i] : kIpOutOfRange, soff, 0));
+            rx[i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, inside ? x_off[i] : kIpOutOfRange, soff, 0));
         }
     };
-    // batch rows past XR do not exist: their lanes read a row of zeros
-    const int x_row = l32 < XR ? l32 : XR;
-    if (XR < 32) {
-        for (int i = tid; i < kIpLdsRow / 16; i += 256)
-            *(ip_u32x4 *)(Xs + XR * kIpLdsRow + i * 16) = ip_u32x4{0u, 0u, 0u, 0u};
-    }
-
     ip_f32x16 acc[1];
 #pragma unroll
     for (int r = 0; r < 16; r++)
@@ -318,8 +308,7 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             *(ip_u32x4 *)(Ws + (wave + 4 * i) * kIpLdsRow + lane * 16) = rw[i];
-            if (i < XP)
-                *(ip_u32x4 *)(Xs + (wave + 4 * i) * kIpLdsRow + lane * 16) = rx[i];
+            *(ip_u32x4 *)(Xs + (wave + 4 * i) * kIpLdsRow + lane * 16) = rx[i];
         }
         __syncthreads();
         if (c + 1 < c_end)
@@ -329,7 +318,7 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
         for (int g = 0; g < 8; g++) {
             const int koff = wave * 256 + g * 32 + h * 16;
             const ip_u32x4 fa = *(const ip_u32x4 *)(Ws + l32 * kIpLdsRow + koff);
-            const ip_u32x4 fb = *(const ip_u32x4 *)(Xs + x_row * kIpLdsRow + koff);
+            const ip_u32x4 fb = *(const ip_u32x4 *)(Xs + l32 * kIpLdsRow + koff);
             if constexpr (sizeof(T) == 4) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
@@ -360,6 +349,127 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
             acc[0][r] += red[(q * 16 + r) * 64 + lane];
     ip_finish<T, 1>(a, acc, tile, slice, m0, n0, lane, l32, h);
 }
+
+// ---- small batches: 16 outputs x 16 batch rows per workgroup, the whole reduction in it ----
+// The streaming kernel pays for its K slices with a trip through memory, and its wavefronts wait for each other at two barriers a chunk: 4096 ->
+// 1000 at batch 16 took 15 us, of which the 16 MB of weights are 3.  Here sixteen wavefronts share out the K tiles of 256 bytes per row; each has two
+// K tiles on their way, sixteen lanes to the 256 bytes of a row, and passes them through a part of LDS of its own to operand order.  No
+// barrier, no slices: the partial sums meet in LDS once.  Tiles of 16x16 leave no half of the matrix instruction idle at batch 16, and 4096 outputs
+// are a workgroup for every CU; x comes from the caches, as many bytes of it as of w.
+template <class T>
+__global__ __launch_bounds__(1024) void ip_stream_kernel_16x16(IpArgs a)
+{
+    typedef float acc_t __attribute__((ext_vector_type(4)));
+    constexpr int KW = 16, DEPTH = 2;
+    constexpr int ROW = 256;                   // bytes of a row per K tile
+    extern __shared__ __attribute__((aligned(16))) unsigned char ip_wave_lds[]; // [wavefront][w, x][16 rows][256]
+    float(*const red)[4][64] = reinterpret_cast<float(*)[4][64]>(ip_wave_lds);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int l = lane & 15, h = lane >> 4;
+    int t; // batch tiles fastest, a run of tiles per XCD: tiles that read the same rows of w share an L2
+    {
+        const int nb = gridDim.x, bid = blockIdx.x;
+        const int q = nb >> 3, r = nb & 7;
+        const int xcd = bid & 7, slot = bid >> 3;
+        t = (xcd < r) ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
+    }
+    const int mt = t / a.nchunks;
+    const int n0 = (t - mt * a.nchunks) * 16, m0 = mt * 16;
+
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+    const uint32_t row_bytes = (uint32_t)a.In * (uint32_t)sizeof(T); // a multiple of 16
+    unsigned char *const mine_s = ip_wave_lds + wave * (2 * 16 * ROW);
+    uint32_t w_off[4], x_off[4], slot[4], read[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int r = lane / 16 + 4 * i; // row of the tile this lane loads 16 bytes of, and where they go
+        w_off[i] = m0 + r < a.Out ? (uint32_t)(m0 + r) * row_bytes + (uint32_t)l * 16u : kIpOutOfRange;
+        x_off[i] = n0 + r < a.B ? (uint32_t)(n0 + r) * row_bytes + (uint32_t)l * 16u : kIpOutOfRange;
+        slot[i] = (uint32_t)(r * ROW + (l ^ r) * 16);
+        read[i] = (uint32_t)(l * ROW + ((4 * i + h) ^ l) * 16); // of row l, the k this lane gives to matrix instruction(s) i
+    }
+    const int nkt = (int)((row_bytes + ROW - 1) / ROW);
+    const int kt_begin = wave * nkt / KW, kt_end = (wave + 1) * nkt / KW;
+    ip_u32x4 wv[DEPTH][4], xv[DEPTH][4];
+    auto load = [&](auto q_c, int kt) {
+        constexpr int Q = decltype(q_c)::value;
+        if (kt >= kt_end)
+            return;
+        const uint32_t soff = (uint32_t)kt * (uint32_t)ROW;
+        const bool inside = soff + (uint32_t)l * 16u < row_bytes; // the last K tile of a row may be short: what follows is the next row
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            wv[Q][i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, inside ? w_off[i] : kIpOutOfRange, soff, 0));
+            xv[Q][i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, inside ? x_off[i] : kIpOutOfRange, soff, 0));
+        }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    load(I0{}, kt_begin);
+    load(I1{}, kt_begin + 1);
+
+    // this thread's output: register `wave` of the accumulator is batch row 4 * h + wave, output l
+    const int m = m0 + l, n = n0 + 4 * h + wave;
+    const bool mine = wave < 4 && m < a.Out && n < a.B;
+    const float bias = mine && a.bias ? a.bias[m] : 0.0f;
+
+    // two sums of half of the k each: shorter sums are rounded less (25088 -> 4096 -> 4096 -> 1000: error against 64 bits 6.1e-7 with one, 4.6e-7
+    // with two; four do not fit the registers)
+    acc_t acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    auto step = [&](auto q_c, int kt) {
+        constexpr int Q = decltype(q_c)::value;
+        if (kt >= kt_end)
+            return;
+        // LDS works a wavefront's instructions off in order, and nobody else touches its part
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            *(ip_u32x4 *)(mine_s + slot[i]) = wv[Q][i];
+            *(ip_u32x4 *)(mine_s + 16 * ROW + slot[i]) = xv[Q][i];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        ip_u32x4 fw[4], fx[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            fw[i] = *(const ip_u32x4 *)(mine_s + read[i]);
+            fx[i] = *(const ip_u32x4 *)(mine_s + 16 * ROW + read[i]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        load(q_c, kt + DEPTH);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if constexpr (sizeof(T) == 4) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t xe = fx[i][e], we = fw[i][e];
+                    acc[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, xe), __builtin_bit_cast(float, we), acc[i % 2], 0, 0, 0);
+                }
+            } else
+                acc[i % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ip_bf16x8, fx[i]), __builtin_bit_cast(ip_bf16x8, fw[i]), acc[i % 2], 0, 0, 0);
+        }
+    };
+    for (int kt = kt_begin; kt < kt_end; kt += DEPTH) {
+        step(I0{}, kt);
+        step(I1{}, kt + 1);
+    }
+
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        red[wave][r][lane] = acc[0][r] + acc[1][r];
+    __syncthreads();
+    if (!mine)
+        return;
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < KW; w++)
+        v += red[w][wave][lane];
+    store_plain((T *)a.y + (size_t)n * a.Out + m, apply_act(v + bias, a.act));
+}
+constexpr int kIpWaveLds = 16 * 2 * 16 * 256;
 
 } // namespace
 
@@ -486,11 +596,11 @@ size_t ip_stream_scratch_bytes(int batch, int inputs, int outputs, int dtype, Ip
     p.mblocks = (outputs + 31) / 32;
     p.nchunks = (batch + 31) / 32;
     p.ngroups = (inputs + kc - 1) / kc; // chunks of a row
-    // K slices: as many workgroups as fit the compute units at once (three each with the 16-row tile of x, else two), slices of at
+    // K slices: as many workgroups as fit the compute units at once (two each), slices of at
     // least two chunks, at most 16 slices, and never more than 1024 tiles x slices once K is cut (4 MiB of partial sums, what the
     // entry point that allocates nothing holds)
     const long long tiles = (long long)p.mblocks * p.nchunks;
-    long long s = ((batch <= 16 ? 3ll : 2ll) * dlp_cu_count() + tiles - 1) / tiles;
+    long long s = (2ll * dlp_cu_count() + tiles - 1) / tiles;
     s = std::min<long long>(s, std::max<long long>(1, 1024 / tiles));
     s = std::min<long long>(s, p.ngroups / 2);
     s = std::max<long long>(1, std::min<long long>(s, 16));
@@ -503,41 +613,59 @@ size_t ip_stream_scratch_bytes(int batch, int inputs, int outputs, int dtype, Ip
     return p.cnt_bytes + p.part_bytes;
 }
 
+// Batches in tiles of 16x16 (ip_stream_kernel_16x16) instead: all of at most 16 rows, and up to as many tiles as CUs, twice that where rows are short.
+// us, streaming / these, cold weights: fp32 25088 -> 4096 at batch 16 94 / 78 (5.2 TB/s), 32 102 / 120; 9216 -> 4096 at 32 45 / 51; 4096 -> 4096 at 16 26 / 17,
+// 32 27 / 27, 64 39 / 44; 4096 -> 1000 at 16 15 / 12, 64 20 / 12; 2048 -> 1000 at 128 17 / 12; 512 -> 4096 at 16 8.9 / 4.3, 32 9.2 / 7.0, 64 10 / 12; bf16 25088
+// -> 4096 at 16 39 / 32, 4096 -> 1000 at 16 11 / 5.5, 4096 -> 4096 at 32 17 / 15, 1280 -> 1000 at 1 7.8 / 3.4.
+static bool ip_tiles_16x16(int batch, int inputs, int outputs)
+{
+    const long long tiles = (long long)((batch + 15) / 16) * ((outputs + 15) / 16);
+    return batch <= 16 || tiles <= (inputs <= 4096 ? 512 : 256);
+}
+
 // An instance that needs more than 64 KB of LDS has to ask for it, once per device.  Done when an operator is created (best
 // effort: there may be no device yet) so that a first enqueue inside a stream capture has nothing left to set up; the launch
 // checks again.
-template <class T, int XR>
+template <class T>
 static int ip_stream_instance(const IpArgs *a, dim3 grid, hipStream_t stream, TimingScope *ts)
 {
-    constexpr int lds = ip_stream_lds_bytes(XR);
-    if (lds > 65536) {
-        static std::atomic<bool> asked[64];
-        int dev = 0;
-        DLP_HIP_TRY(hipGetDevice(&dev));
-        if (dev < 0 || dev >= 64 || !asked[dev].load()) {
-            DLP_HIP_TRY(hipFuncSetAttribute((const void *)ip_stream_kernel<T, XR>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-            if (dev >= 0 && dev < 64)
-                asked[dev].store(true);
-        }
+    static std::atomic<bool> asked[64];
+    int dev = 0;
+    DLP_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= 64 || !asked[dev].load()) {
+        DLP_HIP_TRY(hipFuncSetAttribute((const void *)ip_stream_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, kIpStreamLds));
+        if (dev >= 0 && dev < 64)
+            asked[dev].store(true);
     }
     if (a == nullptr) // set-up only
         return DLP_OK;
-    DLP_LAUNCH_TIMED((*ts), (ip_stream_kernel<T, XR>), grid, dim3(256), lds, stream, *a);
+    DLP_LAUNCH_TIMED((*ts), ip_stream_kernel<T>, grid, dim3(256), kIpStreamLds, stream, *a);
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
 }
 template <class T>
-static int ip_stream_dispatch(bool small_batch, const IpArgs *a, dim3 grid, hipStream_t stream, TimingScope *ts)
+static int ip_wave_instance(const IpArgs *a, dim3 grid, hipStream_t stream, TimingScope *ts)
 {
-    return small_batch ? ip_stream_instance<T, 16>(a, grid, stream, ts) : ip_stream_instance<T, 32>(a, grid, stream, ts);
+    static std::atomic<bool> asked[64];
+    int dev = 0;
+    DLP_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= 64 || !asked[dev].load()) {
+        DLP_HIP_TRY(hipFuncSetAttribute((const void *)ip_stream_kernel_16x16<T>, hipFuncAttributeMaxDynamicSharedMemorySize, kIpWaveLds));
+        if (dev >= 0 && dev < 64)
+            asked[dev].store(true);
+    }
+    if (a == nullptr)
+        return DLP_OK;
+    DLP_LAUNCH_TIMED((*ts), ip_stream_kernel_16x16<T>, grid, dim3(1024), kIpWaveLds, stream, *a);
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
 }
 void ip_stream_prepare(int dtype)
 {
     if (dtype != DLP_FLOAT && dtype != DLP_BFLOAT16)
         return;
-    for (int small = 0; small < 2; small++)
-        (void)(dtype == DLP_BFLOAT16 ? ip_stream_dispatch<bf16_t>(small != 0, nullptr, dim3(1), nullptr, nullptr)
-                                     : ip_stream_dispatch<float>(small != 0, nullptr, dim3(1), nullptr, nullptr));
+    (void)(dtype == DLP_BFLOAT16 ? ip_stream_instance<bf16_t>(nullptr, dim3(1), nullptr, nullptr) : ip_stream_instance<float>(nullptr, dim3(1), nullptr, nullptr));
+    (void)(dtype == DLP_BFLOAT16 ? ip_wave_instance<bf16_t>(nullptr, dim3(1), nullptr, nullptr) : ip_wave_instance<float>(nullptr, dim3(1), nullptr, nullptr));
     (void)hipGetLastError(); // no device, no harm: the launch asks again
 }
 
@@ -574,9 +702,12 @@ int ip_stream_launch(int batch, int inputs, int outputs, int dtype, const void *
         return fail(DLP_ERR_NOT_IMPLEMENTED, "inner product too large for a single launch");
     const dim3 grid((unsigned)wgs);
     TimingScope ts("ip_direct", stream);
-    // batches of at most 16 rows keep 16 rows of x in LDS: three workgroups per compute unit instead of two
-    return dtype == DLP_BFLOAT16 ? ip_stream_dispatch<bf16_t>(batch <= 16, &a, grid, stream, &ts)
-                                 : ip_stream_dispatch<float>(batch <= 16, &a, grid, stream, &ts);
+    if (ip_tiles_16x16(batch, inputs, outputs)) {
+        a.nchunks = (batch + 15) / 16;
+        const dim3 tiles((unsigned)((outputs + 15) / 16 * a.nchunks));
+        return dtype == DLP_BFLOAT16 ? ip_wave_instance<bf16_t>(&a, tiles, stream, &ts) : ip_wave_instance<float>(&a, tiles, stream, &ts);
+    }
+    return dtype == DLP_BFLOAT16 ? ip_stream_instance<bf16_t>(&a, grid, stream, &ts) : ip_stream_instance<float>(&a, grid, stream, &ts);
 }
 
 ConvGeom ip_gemm_geom(int batch, int inputs, int outputs, int dtype)
