@@ -229,6 +229,93 @@ __global__ __launch_bounds__(kPwThreads) void conv_pointwise_f32_kernel(PwArgs a
     }
 }
 
+// ---- the other way round: few input channels, many filters (the expansion of an inverted residual block, 24 -> 144 at 56x56), fp32 ----
+// Such a layer writes six times what it reads.  In 32x128 tiles of the gathering kernel every workgroup gathered its 24 channels pixel by pixel for
+// 16 KB of output, five workgroups the same ones.  Here a wavefront keeps four pixels per lane of all K channels in registers (16-byte loads, one
+// pair of channels each, as above) and walks RB blocks of 32 filters over them; a filter block's weights lie in LDS as [k][m].  Stores are 16
+// bytes a lane, 512 consecutive bytes a row, and stay in the caches for the next layer to read.  24 -> 144 at 56x56, batch 64 (135 MB): 56 -> 35 us.
+// (The offset of a store is all in its vector register: with a scalar one besides, the compiler lets the next instruction overwrite the
+// first of the four data registers of a 16-byte store, and lanes 12 to 15 of every 16 stored what came after.)
+template <int KP>
+__global__ __launch_bounds__(kPwThreads) void conv_expand_f32_kernel(PwArgs a, int rb)
+{
+    constexpr int PX = 4;
+    extern __shared__ __attribute__((aligned(16))) float ex_lds[]; // [2 * KP][32 * rb] weights, [32 * rb] bias
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, h = lane >> 5;
+    const int n0 = ((int)blockIdx.x * 4 + wave) * (32 * PX) + l32 * PX; // this lane's first pixel
+    const int rows = 32 * rb, m0 = (int)blockIdx.y * rows;
+    float *const bias_s = ex_lds + 2 * KP * rows;
+
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, a.y_bytes, 0x00020000);
+    const int b_img = (int)fast_div((uint32_t)n0, a.hw_magic, a.hw_shift);
+    const int pix = n0 - b_img * a.HW; // PX divides the plane: the lane's pixels stay in one image
+    const uint32_t xvoff = n0 < a.N ? (uint32_t)(((b_img * a.K + h) * a.HW + pix) * 4) : kPwOutOfRange;
+    const uint32_t pair_bytes = (uint32_t)(2 * a.HW * 4);
+    float x[KP][PX];
+#pragma unroll
+    for (int p = 0; p < KP; p++) {
+        const uint32_t v = 2 * p + h < a.K ? xvoff : kPwOutOfRange;
+        const pw_f32x4 t = __builtin_bit_cast(pw_f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, v, (uint32_t)p * pair_bytes, 0));
+#pragma unroll
+        for (int j = 0; j < PX; j++)
+            x[p][j] = t[j];
+    }
+    for (int i = tid; i < rows * 2 * KP; i += kPwThreads) { // a filter's channels by consecutive lanes
+        const int m = i / (2 * KP), k = i % (2 * KP);
+        ex_lds[k * rows + m] = m0 + m < a.M && k < a.K ? a.w[(m0 + m) * a.K + k] : 0.0f;
+    }
+    for (int i = tid; i < rows; i += kPwThreads)
+        bias_s[i] = a.bias && m0 + i < a.M ? a.bias[m0 + i] : 0.0f;
+    __syncthreads();
+
+    const uint32_t yvoff = n0 < a.N ? (uint32_t)(((b_img * a.M + m0 + 4 * h) * a.HW + pix) * 4) : kPwOutOfRange;
+    const int pairs = (a.K + 1) / 2;
+    for (int i = 0; i < rb; i++) {
+        if (m0 + 32 * i >= a.M)
+            break;
+        pw_f32x16 acc[PX];
+#pragma unroll
+        for (int j = 0; j < PX; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                acc[j][r] = 0.0f;
+        const float *const wl = ex_lds + h * rows + 32 * i + l32;
+#pragma unroll
+        for (int p0 = 0; p0 < KP; p0 += 4) {
+            if (p0 >= pairs)
+                break;
+            float f[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                f[e] = wl[2 * (p0 + e) * rows];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int j = 0; j < PX; j++)
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f[e], x[p0 + e][j], acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int row = 32 * i + 8 * (r >> 2) + (r & 3); // + 4 * h
+            const float bias = bias_s[row + 4 * h];
+            const uint32_t voff = yvoff != kPwOutOfRange && m0 + row + 4 * h < a.M ? yvoff + (uint32_t)(row * a.HW * 4) : kPwOutOfRange;
+            float v[PX];
+#pragma unroll
+            for (int j = 0; j < PX; j++) {
+                v[j] = acc[j][r] + bias;
+                const float c = clamp_med3(v[j], a.clamp_lo, a.clamp_hi);
+                v[j] = a.clamp ? c : v[j]; // identity keeps NaNs: no clamp
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) uint32_t, (pw_f32x4){v[0], v[1], v[2], v[3]}), yr, voff,
+                                                   0, 0);
+        }
+    }
+}
+
 struct PwShape {
     int px, mtw, ms;
 };
@@ -310,6 +397,54 @@ int conv_pointwise_launch(const ConvGeom &g, const void *x, const void *w, void 
     DLP_PW_CASE(4, 1, 1)
 #undef DLP_PW_CASE
     return fail(DLP_ERR_RUNTIME, "pointwise kernel: no instantiation for this shape");
+}
+
+bool conv_expand_serves(const ConvGeom &g, const Epilogue &ep, const void *x, const void *y)
+{
+    if (g.dtype != DLP_FLOAT || g.KH != 1 || g.KW != 1 || g.sh != 1 || g.sw != 1 || g.ph != 0 || g.pw != 0 || g.groups != 1 || g.B <= 0)
+        return false;
+    if (ep.activation == DLP_ACT_TANH || ep.activation == DLP_ACT_SIGMOID || ep.factor != 0.0f || g.Cin > 24 || g.Cout <= 32)
+        return false;
+    if ((g.H * g.W) % 4 != 0 || (((uintptr_t)x | (uintptr_t)y) & 15) != 0)
+        return false;
+    const size_t N = (size_t)g.B * g.H * g.W;
+    // From 40 MB of output on; below, a wavefront that walks many filter blocks takes longer than the gathering kernel's many workgroups.  Cold tensors,
+    // us, gathering / this: 16 -> 96 at 112x112, batch 16 (77 MB) 29 / 21, 8 -> 48 at 112x112, batch 32 (77 MB) 31 / 21, 20 -> 120 at 58x58, batch 10 (16
+    // MB) 11 / 16, 24 -> 144 at 56x56, batch 4 (7 MB) 6 / 17.  More input channels do not fit the registers beside four pixels a lane: with two,
+    // 40 -> 240 at 56x56, batch 24 38 / 41, 64 -> 256 at batch 64 89 / 118.
+    return N * g.Cin * 4 < kPwOutOfRange && N * g.Cout * 4 < kPwOutOfRange && N * g.Cout * 4 >= 40000000;
+}
+
+int conv_expand_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream)
+{
+    PwArgs a = PwArgs();
+    a.x = (const float *)x;
+    a.w = (const float *)w;
+    a.bias = ep.bias;
+    a.y = (float *)y;
+    a.M = g.Cout;
+    a.K = g.Cin;
+    a.HW = g.H * g.W;
+    a.N = g.B * a.HW;
+    a.x_bytes = (uint32_t)((size_t)a.N * a.K * 4);
+    a.y_bytes = (uint32_t)((size_t)a.N * a.M * 4);
+    make_magic((uint32_t)a.HW, a.hw_magic, a.hw_shift);
+    a.clamp = ep.activation != DLP_ACT_IDENTITY;
+    a.clamp_lo = 0.0f;
+    a.clamp_hi = ep.activation == DLP_ACT_RELU6 ? 6.0f : __builtin_huge_valf();
+    const int kp = a.K <= 16 ? 8 : 12, blocks = (a.M + 31) / 32;
+    // filter blocks per wavefront: one to six, as many as leave two workgroups per compute unit (24 -> 144 above: 1, 2, 3, 5 blocks 47, 43, 39, 35 us)
+    const long long gx = (a.N + 511) / 512;
+    const int rb = (int)std::max<long long>(1, std::min<long long>(std::min(blocks, 6), gx * blocks / (2 * dlp_cu_count())));
+    const dim3 grid((unsigned)gx, (unsigned)((blocks + rb - 1) / rb));
+    const size_t lds = (size_t)(2 * kp + 1) * 32 * rb * sizeof(float);
+    void (*kernel)(PwArgs, int) = conv_expand_f32_kernel<12>;
+    if (kp == 8)
+        kernel = conv_expand_f32_kernel<8>;
+    TimingScope ts("conv_gemm", stream);
+    DLP_LAUNCH_TIMED(ts, kernel, grid, dim3(kPwThreads), lds, stream, a, rb);
+    DLP_HIP_TRY(hipGetLastError());
+    return DLP_OK;
 }
 
 } // namespace dlp

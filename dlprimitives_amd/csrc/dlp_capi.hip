@@ -713,6 +713,8 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
         DLP_REQUIRE(ws != nullptr && ws_bytes >= plan.wpack_bytes, "workspace smaller than workspace()");
         if (conv_wave_f32_serves(g, false))
             return conv_wave_f32_launch(g, x, w, y, ep, s);
+        if (conv_expand_serves(g, ep, x, y))
+            return conv_expand_launch(g, x, w, y, ep, s);
         const size_t used = round256(plan.wpack_bytes);
         void *part = ws_bytes > used ? (char *)ws + used : nullptr;
         int *counters = nullptr;
@@ -861,6 +863,8 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
         if (conv_wave_f32_serves(g, true))
             return conv_wave_f32_launch(g, x, w, y, ep, s);
+        if (conv_expand_serves(g, ep, x, y))
+            return conv_expand_launch(g, x, w, y, ep, s);
         void *part = ws_bytes > 0 ? ws : nullptr;
         int *counters = nullptr;
         rc = own_counters(op, g, plan, &counters);

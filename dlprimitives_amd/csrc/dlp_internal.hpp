@@ -341,6 +341,10 @@ int conv_stem_launch(const ConvGeom &g, const void *x, const void *w, void *y, c
 bool conv_pointwise_supported(const ConvGeom &g, int activation);
 int conv_pointwise_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream);
 
+// ... with few input channels and many filters: whether a call is one, and the call (conv_expand_f32_kernel; reads x and w in place)
+bool conv_expand_serves(const ConvGeom &g, const Epilogue &ep, const void *x, const void *y);
+int conv_expand_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream);
+
 // ---- depthwise 3x3 + pointwise 1x1 in one launch (conv_dwpw.hip) ----------------
 // g: the depthwise layer; M: filters of the pointwise layer; act1 / ep.activation: the two activations; bd: depthwise bias or null
 bool conv_dwpw_supported(const ConvGeom &g, int M, int act1, int act2);
