@@ -412,6 +412,68 @@ __global__ __launch_bounds__(256) void depthwise_wgrad3x3_kernel(const float *__
         part[((size_t)slice * Cout + k) * 9 + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
+// The same for undilated filters of stride 1 or 2 (S, of the rows): a thread walks RB output pixels down a column, whose (RB - 1) * S + 3 rows of
+// three input pixels it loads together with dy, before the first is used, instead of ten loads per pixel one pixel after the other.  Work
+// items (image, block of rows, column), columns fastest, so that consecutive lanes read consecutive pixels.  Bound by the loads (the tensors
+// are read 1.25 times); 32 x 192 x 28 x 28: 21.6 -> 15.3 us.
+struct DwWgradArgs {
+    const float *x, *dy;
+    float *part;
+    int B, Cin, Cout, mult, H, W, OH, OW, sw, ph, pw, blocks; // blocks of RB rows
+    uint32_t x_bytes, dy_bytes, ow_magic, ow_shift, bl_magic, bl_shift;
+};
+template <int S, int RB>
+__global__ __launch_bounds__(256) void depthwise_wgrad3x3_columns_kernel(DwWgradArgs a)
+{
+    constexpr int ROWS = (RB - 1) * S + 3;
+    __shared__ float red[4][9];
+    const int k = blockIdx.x, slice = blockIdx.y, slices = gridDim.y;
+    const int c = k / a.mult;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc((void *)a.dy, 0, a.dy_bytes, 0x00020000);
+    float acc[9];
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+        acc[t] = 0.0f;
+    const int images = (a.B - slice + slices - 1) / slices, items = images * a.blocks * a.OW;
+    for (int item = threadIdx.x; item < items; item += 256) {
+        const int q = (int)fast_div((uint32_t)item, a.ow_magic, a.ow_shift), ow = item - q * a.OW;
+        const int i = (int)fast_div((uint32_t)q, a.bl_magic, a.bl_shift), oh0 = (q - i * a.blocks) * RB;
+        const int b = slice + i * slices;
+        const int ih0 = oh0 * S - a.ph, iw0 = ow * a.sw - a.pw;
+        const int xbase = ((b * a.Cin + c) * a.H + ih0) * a.W + iw0, ybase = ((b * a.Cout + k) * a.OH + oh0) * a.OW + ow;
+        float v[ROWS][3], g[RB];
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+            g[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(yr, oh0 + r < a.OH ? (uint32_t)(ybase + r * a.OW) * 4u : kOutOfRange, 0, 0));
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const bool rv = (unsigned)(ih0 + r) < (unsigned)a.H;
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+                v[r][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                        xr, rv && (unsigned)(iw0 + t) < (unsigned)a.W ? (uint32_t)(xbase + r * a.W + t) * 4u : kOutOfRange, 0, 0));
+        }
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int t = 0; t < 9; t++) // (a pixel past the last row has g = 0, but what it meets may be infinite)
+                acc[t] = oh0 + r < a.OH ? fmaf(g[r], v[r * S + t / 3][t % 3], acc[t]) : acc[t];
+    }
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+        float s = acc[t];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1)
+            s += __shfl_down(s, off);
+        if ((threadIdx.x & 63) == 0)
+            red[threadIdx.x >> 6][t] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < 9)
+        a.part[((size_t)slice * a.Cout + k) * 9 + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+}
+
 // out[i] = factor * out[i] + sum over slices.  A wavefront owns 64 consecutive outputs; the four wavefronts of a
 // workgroup take every fourth slice each (slice order within a wavefront, then the four sums in wavefront order:
 // the same bits every run), so a launch with few outputs and many slices still fills the chip.
@@ -1075,9 +1137,22 @@ int dlp_conv2d_bwd_filter_enqueue(dlp_conv2d_bwd_filter *op, const int x_shape[4
         DLP_REQUIRE(c.channels_out <= 0x7FFFFFFF && p.slices <= 65535, "grid");
         {
             TimingScope ts("wgrad_depthwise", st);
-            hipLaunchKernelGGL(depthwise_wgrad3x3_kernel, dim3((unsigned)c.channels_out, (unsigned)p.slices), dim3(256), 0, st, (const float *)x,
-                               (const float *)dy, (float *)ws, batch, c.channels_in, c.channels_out, cout_g, c.shape[2], c.shape[3], op->OH, op->OW,
-                               c.stride[0], c.stride[1], c.pad[0], c.pad[1], c.dilate[0], c.dilate[1]);
+            const dim3 grid((unsigned)c.channels_out, (unsigned)p.slices);
+            if (c.dilate[0] == 1 && c.dilate[1] == 1 && c.stride[0] <= 2) {
+                const int rb = c.stride[0] == 1 ? 8 : 4;
+                DwWgradArgs a = {(const float *)x, (const float *)dy, (float *)ws, batch, c.channels_in, c.channels_out, cout_g, c.shape[2], c.shape[3],
+                                 op->OH, op->OW, c.stride[1], c.pad[0], c.pad[1], (op->OH + rb - 1) / rb, (uint32_t)(x_elems * 4), (uint32_t)(y_elems * 4),
+                                 0, 0, 0, 0};
+                make_magic((uint32_t)a.OW, a.ow_magic, a.ow_shift);
+                make_magic((uint32_t)a.blocks, a.bl_magic, a.bl_shift);
+                if (c.stride[0] == 1)
+                    DLP_LAUNCH_TIMED(ts, (depthwise_wgrad3x3_columns_kernel<1, 8>), grid, dim3(256), 0, st, a);
+                else
+                    DLP_LAUNCH_TIMED(ts, (depthwise_wgrad3x3_columns_kernel<2, 4>), grid, dim3(256), 0, st, a);
+            } else
+                hipLaunchKernelGGL(depthwise_wgrad3x3_kernel, dim3((unsigned)c.channels_out, (unsigned)p.slices), dim3(256), 0, st, (const float *)x,
+                                   (const float *)dy, (float *)ws, batch, c.channels_in, c.channels_out, cout_g, c.shape[2], c.shape[3], op->OH, op->OW,
+                                   c.stride[0], c.stride[1], c.pad[0], c.pad[1], c.dilate[0], c.dilate[1]);
         }
         TimingScope ts("wgrad_reduce", st);
         hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(reduce_grid_for(n_out)), dim3(256), 0, st, (const float *)ws, (float *)dw, n_out, p.slices, factor);

@@ -170,8 +170,10 @@ template <int N, int AUX>
 __device__ __forceinline__ void dw_store(const float *d, __amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s)
 {
     if constexpr (N == 4) {
+        // (all of the offset in the vector register: beside a scalar one the compiler leaves no wait between a 16-byte store and an
+        // instruction that overwrites its data)
         const dw_f32x4 t = {d[0], d[1], d[2], d[3]};
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dw_u32x4, t), r, v, s, AUX);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dw_u32x4, t), r, v + s, 0, AUX);
     } else if constexpr (N == 2) {
         const dw_f32x2 t = {d[0], d[1]};
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(dw_u32x2, t), r, v, s, AUX);

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kPwThreads) void conv_pointwise_f32_kernel(PwArgs a
 // Such a layer writes six times what it reads.  In 32x128 tiles of the gathering kernel every workgroup gathered its 24 channels pixel by pixel for
 // 16 KB of output, five workgroups the same ones.  Here a wavefront keeps four pixels per lane of all K channels in registers (16-byte loads, one
 // pair of channels each, as above) and walks RB blocks of 32 filters over them; a filter block's weights lie in LDS as [k][m].  Stores are 16
-// bytes a lane, 512 consecutive bytes a row, and stay in the caches for the next layer to read.  24 -> 144 at 56x56, batch 64 (135 MB): 56 -> 35 us.
+// bytes a lane, 512 consecutive bytes a row, and stay in the caches for the next layer to read.  24 -> 144 at 56x56, batch 64 (135 MB): 56 -> 37 us.
 // (The offset of a store is all in its vector register: with a scalar one besides, the compiler lets the next instruction overwrite the
 // first of the four data registers of a 16-byte store, and lanes 12 to 15 of every 16 stored what came after.)
 template <int KP>
