@@ -825,6 +825,9 @@ int dlp_conv2d_bwd_data_create(const dlp_conv2d_settings *cfg, const char *algo,
     op->nphases = cfg->stride[0] * cfg->stride[1];
     for (int i = 0; i < op->nphases; i++)
         op->phase[i].fwd = nullptr;
+    // an algorithm that was left open is the one whose phases run in one launch, also for phases of 3x3 taps
+    const bool open = algo == nullptr || *algo == 0 || std::string(algo) == "auto";
+    const char *const phase_algo = open && cfg->channels_out / cfg->groups % 16 == 0 ? "gemm" : algo;
     for (int a = 0; a < cfg->stride[0]; a++)
         for (int b = 0; b < cfg->stride[1]; b++) {
             BwdPhase &ph = op->phase[a * cfg->stride[1] + b];
@@ -840,7 +843,7 @@ int dlp_conv2d_bwd_data_create(const dlp_conv2d_settings *cfg, const char *algo,
             u.dilate[1] = ph.w.dil;
             u.pad[0] = ph.h.pad;
             u.pad[1] = ph.w.pad;
-            rc = dlp_conv2d_fwd_create(&u, 0, DLP_ACT_IDENTITY, algo, &ph.fwd);
+            rc = dlp_conv2d_fwd_create(&u, 0, DLP_ACT_IDENTITY, phase_algo, &ph.fwd);
             if (rc != DLP_OK) {
                 bwd_data_free(op);
                 return rc;

@@ -108,6 +108,7 @@ struct dlp_conv2d_fwd {
     int activation;
     ConvAlgo algo;
     bool automatic; // the algorithm was not asked for by name
+    bool direct;    // ... is Winograd, and large batches run as "gemm" all the same (direct_is_faster); packed weights then are both, Winograd's first
     int device;
     KTabEntry *ktab; // device gather table of the GEMM stage
     WinoPlan wino;
@@ -152,6 +153,21 @@ static int op_geom(const dlp_conv2d_fwd *op, const int x_shape[4], ConvGeom &g)
         g.pool_pw = (g.OW + 2 - 3) / 2 + 1;
     }
     return rc;
+}
+
+// Whether a convolution that the reference's rule gives to Winograd is faster as conv_split_f32_kernel (and less rounded): enough tiles of 64 filters
+// x 128 pixels, none with empty rows.  Filters transformed in the call, cold tensors, Winograd / direct, us: 3x3 64->64 at 56x56, batch 16 (392 tiles) 38 / 39,
+// 32 (784) 63 / 59, 64 (1568) 112 / 100; 128->128 at 28x28, 32 (392) 56 / 59, 48 (588) 81 / 69, 64 (784) 101 / 91; 256->256 at 14x14, 64 (392) 92 / 105, 128 (784)
+// 171 / 161; 192->192 at 35x35, 20 (576) 113 / 106; 32->64 at 112x112, 16 (1568) 76 / 61; 160->96 at 50x50, 16 (626) 78 / 83.
+static bool direct_is_faster(const ConvGeom &g, const GemmPlan &p)
+{
+    const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 127) / 128);
+    return g.dtype == DLP_FLOAT && p.split && p.tile != 6 && p.M % 64 == 0 && tiles >= 560;
+}
+// whether a call runs as "gemm"
+static bool runs_as_gemm(const dlp_conv2d_fwd *op, const ConvGeom &g, const GemmPlan &p)
+{
+    return op->algo == ALGO_GEMM || (op->direct && direct_is_faster(g, p));
 }
 
 struct dlp_ip_fwd {
@@ -283,10 +299,10 @@ bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan)
 {
     ConvGeom g;
     const int x_shape[4] = {batch, op->cfg.channels_in, op->cfg.shape[2], op->cfg.shape[3]};
-    if (op->algo != ALGO_GEMM || op_geom(op, x_shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
+    if (op_geom(op, x_shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
         return false;
     *plan = conv_gemm_plan(g, op->activation);
-    return plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise && !conv_wave_f32_serves(g, false);
+    return runs_as_gemm(op, g, *plan) && plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise && !conv_wave_f32_serves(g, false);
 }
 
 bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab)
@@ -302,7 +318,7 @@ bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const 
 size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op)
 {
     ConvGeom g;
-    if (op->algo != ALGO_GEMM || op_geom(op, op->cfg.shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
+    if ((op->algo != ALGO_GEMM && !op->direct) || op_geom(op, op->cfg.shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
         return 0;
     // (either form; a smaller batch needs no more than the settings' one)
     const GemmPackPlan pp = conv_gemm_pack_plan(g, op->activation);
@@ -596,9 +612,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     // the LDS-patch kernel can serve and that (a) have fewer than 64 input channels, or fewer than 128 with a filter count off 64 (the
     // Winograd kernel then gives a workgroup 32 output channels: 130 against 126 us on 64->64 at 56x56, batch 64), or (b) leave the
     // Winograd kernel fewer than one and a half workgroups per compute unit at the batch of the settings.  These lines were drawn against the
-    // LDS-patch kernel.  From batch 32 to 64 on such layers run on conv_split_f32_kernel, and the choice is then not the faster one
-    // throughout: weights transformed in the call, gemm / winograd, at batch 64 64->64 at 56x56 97 / 111 us, 128->128 at 28x28 91 / 104,
-    // 256->256 at 14x14 107 / 94, 512->512 at 7x7 104 / 106; at batch 16 37 / 37, 42 / 38, 44 / 44 (200 workgroups), 49 / 77 (128).
+    // LDS-patch kernel; from some batch on such layers are faster on conv_split_f32_kernel: those calls run there whatever the name (direct_is_faster).
     const int cin_g = cfg->channels_in / cfg->groups;
     bool gemm_faster = false;
     if (gplan.patch_layer && win) {
@@ -619,6 +633,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     op->activation = activation;
     op->algo = chosen;
     op->automatic = auto_algo;
+    op->direct = chosen == ALGO_WINOGRAD && auto_algo && direct_is_faster(g, gplan);
     op->ktab = nullptr;
     op->workspace = 0;
     for (int i = 0; i < 6; i++)
@@ -631,7 +646,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     op->counter_count = 0;
     if (hipGetDevice(&op->device) != hipSuccess)
         op->device = 0;
-    if (chosen == ALGO_GEMM) {
+    if (chosen == ALGO_GEMM || op->direct) {
         op->workspace = conv_gemm_workspace_bytes(g, activation);
         rc = upload_ktab(g, activation, &op->ktab);
         int *unused = nullptr;
@@ -645,9 +660,10 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
             small.BN = 64;
             rc = own_counters(op, g, small, &unused);
         }
-    } else if (chosen == ALGO_WINOGRAD) {
+    }
+    if (chosen == ALGO_WINOGRAD) {
         op->wino = winograd_plan(g);
-        op->workspace = op->wino.ws_bytes;
+        op->workspace = std::max(op->workspace, op->wino.ws_bytes);
     }
     if (rc != DLP_OK) {
         delete op;
@@ -697,7 +713,9 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
     ep.activation = op->activation;
     ep.accumulate_first = op->accumulate_first;
     hipStream_t s = (hipStream_t)stream;
-    switch (op->algo) {
+    const bool direct = op->direct && ws != nullptr && direct_is_faster(g, conv_gemm_plan(g, op->activation)) &&
+                        ws_bytes >= std::max(op->wino.ws_bytes, conv_gemm_plan(g, op->activation).wpack_bytes);
+    switch (direct ? ALGO_GEMM : op->algo) {
     case ALGO_WINOGRAD:
         if (op->automatic && ws != nullptr && ws_bytes >= op->wino.ws_bytes && conv_wave_f32_serves(g, false))
             return conv_wave_f32_launch(g, x, w, y, ep, s); // (direct: no less exact)
@@ -794,14 +812,13 @@ size_t dlp_conv2d_fwd_packed_bytes(const dlp_conv2d_fwd *op)
 {
     if (!op)
         return 0;
-    if (op->algo == ALGO_WINOGRAD)
-        return round256(op->wino.ws_bytes);
-    if (op->algo == ALGO_DEPTHWISE)
-        return 0;
+    const size_t first = op->algo == ALGO_WINOGRAD ? round256(op->wino.ws_bytes) : 0;
+    if (op->algo == ALGO_DEPTHWISE || (op->algo == ALGO_WINOGRAD && !op->direct))
+        return first;
     ConvGeom g;
     if (op_geom(op, op->cfg.shape, g) != DLP_OK)
         return 0;
-    return round256(conv_gemm_pack_plan(g, op->activation).bytes);
+    return first + round256(conv_gemm_pack_plan(g, op->activation).bytes);
 }
 
 int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *stream)
@@ -816,7 +833,10 @@ int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *s
         return rc;
     if (op->algo == ALGO_WINOGRAD) {
         Epilogue ep = {nullptr, 0.0f, op->activation};
-        return winograd_launch(g, op->wino, nullptr, w, nullptr, packed, op->wino.ws_bytes, ep, (hipStream_t)stream, WINO_FILTER_ONLY);
+        rc = winograd_launch(g, op->wino, nullptr, w, nullptr, packed, op->wino.ws_bytes, ep, (hipStream_t)stream, WINO_FILTER_ONLY);
+        if (rc != DLP_OK || !op->direct)
+            return rc;
+        packed = (char *)packed + round256(op->wino.ws_bytes);
     }
     const GemmPackPlan pp = conv_gemm_pack_plan(g, op->activation);
     layout_of(pp.p, op->packed_layout);
@@ -844,7 +864,10 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
     ep.activation = op->activation;
     ep.accumulate_first = op->accumulate_first;
     hipStream_t s = (hipStream_t)stream;
-    switch (op->algo) {
+    const bool direct = op->direct && packed != nullptr && direct_is_faster(g, conv_gemm_plan(g, op->activation));
+    if (direct)
+        packed = (const char *)packed + round256(op->wino.ws_bytes);
+    switch (direct ? ALGO_GEMM : op->algo) {
     case ALGO_WINOGRAD:
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
         if (op->automatic && conv_wave_f32_serves(g, true))

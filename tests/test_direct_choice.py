@@ -1,0 +1,43 @@
+"""Operators whose algorithm was left open and is Winograd by size: large batches run directly in tiles of the bf16 matrix instruction, with
+filters raw and packed, smaller ones through the transform; gradients alike."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import dlprimitives_amd as dlp
+from test_split_gemm import _kernels
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cin", [64, 40])
+def test_gpu_automatic_choice_by_batch(cin):
+    gen = torch.Generator().manual_seed(cin)
+    h, cout, hint = 40, 64, 48  # 600 tiles of 64 filters x 128 pixels at 48 images, 450 at 36
+    f, bias = torch.randn((cout, cin, 3, 3), generator=gen), torch.randn(cout, generator=gen)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, 3, 1, 1, 1, 1, (hint, cin, h, h)), True, "relu")
+    back = dlp.Conv2DBackwardData.create(dlp.Conv2DSettings(64, 64, 3, 1, 1, 1, 1, (hint, cout, h, h)))
+    assert cin != 64 or op.algo() == "winograd"
+    fd, bd = f.cuda(), bias.cuda()
+    work = torch.empty(max(op.workspace(), back.workspace()), dtype=torch.uint8, device="cuda:0")
+    packed = torch.full((op.packed_size(),), 255, dtype=torch.uint8, device="cuda:0")
+    op.pack(fd, packed)
+    for batch in (48, 36, 2):
+        x = torch.randn((batch, cin, h, h), generator=gen)
+        xd = x.cuda()
+        ref = torch.nn.functional.conv2d(x[-2:].double(), f.double(), bias.double(), 1, 1).relu()
+        scale = torch.nn.functional.conv2d(x[-2:].double().abs(), f.double().abs(), bias.double().abs(), 1, 1)
+        for call in (lambda y: op.enqueue(xd, fd, bd, y, work), lambda y: op.enqueue_packed(xd, fd, packed, bd, y, work)):
+            y = torch.full((batch, cout, h, h), float("nan"), device="cuda:0")
+            names = _kernels(lambda: call(y))
+            if cin == 64:
+                start = {48: ["conv_split_f32_kernel<64, 128,"], 36: [], 2: ["conv_wave_f32_kernel<"]}[batch]
+                assert len(names) == len(start) and all(n.startswith(t) for n, t in zip(names, start)), names
+            # Winograd's transforms round at the size of sixteen products
+            assert ((y[-2:].cpu().double() - ref).abs() <= scale * ((cin * 9 + 16) * 2.0 ** -24)).all()
+    if cin == 64:
+        dy, dx = torch.randn((hint, 64, h, h), generator=gen), torch.full((hint, 64, h, h), float("nan"), device="cuda:0")
+        (name,) = _kernels(lambda: back.enqueue(dx, fd, dy.cuda(), work))
+        assert name.startswith("conv_split_f32_kernel<64, 128,"), name
+        want = torch.nn.functional.conv_transpose2d(dy[-2:].double(), f.double(), None, 1, 1)
+        scale = torch.nn.functional.conv_transpose2d(dy[-2:].double().abs(), f.double().abs(), None, 1, 1)
+        assert ((dx[-2:].cpu().double() - want).abs() <= scale * ((64 * 9 + 16) * 2.0 ** -24)).all()
