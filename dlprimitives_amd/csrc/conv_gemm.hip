@@ -3140,12 +3140,14 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
             p.split = 1;
             p.patch = 0;
             p.tile = tile;
-        } else if (tiles64 * p.nkt >= 12000 && p.nkt >= 48 && !(p.patch && g.sh > 1) && (size_t)g.groups * ((p.M + 63) / 64) * p.nkt * 64 * 96 < kOutOfRange) {
+        } else if (tiles64 * p.nkt >= 12000 && p.nkt >= 48 &&
+                   !(p.patch && (g.sh > 1 || split_cut_64(tiles64, p.nkt, device_cu_count(), 1ll << 30).cost > 1.36e-3 * tiles64 * p.nkt)) && (size_t)g.groups * ((p.M + 63) / 64) * p.nkt * 64 * 96 < kOutOfRange) {
             // below that, long reductions in tiles of 64x64, from some 50 K tiles a CU on.  Filters packed, fp32 instruction / these: 3x3 256->256 at
             // 14x14, batch 16 (196 x 144) 42 / 34 us, batch 4 (52 x 144) 17 / 21, 512->512 at 7x7, batch 16 (104 x 288) 42 / 40, 128->128 at 28x28, batch
             // 16 (392 x 72) 41 / 35, 64->64 at 56x56, batch 4 (196 x 36) 13 / 17, 5x5 48->80 at 31x31, batch 9 (272 x 75) 34 / 28, 1x1 2048->512 at 7x7,
             // batch 16 (104 x 128) 28 / 24, 512->128 at 28x28 (392 x 32) 25 / 25, 3x3 stride 2 128->128 at 56x56 45 / 50 on cold tensors.  (1x1 filters
-            // read in place: 2048->512 29 / 32.  Those calls stay.)
+            // read in place: 2048->512 29 / 32.  Those calls stay.)  The LDS-patch kernel takes some 1.36 us per thousand K tiles and cuts finer: 256->256 at
+            // 14x14, batch 21, whose 260 tiles are just more than a workgroup for every CU, 52 / 56.
             p.split = 1;
             p.patch = 0;
             p.tile = 6;
