@@ -159,9 +159,10 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4],
  * takes the raw filter every time; dlp_conv2d_fwd_enqueue does the same and transforms the filter on
  * every call.  Here the caller transforms it once: `packed` is a device buffer of
  * dlp_conv2d_fwd_packed_bytes(op) bytes (0 for "depthwise_separable") that dlp_conv2d_fwd_pack fills
- * (tile-ordered weights of "gemm", the transformed filter of "winograd") and that
- * dlp_conv2d_fwd_enqueue_packed reads instead of transforming `w` again (`w` is still passed: 1x1
- * bf16 and small float convolutions read it in place).  `ws` then only holds the per-call scratch: workspace() bytes
+ * (tile-ordered weights of "gemm", the transformed filter of "winograd", both where the choice was left
+ * open and large batches run directly) and that dlp_conv2d_fwd_enqueue_packed reads instead of
+ * transforming `w` again (`w` is still passed: 1x1 bf16, 1x1 float of few channels and small float
+ * convolutions read it in place).  `ws` then only holds the per-call scratch: workspace() bytes
  * are always enough, and convolutions that run one after another on a stream may share it.  The
  * buffer serves every batch (float "gemm" weights that a large batch wants as three bf16 parts are
  * held as fp32 tiles too, for small ones).  Pack again after the weights change. */

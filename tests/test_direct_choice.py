@@ -41,3 +41,22 @@ def test_gpu_automatic_choice_by_batch(cin):
         want = torch.nn.functional.conv_transpose2d(dy[-2:].double(), f.double(), None, 1, 1)
         scale = torch.nn.functional.conv_transpose2d(dy[-2:].double().abs(), f.double().abs(), None, 1, 1)
         assert ((dx[-2:].cpu().double() - want).abs() <= scale * ((64 * 9 + 16) * 2.0 ** -24)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch, start", [(16, "conv_split_f32_kernel<64, 64,"), (21, "conv_patch_f32_kernel<")])
+def test_gpu_tiles_of_64_or_patch_by_rounds(batch, start):
+    """144 K tiles a tile: 196 tiles of 64x64 are cut to fill 256 CUs, 260 would leave four of them a round of their own."""
+    gen = torch.Generator().manual_seed(batch)
+    x, f = torch.randn((batch, 256, 14, 14), generator=gen), torch.randn((256, 256, 3, 3), generator=gen)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(256, 256, 3, 1, 1, 1, 1, (batch, 256, 14, 14)), False, "identity", algo="gemm")
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    packed = torch.full((op.packed_size(),), 255, dtype=torch.uint8, device="cuda:0")
+    xd, fd, y = x.cuda(), f.cuda(), torch.full((batch, 256, 14, 14), float("nan"), device="cuda:0")
+    op.pack(fd, packed)
+    (name,) = _kernels(lambda: op.enqueue_packed(xd, fd, packed, None, y, work))
+    assert name.startswith(start), name
+    pick = slice(batch - 2, batch)
+    want = torch.nn.functional.conv2d(x[pick].double(), f.double(), None, 1, 1)
+    scale = torch.nn.functional.conv2d(x[pick].double().abs(), f.double().abs(), None, 1, 1)
+    assert ((y[pick].cpu().double() - want).abs() <= scale * (256 * 9 * 2.0 ** -24)).all()
