@@ -3131,26 +3131,36 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
     // 39 / 39 / 45.  128x128 tiles want twice as much work: 3x3 128->128 at batch 32 (392 x 72) 63 / 53 / 57, 256->256 at 14x14,
     // batch 40 (248 x 144) 81 / 99 / 69.
     if (g.dtype == DLP_FLOAT && p.order == GEMM_ORDER_TAP && !p.stem && !p.pointwise && p.M > 32) {
-        const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 127) / 128), work = tiles * p.nkt;
-        const long long tiles64 = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 63) / 64);
         const int rest = p.M % 128;
-        const int tile = (rest == 0 || rest > 64) && (tiles >= 700 || work >= 30000) ? 4 : 5;
-        const int bm = tile == 4 ? 128 : 64;
-        if ((tiles >= 350 || work >= (p.patch ? 20000 : 12000)) && (size_t)g.groups * ((p.M + bm - 1) / bm) * p.nkt * bm * 96 < kOutOfRange) {
-            p.split = 1;
-            p.patch = 0;
-            p.tile = tile;
-        } else if (tiles64 * p.nkt >= 12000 && p.nkt >= 48 &&
-                   !(p.patch && (g.sh > 1 || split_cut_64(tiles64, p.nkt, device_cu_count(), 1ll << 30).cost > 1.36e-3 * tiles64 * p.nkt)) && (size_t)g.groups * ((p.M + 63) / 64) * p.nkt * 64 * 96 < kOutOfRange) {
+        const auto fits = [&](int bm) { return (size_t)g.groups * ((p.M + bm - 1) / bm) * p.nkt * bm * 96 < kOutOfRange; };
+        const auto split_tile = [&](int batch) { // at this batch; -1: the fp32 instruction
+            const long long rows = (long long)g.groups * ((p.M + 63) / 64), N = (long long)batch * g.OH * g.OW;
+            const long long tiles = rows * ((N + 127) / 128), work = tiles * p.nkt, tiles64 = rows * ((N + 63) / 64);
+            const int tile = (rest == 0 || rest > 64) && (tiles >= 700 || work >= 30000) ? 4 : 5;
+            if ((tiles >= 350 || work >= (p.patch ? 20000 : 12000)) && fits(tile == 4 ? 128 : 64))
+                return tile;
             // below that, long reductions in tiles of 64x64, from some 50 K tiles a CU on.  Filters packed, fp32 instruction / these: 3x3 256->256 at
             // 14x14, batch 16 (196 x 144) 42 / 34 us, batch 4 (52 x 144) 17 / 21, 512->512 at 7x7, batch 16 (104 x 288) 42 / 40, 128->128 at 28x28, batch
             // 16 (392 x 72) 41 / 35, 64->64 at 56x56, batch 4 (196 x 36) 13 / 17, 5x5 48->80 at 31x31, batch 9 (272 x 75) 34 / 28, 1x1 2048->512 at 7x7,
             // batch 16 (104 x 128) 28 / 24, 512->128 at 28x28 (392 x 32) 25 / 25, 3x3 stride 2 128->128 at 56x56 45 / 50 on cold tensors.  (1x1 filters
-            // read in place: 2048->512 29 / 32.  Those calls stay.)  The LDS-patch kernel takes some 1.36 us per thousand K tiles and cuts finer: 256->256 at
-            // 14x14, batch 21, whose 260 tiles are just more than a workgroup for every CU, 52 / 56.
+            // read in place: 2048->512 29 / 32.  Those calls stay.)
+            if (tiles64 * p.nkt < 12000 || p.nkt < 48 || !fits(64))
+                return -1;
+            // The LDS-patch kernel takes some 1.36 us per thousand K tiles and cuts finer: 256->256 at 14x14, batch 21, whose 260 tiles are just
+            // more than a workgroup for every CU, 52 / 56.
+            if (p.patch && (g.sh > 1 || split_cut_64(tiles64, p.nkt, device_cu_count(), 1ll << 30).cost > 1.36e-3 * tiles64 * p.nkt))
+                return -1;
+            return 6;
+        };
+        int tile = split_tile(std::min(g.B, g.B_hint));
+        // What the LDS-patch kernel is left with does not only grow with the batch.  Weights packed ahead, and the place of tiles packed in a call, are
+        // laid out for the batch of the settings: without bf16 parts there, no smaller batch runs on them.
+        if (tile == 6 && g.B < g.B_hint && split_tile(g.B_hint) < 0)
+            tile = -1;
+        if (tile >= 0) {
             p.split = 1;
             p.patch = 0;
-            p.tile = 6;
+            p.tile = tile;
         }
     }
     p.BM = 64;

@@ -884,6 +884,7 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
         for (int i = 0; i < 6; i++)
             DLP_REQUIRE(sig[i] == op->packed_layout[i], "the weights were packed for another tile plan (pack again for this batch)");
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
+        DLP_REQUIRE(hint_plan.split || !plan.split, "the weights were not packed as bf16 parts");
         if (conv_wave_f32_serves(g, true))
             return conv_wave_f32_launch(g, x, w, y, ep, s);
         if (conv_expand_serves(g, ep, x, y))

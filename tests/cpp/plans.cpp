@@ -1,0 +1,97 @@
+// The plans of float convolutions over pairs of batches, the one that an operator is created with and the one that it is called with: what a call
+// reads is what was packed, in the form and in the bytes that it was packed in.  Host code only, run without a GPU by tests/test_plans.py.
+#include "dlp_internal.hpp"
+
+#include <algorithm>
+#include <cstdio>
+#include <cstring>
+
+using namespace dlp;
+
+namespace {
+int failures = 0, checked = 0;
+
+void expect(bool ok, const char *what, const ConvGeom &g)
+{
+    checked++;
+    if (ok)
+        return;
+    if (failures++ < 20)
+        std::printf("%s: %dx%d %d->%d at %dx%d stride %d groups %d, created at batch %d, called at %d\n", what, g.KH, g.KW, g.Cin, g.Cout, g.H, g.W, g.sh, g.groups,
+                    g.B_hint, g.B);
+}
+
+ConvGeom geometry(int cin, int cout, int k, int s, int groups, int h, int w)
+{
+    ConvGeom g = ConvGeom();
+    g.Cin = cin;
+    g.Cout = cout;
+    g.KH = g.KW = k;
+    g.sh = g.sw = s;
+    g.ph = g.pw = k / 2;
+    g.dh = g.dw = 1;
+    g.H = h;
+    g.W = w;
+    g.OH = (h + 2 * g.ph - k) / s + 1;
+    g.OW = (w + 2 * g.pw - k) / s + 1;
+    g.groups = groups;
+    g.dtype = DLP_FLOAT;
+    return g;
+}
+
+template <class F>
+void shapes(F f)
+{
+    const int channels[][2] = {{64, 64}, {128, 128}, {256, 256}, {192, 192}, {384, 384}, {512, 512}, {48, 80}, {320, 96}, {96, 200}, {256, 33}, {768, 512}, {100, 72}};
+    const int sizes[][2] = {{7, 7}, {14, 14}, {28, 28}, {35, 35}, {56, 56}, {19, 23}};
+    for (const auto &c : channels)
+        for (const auto &hw : sizes)
+            for (int k : {1, 3, 5})
+                for (int s : {1, 2})
+                    for (int groups : {1, 2})
+                        f(geometry(c[0] * groups, c[1] * groups, k, s, groups, hw[0], hw[1]));
+}
+
+// weights packed for the settings' batch, run at another one
+void packed()
+{
+    shapes([](ConvGeom g) {
+        for (g.B_hint = 1; g.B_hint <= 72; g.B_hint += g.B_hint < 40 ? 1 : 8) {
+            const GemmPackPlan packs = conv_gemm_pack_plan(g, DLP_ACT_RELU);
+            for (g.B = 1; g.B <= g.B_hint + 1; g.B += g.B < 40 ? 1 : 8) {
+                size_t offset = 0;
+                const GemmPlan p = conv_gemm_plan_on_packed(g, DLP_ACT_RELU, packs.p, offset);
+                const GemmPlan &form = offset ? packs.floats : packs.p;
+                expect(p.split == form.split && offset == (packs.p.split && !p.split ? packs.p.wpack_bytes : 0), "another form than was packed", g);
+                expect(offset + p.wpack_bytes <= packs.bytes, "more bytes than were packed", g);
+                expect(p.pack_bm == form.BM && p.BM <= form.BM && p.nkt == form.nkt && p.order == form.order, "other tiles than were packed", g);
+            }
+        }
+    });
+}
+
+// tiles that a gradient packs in the call, for that call's batch, into a place laid out at create
+void tiles()
+{
+    shapes([](ConvGeom g) {
+        for (g.B_hint = 1; g.B_hint <= 72; g.B_hint += g.B_hint < 40 ? 1 : 8) {
+            const GemmPackPlan packs = conv_gemm_pack_plan(g, DLP_ACT_IDENTITY);
+            const size_t place = packs.p.split ? std::max(packs.p.wpack_bytes, packs.floats.wpack_bytes) : packs.p.wpack_bytes;
+            for (g.B = 1; g.B <= g.B_hint + 1; g.B += g.B < 40 ? 1 : 8)
+                expect(conv_gemm_plan(g, DLP_ACT_IDENTITY).wpack_bytes <= place, "tiles larger than their place", g);
+        }
+    });
+}
+} // namespace
+
+int main(int argc, char **argv)
+{
+    if (argc == 2 && !std::strcmp(argv[1], "packed"))
+        packed();
+    else if (argc == 2 && !std::strcmp(argv[1], "tiles"))
+        tiles();
+    else
+        return 2;
+    std::printf("%d checked, %d failed\n", checked, failures);
+    return failures ? 1 : 0;
+}
