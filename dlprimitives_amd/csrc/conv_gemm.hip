@@ -2762,18 +2762,22 @@ int launch_wave_bf16(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStrea
     return DLP_OK;
 }
 
+// LDS of conv_wave_f32_kernel: operands, later the sums, and the table of its k (none for 1x1)
+constexpr size_t wave_f32_lds(int tile, int wavefronts, long long K, bool point)
+{
+    const int kt = tile == 32 ? 16 : 32;
+    return (size_t)wavefronts * tile * std::max(kt, tile) * 4 + (point ? 0 : (size_t)((K + kt - 1) / kt * kt * 8));
+}
+
 template <int TILE, int KW>
 int launch_wave_f32(const GemmArgs &a, unsigned blocks, hipStream_t stream)
 {
-    constexpr int KT = TILE == 32 ? 16 : 32;
-    constexpr size_t operands = (size_t)KW * TILE * KT * 4, sums = (size_t)KW * TILE * TILE * 4;
     const bool point = a.KH * a.KW == 1;
-    const size_t lds = std::max(operands, sums) + (point ? 0 : (size_t)(a.K + KT - 1) / KT * KT * 8);
     void (*kernel)(GemmArgs) = conv_wave_f32_kernel<TILE, KW, false>;
     if (point)
         kernel = conv_wave_f32_kernel<TILE, KW, true>;
     TimingScope ts("conv_gemm", stream);
-    DLP_LAUNCH_TIMED(ts, kernel, dim3(blocks), dim3(KW * 64), lds, stream, a);
+    DLP_LAUNCH_TIMED(ts, kernel, dim3(blocks), dim3(KW * 64), wave_f32_lds(TILE, KW, a.K, point), stream, a);
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
 }
@@ -3612,6 +3616,26 @@ int conv_gemm_phases_launch(const PhaseConv *ph, int n, const PhasesPlan &pl, co
     return DLP_OK;
 }
 
+// Tiles of 16x16 where those of 32x32 would leave half of the CUs idle (3x3 256->256 at 14x14, one image, 56 tiles: 18.3 us, in tiles of 16x16 12.7;
+// 64->64 at 56x56, 196 tiles: 10.1 and 11.8); four wavefronts for short reductions (15 K tiles, 750 tiles: 11.8 us, eight 12.4).
+struct WaveF32Shape {
+    int tile, wavefronts;
+};
+static WaveF32Shape wave_f32_shape(const ConvGeom &g)
+{
+    const int M = g.Cout / g.groups;
+    const long long tiles32 = (long long)g.groups * ((M + 31) / 32) * (((long long)g.B * g.OH * g.OW + 31) / 32);
+    if (tiles32 <= 128)
+        return {16, 8};
+    return {32, (long long)g.Cin / g.groups * g.KH * g.KW > 15 * 16 ? 8 : 4};
+}
+
+size_t conv_wave_f32_lds_bytes(const ConvGeom &g)
+{
+    const WaveF32Shape s = wave_f32_shape(g);
+    return wave_f32_lds(s.tile, s.wavefronts, (long long)g.Cin / g.groups * g.KH * g.KW, g.KH * g.KW == 1);
+}
+
 // Which float convolutions run on conv_wave_f32_kernel: long reductions in few tiles.  Its time goes with U = tiles of 32x32 x K tiles of 16,
 // about 4 us + 0.35 us per thousand; the other kernels take 9 to 30 us however small the layer, and a packing launch where the filter comes
 // raw.  Measured, us, raw filters, others / this one: 3x3 512->512 at 7x7 batch 1 (U 9200) 26 / 21, 256->256 at 14x14 batch 1 20 / 13, batch 4
@@ -3628,6 +3652,9 @@ bool conv_wave_f32_serves(const ConvGeom &g, bool packed)
     const long long N = (long long)g.B * g.OH * g.OW;
     if (((size_t)g.B * g.Cin * g.H * g.W + (size_t)g.ph * g.W + g.pw) * 4 >= kOutOfRange || (size_t)N * g.Cout * 4 >= kOutOfRange ||
         (size_t)g.Cout * K * 4 >= kOutOfRange)
+        return false;
+    // the table of k beside the operands: up to 4096 k in tiles of 32x32, 6144 in tiles of 16x16, fit the LDS that a launch gets without asking for it
+    if (conv_wave_f32_lds_bytes(g) > 65536)
         return false;
     const long long tiles = (long long)g.groups * ((M + 31) / 32) * ((N + 31) / 32), kt = (K + 15) / 16, u = tiles * kt;
     if (taps == 1) // (not filters that leave conv_gemm_f32_kernel's last tile of 64 half empty: it has tiles of 32 rows for those)
@@ -3679,17 +3706,15 @@ int conv_wave_f32_launch(const ConvGeom &g, const void *x, const void *w, void *
         a.clamp_lo = 0.0f;
     if (ep.activation == DLP_ACT_RELU6)
         a.clamp_hi = 6.0f;
-    // tiles of 16x16 where those of 32x32 would leave half of the CUs idle (3x3 256->256 at 14x14, one image, 56 tiles: 18.3 us, in tiles of 16x16 12.7;
-    // 64->64 at 56x56, 196 tiles: 10.1 and 11.8); four wavefronts for short reductions (15 K tiles, 750 tiles: 11.8 us, eight 12.4)
-    const long long tiles32 = (long long)g.groups * ((a.M + 31) / 32) * ((a.N + 31) / 32);
-    const int tile = tiles32 <= 128 ? 16 : 32;
+    const WaveF32Shape shape = wave_f32_shape(g);
+    const int tile = shape.tile;
     a.mtiles = (a.M + tile - 1) / tile;
     a.ntiles = (a.N + tile - 1) / tile;
     set_tile_magics(a, g.groups);
     const unsigned tiles = (unsigned)((long long)a.mtiles * a.ntiles * g.groups); // (conv_wave_f32_serves bounds them)
     if (tile == 16)
         return launch_wave_f32<16, 8>(a, tiles, stream);
-    return a.K > 15 * 16 ? launch_wave_f32<32, 8>(a, tiles, stream) : launch_wave_f32<32, 4>(a, tiles, stream);
+    return shape.wavefronts == 8 ? launch_wave_f32<32, 8>(a, tiles, stream) : launch_wave_f32<32, 4>(a, tiles, stream);
 }
 
 // Channels-last x and / or y: served by the bf16 matrix-instruction kernels only (x: the channels-last loader, i.e. input

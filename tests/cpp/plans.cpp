@@ -82,6 +82,21 @@ void tiles()
         }
     });
 }
+
+// calls of the small float kernel: no more LDS than a launch gets without asking for it
+void lds()
+{
+    for (int k : {1, 3, 5})
+        for (int cin = 16; cin * k * k <= 9000; cin += cin < 200 ? 7 : 1)
+            for (int cout : {8, 40, 64, 256, 512})
+                for (int size : {1, 7, 10, 14})
+                    for (int batch : {1, 2, 4, 9}) {
+                        ConvGeom g = geometry(cin, cout, k, 1, 1, size, size);
+                        g.B = g.B_hint = batch;
+                        for (bool packed : {false, true})
+                            expect(!conv_wave_f32_serves(g, packed) || conv_wave_f32_lds_bytes(g) <= 65536, "more than 64 KB of LDS", g);
+                    }
+}
 } // namespace
 
 int main(int argc, char **argv)
@@ -90,6 +105,8 @@ int main(int argc, char **argv)
         packed();
     else if (argc == 2 && !std::strcmp(argv[1], "tiles"))
         tiles();
+    else if (argc == 2 && !std::strcmp(argv[1], "lds"))
+        lds();
     else
         return 2;
     std::printf("%d checked, %d failed\n", checked, failures);

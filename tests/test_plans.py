@@ -12,7 +12,7 @@ import dlprimitives_amd as dlp
 BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "bin", "plans")
 
 
-@pytest.mark.parametrize("part", ["packed", "tiles"])
+@pytest.mark.parametrize("part", ["packed", "tiles", "lds"])
 def test_plans(part):
     if not os.path.exists(BIN):
         pytest.fail("tests/bin/plans is not built: run `make -C tests/cpp` (or __graft_entry__.build())")

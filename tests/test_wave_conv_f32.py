@@ -20,6 +20,8 @@ CASES = {
     (64, 40, 3, 1, 2, 2, 1, 2, 40, 41): (32, 8),         # dilated
     (60, 46, 3, 1, 1, 1, 2, 6, 30, 30): (32, 8),         # groups, everything off the tiles
     (20, 40, 5, 1, 2, 1, 1, 3, 33, 31): (32, 8),
+    (455, 256, 3, 1, 1, 1, 1, 4, 14, 14): (32, 8),       # 4095 and 6125 k: all of the 64 KB of LDS
+    (245, 64, 5, 1, 2, 1, 1, 1, 7, 7): (16, 8),
 }
 
 
@@ -49,6 +51,24 @@ def test_gpu_wave_conv_f32(c):
         v = conv(x, f) + chan
         res = {"relu6": lambda: v.clamp(0, 6), "identity": lambda: v + factor * old.double(), "tanh": lambda: v.tanh() + factor * old.double()}[act]()
         assert ((y.cpu().double() - res).abs() <= bound + (4e-7 if act == "tanh" else 0)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(456, 256, 3, 1, 1, 1, 1, 4, 14, 14), (246, 64, 5, 1, 2, 1, 1, 1, 7, 7), (256, 256, 5, 1, 2, 1, 1, 1, 10, 10)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_gpu_wave_conv_f32_longer_reductions(c):
+    """more k than the table has room for: the other kernels"""
+    cin, cout, k, s, p, d, g, b, h, w = c
+    gen, xs, ws, ys = _tensors(c)
+    x, f = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs), False, "identity", "gemm")
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    y = torch.full(ys, float("nan"), device="cuda:0")
+    names = _kernels(lambda: op.enqueue(x.cuda(), f.cuda(), None, y, work))
+    assert names and not any(n.startswith("conv_wave_f32_kernel") for n in names), names
+    conv = lambda x, f: torch.nn.functional.conv2d(x.double(), f.double(), None, s, p, d, g)
+    # a rounding per product
+    assert ((y.cpu().double() - conv(x, f)).abs() <= conv(x.abs(), f.abs()) * ((cin * k * k + 8) * 2.0 ** -24)).all()
 
 
 @pytest.mark.gpu
