@@ -225,8 +225,8 @@ __global__ __launch_bounds__(KW * 64) void conv_wave_bf16_kernel(GemmArgs a)
 //  * Input: a load a k, consecutive lanes on consecutive pixels, straight into the register of that k.  Where k lies and which tap of the window it
 //    is comes from a table in LDS, made when the workgroup starts (POINT: 1x1, no table).
 //  * Both are split into three bf16 parts as in conv_split_f32_kernel, by every lane for the eight k it has of its row and of its pixel: six
-//    products in two accumulators.  What such products cannot hold (operands above 2^16, sums not finite or too small) is summed again in
-//    fp32, output by output, from memory.
+//    products in two accumulators.  A tile that such products cannot hold (operands above 2^16, sums not finite or too small) is computed again,
+//    whole, on the fp32 instruction.
 // A K tile of a 32x32 tile takes a CU some 140 clocks of vector instructions (two splits), 100 of loads, 48 of matrix instructions.
 template <int TILE, int KW, bool POINT>
 __global__ __launch_bounds__(KW * 64) void conv_wave_f32_kernel(GemmArgs a)
@@ -386,51 +386,83 @@ __global__ __launch_bounds__(KW * 64) void conv_wave_f32_kernel(GemmArgs a)
         else
             c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, c, 0, 0, 0);
     };
-    for (int kt = kt_begin; kt < kt_end; kt += DEPTH)
-        static_for_n<DEPTH>([&](auto slot_c) {
-            constexpr int Q = decltype(slot_c)::value;
-            if (kt + Q < kt_end) {
-                // LDS works a wavefront's instructions off in order, and nobody else touches its part: no barrier, no second buffer
+    // IN_FLOATS: the products on the fp32 instruction, whose k a lane gives one at a time
+    auto reduce = [&](auto in_floats_c) {
+        constexpr bool IN_FLOATS = decltype(in_floats_c)::value;
+        for (int kt = kt_begin; kt < kt_end; kt += DEPTH)
+            static_for_n<DEPTH>([&](auto slot_c) {
+                constexpr int Q = decltype(slot_c)::value;
+                if (kt + Q < kt_end) {
+                    // LDS works a wavefront's instructions off in order, and nobody else touches its part: no barrier, no second buffer
 #pragma unroll
-                for (int s = 0; s < 2; s++)
-                    *(u32x4 *)(mine_s + slot[s]) = wv[Q][s];
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                float w[8], x[8];
+                    for (int s = 0; s < 2; s++)
+                        *(u32x4 *)(mine_s + slot[s]) = wv[Q][s];
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    float w[8], x[8];
 #pragma unroll
-                for (int s = 0; s < 2; s++) {
-                    const f32x4 p = *(const f32x4 *)(mine_s + read[s]);
+                    for (int s = 0; s < 2; s++) {
+                        const f32x4 p = *(const f32x4 *)(mine_s + read[s]);
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        w[4 * s + e] = p[e];
+                        for (int e = 0; e < 4; e++)
+                            w[4 * s + e] = p[e];
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        x[e] = xv[Q][e];
+                    load(slot_c, kt + Q + DEPTH);
+                    if constexpr (IN_FLOATS) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            if constexpr (TILE == 32)
+                                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w[e], x[e], acc, 0, 0, 0);
+                            else
+                                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], acc, 0, 0, 0);
+                        }
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; e += 2) {
+                            largest = split_largest(largest, w[e], w[e + 1]);
+                            largest = split_largest(largest, x[e], x[e + 1]);
+                        }
+                        u32x4 wp[3], xp[3];
+                        split8(w, wp);
+                        split8(x, xp);
+                        multiply(acc, wp[0], xp[0]);
+                        multiply(small, wp[1], xp[1]);
+                        multiply(small, wp[1], xp[0]);
+                        multiply(small, wp[0], xp[1]);
+                        multiply(small, wp[2], xp[0]);
+                        multiply(small, wp[0], xp[2]);
+                    }
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-                    x[e] = xv[Q][e];
-                load(slot_c, kt + Q + DEPTH);
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    largest = split_largest(largest, w[e], w[e + 1]);
-                    largest = split_largest(largest, x[e], x[e + 1]);
-                }
-                u32x4 wp[3], xp[3];
-                split8(w, wp);
-                split8(x, xp);
-                multiply(acc, wp[0], xp[0]);
-                multiply(small, wp[1], xp[1]);
-                multiply(small, wp[1], xp[0]);
-                multiply(small, wp[0], xp[1]);
-                multiply(small, wp[2], xp[0]);
-                multiply(small, wp[0], xp[2]);
-            }
-        });
+            });
+    };
+    reduce(std::false_type{});
 
-    const bool large = __syncthreads_or(largest > kSplitLarge);
+    // sums that are not finite or too small, operands too large: the whole tile again on the fp32 instruction
+    float sums[R], finite = 0.0f; // 0 * infinity and 0 * NaN are NaN, which is not equal to zero
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        sums[r] = acc[r] + small[r];
+        finite = fmaf(sums[r], 0.0f, finite);
+    }
+    if (__syncthreads_or(finite != 0.0f || split_small_sum(sums) || largest > kSplitLarge)) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            acc[r] = 0.0f;
+        static_for_n<DEPTH>([&](auto slot_c) { load(slot_c, kt_begin + decltype(slot_c)::value); });
+        reduce(std::true_type{});
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            sums[r] = acc[r];
+        __syncthreads();
+    }
 #pragma unroll
     for (int r = 0; r < R; r++)
-        red[wave][r][lane] = acc[r] + small[r];
+        red[wave][r][lane] = sums[r];
     __syncthreads();
     if (!mine)
         return;
@@ -441,18 +473,6 @@ __global__ __launch_bounds__(KW * 64) void conv_wave_f32_kernel(GemmArgs a)
 #pragma unroll
         for (int w = 0; w < KW; w++)
             sum += red[w][r][lane];
-        const float one[2] = {sum, sum};
-        if ((large || !(fabsf(sum) < __builtin_huge_valf()) || split_small_sum(one)) && yoff[v] != kOutOfRange) {
-            const int m = m0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            const uint32_t pixel = POINT ? xbase - (uint32_t)(8 * h) * a.hw4 : xbase;
-            sum = 0.0f;
-            for (int c = 0, k = 0; c < a.Cin_g; c++)
-                for (int ky = 0; ky < a.KH; ky++)
-                    for (int kx = 0; kx < a.KW; kx++, k++)
-                        if ((xmask >> (ky * a.KW + kx)) & 1u)
-                            sum = fmaf(buf_load<float>(wr, (uint32_t)((g * a.M + m) * a.K + k) * 4u, 0),
-                                       buf_load<float>(xr, pixel + (uint32_t)(((c * a.H + ky * a.dh) * a.W + kx * a.dw) * 4), 0), sum);
-        }
         sum += bias[v];
         if (pre)
             sum = fmaf(old[v], a.factor, sum);

@@ -121,3 +121,34 @@ def test_gpu_wave_conv_f32_automatic_choice():
             y = torch.full(xs, float("nan"), device="cuda:0")
             assert len(_kernels(lambda: call(y), section)) == 1
             assert (y.cpu() - want).abs().max() <= 2e-3 and (algo or torch.equal(y.cpu(), want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(512, 512, 3, 1, 1, 1, 1, 1, 7, 7), (60, 46, 3, 1, 1, 1, 2, 6, 30, 30), (256, 120, 1, 2, 0, 1, 1, 4, 41, 27)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_gpu_wave_conv_f32_large_operands(c):
+    """operands above 2^16 in every tile: the fp32 sums, in little more time than others take (the tile again on the fp32 instruction; one thread an
+    output, a product at a time, took 11 to 34 times as long)"""
+    cin, cout, k, s, p, d, g, b, h, w = c
+    gen, xs, ws, ys = _tensors(c)
+    x, f = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+    large = x.clone()
+    large[:, 1::2] *= 2.0 ** 17
+    conv = lambda x, f: torch.nn.functional.conv2d(x.double(), f.double(), None, s, p, d, g)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs), False, "identity", "gemm")
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    y, fd, times = torch.full(ys, float("nan"), device="cuda:0"), f.cuda(), []
+    for v in (x, large):
+        vd = v.cuda()
+        (name,) = _kernels(lambda: op.enqueue(vd, fd, None, y, work))
+        assert name.startswith("conv_wave_f32_kernel"), name
+        # a rounding per product
+        assert ((y.cpu().double() - conv(v, f)).abs() <= conv(v.abs(), f.abs()) * ((cin // g * k * k + 8) * 2.0 ** -24)).all()
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        for _ in range(50):
+            op.enqueue(vd, fd, None, y, work)
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    assert times[1] <= 8 * times[0], times
