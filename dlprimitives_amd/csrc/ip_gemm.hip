@@ -256,13 +256,14 @@ __global__ __launch_bounds__(256) void ip_direct_kernel(IpArgs a)
 // accumulators are added in wavefront order through LDS; wavefront 0 then finishes the slice like the direct kernel does.
 constexpr int kIpRowBytes = 1024;            // bytes of a row per chunk
 constexpr int kIpLdsRow = kIpRowBytes + 16;  // LDS bytes per row
-// LDS: the tiles of w and x, 65 KB, two workgroups per compute unit.
-constexpr int kIpStreamLds = 64 * kIpLdsRow;
+// LDS of an instance: the tile of w and XR (+ 1 row of zeros when XR < 32) rows of x.  32 rows of x: 65 KB, two workgroups per
+// compute unit; 16 rows (batches of at most 16): 50 KB, three.
+constexpr int ip_stream_lds_bytes(int xr) { return (32 + xr + (xr < 32 ? 1 : 0)) * kIpLdsRow; }
 
-template <class T>
+template <class T, int XR>
 __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
 {
-    extern __shared__ __attribute__((aligned(16))) unsigned char ip_lds[]; // kIpStreamLds, asked for at launch
+    extern __shared__ __attribute__((aligned(16))) unsigned char ip_lds[]; // ip_stream_lds_bytes(XR), asked for at launch
     unsigned char *Ws = ip_lds, *Xs = ip_lds + 32 * kIpLdsRow;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -286,16 +287,25 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
         w_off[i] = (uint32_t)min(m0 + r, a.Out - 1) * row_bytes + (uint32_t)lane * 16u;
         x_off[i] = n0 + r < a.B ? (uint32_t)(n0 + r) * row_bytes + (uint32_t)lane * 16u : kIpOutOfRange;
     }
-    ip_u32x4 rw[8], rx[8];
+    constexpr int XP = XR / 4; // pieces of x per thread
+    ip_u32x4 rw[8], rx[XP];
     auto load_chunk = [&](int c) {
         const uint32_t soff = (uint32_t)c * (uint32_t)kIpRowBytes;
         const bool inside = soff + (uint32_t)lane * 16u < row_bytes; // the last chunk of a row may be short: what follows is the next row
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             rw[i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, inside ? w_off[i] : kIpOutOfRange, soff, 0));
-            rx[i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, inside ? x_off[i] : kIpOutOfRange, soff, 0));
+            if (i < XP)
+                rx[i] = __builtin_bit_cast(ip_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, inside ? x_off[i] : kIpOutOfRange, soff, 0));
         }
     };
+    // batch rows past XR do not exist: their lanes read a row of zeros
+    const int x_row = l32 < XR ? l32 : XR;
+    if (XR < 32) {
+        for (int i = tid; i < kIpLdsRow / 16; i += 256)
+            *(ip_u32x4 *)(Xs + XR * kIpLdsRow + i * 16) = ip_u32x4{0u, 0u, 0u, 0u};
+    }
+
     ip_f32x16 acc[1];
 #pragma unroll
     for (int r = 0; r < 16; r++)
@@ -308,7 +318,8 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             *(ip_u32x4 *)(Ws + (wave + 4 * i) * kIpLdsRow + lane * 16) = rw[i];
-            *(ip_u32x4 *)(Xs + (wave + 4 * i) * kIpLdsRow + lane * 16) = rx[i];
+            if (i < XP)
+                *(ip_u32x4 *)(Xs + (wave + 4 * i) * kIpLdsRow + lane * 16) = rx[i];
         }
         __syncthreads();
         if (c + 1 < c_end)
@@ -318,7 +329,7 @@ __global__ __launch_bounds__(256) void ip_stream_kernel(IpArgs a)
         for (int g = 0; g < 8; g++) {
             const int koff = wave * 256 + g * 32 + h * 16;
             const ip_u32x4 fa = *(const ip_u32x4 *)(Ws + l32 * kIpLdsRow + koff);
-            const ip_u32x4 fb = *(const ip_u32x4 *)(Xs + l32 * kIpLdsRow + koff);
+            const ip_u32x4 fb = *(const ip_u32x4 *)(Xs + x_row * kIpLdsRow + koff);
             if constexpr (sizeof(T) == 4) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
@@ -596,11 +607,11 @@ size_t ip_stream_scratch_bytes(int batch, int inputs, int outputs, int dtype, Ip
     p.mblocks = (outputs + 31) / 32;
     p.nchunks = (batch + 31) / 32;
     p.ngroups = (inputs + kc - 1) / kc; // chunks of a row
-    // K slices: as many workgroups as fit the compute units at once (two each), slices of at
+    // K slices: as many workgroups as fit the compute units at once (three each with the 16-row tile of x, else two), slices of at
     // least two chunks, at most 16 slices, and never more than 1024 tiles x slices once K is cut (4 MiB of partial sums, what the
     // entry point that allocates nothing holds)
     const long long tiles = (long long)p.mblocks * p.nchunks;
-    long long s = (2ll * dlp_cu_count() + tiles - 1) / tiles;
+    long long s = ((batch <= 16 ? 3ll : 2ll) * dlp_cu_count() + tiles - 1) / tiles;
     s = std::min<long long>(s, std::max<long long>(1, 1024 / tiles));
     s = std::min<long long>(s, p.ngroups / 2);
     s = std::max<long long>(1, std::min<long long>(s, 16));
@@ -613,35 +624,56 @@ size_t ip_stream_scratch_bytes(int batch, int inputs, int outputs, int dtype, Ip
     return p.cnt_bytes + p.part_bytes;
 }
 
-// Batches in tiles of 16x16 (ip_stream_kernel_16x16) instead: all of at most 16 rows, and up to as many tiles as CUs, twice that where rows are short.
-// us, streaming / these, cold weights: fp32 25088 -> 4096 at batch 16 94 / 78 (5.2 TB/s), 32 102 / 120; 9216 -> 4096 at 32 45 / 51; 4096 -> 4096 at 16 26 / 17,
-// 32 27 / 27, 64 39 / 44; 4096 -> 1000 at 16 15 / 12, 64 20 / 12; 2048 -> 1000 at 128 17 / 12; 512 -> 4096 at 16 8.9 / 4.3, 32 9.2 / 7.0, 64 10 / 12; bf16 25088
-// -> 4096 at 16 39 / 32, 4096 -> 1000 at 16 11 / 5.5, 4096 -> 4096 at 32 17 / 15, 1280 -> 1000 at 1 7.8 / 3.4.
-static bool ip_tiles_16x16(int batch, int inputs, int outputs)
+// Batches in tiles of 16x16 (ip_stream_kernel_16x16) instead.  One workgroup of sixteen wavefronts fills a CU, so what counts is the tiles a CU
+// has to go through and the bytes of a row that a tile's workgroup reads alone.  us, streaming / these, warm weights:
+//  * up to as many tiles as CUs, twice that where rows are short: cold weights, fp32 25088 -> 4096 at batch 16 94 / 78 (5.2 TB/s), 32 102 / 120;
+//    9216 -> 4096 at 32 45 / 51; 4096 -> 4096 at 16 26 / 17, 32 27 / 27, 64 39 / 44; 4096 -> 1000 at 16 15 / 12, 64 20 / 12; 2048 -> 1000 at 128 17 /
+//    12; 512 -> 4096 at 16 8.9 / 4.3, 32 9.2 / 7.0, 64 10 / 12; bf16 25088 -> 4096 at 16 39 / 32, 4096 -> 1000 at 16 11 / 5.5, 4096 -> 4096 at 32 17 / 15,
+//    1280 -> 1000 at 1 7.8 / 3.4;
+//  * batches of 16 and fewer, whose one tile of x every workgroup reads, up to more tiles: a workgroup costs most where its rows are short
+//    (fp32 504 -> 21872 at batch 1, 2 KB and 1367 tiles, 15 / 16; 240 -> 51562 at 4 25 / 34; bf16 440 -> 47120 at 16 16 / 22, 3064 -> 22879 at 1 26 / 29);
+//  * but few tiles with long rows leave the chip to the K slices (fp32 24928 -> 32 at 1, 2 tiles of 100 KB, 22 / 30; 23592 -> 201 at 128 33 / 45), and
+//    so do a few tiles more than CUs, which take a round of their own (27304 -> 4192 at 4, 262 tiles, 110 / 131).
+static bool ip_tiles_16x16(int batch, int inputs, int outputs, int dtype)
 {
-    const long long tiles = (long long)((batch + 15) / 16) * ((outputs + 15) / 16);
-    return batch <= 16 || tiles <= (inputs <= 4096 ? 512 : 256);
+    const long long tiles = (long long)((batch + 15) / 16) * ((outputs + 15) / 16), row = (long long)inputs * (long long)dtype_size(dtype);
+    const long long cus = dlp_cu_count(), rounds = (tiles + cus - 1) / cus;
+    if (row > 36000 && tiles * 640 < row)
+        return false;
+    if (batch > 16)
+        return tiles <= (inputs <= 4096 ? 512 : 256);
+    if (row >= 8000)
+        return tiles <= cus || (tiles <= 1024 && 10 * tiles >= 7 * rounds * cus);
+    return tiles <= (row < 2000 ? 512 : dtype == DLP_BFLOAT16 ? 1024 : 2000);
 }
 
 // An instance that needs more than 64 KB of LDS has to ask for it, once per device.  Done when an operator is created (best
 // effort: there may be no device yet) so that a first enqueue inside a stream capture has nothing left to set up; the launch
 // checks again.
-template <class T>
+template <class T, int XR>
 static int ip_stream_instance(const IpArgs *a, dim3 grid, hipStream_t stream, TimingScope *ts)
 {
-    static std::atomic<bool> asked[64];
-    int dev = 0;
-    DLP_HIP_TRY(hipGetDevice(&dev));
-    if (dev < 0 || dev >= 64 || !asked[dev].load()) {
-        DLP_HIP_TRY(hipFuncSetAttribute((const void *)ip_stream_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, kIpStreamLds));
-        if (dev >= 0 && dev < 64)
-            asked[dev].store(true);
+    constexpr int lds = ip_stream_lds_bytes(XR);
+    if (lds > 65536) {
+        static std::atomic<bool> asked[64];
+        int dev = 0;
+        DLP_HIP_TRY(hipGetDevice(&dev));
+        if (dev < 0 || dev >= 64 || !asked[dev].load()) {
+            DLP_HIP_TRY(hipFuncSetAttribute((const void *)ip_stream_kernel<T, XR>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+            if (dev >= 0 && dev < 64)
+                asked[dev].store(true);
+        }
     }
     if (a == nullptr) // set-up only
         return DLP_OK;
-    DLP_LAUNCH_TIMED((*ts), ip_stream_kernel<T>, grid, dim3(256), kIpStreamLds, stream, *a);
+    DLP_LAUNCH_TIMED((*ts), (ip_stream_kernel<T, XR>), grid, dim3(256), lds, stream, *a);
     DLP_HIP_TRY(hipGetLastError());
     return DLP_OK;
+}
+template <class T>
+static int ip_stream_dispatch(bool small_batch, const IpArgs *a, dim3 grid, hipStream_t stream, TimingScope *ts)
+{
+    return small_batch ? ip_stream_instance<T, 16>(a, grid, stream, ts) : ip_stream_instance<T, 32>(a, grid, stream, ts);
 }
 template <class T>
 static int ip_wave_instance(const IpArgs *a, dim3 grid, hipStream_t stream, TimingScope *ts)
@@ -664,7 +696,9 @@ void ip_stream_prepare(int dtype)
 {
     if (dtype != DLP_FLOAT && dtype != DLP_BFLOAT16)
         return;
-    (void)(dtype == DLP_BFLOAT16 ? ip_stream_instance<bf16_t>(nullptr, dim3(1), nullptr, nullptr) : ip_stream_instance<float>(nullptr, dim3(1), nullptr, nullptr));
+    for (int small = 0; small < 2; small++)
+        (void)(dtype == DLP_BFLOAT16 ? ip_stream_dispatch<bf16_t>(small != 0, nullptr, dim3(1), nullptr, nullptr)
+                                     : ip_stream_dispatch<float>(small != 0, nullptr, dim3(1), nullptr, nullptr));
     (void)(dtype == DLP_BFLOAT16 ? ip_wave_instance<bf16_t>(nullptr, dim3(1), nullptr, nullptr) : ip_wave_instance<float>(nullptr, dim3(1), nullptr, nullptr));
     (void)hipGetLastError(); // no device, no harm: the launch asks again
 }
@@ -702,12 +736,14 @@ int ip_stream_launch(int batch, int inputs, int outputs, int dtype, const void *
         return fail(DLP_ERR_NOT_IMPLEMENTED, "inner product too large for a single launch");
     const dim3 grid((unsigned)wgs);
     TimingScope ts("ip_direct", stream);
-    if (ip_tiles_16x16(batch, inputs, outputs)) {
+    if (ip_tiles_16x16(batch, inputs, outputs, dtype)) {
         a.nchunks = (batch + 15) / 16;
         const dim3 tiles((unsigned)((outputs + 15) / 16 * a.nchunks));
         return dtype == DLP_BFLOAT16 ? ip_wave_instance<bf16_t>(&a, tiles, stream, &ts) : ip_wave_instance<float>(&a, tiles, stream, &ts);
     }
-    return dtype == DLP_BFLOAT16 ? ip_stream_instance<bf16_t>(&a, grid, stream, &ts) : ip_stream_instance<float>(&a, grid, stream, &ts);
+    // batches of at most 16 rows keep 16 rows of x in LDS: three workgroups per compute unit instead of two
+    return dtype == DLP_BFLOAT16 ? ip_stream_dispatch<bf16_t>(batch <= 16, &a, grid, stream, &ts)
+                                 : ip_stream_dispatch<float>(batch <= 16, &a, grid, stream, &ts);
 }
 
 ConvGeom ip_gemm_geom(int batch, int inputs, int outputs, int dtype)

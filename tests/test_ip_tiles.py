@@ -18,6 +18,11 @@ CASES = {
     (17, 520, 4112): False,
     (33, 8192, 1360): True,   # 255 tiles of long rows
     (49, 8192, 1040): False,
+    (4, 240, 8192): True,     # short rows: two tiles a CU
+    (4, 240, 8208): False,
+    (2, 8192, 4112): False,   # a tile more than CUs
+    (16, 20000, 2000): True,  # rows of 80 KB (40 in bf16): enough tiles
+    (1, 24576, 32): False,    # ... and too few
 }
 
 
