@@ -3657,13 +3657,23 @@ bool conv_wave_f32_serves(const ConvGeom &g, bool packed)
     if (conv_wave_f32_lds_bytes(g) > 65536)
         return false;
     const long long tiles = (long long)g.groups * ((M + 31) / 32) * ((N + 31) / 32), kt = (K + 15) / 16, u = tiles * kt;
-    if (taps == 1) // (not filters that leave conv_gemm_f32_kernel's last tile of 64 half empty: it has tiles of 32 rows for those)
-        return kt >= 14 && (M <= 32 || M % 64 == 0 || M % 64 > 32) && u <= (kt >= 32 ? 20000 : 8000);
+    // (1x1: not filters that leave conv_gemm_f32_kernel's last tile of 64 half empty, it has tiles of 32 rows for those; strided ones use a part of
+    // every line they load: 1024->256 at 28x28 stride 2, batch 6, u 18900, 19 / 31)
+    const bool strided = g.sh > 1 || g.sw > 1;
+    if (taps == 1)
+        return kt >= 14 && (M <= 32 || M % 64 == 0 || M % 64 > 32) && u <= (kt >= 32 ? (strided ? 16000 : 20000) : strided ? 6000 : 8000);
     if (kt < 9)
         return false;
-    if (cin_g % BK != 0)
-        return u <= 54000;
-    if (kt < 14 && M <= 32) // 3x3 of 16 channels: 64 filters at 40x40, batch 6, 26 / 10; 16 at 60x60, batch 12, 14 / 16
+    // Short reductions in many tiles are the other kernels' again: channels off 16 3x3 15->256 at 56x14, batch 16, 3136 tiles, packed 16 / 26 us, 18->128
+    // at 56x56, batch 4, 1568, packed 11.5 / 16, 25->192 at 14x71, batch 16, 2982, raw 20 / 26; 16->512 at 56x56 stride 2, batch 2, 784, packed 7.3 / 10.3
+    // (of stride 1, on the LDS-patch kernel, 16->128 at 28x28, batch 8, 784, packed 20 / 11).  Strided ones load a part of every line: 422->1024 at
+    // 58x9, u 38000, packed 28 / 33, 154->256 at 68x8, batch 16, 47000, raw 30 / 38.
+    if (cin_g % BK != 0) {
+        if (kt <= 30 && tiles > (M <= 32 ? 1900 : packed ? 1000 : 1500))
+            return false;
+        return u <= (!strided ? 54000 : packed ? 36000 : 46000);
+    }
+    if (kt < 14 && (M <= 32 || (strided && tiles > (packed ? 700 : 1500)))) // 3x3 of 16 channels: 64 filters at 40x40, batch 6, 26 / 10; 16 at 60x60, batch 12, 14 / 16
         return false;
     return packed ? u <= 10000 && tiles >= 48 : u <= 24000;
 }

@@ -72,6 +72,32 @@ def test_gpu_wave_conv_f32_longer_reductions(c):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("c, packed, wave", [
+    ((18, 128, 3, 1, 1, 1, 1, 4, 56, 56), True, False),     # 1568 tiles of 11 K tiles
+    ((18, 128, 3, 1, 1, 1, 1, 2, 56, 56), True, True),
+    ((25, 192, 3, 1, 1, 1, 1, 16, 14, 71), False, False),   # 2982 of 15
+    ((154, 256, 3, 2, 1, 1, 1, 16, 68, 8), False, False),   # strided
+    ((1024, 256, 1, 2, 0, 1, 1, 6, 28, 28), False, False),
+    ((1024, 256, 1, 2, 0, 1, 1, 2, 28, 28), False, True),
+], ids=str)
+def test_gpu_wave_conv_f32_lines(c, packed, wave):
+    """calls on either side of the lines to the other kernels"""
+    cin, cout, k, s, p, d, g, b, h, w = c
+    gen, xs, ws, ys = _tensors(c)
+    x, f = torch.randn(xs, generator=gen), torch.randn(ws, generator=gen)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs), False, "identity", "gemm")
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    y, xd, fd = torch.full(ys, float("nan"), device="cuda:0"), x.cuda(), f.cuda()
+    buf = torch.empty(op.packed_size(), dtype=torch.uint8, device="cuda:0")
+    op.pack(fd, buf)
+    names = _kernels(lambda: op.enqueue_packed(xd, fd, buf, None, y, work) if packed else op.enqueue(xd, fd, None, y, work))
+    assert len(names) == 1 and names[0].startswith("conv_wave_f32_kernel") == wave, names
+    conv = lambda x, f: torch.nn.functional.conv2d(x.double(), f.double(), None, s, p, d, g)
+    # a rounding per product
+    assert ((y.cpu().double() - conv(x, f)).abs() <= conv(x.abs(), f.abs()) * ((cin * k * k + 8) * 2.0 ** -24)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("c", [(237, 58, 1, 1, 0, 1, 1, 2, 9, 7), (26, 48, 3, 1, 1, 1, 1, 11, 33, 33)], ids=lambda c: "x".join(map(str, c)))
 def test_gpu_wave_conv_f32_special_values(c):
     """infinities, NaN, operands near the ends of the range: what the fp32 sum of the products is"""
