@@ -955,7 +955,7 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
         float *wt = (float *)ws;
         void *fws = (char *)ws + op->wt_bytes;
         PhaseFilter pf = {{}, wt, c.kernel[0], c.kernel[1], 0, 1, 0, 1};
-        if (conv_fwd_tiles_plan(op->fwd, batch, &pf.plan)) {
+        if (conv_fwd_tiles_plan(op->fwd, batch, false, &pf.plan)) {
             DLP_REQUIRE(pf.plan.wpack_bytes <= op->wt_bytes, "tiles larger than their place in the workspace");
             const int rc = conv_gemm_pack_phases((const float *)w, c.groups, cout_g, cin_g, c.kernel[0], c.kernel[1], &pf, 1, st);
             if (rc != DLP_OK)
@@ -1029,7 +1029,7 @@ static int bwd_data_run(dlp_conv2d_bwd_data *op, const int x_shape[4], void *dx,
         cursor += round256(planes * ph.h.out * ph.w.out * sizeof(float));
         GemmPlan plan;
         packed_as[i] = -1;
-        if (conv_fwd_tiles_plan(ph.fwd, batch, &plan)) {
+        if (conv_fwd_tiles_plan(ph.fwd, batch, true, &plan)) {
             DLP_REQUIRE(plan.wpack_bytes <= ph.wt_bytes, "tiles larger than their place in the workspace");
             packed_as[i] = npf;
             pf[npf++] = {plan, wt[i], ph.h.n, ph.w.n, ph.h.r0, ph.h.rstep, ph.w.r0, ph.w.rstep};

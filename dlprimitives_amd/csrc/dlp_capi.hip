@@ -295,14 +295,18 @@ static void layout_of(const GemmPlan &p, int (&sig)[6])
 }
 
 namespace dlp {
-bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan)
+bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, bool one_of_several, GemmPlan *plan)
 {
     ConvGeom g;
     const int x_shape[4] = {batch, op->cfg.channels_in, op->cfg.shape[2], op->cfg.shape[3]};
     if (op_geom(op, x_shape, g) != DLP_OK || g.dtype != DLP_FLOAT)
         return false;
     *plan = conv_gemm_plan(g, op->activation);
-    return runs_as_gemm(op, g, *plan) && plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise && !conv_wave_f32_serves(g, false);
+    // One of several phases has its tiles packed along with the others', and would have its filter picked by a launch of its own: worth it from 24
+    // K tiles on (transposed 3x3 stride 2 128->64 at 28x28, batch 16, tanh, phases of 32, 16, 16 and 8 K tiles 60 us, the two of 16 on the small kernel
+    // 70; 6x6 64->32 at 32x32, batch 16, four of 36, 79 and 61), and for phases of one tap (2x2 stride 3 64->256 at 7x8, batch 17, 41 and 27).
+    return runs_as_gemm(op, g, *plan) && plan->order == GEMM_ORDER_TAP && !plan->stem && !plan->pointwise &&
+           ((one_of_several && plan->nkt < 24 && g.KH * g.KW > 1) || !conv_wave_f32_serves(g, false));
 }
 
 bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab)

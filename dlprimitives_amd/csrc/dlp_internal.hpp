@@ -313,8 +313,9 @@ int conv_wave_f32_launch(const ConvGeom &g, const void *x, const void *w, void *
 // the gather table of a float operator of algorithm gemm in the tap-major order (not where the kernel reads the filter as it is), and the geometry of its convolution at this batch
 bool conv_fwd_tap_table(const dlp_conv2d_fwd *op, int batch, ConvGeom &g, const KTabEntry **ktab);
 // Whether a call at this batch can run on tiles that conv_gemm_pack_phases writes, and by which plan (float, algorithm gemm, K tiles of one
-// tap x 16 channels; not where the kernel of the call reads the filter as it is, which depends on the batch too).
-bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, GemmPlan *plan);
+// tap x 16 channels; not where the kernel of the call reads the filter as it is, which depends on the batch too).  one_of_several: of
+// the phases of a strided pass.
+bool conv_fwd_tiles_plan(const dlp_conv2d_fwd *op, int batch, bool one_of_several, GemmPlan *plan);
 // ... the bytes of the tiles, enough for every batch (0: no call of this operator runs on them)
 size_t conv_fwd_tiles_bytes(const dlp_conv2d_fwd *op);
 // ... and the call (an operator without bias)

@@ -1,0 +1,34 @@
+"""Stride phases that run one by one (an activation that the one launch of all phases does not have): which kernels serve them, and the sums."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import dlprimitives_amd as dlp
+from test_split_gemm import _kernels
+
+
+# (cin, cout, k, pad, output pad, batch, h): phases on the small-tile kernel
+CASES = {
+    (128, 64, 3, 1, 1, 16, 28): 0,  # 32, 16, 16 and 8 K tiles a phase
+    (64, 32, 6, 2, 0, 16, 32): 4,   # four of 36
+    (256, 40, 1, 0, 1, 4, 14): 1,   # one phase of one tap
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_gpu_phases_one_by_one(c):
+    cin, cout, k, p, extra, b, h = c
+    gen = torch.Generator().manual_seed(sum(c))
+    x, f, bias = torch.randn((b, cin, h, h), generator=gen), torch.randn((cin, cout, k, k), generator=gen), torch.randn(cout, generator=gen)
+    x, bias = x / (cin * k * k / 4) ** 0.5, bias / 4
+    op = dlp.TransposedConv2DForward.create(dlp.Conv2DSettings(cin, cout, k, 2, 1, p, 1, tuple(x.shape)), (extra, extra), True, "tanh")
+    y = torch.full(op.output_shape(tuple(x.shape)), float("nan"), device="cuda:0")
+    work = torch.empty(op.workspace(), dtype=torch.uint8, device="cuda:0")
+    names = _kernels(lambda: op.enqueue(x.cuda(), f.cuda(), bias.cuda(), y, work))
+    assert sum(n.startswith("conv_wave_f32_kernel") for n in names) == CASES[c], names
+    back = lambda x, f: torch.nn.functional.conv_transpose2d(x.double(), f.double(), None, 2, p, extra)
+    chan = bias.double().view(1, -1, 1, 1)
+    # a rounding per product ahead of tanh, which shrinks every difference, and a few of its own
+    bound = (back(x.abs(), f.abs()) + chan.abs()) * ((cin * k * k + 8) * 2.0 ** -24) + 4e-7
+    assert ((y.cpu().double() - (back(x, f) + chan).tanh()).abs() <= bound).all()
