@@ -774,6 +774,34 @@ static void bwd_data_free(dlp_conv2d_bwd_data *op)
     delete op;
 }
 
+// The phases as one launch, longest first (place[i]: of phase i), where all of them have filter taps and are convolutions on tiles of 16 channels
+// of a tap (conv_gemm_phases_plan).
+static bool merged_phases(const dlp_conv2d_bwd_data *op, int batch, int act, size_t ws_bytes, PhaseConv *ph, int *order, PhasesPlan &plan)
+{
+    if (!op->strided || op->nphases > kMaxPhases)
+        return false;
+    for (int i = 0; i < op->nphases; i++) {
+        if (!op->phase[i].fwd)
+            return false;
+        order[i] = i;
+    }
+    std::stable_sort(order, order + op->nphases, [&](int x, int y) {
+        return op->phase[x].h.n * op->phase[x].w.n > op->phase[y].h.n * op->phase[y].w.n;
+    });
+    const dlp_conv2d_settings &c = op->cfg;
+    for (int j = 0; j < op->nphases; j++) {
+        const BwdPhase &p = op->phase[order[j]];
+        if (!conv_fwd_tap_table(p.fwd, batch, ph[j].g, &ph[j].ktab))
+            return false;
+        ph[j].off_h = p.h.off;
+        ph[j].off_w = p.w.off;
+        ph[j].len_h = p.h.len;
+        ph[j].len_w = p.w.len;
+        ph[j].out_off = order[j] / c.stride[1] * c.shape[3] + order[j] % c.stride[1];
+    }
+    return conv_gemm_phases_plan(ph, op->nphases, act, ws_bytes, plan);
+}
+
 int dlp_conv2d_bwd_data_create(const dlp_conv2d_settings *cfg, const char *algo, dlp_conv2d_bwd_data **out)
 {
     DLP_REQUIRE(out != nullptr, "null argument");
@@ -825,32 +853,48 @@ int dlp_conv2d_bwd_data_create(const dlp_conv2d_settings *cfg, const char *algo,
     op->nphases = cfg->stride[0] * cfg->stride[1];
     for (int i = 0; i < op->nphases; i++)
         op->phase[i].fwd = nullptr;
-    // an algorithm that was left open is the one whose phases run in one launch, also for phases of 3x3 taps
-    const bool open = algo == nullptr || *algo == 0 || std::string(algo) == "auto";
-    const char *const phase_algo = open && cfg->channels_out / cfg->groups % 16 == 0 ? "gemm" : algo;
-    for (int a = 0; a < cfg->stride[0]; a++)
-        for (int b = 0; b < cfg->stride[1]; b++) {
-            BwdPhase &ph = op->phase[a * cfg->stride[1] + b];
-            ph.h = phase_axis(a, cfg->shape[2], op->OH, cfg->kernel[0], cfg->stride[0], cfg->dilate[0], cfg->pad[0]);
-            ph.w = phase_axis(b, cfg->shape[3], op->OW, cfg->kernel[1], cfg->stride[1], cfg->dilate[1], cfg->pad[1]);
-            ph.wt_bytes = ph.fwd_ws = 0;
-            if (ph.h.n == 0 || ph.w.n == 0)
-                continue; // no filter tap meets this phase: its part of dx is zero
-            dlp_conv2d_settings u = t;
-            u.kernel[0] = ph.h.n;
-            u.kernel[1] = ph.w.n;
-            u.dilate[0] = ph.h.dil;
-            u.dilate[1] = ph.w.dil;
-            u.pad[0] = ph.h.pad;
-            u.pad[1] = ph.w.pad;
-            rc = dlp_conv2d_fwd_create(&u, 0, DLP_ACT_IDENTITY, phase_algo, &ph.fwd);
-            if (rc != DLP_OK) {
-                bwd_data_free(op);
-                return rc;
+    const auto create_phases = [&](const char *phase_algo) {
+        for (int a = 0; a < cfg->stride[0]; a++)
+            for (int b = 0; b < cfg->stride[1]; b++) {
+                BwdPhase &ph = op->phase[a * cfg->stride[1] + b];
+                dlp_conv2d_fwd_destroy(ph.fwd);
+                ph.fwd = nullptr;
+                ph.h = phase_axis(a, cfg->shape[2], op->OH, cfg->kernel[0], cfg->stride[0], cfg->dilate[0], cfg->pad[0]);
+                ph.w = phase_axis(b, cfg->shape[3], op->OW, cfg->kernel[1], cfg->stride[1], cfg->dilate[1], cfg->pad[1]);
+                ph.wt_bytes = ph.fwd_ws = 0;
+                if (ph.h.n == 0 || ph.w.n == 0)
+                    continue; // no filter tap meets this phase: its part of dx is zero
+                dlp_conv2d_settings u = t;
+                u.kernel[0] = ph.h.n;
+                u.kernel[1] = ph.w.n;
+                u.dilate[0] = ph.h.dil;
+                u.dilate[1] = ph.w.dil;
+                u.pad[0] = ph.h.pad;
+                u.pad[1] = ph.w.pad;
+                const int rc = dlp_conv2d_fwd_create(&u, 0, DLP_ACT_IDENTITY, phase_algo, &ph.fwd);
+                if (rc != DLP_OK)
+                    return rc;
+                ph.wt_bytes = std::max(conv_fwd_tiles_bytes(ph.fwd), round256((size_t)cfg->channels_out * cin_g * ph.h.n * ph.w.n * sizeof(float)));
+                ph.fwd_ws = round256(dlp_conv2d_fwd_workspace(ph.fwd));
             }
-            ph.wt_bytes = std::max(conv_fwd_tiles_bytes(ph.fwd), round256((size_t)cfg->channels_out * cin_g * ph.h.n * ph.w.n * sizeof(float)));
-            ph.fwd_ws = round256(dlp_conv2d_fwd_workspace(ph.fwd));
-        }
+        return (int)DLP_OK;
+    };
+    // An algorithm that was left open is the one whose phases run in one launch, also for phases of 3x3 taps; where they don't at the batch of the
+    // settings, every phase has its own choice (6x6 stride 2 8->128 at 56x56, batch 64: 153 us, phases on "gemm" 162).
+    const bool open = algo == nullptr || *algo == 0 || std::string(algo) == "auto";
+    const bool gemm = open && cfg->channels_out / cfg->groups % 16 == 0;
+    rc = create_phases(gemm ? "gemm" : algo);
+    if (rc == DLP_OK && gemm) {
+        PhaseConv ph[kMaxPhases];
+        int order[kMaxPhases];
+        PhasesPlan plan;
+        if (!merged_phases(op, std::max(cfg->shape[0], 1), DLP_ACT_IDENTITY, (size_t)-1, ph, order, plan))
+            rc = create_phases(algo);
+    }
+    if (rc != DLP_OK) {
+        bwd_data_free(op);
+        return rc;
+    }
     *out = op;
     return DLP_OK;
 }
@@ -886,34 +930,6 @@ static size_t bwd_data_need(const dlp_conv2d_bwd_data *op, int batch, size_t *fw
     if (fwd_ws_out)
         *fwd_ws_out = fws;
     return total + fws;
-}
-
-// The phases as one launch, longest first (place[i]: of phase i), where all of them have filter taps and are convolutions on tiles of 16 channels
-// of a tap (conv_gemm_phases_plan).
-static bool merged_phases(const dlp_conv2d_bwd_data *op, int batch, int act, size_t ws_bytes, PhaseConv *ph, int *order, PhasesPlan &plan)
-{
-    if (!op->strided || op->nphases > kMaxPhases)
-        return false;
-    for (int i = 0; i < op->nphases; i++) {
-        if (!op->phase[i].fwd)
-            return false;
-        order[i] = i;
-    }
-    std::stable_sort(order, order + op->nphases, [&](int x, int y) {
-        return op->phase[x].h.n * op->phase[x].w.n > op->phase[y].h.n * op->phase[y].w.n;
-    });
-    const dlp_conv2d_settings &c = op->cfg;
-    for (int j = 0; j < op->nphases; j++) {
-        const BwdPhase &p = op->phase[order[j]];
-        if (!conv_fwd_tap_table(p.fwd, batch, ph[j].g, &ph[j].ktab))
-            return false;
-        ph[j].off_h = p.h.off;
-        ph[j].off_w = p.w.off;
-        ph[j].len_h = p.h.len;
-        ph[j].len_w = p.w.len;
-        ph[j].out_off = order[j] / c.stride[1] * c.shape[3] + order[j] % c.stride[1];
-    }
-    return conv_gemm_phases_plan(ph, op->nphases, act, ws_bytes, plan);
 }
 
 size_t dlp_conv2d_bwd_data_workspace(const dlp_conv2d_bwd_data *op)

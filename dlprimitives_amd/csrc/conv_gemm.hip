@@ -3475,10 +3475,12 @@ bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws
     // Tiles: what the phases would take by themselves, and 64x64 below that, measured against one launch a phase and the interleaving (transposed,
     // packing included, us; interleaved / 64x64 / 64x128 / 128x128): 256->128 at 14x14, 4x4, batch 1 73 / 22 / 28 / 37, batch 4 77 / 26 / 31 / 40, batch
     // 16 91 / 45 / 46 / 49; 512->256 at 7x7, 4x4, batch 8 87 / 36 / 42 / 53; 512->16 at 20x20, 3x3, batch 4 72 / 24 / 31 / 41; 128->128 at 28x28,
-    // 4x4, batch 32 175 / 120 / 115 / 108, 128->64 at 56x56 278 / 202 / 195 / 264.  No size was found where one launch a phase is the better one.
+    // 4x4, batch 32 175 / 120 / 115 / 108, 128->64 at 56x56 278 / 202 / 195 / 264.
     const int bm = tile == 4 ? 128 : 64, bn = tile == 0 ? 64 : 128;
     pl.packed_bytes = 0;
     long long ntiles = 0;
+    double half_empty = 0.0;
+    bool winograd = true; // every phase would be Winograd's by itself, on images that do not leave its tiles half empty
     for (int i = 0; i < n; i++) {
         const ConvGeom &g = ph[i].g;
         GemmPlan &p = pl.plan[i];
@@ -3495,8 +3497,17 @@ bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws
         p.mtiles = (M + bm - 1) / bm;
         p.wpack_bytes = (size_t)g.groups * p.mtiles * p.nkt * bm * 96;
         pl.packed_bytes += p.wpack_bytes;
-        ntiles += (long long)g.groups * p.mtiles * (((long long)g.B * ph[i].len_h * ph[i].len_w + p.BN - 1) / p.BN);
+        const long long N = (long long)g.B * ph[i].len_h * ph[i].len_w;
+        ntiles += (long long)g.groups * p.mtiles * ((N + p.BN - 1) / p.BN);
+        winograd = winograd && g.KH == 3 && g.KW == 3 && ph[i].len_h >= 14 && ph[i].len_w >= 14;
+        half_empty += M <= 32 ? (double)g.groups * p.nkt * ((N + 63) / 64) - 6e-3 * g.groups * M * N : 0.0;
     }
+    // Up to 32 rows leave half of these tiles empty: in large launches, less what one launch a phase writes twice, tiles of 32 rows (Winograd's for 3x3
+    // phases) and the interleaving are faster.  One launch a phase / this one, stride 2, us: 6x6 8->128 at 56x56, batch 64, 226000 K tiles 153 / 169, batch
+    // 200 339 / 485, 32->128 at 64 171 / 185, 8->64 at 128 176 / 167, 8->512 at 14x14, batch 256, 260 / 188; 5x5 8->128 at 128, 314000 194 / 224, 32->128
+    // 226 / 251, 8->256 at 28x28, batch 200, 245000 200 / 184; 4x4 8->128 at 200, 314000 209 / 232.
+    if (half_empty > (winograd ? 185000.0 : 235000.0))
+        return false;
     pl.packed_bytes = (pl.packed_bytes + 255) / 256 * 256;
     const size_t fixed = pl.packed_bytes + split_counter_bytes(ntiles);
     if (pl.packed_bytes >= kOutOfRange || ntiles * 16 > 0x7fffffffLL || fixed > ws_bytes)

@@ -32,3 +32,30 @@ def test_gpu_phases_one_by_one(c):
     # a rounding per product ahead of tanh, which shrinks every difference, and a few of its own
     bound = (back(x.abs(), f.abs()) + chan.abs()) * ((cin * k * k + 8) * 2.0 ** -24) + 4e-7
     assert ((y.cpu().double() - (back(x, f) + chan).tanh()).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c, merged", [((8, 128, 6, 2, 64, 56), False), ((8, 128, 6, 2, 32, 56), True), ((32, 128, 5, 2, 136, 56), False), ((33, 128, 6, 2, 64, 56), True)], ids=str)
+def test_gpu_few_rows(c, merged):
+    """at most 32 rows leave half of a tile of the one launch empty, which large calls do not take: whole numbers, exact in any order (Winograd's: rounded)"""
+    cin, cout, k, p, b, h = c
+    gen = torch.Generator().manual_seed(sum(c))
+    oh = (h + 2 * p - k) // 2 + 1
+    f, dy = (torch.randint(-2, 3, n, generator=gen).float() for n in ((cout, cin, k, k), (b, cout, oh, oh)))
+    op = dlp.Conv2DBackwardData.create(dlp.Conv2DSettings(cin, cout, k, 2, 1, p, 1, (b, cin, h, h)))
+    dx, work = torch.full((b, cin, h, h), float("nan"), device="cuda:0"), torch.empty(op.workspace(), dtype=torch.uint8, device="cuda:0")
+    dlp.timing_enable(True)
+    dlp.timing_reset()
+    try:
+        op.enqueue(dx, f.cuda(), dy.cuda(), work)
+        sections = [s for s, _ in dlp.timing_records()]
+    finally:
+        dlp.timing_enable(False)
+        dlp.timing_reset()
+    assert ("bwd_data_interleave" not in sections) == merged, sections
+    pick = slice(b - 2, b)
+    extra = h - ((oh - 1) * 2 - 2 * p + k)
+    want = torch.nn.functional.conv_transpose2d(dy[pick], f, None, 2, p, extra)
+    # Winograd's transforms: values of up to four times the operands', in sums of every channel
+    bound = 0.0 if merged else cout * 4 * 9 * 2.0 ** -20
+    assert (dx[pick].cpu() - want).abs().max() <= bound
