@@ -399,13 +399,17 @@ int conv_pointwise_launch(const ConvGeom &g, const void *x, const void *w, void 
     return fail(DLP_ERR_RUNTIME, "pointwise kernel: no instantiation for this shape");
 }
 
+bool conv_expand_geometry(const ConvGeom &g)
+{
+    return g.dtype == DLP_FLOAT && g.KH == 1 && g.KW == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0 && g.groups == 1 && g.Cin <= 24 && g.Cout > 32 &&
+           (g.H * g.W) % 4 == 0;
+}
+
 bool conv_expand_serves(const ConvGeom &g, const Epilogue &ep, const void *x, const void *y)
 {
-    if (g.dtype != DLP_FLOAT || g.KH != 1 || g.KW != 1 || g.sh != 1 || g.sw != 1 || g.ph != 0 || g.pw != 0 || g.groups != 1 || g.B <= 0)
+    if (!conv_expand_geometry(g) || g.B <= 0 || ep.activation == DLP_ACT_TANH || ep.activation == DLP_ACT_SIGMOID || ep.factor != 0.0f)
         return false;
-    if (ep.activation == DLP_ACT_TANH || ep.activation == DLP_ACT_SIGMOID || ep.factor != 0.0f || g.Cin > 24 || g.Cout <= 32)
-        return false;
-    if ((g.H * g.W) % 4 != 0 || (((uintptr_t)x | (uintptr_t)y) & 15) != 0)
+    if ((((uintptr_t)x | (uintptr_t)y) & 15) != 0)
         return false;
     const size_t N = (size_t)g.B * g.H * g.W;
     // From 40 MB of output on; below, a wavefront that walks many filter blocks takes longer than the gathering kernel's many workgroups.  Cold tensors,

@@ -113,6 +113,7 @@ struct dlp_conv2d_fwd {
     KTabEntry *ktab; // device gather table of the GEMM stage
     WinoPlan wino;
     size_t workspace;
+    size_t filter_copy, filter_at; // packed weights end in the filter as it lies, for the kernels that read it so: bytes (0: no call wants it) and place
     int packed_layout[6]; // of the last dlp_conv2d_fwd_pack: order, BM, K tiles, m tiles, patch, in-place
     int accumulate_first; // y = act(conv + bias + factor * y) instead of factor * y + act(conv + bias)
     int x_channels_last, y_channels_last; // tensor layouts of the gemm algorithm on bf16 tensors (dlp_conv2d_fwd_set_channels_last)
@@ -168,6 +169,32 @@ static bool direct_is_faster(const ConvGeom &g, const GemmPlan &p)
 static bool runs_as_gemm(const dlp_conv2d_fwd *op, const ConvGeom &g, const GemmPlan &p)
 {
     return op->algo == ALGO_GEMM || (op->direct && direct_is_faster(g, p));
+}
+
+// Whether a call on packed weights may read the filter as it lies (conv_wave_f32_kernel up to the settings' batch, conv_expand_f32_kernel at any): it
+// is packed along then.  A caller may have released the filter itself, as most kernels do not look at it.
+static bool packed_calls_read_filter(const dlp_conv2d_fwd *op, ConvGeom g)
+{
+    if (g.dtype != DLP_FLOAT || (op->algo != ALGO_GEMM && !(op->algo == ALGO_WINOGRAD && op->automatic)))
+        return false;
+    if (op->algo == ALGO_GEMM && conv_expand_geometry(g))
+        return true;
+    for (g.B = std::max(g.B, 1); g.B >= 1; g.B -= std::max(1, g.B / 64))
+        if (conv_wave_f32_serves(g, true))
+            return true;
+    return false;
+}
+
+// bytes of packed weights without the copy of the filter
+static size_t packed_form_bytes(const dlp_conv2d_fwd *op)
+{
+    const size_t first = op->algo == ALGO_WINOGRAD ? round256(op->wino.ws_bytes) : 0;
+    if (op->algo == ALGO_DEPTHWISE || (op->algo == ALGO_WINOGRAD && !op->direct))
+        return first;
+    ConvGeom g;
+    if (op_geom(op, op->cfg.shape, g) != DLP_OK)
+        return 0;
+    return first + round256(conv_gemm_pack_plan(g, op->activation).bytes);
 }
 
 struct dlp_ip_fwd {
@@ -272,6 +299,13 @@ int scratch_on_current_device(void **out)
     }
     *out = g_scratch_ptr[device];
     return DLP_OK;
+}
+
+__global__ void copy_floats_kernel(float *__restrict__ y, const float *__restrict__ x, int n)
+{
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i < n)
+        y[i] = x[i];
 }
 
 // a fill kernel, not hipMemsetAsync: the call may be recorded into a HIP graph
@@ -638,6 +672,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     op->algo = chosen;
     op->automatic = auto_algo;
     op->direct = chosen == ALGO_WINOGRAD && auto_algo && direct_is_faster(g, gplan);
+    op->filter_copy = op->filter_at = 0;
     op->ktab = nullptr;
     op->workspace = 0;
     for (int i = 0; i < 6; i++)
@@ -673,6 +708,9 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
         delete op;
         return rc;
     }
+    op->filter_copy = packed_calls_read_filter(op, g) ? round256((size_t)g.Cout * (g.Cin / g.groups) * g.KH * g.KW * sizeof(float)) : 0;
+    op->filter_at = packed_form_bytes(op);
+    op->workspace = std::max(op->workspace, op->filter_at + op->filter_copy);
     *out = op;
     return DLP_OK;
 }
@@ -812,18 +850,7 @@ int dlp_conv2d_fwd_fuse_max_pool(dlp_conv2d_fwd *op, int kernel, int stride, int
     return DLP_OK;
 }
 
-size_t dlp_conv2d_fwd_packed_bytes(const dlp_conv2d_fwd *op)
-{
-    if (!op)
-        return 0;
-    const size_t first = op->algo == ALGO_WINOGRAD ? round256(op->wino.ws_bytes) : 0;
-    if (op->algo == ALGO_DEPTHWISE || (op->algo == ALGO_WINOGRAD && !op->direct))
-        return first;
-    ConvGeom g;
-    if (op_geom(op, op->cfg.shape, g) != DLP_OK)
-        return 0;
-    return first + round256(conv_gemm_pack_plan(g, op->activation).bytes);
-}
+size_t dlp_conv2d_fwd_packed_bytes(const dlp_conv2d_fwd *op) { return op ? packed_form_bytes(op) + op->filter_copy : 0; }
 
 int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *stream)
 {
@@ -835,6 +862,13 @@ int dlp_conv2d_fwd_pack(dlp_conv2d_fwd *op, const void *w, void *packed, void *s
     int rc = op_geom(op, op->cfg.shape, g);
     if (rc != DLP_OK)
         return rc;
+    if (op->filter_copy) {
+        const int n = g.Cout * (g.Cin / g.groups) * g.KH * g.KW;
+        TimingScope ts("pack_weights", (hipStream_t)stream);
+        hipLaunchKernelGGL(copy_floats_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                           (float *)((char *)packed + op->filter_at), (const float *)w, n);
+        DLP_HIP_TRY(hipGetLastError());
+    }
     if (op->algo == ALGO_WINOGRAD) {
         Epilogue ep = {nullptr, 0.0f, op->activation};
         rc = winograd_launch(g, op->wino, nullptr, w, nullptr, packed, op->wino.ws_bytes, ep, (hipStream_t)stream, WINO_FILTER_ONLY);
@@ -869,13 +903,15 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
     ep.accumulate_first = op->accumulate_first;
     hipStream_t s = (hipStream_t)stream;
     const bool direct = op->direct && packed != nullptr && direct_is_faster(g, conv_gemm_plan(g, op->activation));
+    const bool small = op->filter_copy && conv_wave_f32_serves(g, true);
+    const void *const filter = op->filter_copy && packed ? (const char *)packed + op->filter_at : nullptr;
     if (direct)
         packed = (const char *)packed + round256(op->wino.ws_bytes);
     switch (direct ? ALGO_GEMM : op->algo) {
     case ALGO_WINOGRAD:
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
-        if (op->automatic && conv_wave_f32_serves(g, true))
-            return conv_wave_f32_launch(g, x, w, y, ep, s);
+        if (small)
+            return conv_wave_f32_launch(g, x, filter, y, ep, s);
         return winograd_launch(g, op->wino, x, w, y, const_cast<void *>(packed), op->wino.ws_bytes, ep, s, WINO_RUN_ONLY);
     case ALGO_DEPTHWISE:
         return depthwise_launch(g, x, w, y, ep, s);
@@ -889,10 +925,10 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
             DLP_REQUIRE(sig[i] == op->packed_layout[i], "the weights were packed for another tile plan (pack again for this batch)");
         DLP_REQUIRE(packed != nullptr, "null buffer of packed weights");
         DLP_REQUIRE(hint_plan.split || !plan.split, "the weights were not packed as bf16 parts");
-        if (conv_wave_f32_serves(g, true))
-            return conv_wave_f32_launch(g, x, w, y, ep, s);
-        if (conv_expand_serves(g, ep, x, y))
-            return conv_expand_launch(g, x, w, y, ep, s);
+        if (small)
+            return conv_wave_f32_launch(g, x, filter, y, ep, s);
+        if (op->filter_copy && conv_expand_serves(g, ep, x, y))
+            return conv_expand_launch(g, x, filter, y, ep, s);
         void *part = ws_bytes > 0 ? ws : nullptr;
         int *counters = nullptr;
         rc = own_counters(op, g, plan, &counters);

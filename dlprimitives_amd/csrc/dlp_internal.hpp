@@ -344,6 +344,7 @@ bool conv_pointwise_supported(const ConvGeom &g, int activation);
 int conv_pointwise_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream);
 
 // ... with few input channels and many filters: whether a call is one, and the call (conv_expand_f32_kernel; reads x and w in place)
+bool conv_expand_geometry(const ConvGeom &g); // whether a call at some batch can be one
 bool conv_expand_serves(const ConvGeom &g, const Epilogue &ep, const void *x, const void *y);
 int conv_expand_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream);
 

@@ -160,9 +160,10 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4],
  * every call.  Here the caller transforms it once: `packed` is a device buffer of
  * dlp_conv2d_fwd_packed_bytes(op) bytes (0 for "depthwise_separable") that dlp_conv2d_fwd_pack fills
  * (tile-ordered weights of "gemm", the transformed filter of "winograd", both where the choice was left
- * open and large batches run directly) and that dlp_conv2d_fwd_enqueue_packed reads instead of
- * transforming `w` again (`w` is still passed: 1x1 bf16, 1x1 float of few channels and small float
- * convolutions read it in place).  `ws` then only holds the per-call scratch: workspace() bytes
+ * open and large batches run directly, and a copy of the filter where small or widening float convolutions
+ * read it as it is) and that dlp_conv2d_fwd_enqueue_packed reads instead of transforming `w` again.  `w` is
+ * still passed, and read in place by 1x1 bf16 convolutions, the 7x7 stride-2 ones of 3 channels and 1x1
+ * float ones of so few filters that they stream their input.  `ws` then only holds the per-call scratch: workspace() bytes
  * are always enough, and convolutions that run one after another on a stream may share it.  The
  * buffer serves every batch (float "gemm" weights that a large batch wants as three bf16 parts are
  * held as fp32 tiles too, for small ones).  Pack again after the weights change. */
