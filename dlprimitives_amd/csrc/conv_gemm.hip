@@ -2970,8 +2970,9 @@ template <int BM, int BN, int WM, int WN, bool RAGGED>
 void launch_split_inst(TimingScope &ts, const GemmArgs &a, unsigned blocks, hipStream_t stream)
 {
     void (*kernel)(GemmArgs) = conv_split_f32_kernel<BM, BN, WM, WN, false, RAGGED>;
-    if (a.wdirect)
-        kernel = conv_split_f32_kernel<BM, BN, WM, WN, true, RAGGED>;
+    if constexpr (BN == 128) // (64x64: calls with a filter in place are on the fp32 instruction)
+        if (a.wdirect)
+            kernel = conv_split_f32_kernel<BM, BN, WM, WN, true, RAGGED>;
     DLP_LAUNCH_TIMED(ts, kernel, dim3(blocks), dim3(kThreads), 0, stream, a);
 }
 
@@ -2980,6 +2981,8 @@ int launch_split(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t 
     const long long blocks = (long long)a.main_wgs + (long long)a.tail_tiles * a.tail_splitk;
     if ((long long)a.mtiles * a.ntiles * g.groups * a.splitk > 0x7fffffffLL)
         return fail(DLP_ERR_NOT_IMPLEMENTED, "convolution too large for a single launch");
+    if (p.tile == 6 && a.wdirect)
+        return fail(DLP_ERR_RUNTIME, "tiles of 64x64 read packed weights");
     {
         TimingScope ts("conv_gemm", stream);
         const bool ragged = (a.M & 7) != 0;
