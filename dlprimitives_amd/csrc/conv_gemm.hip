@@ -3151,13 +3151,14 @@ GemmPlan conv_gemm_plan(const ConvGeom &g, int activation)
             // 16 (392 x 72) 41 / 35, 64->64 at 56x56, batch 4 (196 x 36) 13 / 17, 5x5 48->80 at 31x31, batch 9 (272 x 75) 34 / 28, 1x1 2048->512 at 7x7,
             // batch 16 (104 x 128) 28 / 24, 512->128 at 28x28 (392 x 32) 25 / 25, 3x3 stride 2 128->128 at 56x56 45 / 50 on cold tensors.  (1x1 filters
             // read in place: 2048->512 29 / 32.  Those calls stay.)
-            if (tiles64 * p.nkt < 12000 || p.nkt < 48 || !fits(64))
+            if (tiles64 * p.nkt < 12000 || p.nkt < 48 || !fits(64) || (p.patch && g.sh > 1))
                 return -1;
-            // The LDS-patch kernel takes some 1.36 us per thousand K tiles and cuts finer: 256->256 at 14x14, batch 21, whose 260 tiles are just
-            // more than a workgroup for every CU, 52 / 56.
-            if (p.patch && (g.sh > 1 || split_cut_64(tiles64, p.nkt, device_cu_count(), 1ll << 30).cost > 1.36e-3 * tiles64 * p.nkt))
-                return -1;
-            return 6;
+            // The kernels on the fp32 instruction cut finer.  The LDS-patch one takes some 1.36 us per thousand K tiles: 256->256 at 14x14, batch 21,
+            // whose 260 tiles are just more than a workgroup for every CU, 52 / 56.  The gathering one takes 2 to 4, the more the longer the sums: where
+            // eight slices of few tiles leave CUs without work it is the faster one (5x5 912->64 at 12x12, batch 5, 12 tiles of 1425 K tiles, 43 / 75 us,
+            // 640->171 stride 2 at 32x46, 18 of 1000, 51 / 64, 336->448 stride 2 at 8x8, batch 15, 28 of 525, 35 / 40; 176->512 at 22x30 stride 2, batch 2, 48 of 275, 36 / 28;
+            // 96->464 at 11x11 stride 2, batch 22, 104 of 150, 32 / 27).
+            return split_cut_64(tiles64, p.nkt, device_cu_count(), 1ll << 30).cost <= (p.patch ? 1.36e-3 : 2.0e-3) * tiles64 * p.nkt ? 6 : -1;
         };
         int tile = split_tile(std::min(g.B, g.B_hint));
         // What the LDS-patch kernel is left with does not only grow with the batch.  Weights packed ahead, and the place of tiles packed in a call, are

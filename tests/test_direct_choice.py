@@ -60,3 +60,30 @@ def test_gpu_tiles_of_64_or_patch_by_rounds(batch, start):
     want = torch.nn.functional.conv2d(x[pick].double(), f.double(), None, 1, 1)
     scale = torch.nn.functional.conv2d(x[pick].double().abs(), f.double().abs(), None, 1, 1)
     assert ((y[pick].cpu().double() - want).abs() <= scale * (256 * 9 * 2.0 ** -24)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c, start", [
+    ((912, 64, 5, 1, 5, 12, 12), "conv_gemm_f32_kernel<"),         # 12 tiles of 1425 K tiles: eight slices leave most CUs without work
+    ((336, 448, 5, 2, 15, 8, 8), "conv_gemm_f32_kernel<"),         # 28 of 525
+    ((176, 512, 5, 2, 2, 22, 30), "conv_split_f32_kernel<64, 64,"),  # 48 of 275
+    ((96, 64, 5, 1, 13, 21, 21), "conv_split_f32_kernel<64, 64,"),   # 90 of 150
+], ids=str)
+def test_gpu_tiles_of_64_by_slices(c, start):
+    """both sides of the line where K slices of 64x64 tiles no longer fill the chip"""
+    cin, cout, k, s, b, h, w = c
+    gen = torch.Generator().manual_seed(sum(c))
+    x, f = torch.randn((b, cin, h, w), generator=gen), torch.randn((cout, cin, k, k), generator=gen)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, 1, k // 2, 1, tuple(x.shape)), False, "identity", "gemm")
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    packed = torch.full((op.packed_size(),), 255, dtype=torch.uint8, device="cuda:0")
+    xd, fd = x.cuda(), f.cuda()
+    op.pack(fd, packed)
+    want = torch.nn.functional.conv2d(x.double(), f.double(), None, s, k // 2)
+    scale = torch.nn.functional.conv2d(x.double().abs(), f.double().abs(), None, s, k // 2)
+    for call in (lambda y: op.enqueue(xd, fd, None, y, work), lambda y: op.enqueue_packed(xd, fd, packed, None, y, work)):
+        y = torch.full(tuple(want.shape), float("nan"), device="cuda:0")
+        (name,) = _kernels(lambda: call(y))
+        assert name.startswith(start), name
+        # a rounding per product
+        assert ((y.cpu().double() - want).abs() <= scale * ((cin * k * k + 8) * 2.0 ** -24)).all()
