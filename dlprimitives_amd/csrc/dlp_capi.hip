@@ -157,13 +157,19 @@ static int op_geom(const dlp_conv2d_fwd *op, const int x_shape[4], ConvGeom &g)
 }
 
 // Whether a convolution that the reference's rule gives to Winograd is faster as conv_split_f32_kernel (and less rounded): enough tiles of 64 filters
-// x 128 pixels, none with empty rows.  Filters transformed in the call, cold tensors, Winograd / direct, us: 3x3 64->64 at 56x56, batch 16 (392 tiles) 38 / 39,
-// 32 (784) 63 / 59, 64 (1568) 112 / 100; 128->128 at 28x28, 32 (392) 56 / 59, 48 (588) 81 / 69, 64 (784) 101 / 91; 256->256 at 14x14, 64 (392) 92 / 105, 128 (784)
-// 171 / 161; 192->192 at 35x35, 20 (576) 113 / 106; 32->64 at 112x112, 16 (1568) 76 / 61; 160->96 at 50x50, 16 (626) 78 / 83.
+// x 128 pixels, none with empty rows, and sums short enough that 2.25 times the products are no more than what the transforms cost.  Winograd / direct, us,
+// filters transformed in the call, cold tensors: 3x3 64->64 at 56x56, batch 16 (392 tiles) 38 / 39, 32 (784) 63 / 59, 64 (1568) 112 / 100; 128->128 at 28x28, 32
+// (392) 56 / 59, 48 (588) 81 / 69, 64 (784) 101 / 91; 256->256 at 14x14, 64 (392) 92 / 105, 128 (784) 171 / 161; 32->64 at 112x112, 16 (1568) 76 / 61; 160->96 at
+// 50x50, 16 (626) 78 / 83.  In tiles of 64 rows, warm, transformed ahead or in the call: 64->320 at 84x84, 4 (1105 tiles of 36 K tiles) 89 / 78, 128->320 at 34x34, 13 (590
+// of 72) 87 / 78, but from some 650 tiles on, which a second round of workgroups begins, 144->448 at 24x24, 29 (917 of 81) 112 / 144, 208->192 at 20x15, 102
+// (720 of 117) 116 / 148, 96->64 at 83x76, 19 (937 of 54) 86 / 97, 80->64 at 68x68, 26 (940 of 45) 72 / 79.  In tiles of 128 rows 208->256 at 23x23, 55 (912 of
+// 117) 141 / 152, 144->384 at 25x25, 47 (1380 of 81) 157 / 166; 272->384 at 23x23, 30 (744 of 153) 182 / 161.
 static bool direct_is_faster(const ConvGeom &g, const GemmPlan &p)
 {
     const long long tiles = (long long)g.groups * ((p.M + 63) / 64) * (((long long)std::min(g.B, g.B_hint) * g.OH * g.OW + 127) / 128);
-    return g.dtype == DLP_FLOAT && p.split && p.tile != 6 && p.M % 64 == 0 && tiles >= 560;
+    if (g.dtype != DLP_FLOAT || !p.split || p.tile == 6 || p.M % 64 != 0 || tiles < 560)
+        return false;
+    return p.tile == 4 ? p.nkt <= 72 || tiles < 900 : p.nkt <= 36 || (p.nkt <= 90 && tiles <= 640);
 }
 // whether a call runs as "gemm"
 static bool runs_as_gemm(const dlp_conv2d_fwd *op, const ConvGeom &g, const GemmPlan &p)
@@ -650,7 +656,7 @@ int dlp_conv2d_fwd_create(const dlp_conv2d_settings *cfg, int bias, int activati
     // the LDS-patch kernel can serve and that (a) have fewer than 64 input channels, or fewer than 128 with a filter count off 64 (the
     // Winograd kernel then gives a workgroup 32 output channels: 130 against 126 us on 64->64 at 56x56, batch 64), or (b) leave the
     // Winograd kernel fewer than one and a half workgroups per compute unit at the batch of the settings.  These lines were drawn against the
-    // LDS-patch kernel; from some batch on such layers are faster on conv_split_f32_kernel: those calls run there whatever the name (direct_is_faster).
+    // LDS-patch kernel; from some batch on such layers are faster on conv_split_f32_kernel: those calls run there all the same (direct_is_faster).
     const int cin_g = cfg->channels_in / cfg->groups;
     bool gemm_faster = false;
     if (gplan.patch_layer && win) {

@@ -87,3 +87,30 @@ def test_gpu_tiles_of_64_by_slices(c, start):
         assert name.startswith(start), name
         # a rounding per product
         assert ((y.cpu().double() - want).abs() <= scale * ((cin * k * k + 8) * 2.0 ** -24)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c, direct", [
+    ((96, 64, 19, 83, 76), False),    # 937 tiles of 54 K tiles, a second round of workgroups
+    ((96, 64, 12, 83, 76), True),     # 592
+    ((64, 64, 13, 83, 76), True),     # 641 of 36
+    ((208, 256, 55, 23, 23), False),  # rows of 128: 912 of 117
+    ((208, 256, 40, 23, 23), True),   # 664
+], ids=str)
+def test_gpu_automatic_choice_by_length_of_sums(c, direct):
+    """both sides of the lines between Winograd and the direct kernel for long sums, filters packed"""
+    cin, cout, b, h, w = c
+    gen = torch.Generator().manual_seed(sum(c))
+    x, f = torch.randn((b, cin, h, w), generator=gen), torch.randn((cout, cin, 3, 3), generator=gen)
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, 3, 1, 1, 1, 1, tuple(x.shape)), False)
+    assert op.algo() == "winograd"
+    work = torch.empty(op.workspace(), dtype=torch.uint8, device="cuda:0")
+    packed = torch.full((op.packed_size(),), 255, dtype=torch.uint8, device="cuda:0")
+    xd, fd, y = x.cuda(), f.cuda(), torch.full((b, cout, h, w), float("nan"), device="cuda:0")
+    op.pack(fd, packed)
+    names = _kernels(lambda: op.enqueue_packed(xd, fd, packed, None, y, work))
+    assert [n.startswith("conv_split_f32_kernel<") for n in names] == [True] * direct, names
+    want = torch.nn.functional.conv2d(x[-2:].double(), f.double(), None, 1, 1)
+    scale = torch.nn.functional.conv2d(x[-2:].double().abs(), f.double().abs(), None, 1, 1)
+    # Winograd's transforms round at the size of sixteen products
+    assert ((y[-2:].cpu().double() - want).abs() <= scale * ((cin * 9 + 16) * 2.0 ** -24)).all()
