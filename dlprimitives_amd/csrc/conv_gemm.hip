@@ -2726,10 +2726,15 @@ void launch_wave_bf16(TimingScope &ts, const GemmArgs &a, unsigned blocks, hipSt
 // of ResNet-50, us, those / these: 3x3 512->512 at 7x7 (144 K tiles) batch 1 13.9 / 6.4, batch 16 24.5 / 16.7, batch 32 28.3 / 28.3; 1x1
 // 1024->256 at 14x14 (32) batch 1 10.2 / 3.8, 16 17.6 / 13.5, 32 22.9 / 20.6; 1x1 512->256 at 28x28 (16) batch 8 19.1 / 12.8, 32 15.2 / 35.4.
 // Short reductions end sooner: 1x1 256->64 at 56x56 (8) batch 4 7.4 / 5.6, 8 7.8 / 7.4, 16 8.8 / 13.7; 64->256 (2) batch 1 5.2 / 4.5, 4 5.9 / 8.7.
+// Between them the tiles of the others count, 128 rows or 64, and K tiles too: 1x1 448->200 at 31x31, batch 7 (1477 tiles of 14) 9.5 / 11.9, 320->80 at 22x22, 35
+// (1590 of 10) 8.3 / 9.8, 352->160 at 39x38 stride 2, 23 (1370 of 11) 8.5 / 9.5, 384->384 at 20x20, 8 (1200 of 12) 8.5 / 7.5; 384->48 at 53x33, 14 (1532 of 12)
+// 10.1 / 10.3, 352->32 at 78x78, 8 (1521 of 11) 11.1 / 9.4.
 bool bf16_wave(const GemmPlan &p, long long N, int groups)
 {
     const long long tiles = (long long)groups * ((p.M + 31) / 32) * ((N + 31) / 32);
-    return p.nkt >= 16 ? tiles * p.nkt <= 58000 : tiles <= (p.nkt >= 8 ? 1600 : 1000);
+    if (p.nkt >= 16)
+        return tiles * p.nkt <= 58000;
+    return p.nkt >= 8 ? tiles <= (p.M > 64 ? 1300 : 1600) && tiles * p.nkt <= 17000 : tiles <= 1000;
 }
 
 int launch_wave_bf16(const ConvGeom &g, const GemmPlan &p, GemmArgs &a, hipStream_t stream)

@@ -53,3 +53,23 @@ def test_gpu_wave_conv(c, ycl):
             res = want + factor * old.double() if first else want.relu()
             got = (y.permute(0, 3, 1, 2) if ycl else y).cpu().double()
             assert ((got - res).abs() <= res.abs() * 2.0 ** -8 + slack).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c, wave", [((448, 200, 7, 31, 31), False), ((448, 200, 5, 31, 31), True), ((352, 144, 38, 19, 14), False), ((256, 320, 18, 15, 15), True),
+                                     ((320, 80, 35, 22, 22), False), ((352, 32, 8, 78, 78), True), ((512, 200, 16, 31, 31), True)], ids=str)
+def test_gpu_wave_conv_lines(c, wave):
+    """1x1 of 8 to 15 K tiles: up to 1300 tiles (1600 of up to 64 filters) and 17000 K tiles; whole numbers, their sums exact in any order before the one rounding"""
+    cin, cout, b, h, w = c
+    gen = torch.Generator().manual_seed(sum(c))
+    x, f = torch.randint(-3, 4, (b, h, w, cin), generator=gen).bfloat16().cuda(), torch.randint(-3, 4, (cout, cin, 1, 1), generator=gen).bfloat16().cuda()
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, 1, 1, 1, 0, 1, (b, cin, h, w), dtype=BFLOAT16_DATA), False, "identity", "gemm")
+    op.channels_last(True, True)
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    packed = torch.empty(max(op.packed_size(), 1), dtype=torch.uint8, device="cuda:0")
+    op.pack(f, packed)
+    y = torch.full((b, h, w, cout), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    (name,) = _kernels(lambda: op.enqueue_packed(x, f, packed, None, y, work))
+    assert name.startswith("conv_wave_bf16_kernel<") == wave, name
+    want = torch.matmul(x.view(-1, cin).float().cpu(), f.view(cout, cin).float().cpu().t().contiguous())
+    assert torch.equal(y.view(-1, cout).cpu(), want.bfloat16())
