@@ -34,3 +34,20 @@ def test_gpu_depthwise_wgrad_columns(c):
     dw = torch.full(f, float("nan"), device="cuda:0")
     op.enqueue(x.cuda(), dw, dy.abs().cuda() + 0.5, work)
     assert torch.equal(torch.isfinite(dw.cpu()), torch.isfinite(grad(x, dy.abs() + 0.5)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c, rows", [((40, 1, 1, 1, 26, 16, 16), 1), ((40, 1, 1, 1, 26, 16, 17), 8), ((40, 1, 1, 1, 27, 16, 16), 8), ((40, 1, 2, 1, 26, 31, 32), 1), ((40, 1, 2, 1, 26, 33, 31), 4),
+                                     ((1, 2, 2, 0, 1, 3, 3), 1)], ids=str)
+def test_gpu_depthwise_wgrad_rows_of_a_lane(c, rows):
+    """one pixel a lane up to 256 of one image a workgroup, more down a column: whole numbers, exact in any order"""
+    ch, mult, s, p, b, h, w = c
+    gen = torch.Generator().manual_seed(sum(c))
+    x, f = torch.randint(-3, 4, (b, ch, h, w), generator=gen).float(), (ch * mult, 1, 3, 3)
+    st = dlp.Conv2DSettings(ch, ch * mult, 3, s, 1, p, ch, tuple(x.shape))
+    dy = torch.randint(-3, 4, dlp.conv2d_output_shape(st, x.shape), generator=gen).float()
+    op = dlp.Conv2DBackwardFilter.create(st)
+    work, dw = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0"), torch.full(f, float("nan"), device="cuda:0")
+    (name,) = _kernels(lambda: op.enqueue(x.cuda(), dw, dy.cuda(), work), "wgrad_depthwise")
+    assert name == "depthwise_wgrad3x3_columns_kernel<%d, %d>" % (s, rows), name
+    assert torch.equal(dw.cpu().double(), torch.nn.grad.conv2d_weight(x.double(), f, dy.double(), s, p, 1, ch))
