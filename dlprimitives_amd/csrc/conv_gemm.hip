@@ -3511,11 +3511,11 @@ bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws
         winograd = winograd && g.KH == 3 && g.KW == 3 && ph[i].len_h >= 14 && ph[i].len_w >= 14;
         half_empty += M <= 32 ? (double)g.groups * p.nkt * ((N + 63) / 64) - 6e-3 * g.groups * M * N : 0.0;
     }
-    // Up to 32 rows leave half of these tiles empty: in large launches, less what one launch a phase writes twice, tiles of 32 rows (Winograd's for 3x3
-    // phases) and the interleaving are faster.  One launch a phase / this one, stride 2, us: 6x6 8->128 at 56x56, batch 64, 226000 K tiles 153 / 169, batch
-    // 200 339 / 485, 32->128 at 64 171 / 185, 8->64 at 128 176 / 167, 8->512 at 14x14, batch 256, 260 / 188; 5x5 8->128 at 128, 314000 194 / 224, 32->128
-    // 226 / 251, 8->256 at 28x28, batch 200, 245000 200 / 184; 4x4 8->128 at 200, 314000 209 / 232.
-    if (half_empty > (winograd ? 185000.0 : 235000.0))
+    // Up to 32 rows leave half of these tiles empty or more: in large launches, less what one launch a phase writes twice, tiles of 32 rows (Winograd's for 3x3
+    // phases) and the interleaving are faster.  One launch a phase / this one, stride 2, us, by thousands of K tiles less those writes: up to 16 rows 6x6 8->128 at
+    // 56x56, batch 64, 153 / 169, batch 32 (110) 92 / 89, 4x4 176->8 (transposed) at 43x30, batch 48, 120 / 143, 32->3 at 92x92, 44 (159) 152 / 181, 64->1 at
+    // 65x65, 30 (124) 88 / 109; more rows 5x5 192->24 (transposed) at 64x64, 13 (219) 175 / 190, 32->128 at 56x56, batch 128, 226 / 251, 6x6 at batch 64 171 / 185.
+    if (half_empty > (M <= 16 ? 125000.0 : winograd ? 150000.0 : 185000.0))
         return false;
     pl.packed_bytes = (pl.packed_bytes + 255) / 256 * 256;
     const size_t fixed = pl.packed_bytes + split_counter_bytes(ntiles);

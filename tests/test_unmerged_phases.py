@@ -59,3 +59,20 @@ def test_gpu_few_rows(c, merged):
     # Winograd's transforms: values of up to four times the operands', in sums of every channel
     bound = 0.0 if merged else cout * 4 * 9 * 2.0 ** -20
     assert (dx[pick].cpu() - want).abs().max() <= bound
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c, merged", [((176, 8, 4, 1, 0, 48, 43, 30), False), ((176, 8, 4, 1, 0, 24, 43, 30), True), ((192, 24, 5, 2, 1, 13, 64, 64), False), ((192, 24, 5, 2, 1, 9, 64, 64), True),
+                                       ((32, 3, 4, 1, 0, 44, 92, 92), False)], ids=str)
+def test_gpu_few_filters(c, merged):
+    """... and up to 16 rows leave three quarters of it empty: whole numbers, exact in any order"""
+    cin, cout, k, p, extra, b, h, w = c
+    gen = torch.Generator().manual_seed(sum(c))
+    x, f = torch.randint(-2, 3, (b, cin, h, w), generator=gen).float(), torch.randint(-2, 3, (cin, cout, k, k), generator=gen).float()
+    op = dlp.TransposedConv2DForward.create(dlp.Conv2DSettings(cin, cout, k, 2, 1, p, 1, tuple(x.shape)), (extra, extra), False, "identity", "gemm")
+    y = torch.full(op.output_shape(tuple(x.shape)), float("nan"), device="cuda:0")
+    work = torch.empty(op.workspace(), dtype=torch.uint8, device="cuda:0")
+    names = _kernels(lambda: op.enqueue(x.cuda(), f.cuda(), None, y, work))
+    assert (len(names) == 1) == merged, names
+    pick = slice(b - 2, b)
+    assert torch.equal(y[pick].cpu(), torch.nn.functional.conv_transpose2d(x[pick], f, None, 2, p, extra))
