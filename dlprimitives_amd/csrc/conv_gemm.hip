@@ -3663,7 +3663,7 @@ size_t conv_wave_f32_lds_bytes(const ConvGeom &g)
 // 17 / 6, batch 16 (50000) 26 / 28, 256->64 at 56x56 batch 2 (6300, 16 K tiles) 9.3 / 7.0, 192->32 at 28x28 batch 32 (9400, 12) 8.8 / 10.5, 64->256 at 56x56 (4) 5.3 / 8;
 // channels off multiples of 16, which the others gather k by k: 3x3 52->16 at 107x107 batch 5 (54000) 31 / 26, 215->489 at 7x8 33 / 14.  With filters
 // packed ahead: 3x3 64->64 at 56x56 batch 1 13 / 10, 512->512 at 7x7 (32 tiles) 18 / 21.
-bool conv_wave_f32_serves(const ConvGeom &g, bool packed)
+bool conv_wave_f32_serves(const ConvGeom &g, bool packed, bool winograd)
 {
     const int cin_g = g.Cin / g.groups, M = g.Cout / g.groups, taps = g.KH * g.KW;
     const long long K = (long long)cin_g * taps;
@@ -3693,6 +3693,11 @@ bool conv_wave_f32_serves(const ConvGeom &g, bool packed)
             return false;
         return u <= (!strided ? 54000 : packed ? 36000 : 46000);
     }
+    // Nine K tiles in many tiles on images too wide for the LDS-patch kernel are the gathering kernel's again: 3x3 16->64 at 115x115, batch 3, 2480 tiles, raw 16 / 20,
+    // 16->240 at 86x86, 1856, 13 / 16, 16->64 at 134x134, 1124, 12 / 11, packed 16->48 at 81x81, batch 2, 822, 7.2 / 9.9 (Winograd's: 16->112 at 94x94, batch 2, 2212,
+    // raw 22 / 18, 16->80 at 69x69, 894, packed 11.2 / 10.3).
+    if (kt < 14 && !winograd && !strided && g.W > 62 && tiles > (packed ? 700 : 1800))
+        return false;
     if (kt < 14 && (M <= 32 || (strided && tiles > (packed ? 700 : 1500)))) // 3x3 of 16 channels: 64 filters at 40x40, batch 6, 26 / 10; 16 at 60x60, batch 12, 14 / 16
         return false;
     return packed ? u <= 10000 && tiles >= 48 : u <= 24000;

@@ -186,7 +186,7 @@ static bool packed_calls_read_filter(const dlp_conv2d_fwd *op, ConvGeom g)
     if (op->algo == ALGO_GEMM && conv_expand_geometry(g))
         return true;
     for (g.B = std::max(g.B, 1); g.B >= 1; g.B -= std::max(1, g.B / 64))
-        if (conv_wave_f32_serves(g, true))
+        if (conv_wave_f32_serves(g, true, op->algo == ALGO_WINOGRAD))
             return true;
     return false;
 }
@@ -765,7 +765,7 @@ int dlp_conv2d_fwd_enqueue(dlp_conv2d_fwd *op, const int x_shape[4], const void 
                         ws_bytes >= std::max(op->wino.ws_bytes, conv_gemm_plan(g, op->activation).wpack_bytes);
     switch (direct ? ALGO_GEMM : op->algo) {
     case ALGO_WINOGRAD:
-        if (op->automatic && ws != nullptr && ws_bytes >= op->wino.ws_bytes && conv_wave_f32_serves(g, false))
+        if (op->automatic && ws != nullptr && ws_bytes >= op->wino.ws_bytes && conv_wave_f32_serves(g, false, true))
             return conv_wave_f32_launch(g, x, w, y, ep, s); // (direct: no less exact)
         return winograd_launch(g, op->wino, x, w, y, ws, ws_bytes, ep, s);
     case ALGO_DEPTHWISE:
@@ -909,7 +909,7 @@ int dlp_conv2d_fwd_enqueue_packed(dlp_conv2d_fwd *op, const int x_shape[4], cons
     ep.accumulate_first = op->accumulate_first;
     hipStream_t s = (hipStream_t)stream;
     const bool direct = op->direct && packed != nullptr && direct_is_faster(g, conv_gemm_plan(g, op->activation));
-    const bool small = op->filter_copy && conv_wave_f32_serves(g, true);
+    const bool small = op->filter_copy && conv_wave_f32_serves(g, true, op->algo == ALGO_WINOGRAD);
     const void *const filter = op->filter_copy && packed ? (const char *)packed + op->filter_at : nullptr;
     if (direct)
         packed = (const char *)packed + round256(op->wino.ws_bytes);

@@ -306,8 +306,8 @@ bool conv_gemm_phases_plan(const PhaseConv *ph, int n, int activation, size_t ws
 int conv_gemm_phases_launch(const PhaseConv *ph, int n, const PhasesPlan &plan, const void *dy, const void *packed, int *counters, float *images, void *dx,
                             int out_h, int out_w, int out_sh, int out_sw, const Epilogue &ep, hipStream_t stream);
 // Small float convolutions, read as they lie (conv_wave_f32_kernel): whether a call is one, given that its filter could be packed ahead or has to be
-// in the call, and the call.
-bool conv_wave_f32_serves(const ConvGeom &g, bool packed);
+// in the call (winograd: and that it is Winograd's otherwise), and the call.
+bool conv_wave_f32_serves(const ConvGeom &g, bool packed, bool winograd = false);
 size_t conv_wave_f32_lds_bytes(const ConvGeom &g); // that the call asks for
 int conv_wave_f32_launch(const ConvGeom &g, const void *x, const void *w, void *y, const Epilogue &ep, hipStream_t stream);
 // the gather table of a float operator of algorithm gemm in the tap-major order (not where the kernel reads the filter as it is), and the geometry of its convolution at this batch

@@ -98,6 +98,30 @@ def test_gpu_wave_conv_f32_lines(c, packed, wave):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("c, packed, algo, wave", [
+    ((16, 64, 3, 1, 1, 1, 1, 2, 140, 140), False, "gemm", False),  # 2450 tiles
+    ((16, 64, 3, 1, 1, 1, 1, 1, 140, 140), False, "gemm", True),
+    ((16, 64, 3, 1, 1, 1, 1, 2, 140, 140), False, "", True),       # Winograd otherwise
+    ((16, 48, 3, 1, 1, 1, 1, 2, 81, 81), True, "gemm", False),     # 822
+    ((16, 48, 3, 1, 1, 1, 1, 1, 81, 81), True, "gemm", True),
+    ((16, 48, 3, 1, 1, 1, 1, 4, 56, 56), True, "gemm", True),      # the LDS-patch kernel otherwise
+], ids=str)
+def test_gpu_wave_conv_f32_wide_images(c, packed, algo, wave):
+    """3x3 of 16 channels: both sides of the lines to the gathering kernel, whole numbers, exact in any order"""
+    cin, cout, k, s, p, d, g, b, h, w = c
+    gen, xs, ws, ys = _tensors(c)
+    x, f = torch.randint(-3, 4, xs, generator=gen).float(), torch.randint(-3, 4, ws, generator=gen).float()
+    op = dlp.Conv2DForward.create(dlp.Conv2DSettings(cin, cout, k, s, d, p, g, xs), False, "identity", algo)
+    work = torch.empty(max(op.workspace(), 1), dtype=torch.uint8, device="cuda:0")
+    y, xd, fd = torch.full(ys, float("nan"), device="cuda:0"), x.cuda(), f.cuda()
+    buf = torch.empty(op.packed_size(), dtype=torch.uint8, device="cuda:0")
+    op.pack(fd, buf)
+    (name,) = _kernels(lambda: op.enqueue_packed(xd, fd, buf, None, y, work) if packed else op.enqueue(xd, fd, None, y, work))
+    assert name.startswith("conv_wave_f32_kernel") == wave, name
+    assert torch.equal(y.cpu(), torch.nn.functional.conv2d(x, f, None, s, p))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("c", [(237, 58, 1, 1, 0, 1, 1, 2, 9, 7), (26, 48, 3, 1, 1, 1, 1, 11, 33, 33)], ids=lambda c: "x".join(map(str, c)))
 def test_gpu_wave_conv_f32_special_values(c):
     """infinities, NaN, operands near the ends of the range: what the fp32 sum of the products is"""
