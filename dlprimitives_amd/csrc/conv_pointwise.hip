@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kPwThreads) void conv_pointwise_f32_kernel(PwArgs a
 // Such a layer writes six times what it reads.  In 32x128 tiles of the gathering kernel every workgroup gathered its 24 channels pixel by pixel for
 // 16 KB of output, five workgroups the same ones.  Here a wavefront keeps four pixels per lane of all K channels in registers (16-byte loads, one
 // pair of channels each, as above) and walks RB blocks of 32 filters over them; a filter block's weights lie in LDS as [k][m].  Stores are 16
-// bytes a lane, 512 consecutive bytes a row, and stay in the caches for the next layer to read.  24 -> 144 at 56x56, batch 64 (135 MB): 56 -> 39 us.
+// bytes a lane, 512 consecutive bytes a row, and stay in the caches for the next layer to read.  24 -> 144 at 56x56, batch 64 (135 MB): 56 -> 37 us.
 // (The offset of a store is all in its vector register: with a scalar one besides, the compiler lets the next instruction overwrite the
 // first of the four data registers of a 16-byte store, and lanes 12 to 15 of every 16 stored what came after.)
 template <int KP>
@@ -417,8 +417,7 @@ bool conv_expand_serves(const ConvGeom &g, const Epilogue &ep, const void *x, co
     //  * 40 MB: filters off multiples of 8, which the others store element by element (8 -> 142 at 38x38, batch 80, 66 MB 32 / 18; 24 -> 162 at 54x54,
     //    batch 51, 96 MB 54 / 36); up to 8 channels into up to 128 filters (8 -> 48 at 42x42, batch 128, 43 MB 16 / 15; 8 -> 128 at 86x86, 33, 125 MB
     //    29 / 26; but 8 -> 256 at 42x42, 75, 135 MB 31 / 34); filters that leave a last tile of 64 at least half empty (17 -> 144 at 38x38, 79, 66 MB 28 / 24, 24 -> 144 at
-    //    106x106, 15, 97 MB 39 / 35, 24 -> 144 at 56x56, batch 64, 116 MB 56 / 39; up to 65 MB, a filter block per wavefront, within
-    //    10 % either way, 24 -> 96 at 48x48, 56, 58 MB 24 / 25);
+    //    106x106, 15, 97 MB 39 / 35, 24 -> 144 at 56x56, batch 64, 116 MB 56 / 37);
     //  * 190 MB: the rest (24 -> 128 at 68x68, 28, 66 MB 22 / 28, 16 -> 64 at 112x112, 42, 135 MB 31 / 37, 20 -> 128 at 68x68, 61, 144 MB 42 / 43; 24 -> 64 at
     //    106x106, 69, 198 MB 77 / 59, 20 -> 256 at 60x60, 60, 221 MB 59 / 52).
     // More than 24 channels were tried with two pixels a lane only: 40 -> 240 at 56x56, batch 24 38 / 41, 64 -> 256 at batch 64 89 / 118.  (24 channels take 100
@@ -446,9 +445,10 @@ int conv_expand_launch(const ConvGeom &g, const void *x, const void *w, void *y,
     a.clamp_lo = 0.0f;
     a.clamp_hi = ep.activation == DLP_ACT_RELU6 ? 6.0f : __builtin_huge_valf();
     const int kp = a.K <= 16 ? 8 : 12, blocks = (a.M + 31) / 32;
-    // filter blocks per wavefront: one to six, as many as leave two workgroups per compute unit (24 -> 144 above, warm: 1, 2, 3, 5 blocks 47, 43, 39, 35 us)
-    const long long gx = (a.N + 511) / 512;
-    const int rb = (int)std::max<long long>(1, std::min<long long>(std::min(blocks, 6), gx * blocks / (2 * dlp_cu_count())));
+    // filter blocks per wavefront: one to six, as many as leave nearly two workgroups per compute unit (24 -> 144 above: 1, 2, 3, 4, 5 blocks 48, 43, 40, 37, 36 us, the
+    // same tensors again 45, 39, 36, 33, 35; 24 -> 96 at batch 48: 1, 2, 3 blocks 25, 23, 24)
+    const long long gx = (a.N + 511) / 512, two = 2 * dlp_cu_count();
+    const int rb = (int)std::max<long long>(1, std::min<long long>(std::min(blocks, 6), (gx * blocks + two - 1) / two));
     const dim3 grid((unsigned)gx, (unsigned)((blocks + rb - 1) / rb));
     const size_t lds = (size_t)(2 * kp + 1) * 32 * rb * sizeof(float);
     void (*kernel)(PwArgs, int) = conv_expand_f32_kernel<12>;
