@@ -3694,9 +3694,9 @@ bool conv_wave_f32_serves(const ConvGeom &g, bool packed, bool winograd)
         return u <= (!strided ? 54000 : packed ? 36000 : 46000);
     }
     // Nine K tiles in many tiles on images too wide for the LDS-patch kernel are the gathering kernel's again: 3x3 16->64 at 115x115, batch 3, 2480 tiles, raw 16 / 20,
-    // 16->240 at 86x86, 1856, 13 / 16, 16->64 at 134x134, 1124, 12 / 11, packed 16->48 at 81x81, batch 2, 822, 7.2 / 9.9 (Winograd's: 16->112 at 94x94, batch 2, 2212,
+    // 16->240 at 86x86, 1856, 13 / 16, 16->48 at 160x160, 1600, 12 / 15, 16->64 at 134x134, 1124, 12 / 11, packed 16->48 at 81x81, batch 2, 822, 7.2 / 9.9 (Winograd's: 16->112 at 94x94, batch 2, 2212,
     // raw 22 / 18, 16->80 at 69x69, 894, packed 11.2 / 10.3).
-    if (kt < 14 && !winograd && !strided && g.W > 62 && tiles > (packed ? 700 : 1800))
+    if (kt < 14 && !winograd && !strided && g.W > 62 && tiles > (packed ? 700 : 1450))
         return false;
     if (kt < 14 && (M <= 32 || (strided && tiles > (packed ? 700 : 1500)))) // 3x3 of 16 channels: 64 filters at 40x40, batch 6, 26 / 10; 16 at 60x60, batch 12, 14 / 16
         return false;

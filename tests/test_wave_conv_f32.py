@@ -101,6 +101,7 @@ def test_gpu_wave_conv_f32_lines(c, packed, wave):
 @pytest.mark.parametrize("c, packed, algo, wave", [
     ((16, 64, 3, 1, 1, 1, 1, 2, 140, 140), False, "gemm", False),  # 2450 tiles
     ((16, 64, 3, 1, 1, 1, 1, 1, 140, 140), False, "gemm", True),
+    ((16, 48, 3, 1, 1, 1, 1, 1, 160, 160), False, "gemm", False),  # 1600
     ((16, 64, 3, 1, 1, 1, 1, 2, 140, 140), False, "", True),       # Winograd otherwise
     ((16, 48, 3, 1, 1, 1, 1, 2, 81, 81), True, "gemm", False),     # 822
     ((16, 48, 3, 1, 1, 1, 1, 1, 81, 81), True, "gemm", True),
